@@ -30,6 +30,7 @@ struct ContractArgs {
   int chunk_rows;
   int n_qgroups;
   int n_lanes;  // persistent kernels: entity-chunk lanes per (XCD, query group)
+  int lanes_flat = 0;  // persistent kernels: 0, or the entity-chunk lanes per query group over the whole chip (walk_of_wg)
   // ksplit_kernel only: row strides of Q and E in elements (0: d), and the length of the K range one
   // workgroup sums (0: all of d; otherwise a multiple of 32, and blockIdx.y selects the range)
   int ldq, lde;
@@ -121,6 +122,25 @@ __device__ __forceinline__ bool decompose_wg(const ContractArgs& a, int& qg, int
   qg = (int)(slot % a.n_qgroups);
   chunk = (slot / a.n_qgroups) * 8 + xcd;
   return chunk < a.n_chunks;
+}
+
+// The walk of a persistent workgroup: its query group and the entity chunks c_first + c_stride * i it takes.  Two forms:
+// * per XCD (lanes_flat = 0): flat id -> (xcd = id % 8, query group, lane), chunks xcd + 8 * (lane + n_lanes * i);
+// * flat: the chunks of a group are dealt over lanes_flat workgroups wherever they run, chunks lane + lanes_flat * i.
+//   A lane's query groups are numbered consecutively along an XCD's workgroups, so that most of them walk the same rows
+//   behind the same L2.  The host takes it where 32 workgroups per XCD do not divide evenly by the query groups
+//   (host::flat_walk).
+// (rank128_kernel and topk_i8_filter_kernel, 1024 queries per workgroup, keep the first form: at most a ninth of the chip
+// is idle up to 8192 queries, and the hand-allocated kernel ran 2.5 % slower with the choice in its prologue.)
+// Ids past the last lane get a first chunk past the end.
+__device__ __forceinline__ void walk_of_wg(const ContractArgs& a, int64_t wg, int& qg, int64_t& c_first, int64_t& c_stride) {
+  const int xcd = (int)(wg & 7);
+  const int64_t slot = wg >> 3;
+  const int64_t idx = a.lanes_flat ? (int64_t)xcd * (gridDim.x >> 3) + slot : slot;
+  qg = (int)(idx % a.n_qgroups);
+  const int64_t wlane = idx / a.n_qgroups;
+  c_first = a.lanes_flat ? (wlane < a.lanes_flat ? wlane : a.n_chunks) : xcd + 8 * wlane;
+  c_stride = a.lanes_flat ? (int64_t)a.lanes_flat : 8 * (int64_t)a.n_lanes;
 }
 
 // ============================================================================================
@@ -978,17 +998,14 @@ __global__ void __launch_bounds__(64 * QA_WG_WAVES, QA_WAVES_PER_SIMD) qreg_asyn
   __shared__ __attribute__((aligned(1024))) unsigned char lds_e[2 * BUF_BYTES];
 
   const int64_t wg = blockIdx.x;
-  const int xcd = (int)(wg & 7);
-  const int64_t slot = wg >> 3;
-  const int qg = (int)(slot % a.n_qgroups);
-  const int wlane = (int)(slot / a.n_qgroups);
+  int qg;
+  int64_t c_first, c_stride;
+  walk_of_wg(a, wg, qg, c_first, c_stride);
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t q0 = (int64_t)qg * (QA_WG_WAVES * 32 * NQT) + wave * (32 * NQT);
 
   // chunks of this workgroup: first, stride, count
-  const int64_t c_first = xcd + 8 * (int64_t)wlane;
-  const int64_t c_stride = 8 * (int64_t)a.n_lanes;
   if (c_first >= a.n_chunks) return;
   const int my_chunks = (int)((a.n_chunks - 1 - c_first) / c_stride) + 1;
   const int spc = a.chunk_rows / QA_STAGE_ROWS;  // stages per chunk
@@ -1158,17 +1175,14 @@ __global__ void __launch_bounds__(64 * W, OCC) qstream_kernel(ContractArgs a, ty
   __shared__ __attribute__((aligned(1024))) unsigned char lds_e[QS_NBUF * STAGE_BYTES];
 
   const int64_t wg = blockIdx.x;
-  const int xcd = (int)(wg & 7);
-  const int64_t slot = wg >> 3;
-  const int qg = (int)(slot % a.n_qgroups);
-  const int wlane = (int)(slot / a.n_qgroups);
+  int qg;
+  int64_t c_first, c_stride;
+  walk_of_wg(a, wg, qg, c_first, c_stride);
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t q0 = (int64_t)qg * (W * 32 * NQT) + wave * (32 * NQT);
 
   // chunks of this workgroup: first, stride, count; stages that hold at least one valid row
-  const int64_t c_first = xcd + 8 * (int64_t)wlane;
-  const int64_t c_stride = 8 * (int64_t)a.n_lanes;
   if (c_first >= a.n_chunks) return;
   const int my_chunks = (int)((a.n_chunks - 1 - c_first) / c_stride) + 1;
   const int spc = a.chunk_rows / QS_STAGE_ROWS;  // stages per chunk
@@ -1425,16 +1439,13 @@ __global__ void __launch_bounds__(64 * I8_WG_WAVES, 2) qreg_i8_kernel(ContractAr
   constexpr int NPIECE = QA_STAGE_ROWS * PPR / NT;  // 16-byte pieces of int8 a thread stages per stage
 
   const int64_t wg = blockIdx.x;
-  const int xcd = (int)(wg & 7);
-  const int64_t slot = wg >> 3;
-  const int qg = (int)(slot % a.n_qgroups);
-  const int wlane = (int)(slot / a.n_qgroups);
+  int qg;
+  int64_t c_first, c_stride;
+  walk_of_wg(a, wg, qg, c_first, c_stride);
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t q0 = (int64_t)qg * (I8_WG_WAVES * 32 * NQT) + wave * (32 * NQT);
 
-  const int64_t c_first = xcd + 8 * (int64_t)wlane;
-  const int64_t c_stride = 8 * (int64_t)a.n_lanes;
   if (c_first >= a.n_chunks) return;
   const int my_chunks = (int)((a.n_chunks - 1 - c_first) / c_stride) + 1;
   const int spc = a.chunk_rows / QA_STAGE_ROWS;

@@ -60,6 +60,39 @@ inline void rank128_plan(int64_t B, int64_t rows, int* n_qgroups, int* n_lanes, 
   *n_chunks = (rows + chunk - 1) / chunk;
 }
 
+// The other way to deal a persistent launch's entity chunks (walk_of_wg): every query group gets `lanes_flat` =
+// 256 / groups workgroups, on whichever XCDs they fall.  With whole lanes per (XCD, group) a launch of 20 groups runs
+// 20 of the 32 workgroups an XCD holds (5000 queries, heads and tails, on an int8 d = 240 table of 123k rows: 1554 us a pass
+// with the main loop on 160 CUs, 1265 us on 240), one of 33
+// groups a second round for the thirty-third; a group's rows are then read behind fewer L2s, which is why the per-XCD
+// form stays wherever it fills the chip to within a tenth as well.  The chunk length is the one whose busiest lane has
+// the fewest rows (longer chunks among equals).
+inline void flat_walk(int groups, int64_t rows, int stage_rows, int max_chunk, int* lanes_flat, int* chunk_rows,
+                      int64_t* n_chunks) {
+  *lanes_flat = 0;
+  if (groups < 1 || groups > 256) return;
+  const int per_xcd = 32 / groups > 1 ? 32 / groups : 1;
+  const int wgs = 8 * groups * per_xcd;
+  const double fill = (double)wgs / (256.0 * ((wgs + 255) / 256));
+  const int lanes = 256 / groups;
+  if (lanes * groups / 256.0 < 1.1 * fill) return;
+  int64_t best = -1;
+  for (int chunk = max_chunk; chunk >= stage_rows; chunk -= stage_rows) {
+    const int64_t n = (rows + chunk - 1) / chunk;
+    const int64_t busiest = (n + lanes - 1) / lanes * chunk;
+    if (best < 0 || busiest < best) {
+      best = busiest;
+      *chunk_rows = chunk;
+      *n_chunks = n;
+    }
+  }
+  *lanes_flat = lanes;
+}
+// workgroups of a persistent launch of either form
+inline int64_t walk_grid(int groups, int n_lanes, int lanes_flat) {
+  return lanes_flat ? ((int64_t)groups * lanes_flat + 7) / 8 * 8 : 8 * (int64_t)groups * n_lanes;
+}
+
 struct Status {
   int code = KGE_OK;
   char msg[256] = "";

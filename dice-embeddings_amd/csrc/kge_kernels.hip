@@ -1243,6 +1243,7 @@ ContractArgs make_args(const float* Q, const void* E, int dtype, const float* sc
     if (chunk > 1024) chunk = 1024;
     a.chunk_rows = (int)chunk;
     a.n_chunks = (rows + chunk - 1) / chunk;
+    host::flat_walk(a.n_qgroups, rows, QA_STAGE_ROWS, 1024, &a.lanes_flat, &a.chunk_rows, &a.n_chunks);
     a.persistent = 1;
     return a;
   }
@@ -1328,7 +1329,7 @@ int launch_contract(int dtype, const ContractArgs& a, const EArgs& ea, hipStream
   // (make_args and this function both decide, from the table, between the persistent and the tiled kernels; a plan
   // made for the other kind would be read as garbage, so the two must not drift apart)
   KGE_REQUIRE((a.persistent != 0) == persistent, KGE_ERR_INVALID, "%s: work decomposition planned for another kernel", name);
-  const int64_t nwg = persistent ? 8 * (int64_t)a.n_qgroups * a.n_lanes : contract_grid_wgs(a);
+  const int64_t nwg = persistent ? host::walk_grid(a.n_qgroups, a.n_lanes, a.lanes_flat) : contract_grid_wgs(a);
   KGE_REQUIRE(nwg <= 0x7fffffffLL, KGE_ERR_INVALID, "%s: grid of %lld workgroups too large", name, (long long)nwg);
   const bool f32_split = (dtype == KGE_F32);
   const bool wide_bf16 = (dtype == KGE_BF16 || dtype == KGE_I8) && rc.lds_d == 0 && !wide_q;
@@ -1432,6 +1433,7 @@ int launch_rank128(const ContractArgs& base, const RankArgs& ea, hipStream_t st,
     eb.n_eq += s;
     eb.n_eql += s;
     host::rank128_plan(a.B, a.e_end - a.e_begin, &a.n_qgroups, &a.n_lanes, &a.chunk_rows, &a.n_chunks);
+    a.lanes_flat = 0;
     const int64_t nwg = 8 * (int64_t)a.n_qgroups * a.n_lanes;
     KGE_REQUIRE(nwg <= 0x7fffffffLL, KGE_ERR_INVALID, "%s: grid of %lld workgroups too large", name, (long long)nwg);
     hipLaunchKernelGGL((rank128_kernel<host::R128_WG_WAVES>), dim3((unsigned)nwg), dim3(64 * host::R128_WG_WAVES), 0, st, a, eb);
@@ -2007,6 +2009,7 @@ int topk_impl(const char* who, const float* Q, const float* bias, const void* E,
     if (chunk > 1024) chunk = 1024;
     a.chunk_rows = (int)chunk;
     a.n_chunks = (e1 - e0 + chunk - 1) / chunk;
+    a.lanes_flat = 0;
     const int64_t nwg = 8 * (int64_t)a.n_qgroups * a.n_lanes;
     KGE_REQUIRE(nwg <= 0x7fffffffLL, KGE_ERR_INVALID, "%s: grid of %lld workgroups too large", name, (long long)nwg);
     I8FilterArgs ea{tau, active, ws.cnt, ws.cand_id, TOPK_CAP, ws.requant, ws.rowmeta, ws.qh, ws.qc};

@@ -42,17 +42,14 @@ __global__ void __launch_bounds__(64 * QW_WG_WAVES, 2) qwide_kernel(ContractArgs
   __shared__ __attribute__((aligned(16))) float lds_sc[I8 ? QW_NBUF : 1][QW_STAGE_ROWS];
 
   const int64_t wg = blockIdx.x;
-  const int xcd = (int)(wg & 7);
-  const int64_t slot = wg >> 3;
-  const int qg = (int)(slot % a.n_qgroups);
-  const int wlane = (int)(slot / a.n_qgroups);
+  int qg;
+  int64_t c_first, c_stride;
+  walk_of_wg(a, wg, qg, c_first, c_stride);
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t q0 = (int64_t)qg * QW_WG_QUERIES + wave * 32;
 
   // chunks of this workgroup: first, stride, count; stages that hold at least one valid row
-  const int64_t c_first = xcd + 8 * (int64_t)wlane;
-  const int64_t c_stride = 8 * (int64_t)a.n_lanes;
   if (c_first >= a.n_chunks) return;
   const int my_chunks = (int)((a.n_chunks - 1 - c_first) / c_stride) + 1;
   const int spc = a.chunk_rows / QW_STAGE_ROWS;  // stages per chunk

@@ -261,7 +261,34 @@ static void test_plan() {
   }
 }
 
+// every chunk of every query group is walked by exactly one workgroup of a flat launch, and the form is only taken
+// where it fills more of the chip
+static void test_flat_walk() {
+  for (int groups = 1; groups <= 300; ++groups)
+    for (int64_t rows : {1LL, 128LL, 129LL, 5003LL, 123182LL, 2500000LL}) {
+      int lanes = -1, chunk = 0;
+      int64_t n = 0;
+      flat_walk(groups, rows, 128, 1024, &lanes, &chunk, &n);
+      if (lanes == 0) {
+        CHECK(chunk == 0 && n == 0 && walk_grid(groups, 3, 0) == 24 * (int64_t)groups);
+        continue;
+      }
+      CHECK(chunk >= 128 && chunk <= 1024 && chunk % 128 == 0 && n == (rows + chunk - 1) / chunk);
+      const int per_xcd = 32 / groups > 1 ? 32 / groups : 1, wgs = 8 * groups * per_xcd, rounds = (wgs + 255) / 256;
+      CHECK(lanes * groups <= 256 && lanes * groups * rounds > wgs);
+      const int64_t grid = walk_grid(groups, per_xcd, lanes);
+      CHECK(grid % 8 == 0 && grid <= 256 && grid >= (int64_t)groups * lanes);
+      std::vector<int> seen((size_t)groups * lanes, 0);
+      for (int64_t wg = 0; wg < grid; ++wg) {
+        const int64_t idx = (wg & 7) * (grid >> 3) + (wg >> 3);
+        if (idx / groups < lanes) ++seen[(size_t)((idx % groups) * lanes + idx / groups)];
+      }
+      for (int v : seen) CHECK(v == 1);
+    }
+}
+
 int main() {
+  test_flat_walk();
   test_contract_rules();
   test_layouts();
   test_csr_keys();
