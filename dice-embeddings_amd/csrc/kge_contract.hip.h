@@ -107,6 +107,106 @@ __device__ __forceinline__ u32x4 i8x8_to_bf16x8(uint32_t w0, uint32_t w1) {
   return r;
 }
 
+// ============================================================================================
+// One 32x32 tile straight from global memory: entity rows as A, query rows as B, in the same
+// reduction order as the two main loops.  Lane (c, hf) supplies entity row `e_row` and query row
+// `q_row` (either may be -1: a zero row).  Used where rows are gathered (targets, filter lists).
+// ============================================================================================
+template <int EDT>
+__device__ __forceinline__ f32x16 chain_direct(const void* E, int d, int64_t e_row, const float* Q, int64_t q_row,
+                                               int hf) {
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  if (EDT == KGE_F32) {
+    // fp32 rows on the bf16 MFMA: both rows split into three bf16 parts, six products per K step of 16
+    // (the order of ksplit_kernel).  Four K steps per trip: all sixteen loads are issued first.
+    const bool e_ok = e_row >= 0, q_ok = q_row >= 0;
+    const float* e_ptr = (const float*)E + (e_ok ? e_row : 0) * d;
+    const float* q_ptr = Q + (q_ok ? q_row : 0) * d;
+    const bool vec_ok = (d & 3) == 0;
+    const int nks = (d + 15) >> 4;
+    // Branch-free loads (a missing row or a column past d reads a clamped address and is zeroed after), so
+    // that the sixteen loads of a trip of four K steps are in flight together.
+    auto load_trip = [&](int ks0, f32x4 (&fe)[4][2], f32x4 (&fq)[4][2]) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = (ks0 + u) * 16 + 8 * hf + 4 * h;
+          if (vec_ok) {
+            const int kk = (k < d) ? k : 0;
+            fe[u][h] = *(const f32x4*)(e_ptr + kk);
+            fq[u][h] = *(const f32x4*)(q_ptr + kk);
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const int kk = (k + j < d) ? k + j : 0;
+              fe[u][h][j] = e_ptr[kk];
+              fq[u][h][j] = q_ptr[kk];
+            }
+          }
+        }
+      }
+    };
+    auto mul_trip = [&](int ks0, f32x4 (&fe)[4][2], f32x4 (&fq)[4][2]) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (ks0 + u < nks) {  // uniform: whole K steps past d are skipped (they would only add zeros)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int k = (ks0 + u) * 16 + 8 * hf + 4 * h;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const bool in = k + j < d;
+              fe[u][h][j] = (in && e_ok) ? fe[u][h][j] : 0.f;
+              fq[u][h][j] = (in && q_ok) ? fq[u][h][j] : 0.f;
+            }
+          }
+          bf16x8 se[3], sq[3];
+          split3_bf16x8(fe[u][0], fe[u][1], se);
+          split3_bf16x8(fq[u][0], fq[u][1], sq);
+#pragma unroll
+          for (int p = 0; p < SPLIT_PRODUCTS; ++p) acc = mfma_bf16(se[SPLIT_A[p]], sq[SPLIT_B[p]], acc);
+        }
+      }
+    };
+    // (Issuing the next trip's loads before this trip is multiplied was measured slower: the second register
+    // set costs the gather kernels more in occupancy than the overlap returns.)
+    for (int ks0 = 0; ks0 < nks; ks0 += 4) {
+      f32x4 fe[4][2], fq[4][2];
+      load_trip(ks0, fe, fq);
+      mul_trip(ks0, fe, fq);
+    }
+  } else {
+    for (int s0 = 0; s0 < d; s0 += 128)  // eight K steps per trip (one trip for d <= 128)
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int k = s0 + 16 * s + 8 * hf;
+      u32x4 ev = {0u, 0u, 0u, 0u};
+      f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+      if (k < d) {
+        if (e_row >= 0) {
+          if (EDT == KGE_BF16) {
+            ev = *(const u32x4*)((const uint16_t*)E + e_row * d + k);
+          } else {
+            const u32x2 w = *(const u32x2*)((const int8_t*)E + e_row * d + k);
+            ev = i8x8_to_bf16x8(w[0], w[1]);
+          }
+        }
+        if (q_row >= 0) {
+          const f32x4* src = (const f32x4*)(Q + q_row * d + k);
+          lo = src[0];
+          hi = src[1];
+        }
+      }
+      bf16x8 ef = __builtin_bit_cast(bf16x8, ev);
+      acc = mfma_bf16(ef, cvt_bf16x8(lo, hi), acc);
+    }
+  }
+  return acc;
+}
+
 // XCD-aware decomposition of a flat workgroup id: hardware deals consecutive ids round-robin over
 // the 8 XCDs, so ids with the same (id % 8) share an L2.  Consecutive slots on one XCD walk the
 // query groups of ONE entity chunk, which keeps that chunk's rows hot in that XCD's L2.

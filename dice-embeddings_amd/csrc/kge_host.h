@@ -229,6 +229,29 @@ inline TopkWsOffsets topk_ws_offsets(int64_t B, int64_t N, int64_t k, bool with_
   return o;
 }
 
+// Few queries (kge_few.hip): every wave holds the same queries and the rows are shared out, so the table is read once per
+// 32 .. 128 queries at the rate of memory.  The top-k form keeps the maximum of every 32-row tile per query in the
+// workspace: 4 N / 32 bytes per query.
+constexpr int FEW_MAX_B = 128;            // top-k
+constexpr int FEW_SCORES_MAX_B = 64;
+constexpr int FEW_MAX_K = 128;            // tiles scored again per query: one workgroup's work
+constexpr int FEW_TILES_DIRECT = 16384;   // tile maxima one workgroup selects from; more go through maxima of 32 tiles
+constexpr int64_t FEW_MAX_N = (int64_t)FEW_TILES_DIRECT * 32 * 32;
+constexpr int FEW_LDS_KB = 64;            // LDS for the query fragments: 1 KB per K step of 16, bf16 part and query tile
+inline int64_t few_maxima_pitch(int64_t N) { return ((N + 31) / 32 + 31) / 32 * 32; }
+inline bool few_rows_ok(int dtype, int64_t d) {
+  return (d + 15) / 16 * (dtype == KGE_F32 ? 3 : 1) <= FEW_LDS_KB && (dtype != KGE_F32 || d % 4 == 0);
+}
+inline bool few_topk_applies(int dtype, int64_t B, int64_t d, int64_t N, int64_t k) {
+  return B >= 1 && B <= FEW_MAX_B && k <= FEW_MAX_K && N <= FEW_MAX_N && few_rows_ok(dtype, d);
+}
+inline bool few_scores_applies(int dtype, int64_t B, int64_t d) {
+  return B >= 1 && B <= FEW_SCORES_MAX_B && few_rows_ok(dtype, d);
+}
+inline size_t few_topk_ws_bytes(int64_t B, int64_t N, int64_t k) {
+  return (B <= FEW_MAX_B && k <= FEW_MAX_K && N <= FEW_MAX_N) ? (size_t)B * (size_t)few_maxima_pitch(N) * 4 : 0;
+}
+
 // The threshold a scan of `n_next` more rows may use once `ranked` rows are ranked: the j-th best score so far, j as
 // small as the order statistics allow.  Of the best k of all ranked + n_next rows, the number X that are among
 // the rows already ranked is hypergeometric (rows in exchangeable order), mean k rho, variance below

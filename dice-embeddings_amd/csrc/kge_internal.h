@@ -41,6 +41,13 @@ void clear_error();
       return ::kge::set_error(KGE_ERR_HIP, "launch of %s failed: %s", name, hipGetErrorString(_e)); \
   } while (0)
 
+// ---- few queries against the whole table (kge_few.hip); the caller has asked host::few_topk_applies / few_scores_applies
+int few_topk_launch(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
+                    int64_t N, int64_t k, float* out_scores, int64_t* out_idx, int apply_sigmoid, void* workspace,
+                    hipStream_t st);
+int few_scores_launch(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
+                      int64_t N, float* out, int64_t ldo, hipStream_t st);
+
 // ---- MFMA 32x32 accumulator layout --------------------------------------------------------
 // acc[i] of lane l holds output (row_of(i, l / 32), l % 32).
 __device__ __forceinline__ int row_of(int i, int hf) { return ((i >> 2) << 3) + (hf << 2) + (i & 3); }

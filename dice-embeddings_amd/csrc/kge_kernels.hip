@@ -32,106 +32,6 @@ static char g_prof_kernel[160] = "";  // the main loop most recently bracketed, 
 
 namespace {
 
-// ============================================================================================
-// One 32x32 tile straight from global memory: entity rows as A, query rows as B, in the same
-// reduction order as the two main loops.  Lane (c, hf) supplies entity row `e_row` and query row
-// `q_row` (either may be -1: a zero row).  Used where rows are gathered (targets, filter lists).
-// ============================================================================================
-template <int EDT>
-__device__ __forceinline__ f32x16 chain_direct(const void* E, int d, int64_t e_row, const float* Q, int64_t q_row,
-                                               int hf) {
-  f32x16 acc;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-  if (EDT == KGE_F32) {
-    // fp32 rows on the bf16 MFMA: both rows split into three bf16 parts, six products per K step of 16
-    // (the order of ksplit_kernel).  Four K steps per trip: all sixteen loads are issued first.
-    const bool e_ok = e_row >= 0, q_ok = q_row >= 0;
-    const float* e_ptr = (const float*)E + (e_ok ? e_row : 0) * d;
-    const float* q_ptr = Q + (q_ok ? q_row : 0) * d;
-    const bool vec_ok = (d & 3) == 0;
-    const int nks = (d + 15) >> 4;
-    // Branch-free loads (a missing row or a column past d reads a clamped address and is zeroed after), so
-    // that the sixteen loads of a trip of four K steps are in flight together.
-    auto load_trip = [&](int ks0, f32x4 (&fe)[4][2], f32x4 (&fq)[4][2]) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int k = (ks0 + u) * 16 + 8 * hf + 4 * h;
-          if (vec_ok) {
-            const int kk = (k < d) ? k : 0;
-            fe[u][h] = *(const f32x4*)(e_ptr + kk);
-            fq[u][h] = *(const f32x4*)(q_ptr + kk);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const int kk = (k + j < d) ? k + j : 0;
-              fe[u][h][j] = e_ptr[kk];
-              fq[u][h][j] = q_ptr[kk];
-            }
-          }
-        }
-      }
-    };
-    auto mul_trip = [&](int ks0, f32x4 (&fe)[4][2], f32x4 (&fq)[4][2]) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        if (ks0 + u < nks) {  // uniform: whole K steps past d are skipped (they would only add zeros)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int k = (ks0 + u) * 16 + 8 * hf + 4 * h;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const bool in = k + j < d;
-              fe[u][h][j] = (in && e_ok) ? fe[u][h][j] : 0.f;
-              fq[u][h][j] = (in && q_ok) ? fq[u][h][j] : 0.f;
-            }
-          }
-          bf16x8 se[3], sq[3];
-          split3_bf16x8(fe[u][0], fe[u][1], se);
-          split3_bf16x8(fq[u][0], fq[u][1], sq);
-#pragma unroll
-          for (int p = 0; p < SPLIT_PRODUCTS; ++p) acc = mfma_bf16(se[SPLIT_A[p]], sq[SPLIT_B[p]], acc);
-        }
-      }
-    };
-    // (Issuing the next trip's loads before this trip is multiplied was measured slower: the second register
-    // set costs the gather kernels more in occupancy than the overlap returns.)
-    for (int ks0 = 0; ks0 < nks; ks0 += 4) {
-      f32x4 fe[4][2], fq[4][2];
-      load_trip(ks0, fe, fq);
-      mul_trip(ks0, fe, fq);
-    }
-  } else {
-    for (int s0 = 0; s0 < d; s0 += 128)  // eight K steps per trip (one trip for d <= 128)
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int k = s0 + 16 * s + 8 * hf;
-      u32x4 ev = {0u, 0u, 0u, 0u};
-      f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
-      if (k < d) {
-        if (e_row >= 0) {
-          if (EDT == KGE_BF16) {
-            ev = *(const u32x4*)((const uint16_t*)E + e_row * d + k);
-          } else {
-            const u32x2 w = *(const u32x2*)((const int8_t*)E + e_row * d + k);
-            ev = i8x8_to_bf16x8(w[0], w[1]);
-          }
-        }
-        if (q_row >= 0) {
-          const f32x4* src = (const f32x4*)(Q + q_row * d + k);
-          lo = src[0];
-          hi = src[1];
-        }
-      }
-      bf16x8 ef = __builtin_bit_cast(bf16x8, ev);
-      acc = mfma_bf16(ef, cvt_bf16x8(lo, hi), acc);
-    }
-  }
-  return acc;
-}
-
 // A member that is not its group's leader compares its vector with the leader's: the two halves of the wave
 // take alternate 16-byte pieces of the row (alternate words when the rows are not 16-byte aligned).
 __device__ __forceinline__ void group_vector_check(const ContractArgs& a, int64_t q, int hf, const int32_t* lead,
@@ -1580,6 +1480,12 @@ extern "C" int kge_scores(const float* Q, const float* bias, const void* E, int 
   if (B == 0) return KGE_OK;
   KGE_REQUIRE(S && ldS >= N, KGE_ERR_INVALID, "kge_scores: S is null or ldS=%lld < N=%lld", (long long)ldS,
               (long long)N);
+  if (host::few_scores_applies(dtype, B, d)) {
+    LaunchTimer timer;
+    if ((rc = timer.begin((hipStream_t)stream))) return rc;
+    if ((rc = few_scores_launch(Q, bias, E, dtype, scale, B, d, N, S, ldS, (hipStream_t)stream))) return rc;
+    return timer.end("few_scan_kernel");
+  }
   ContractArgs a = make_args(Q, E, dtype, scale, B, d, N, 0, N);
   StoreArgs ea{S, bias, ldS, 0};
   return launch_contract<StoreEpi>(dtype, a, ea, (hipStream_t)stream, "kge_scores");
@@ -1851,7 +1757,8 @@ extern "C" size_t kge_topk_workspace_bytes(int64_t B, int64_t N, int64_t k) {
   if (N < 1) N = 1;
   if (k < 1) k = 1;
   if (k > TOPK_MAX_K) k = TOPK_MAX_K;
-  return topk_ws_layout(B, N, k, nullptr, nullptr);
+  const size_t rounds = topk_ws_layout(B, N, k, nullptr, nullptr), few = host::few_topk_ws_bytes(B, N, k);
+  return rounds > few ? rounds : few;
 }
 
 namespace {
@@ -1899,7 +1806,8 @@ extern "C" size_t kge_topk_prepared_workspace_bytes(int64_t B, int64_t N, int64_
   if (N < 1) N = 1;
   if (k < 1) k = 1;
   if (k > TOPK_MAX_K) k = TOPK_MAX_K;
-  return topk_ws_layout(B, N, k, nullptr, nullptr, nullptr, false);
+  const size_t rounds = topk_ws_layout(B, N, k, nullptr, nullptr, nullptr, false), few = host::few_topk_ws_bytes(B, N, k);
+  return rounds > few ? rounds : few;
 }
 
 extern "C" int kge_topk(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B,
@@ -1952,6 +1860,12 @@ int topk_impl(const char* who, const float* Q, const float* bias, const void* E,
               int64_t d, int64_t N, int64_t k, float* out_scores, int64_t* out_idx, int apply_sigmoid,
               const void* prepared, void* workspace, hipStream_t st) {
   int rc = KGE_OK;
+  if (host::few_topk_applies(dtype, B, d, N, k)) {
+    LaunchTimer timer;
+    if ((rc = timer.begin(st))) return rc;
+    if ((rc = few_topk_launch(Q, bias, E, dtype, scale, B, d, N, k, out_scores, out_idx, apply_sigmoid, workspace, st))) return rc;
+    return timer.end("few_scan_kernel");
+  }
   TopkWs ws;
   topk_ws_layout(B, N, k, workspace, &ws, prepared, prepared == nullptr);
   const int64_t first_rows = (N < TOPK_FIRST_ROWS) ? N : TOPK_FIRST_ROWS;

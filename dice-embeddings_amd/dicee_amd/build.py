@@ -6,7 +6,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "csrc")
 OUT = os.path.join(HERE, "libkge_hip.so")
-SOURCES = ["kge_query.hip", "kge_kernels.hip", "kge_csr.hip", "kge_probe.hip"]
+SOURCES = ["kge_kernels.hip", "kge_few.hip", "kge_query.hip", "kge_csr.hip", "kge_probe.hip"]
 # -ffp-contract=off: a score is compared bit for bit across kernels, so `acc * scale` must be rounded
 # before it is compared or subtracted; a fused multiply-add would skip that rounding.
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=off",
@@ -14,16 +14,28 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-shared", "-fPIC", "-ffp
 
 
 def build(verbose=False):
-    cmd = ["hipcc"] + FLAGS + [os.path.join(CSRC, s) for s in SOURCES] + ["-o", OUT]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    proc = subprocess.run(cmd, capture_output=True, text=True)
+    """Compile the sources side by side and link them."""
+    import tempfile
     noise = "is not a recognized feature for this target"
-    err = "\n".join(line for line in proc.stderr.splitlines() if noise not in line)
-    if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{err}")
-    if verbose and err.strip():
-        print(err)
+    with tempfile.TemporaryDirectory() as tmp:
+        objs = [os.path.join(tmp, s + ".o") for s in SOURCES]
+        cmds = [["hipcc"] + [f for f in FLAGS if f != "-shared"] + ["-c", os.path.join(CSRC, s), "-o", o]
+                for s, o in zip(SOURCES, objs)]
+        if verbose:
+            print("\n".join(" ".join(c) for c in cmds), flush=True)
+        procs = [subprocess.Popen(c, stdout=subprocess.DEVNULL, stderr=subprocess.PIPE, text=True) for c in cmds]
+        errs = []
+        for p in procs:                       # (all are waited for before any failure is reported)
+            errs.append("\n".join(line for line in p.communicate()[1].splitlines() if noise not in line))
+        for p, s, err in zip(procs, SOURCES, errs):
+            if p.returncode != 0:
+                raise RuntimeError(f"hipcc failed on {s} ({p.returncode}):\n{err}")
+            if verbose and err.strip():
+                print(err)
+        link = subprocess.run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", OUT],
+                              capture_output=True, text=True)
+        if link.returncode != 0:
+            raise RuntimeError(f"hipcc failed to link ({link.returncode}):\n{link.stderr}")
     return OUT
 
 

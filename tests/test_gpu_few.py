@@ -1,0 +1,86 @@
+"""Batches of at most 128 queries: the scan that shares the rows out over the waves, and the selection from tile maxima."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import kge_oracle as ko
+
+pytestmark = pytest.mark.gpu
+
+
+def _table(rng, storage, N, d, pattern):
+    ints = rng.integers(-90, 91, (N, d)).astype(np.int8)
+    if pattern == "pool":                                   # thousands of exact ties, across tiles
+        ints = ints[rng.integers(0, min(3, N), N)]
+    elif pattern == "zero":                                 # ties at zero, of both signs' sums
+        ints[rng.random(N) < 0.7] = 0
+    E = torch.from_numpy(ints).cuda()
+    if storage == "int8":
+        return E, torch.rand(N, device="cuda") * 0.01 + (0.001 if pattern == "random" else 0.0)
+    E = E.float() * 0.01
+    return (E.to(torch.bfloat16) if storage == "bf16" else E), None
+
+
+# edges: one row, a partial tile, whole tiles, one past; one and several query tiles; a partial last K step; every k range;
+# 16384 tiles (the longest table selected from directly) and one more row
+CASES = [("fp32", 1, 4, 1, 1), ("fp32", 33, 20, 2, 33), ("fp32", 4096, 200, 33, 100), ("fp32", 5003, 256, 128, 10),
+         ("fp32", 3001, 340, 5, 7), ("bf16", 31, 8, 3, 31), ("bf16", 4097, 128, 32, 128), ("bf16", 2000, 1024, 65, 10),
+         ("bf16", 524288, 32, 2, 50), ("bf16", 524289, 32, 40, 128), ("int8", 1000, 16, 1, 10), ("int8", 7777, 240, 128, 100),
+         ("int8", 70001, 128, 64, 3)]
+
+
+@pytest.mark.parametrize("storage,N,d,B,k", CASES)
+@pytest.mark.parametrize("pattern", ["random", "pool", "zero"])
+def test_topk_of_few_queries_is_the_top_k_of_the_scores(storage, N, d, B, k, pattern):
+    from dicee_amd import ops
+    rng = np.random.default_rng(N + d + B)
+    E, sc = _table(rng, storage, N, d, pattern)
+    Q = torch.from_numpy((rng.standard_normal((B, d)) * 0.3).astype(np.float32)).cuda()
+    bias = torch.from_numpy(rng.standard_normal(B).astype(np.float32)).cuda()
+    vals, idx = ops.topk(Q, None, E, sc, k)
+    # the scores by the kernels of large batches (the batch repeated past every limit of the few-query forms)
+    S = ops.scores(Q.repeat(-(-130 // B), 1), None, E, sc)[:B]
+    assert torch.equal(ops.scores(Q, None, E, sc), S)
+    assert torch.equal(ops.scores(Q, bias, E, sc), S + bias[:, None])
+    wv, wi = ko.topk(S.cpu().numpy(), k)
+    np.testing.assert_array_equal(vals.cpu().numpy(), wv)
+    np.testing.assert_array_equal(idx.cpu().numpy(), wi)
+    bv, bi = ops.topk(Q, bias, E, sc, k, sigmoid=True)
+    assert torch.equal(bi, idx)
+    torch.testing.assert_close(bv, torch.sigmoid(vals + bias[:, None]), rtol=1e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("storage,d", [("fp32", 32), ("bf16", 64), ("int8", 128)])
+def test_topk_of_few_queries_ranks_no_nan_and_is_capturable(storage, d):
+    """NaN scores (a NaN row) are never ranked, a NaN query yields nothing, padding after the last row is never read as a
+    score; and the call reads nothing back, so it can be captured."""
+    from dicee_amd import ops
+    rng = np.random.default_rng(d)
+    N, B, k = 1003, 9, 20
+    E, sc = _table(rng, storage, N, d, "random")
+    if storage == "int8":
+        sc[5] = float("nan")
+    else:
+        E[5] = float("nan")
+    Q = -torch.rand(B, d, device="cuda")                    # mostly negative scores against ...
+    if storage != "int8":
+        E[:100] = E[:100].abs()
+    Q[3] = float("nan")
+    vals, idx = ops.topk(Q, None, E, sc, k)
+    S = ops.scores(Q.repeat(20, 1), None, E, sc)[:B].cpu().numpy()
+    for b in range(B):
+        if b == 3:
+            assert (idx[b] == -1).all() and torch.isnan(vals[b]).all()
+            continue
+        keep = np.where(np.isnan(S[b]), -np.inf, S[b])
+        want = np.lexsort((np.arange(N), -keep))[:k]
+        np.testing.assert_array_equal(idx[b].cpu().numpy(), want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gv, gi = ops.topk(Q, None, E, sc, k)
+    for _ in range(3):
+        gv.zero_()
+        gi.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(gi, idx) and torch.equal(torch.nan_to_num(gv), torch.nan_to_num(vals))
