@@ -838,6 +838,14 @@ struct BceEpi {
   }
 };
 
+// x / y for y in [1, 2] and x in [0, 1]: the hardware reciprocal (one unit in the last place) and one residual step, which
+// leaves the rounding of a division (nothing here can overflow or lose the residual, which is what the general division's
+// scaling and fix-up instructions, two thirds of it, are for).
+__device__ __forceinline__ float quotient_1_2(float x, float y) {
+  const float r = __builtin_amdgcn_rcpf(y), q = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
+}
+
 // Backward of the multi-hot BCE step: g = (sigmoid(s) - y') * inv_bn for the dense part of y' (the
 // known tails are subtracted afterwards from the CSR), written as G [B, ldG] and, when GT is given, also as its
 // transpose GT [N, ldT] (the operands of the two gradient contractions when they take row-major operands only), plus
@@ -908,7 +916,7 @@ struct GradEpi {
           if (HAS_SCALE) v *= sc_col;
           v += b4[r];
           const float ex = __expf(-fabsf(v));                       // in (0, 1]
-          const float sig = (v >= 0.f ? 1.0f : ex) / (1.0f + ex);    // sigmoid without overflow
+          const float sig = quotient_1_2(v >= 0.f ? 1.0f : ex, 1.0f + ex);  // sigmoid without overflow
           const float gr = sig * a.inv_bn - a.uniform;
           prod = __builtin_fmaf(prod, ex, prod);
           tpos += fmaxf(v, 0.f);
@@ -930,7 +938,7 @@ struct GradEpi {
           v += b4[r];
           const bool ok = qrow + 8 * g + r < B;
           const float ex = __expf(-fabsf(v));
-          const float sig = (v >= 0.f ? 1.0f : ex) / (1.0f + ex);
+          const float sig = quotient_1_2(v >= 0.f ? 1.0f : ex, 1.0f + ex);
           const float gr = ok ? sig * a.inv_bn - a.uniform : 0.f;
           prod = __builtin_fmaf(prod, ok ? ex : 0.f, prod);
           tpos += ok ? fmaxf(v, 0.f) : 0.f;

@@ -934,75 +934,145 @@ __global__ void minmax_final_kernel(uint32_t* kmin, uint32_t* kmax, const float*
 // ---- BCE helpers --------------------------------------------------------------------------------
 // accumulators: BCE_SLOTS partial sums of softplus(s), BCE_SLOTS of s, then BCE_POS_SLOTS of the sum over the positives
 using host::BCE_POS_SLOTS;
-__global__ void bce_init_kernel(double* sums) {
-  for (int i = threadIdx.x; i < 2 * BCE_SLOTS + BCE_POS_SLOTS; i += blockDim.x) sums[i] = 0.0;
+__global__ void bce_init_kernel(double* sums, float* dbias, int64_t B) {  // dbias: a [B] vector to clear as well, or null
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 2 * BCE_SLOTS + BCE_POS_SLOTS) sums[i] = 0.0;
+  if (dbias && i < B) dbias[i] = 0.f;
+}
+constexpr int BCE_INIT_THREADS = 2 * BCE_SLOTS + BCE_POS_SLOTS;
+inline unsigned bce_init_blocks(int64_t B, const float* dbias) {
+  return dbias ? (unsigned)((B + BCE_INIT_THREADS - 1) / BCE_INIT_THREADS) : 1u;
 }
 
-// sum of the logits of the positive (query, tail) pairs.  Grid (queries, BCE_POS_SPLIT): a workgroup is sixteen
+// The positive (query, tail) pairs: the sum of their logits (sums, null: not wanted) and, in the backward, what the label
+// takes from their score gradients (pg.G, null: forward).  Grid (queries, BCE_POS_SPLIT): a workgroup is sixteen
 // groups of sixteen lanes, and positive j of a query's row goes to group j mod (16 * BCE_POS_SPLIT) of that query's
-// workgroups.  The usual row of one or two positives is a single chain of dependent loads (row -> extent -> tail ->
-// embedding row) that runs beside every other query's; a row of hundreds is shared out over 64 groups.  One atomic per
-// workgroup that found work, spread over a few addresses: thousands of double-precision atomics on one address
-// would serialise.
+// workgroups, four of them at a time: what bounds the kernel is the chain of loads (row -> extent -> tail -> embedding
+// row), which the usual row of one or two positives runs through once, beside every other query's, and a hub's row of
+// thousands over and over; with four rows in flight per group, in 16-byte pieces, and both jobs in one launch
+// (2048 pairs of a 41k graph, d = 256: 38 + 13 us in two launches, one row in flight per group -> 17; 1000 pairs of a
+// 14.5k graph, d = 200: 21 + 7 -> 9 us).
+// One atomic per workgroup that found work, spread over a few addresses: thousands of double-precision atomics on one
+// address would serialise.
+struct PosGrad {
+  float* G;  // [B, ldG] score gradients: `pos` is subtracted at the known tails (y = 1 there)
+  int64_t ldG;
+  float* GT;  // the same transposed, or null
+  int64_t ldT;
+  float* dbias;  // row sums of the gradient, or null
+  float pos;
+};
 constexpr int BCE_POS_SPLIT = 4;
+constexpr int BCE_POS_UNROLL = 4;
 template <int EDT>
 __global__ void __launch_bounds__(256) bce_pos_kernel(ContractArgs a, const float* bias, const int64_t* csr_row,
                                                      const int64_t* row_ptr, const int32_t* col, int64_t n_rows,
-                                                     double* sums) {
+                                                     double* sums, PosGrad pg) {
   __shared__ double s_part[16];
+  __shared__ int s_count[16];
   const int tid = threadIdx.x, grp = tid >> 4, sub = tid & 15;
   const int64_t q = blockIdx.x;
   const int64_t row = csr_row[q];
   if (row < 0 || row >= n_rows) return;
   const int64_t j0 = row_ptr[row], j1 = row_ptr[row + 1];
-  const int slot = (int)blockIdx.y * 16 + grp;
+  constexpr int STRIDE = 16 * BCE_POS_SPLIT, U = BCE_POS_UNROLL;
   if (j0 + (int64_t)blockIdx.y * 16 >= j1) return;  // nothing for this workgroup (the same for all of it)
   const float bq = bias ? bias[q] : 0.f;
   const float* qv = a.Q + q * a.d;
   double local = 0.0;  // every lane of a group holds the same sum
-  for (int64_t j = j0 + slot; j < j1; j += 16 * BCE_POS_SPLIT) {
-    const int64_t e = col[j];
-    if (e < 0 || e >= a.N) continue;  // uniform across the group
-    float dot = 0.f;
-    for (int k = sub; k < a.d; k += 16) {
-      float x;
-      float qk = qv[k];
-      if (EDT == KGE_F32) {
-        x = ((const float*)a.E)[e * a.d + k];
-      } else {
-        qk = (float)(__bf16)qk;
-        if (EDT == KGE_BF16)
-          x = __uint_as_float((uint32_t)((const uint16_t*)a.E)[e * a.d + k] << 16);
-        else
-          x = (float)((const int8_t*)a.E)[e * a.d + k];
+  int n_valid = 0;
+  for (int64_t j = j0 + (int)blockIdx.y * 16 + grp; j < j1; j += STRIDE * U) {
+    int64_t e[U];
+    bool ok[U];  // uniform across the group
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      e[u] = j + u * STRIDE < j1 ? col[j + u * STRIDE] : -1;
+      ok[u] = e[u] >= 0 && e[u] < a.N;
+      n_valid += ok[u] ? 1 : 0;
+    }
+    if (pg.G && sub < U) {  // lane u of the group: element u (a row's tails are distinct: no two threads meet)
+      int64_t mine = e[0];
+      bool on = ok[0];
+#pragma unroll
+      for (int u = 1; u < U; ++u) {
+        mine = sub == u ? e[u] : mine;
+        on = sub == u ? ok[u] : on;
       }
-      dot = fmaf(qk, x, dot);
+      if (on) {
+        pg.G[q * pg.ldG + mine] -= pg.pos;
+        if (pg.GT) pg.GT[mine * pg.ldT + q] -= pg.pos;
+      }
+    }
+    if (!sums) continue;
+    float dot[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      dot[u] = 0.f;
+      e[u] = ok[u] ? e[u] : 0;  // (its product is dropped below)
+    }
+    if (EDT == KGE_F32 && (a.d & 3) == 0) {
+      for (int k = 4 * sub; k < a.d; k += 64) {
+        const f32x4 qk = *(const f32x4*)(qv + k);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const f32x4 x = *(const f32x4*)((const float*)a.E + e[u] * a.d + k);
+          dot[u] = fmaf(qk[3], x[3], fmaf(qk[2], x[2], fmaf(qk[1], x[1], fmaf(qk[0], x[0], dot[u]))));
+        }
+      }
+    } else {
+      for (int k = sub; k < a.d; k += 16) {
+        float qk = qv[k];
+        if (EDT != KGE_F32) qk = (float)(__bf16)qk;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float x;
+          if (EDT == KGE_F32) x = ((const float*)a.E)[e[u] * a.d + k];
+          else if (EDT == KGE_BF16) x = __uint_as_float((uint32_t)((const uint16_t*)a.E)[e[u] * a.d + k] << 16);
+          else x = (float)((const int8_t*)a.E)[e[u] * a.d + k];
+          dot[u] = fmaf(qk, x, dot[u]);
+        }
+      }
     }
 #pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) dot += __shfl_xor(dot, o, 64);
-    if (EDT == KGE_I8) dot *= a.scale[e];
-    local += (double)(dot + bq);
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int o = 8; o >= 1; o >>= 1) dot[u] += __shfl_xor(dot[u], o, 64);
+      if (EDT == KGE_I8) dot[u] *= a.scale[e[u]];
+      if (ok[u]) local += (double)(dot[u] + bq);
+    }
   }
-  if (sub == 0) s_part[grp] = local;
+  if (sub == 0) {
+    s_part[grp] = local;
+    s_count[grp] = n_valid;
+  }
   __syncthreads();
   if (tid == 0) {
     double t = 0.0;
+    int n = 0;
 #pragma unroll
-    for (int g = 0; g < 16; ++g) t += s_part[g];
+    for (int g = 0; g < 16; ++g) {
+      t += s_part[g];
+      n += s_count[g];
+    }
     if (t != 0.0) atomicAdd(&sums[2 * BCE_SLOTS + ((blockIdx.x + blockIdx.y) & (BCE_POS_SLOTS - 1))], t);
+    if (pg.dbias && n) atomicAdd(&pg.dbias[q], -pg.pos * (float)n);
   }
 }
 
 // one wave: the partial sums are read side by side (one thread reading 384 doubles in turn is a chain of its own)
-__global__ void bce_final_kernel(const double* sums, double B, double N, float eps, float* loss) {
-  const int lane = threadIdx.x;
-  if (blockIdx.x != 0 || lane >= 64) return;
+struct BceFinal {
+  const double* sums;
+  double B, N;
+  float eps;
+  float* loss;  // null: nothing to do
+};
+__device__ __forceinline__ void bce_final(const BceFinal& f, int lane) {
   double t = 0.0, s = 0.0, pos = 0.0;
   for (int i = lane; i < BCE_SLOTS; i += 64) {
-    t += sums[i];
-    s += sums[BCE_SLOTS + i];
+    t += f.sums[i];
+    s += f.sums[BCE_SLOTS + i];
   }
-  for (int i = lane; i < BCE_POS_SLOTS; i += 64) pos += sums[2 * BCE_SLOTS + i];
+  for (int i = lane; i < BCE_POS_SLOTS; i += 64) pos += f.sums[2 * BCE_SLOTS + i];
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
     t += __shfl_xor(t, o, 64);
@@ -1010,19 +1080,18 @@ __global__ void bce_final_kernel(const double* sums, double B, double N, float e
     pos += __shfl_xor(pos, o, 64);
   }
   if (lane == 0) {
-    if (eps != 0.f)
-      t -= (1.0 - (double)eps) * pos + s / N;
+    if (f.eps != 0.f)
+      t -= (1.0 - (double)f.eps) * pos + s / f.N;
     else
       t -= pos;
-    loss[0] = (float)(t / (B * N));
+    f.loss[0] = (float)(t / (f.B * f.N));
   }
+}
+__global__ void bce_final_kernel(BceFinal f) {
+  if (blockIdx.x == 0 && threadIdx.x < 64) bce_final(f, threadIdx.x);
 }
 
 // ---- backward of the BCE step: helpers -------------------------------------------------------------
-__global__ void fill_zero_kernel(float* p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = 0.f;
-}
-
 // out[c, r] = in[r, c] for a rows x cols matrix (row strides ld_in, ld_out), 32 x 32 tiles through LDS
 __global__ void __launch_bounds__(256) transpose_kernel(const float* in, int64_t rows, int64_t cols, int64_t ld_in,
                                                        float* out, int64_t ld_out) {
@@ -1042,28 +1111,10 @@ __global__ void __launch_bounds__(256) transpose_kernel(const float* in, int64_t
   }
 }
 
-// the known tails: y = 1 there, so `pos` is subtracted from both copies of the gradient and from the row sums
-__global__ void __launch_bounds__(256) grad_pos_kernel(const int64_t* csr_row, const int64_t* row_ptr,
-                                                      const int32_t* col, int64_t n_rows, int64_t B, int64_t N, float* G,
-                                                      int64_t ldG, float* GT, int64_t ldT, float* dbias, float pos) {
-  for (int64_t q = blockIdx.x; q < B; q += gridDim.x) {
-    const int64_t row = csr_row[q];
-    if (row < 0 || row >= n_rows) continue;
-    const int64_t j0 = row_ptr[row], j1 = row_ptr[row + 1];
-    int n_valid = 0;
-    for (int64_t j = j0 + threadIdx.x; j < j1; j += blockDim.x) {
-      const int64_t e = col[j];
-      if (e < 0 || e >= N) continue;
-      G[q * ldG + e] -= pos;  // a row's tails are distinct: no two threads touch one element
-      if (GT) GT[e * ldT + q] -= pos;
-      ++n_valid;
-    }
-    if (dbias && n_valid) atomicAdd(&dbias[q], -pos * (float)n_valid);
-  }
-}
-
 // out[i] = sum over y of partial[y][i], y ascending
-__global__ void reduce_splits_kernel(const float* partial, int n_splits, int64_t n, float* out) {
+// (and, in its first workgroup, the loss from its partial sums: a launch less on the way through the backward)
+__global__ void reduce_splits_kernel(const float* partial, int n_splits, int64_t n, float* out, BceFinal f) {
+  if (f.loss && blockIdx.x == 0 && threadIdx.x < 64) bce_final(f, threadIdx.x);
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     float v = 0.f;
     for (int y = 0; y < n_splits; ++y) v += partial[(int64_t)y * n + i];
@@ -2019,7 +2070,7 @@ extern "C" int kge_bce_multihot(const float* Q, const float* bias, const void* E
   KGE_REQUIRE(((uintptr_t)workspace & 7) == 0, KGE_ERR_WORKSPACE, "kge_bce_multihot: workspace must be 8-byte aligned");
   hipStream_t st = (hipStream_t)stream;
   double* sums = (double*)workspace;
-  hipLaunchKernelGGL(bce_init_kernel, dim3(1), dim3(256), 0, st, sums);
+  hipLaunchKernelGGL(bce_init_kernel, dim3(bce_init_blocks(B, nullptr)), dim3(BCE_INIT_THREADS), 0, st, sums, nullptr, B);
   KGE_LAUNCH_CHECK("bce_init_kernel");
   ContractArgs a = make_args(Q, E, dtype, scale, B, d, N, 0, N);
   BceArgs ea{bias, sums, label_smoothing != 0.f ? 1 : 0};
@@ -2027,10 +2078,10 @@ extern "C" int kge_bce_multihot(const float* Q, const float* bias, const void* E
   if (rc) return rc;
   if (csr_row && n_rows > 0) {
     dim3 grid((unsigned)B, BCE_POS_SPLIT), block(256);
-    KGE_DISPATCH_DTYPE(dtype, bce_pos_kernel, grid, block, 0, st, a, bias, csr_row, row_ptr, col, n_rows, sums);
+    KGE_DISPATCH_DTYPE(dtype, bce_pos_kernel, grid, block, 0, st, a, bias, csr_row, row_ptr, col, n_rows, sums, PosGrad{});
     KGE_LAUNCH_CHECK("bce_pos_kernel");
   }
-  hipLaunchKernelGGL(bce_final_kernel, dim3(1), dim3(64), 0, st, sums, (double)B, (double)N, label_smoothing, loss);
+  hipLaunchKernelGGL(bce_final_kernel, dim3(1), dim3(64), 0, st, BceFinal{sums, (double)B, (double)N, label_smoothing, loss});
   KGE_LAUNCH_CHECK("bce_final_kernel");
   return KGE_OK;
 }
@@ -2078,12 +2129,8 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
   float* part = (float*)(ws + p.off_part);
   const float inv_bn = grad_out / ((float)B * (float)N);
 
-  hipLaunchKernelGGL(bce_init_kernel, dim3(1), dim3(256), 0, st, sums);
+  hipLaunchKernelGGL(bce_init_kernel, dim3(bce_init_blocks(B, dbias)), dim3(BCE_INIT_THREADS), 0, st, sums, dbias, B);
   KGE_LAUNCH_CHECK("bce_init_kernel");
-  if (dbias) {
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, st, dbias, B);
-    KGE_LAUNCH_CHECK("fill_zero_kernel");
-  }
   // (1) scores -> g = (sigmoid(s) - dense part of y') * inv_bn, both layouts, and the loss sums
   ContractArgs a = make_args(Q, E, KGE_F32, nullptr, B, d, N, 0, N);
   GradArgs ga{bias, sums, G, GT, dbias, p.ldG, p.ldT, inv_bn, label_smoothing != 0.f ? inv_bn / (float)N : 0.f,
@@ -2091,19 +2138,14 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
   rc = launch_ksplit<GradEpi>(a, ga, 1, st, "kge_bce_multihot_backward: scores");
   if (rc) return rc;
   if (csr_row && n_rows > 0) {
-    dim3 grid((unsigned)(B < 512 ? B : 512)), block(256);
-    if (loss) {
-      hipLaunchKernelGGL((bce_pos_kernel<KGE_F32>), dim3((unsigned)B, BCE_POS_SPLIT), block, 0, st, a, bias, csr_row,
-                         row_ptr, col, n_rows, sums);
-      KGE_LAUNCH_CHECK("bce_pos_kernel");
-    }
     const float pos = (label_smoothing != 0.f ? 1.0f - label_smoothing : 1.0f) * inv_bn;
-    hipLaunchKernelGGL(grad_pos_kernel, grid, block, 0, st, csr_row, row_ptr, col, n_rows, B, N, G, p.ldG, GT, p.ldT,
-                       dbias, pos);
-    KGE_LAUNCH_CHECK("grad_pos_kernel");
+    hipLaunchKernelGGL((bce_pos_kernel<KGE_F32>), dim3((unsigned)B, BCE_POS_SPLIT), dim3(256), 0, st, a, bias, csr_row,
+                       row_ptr, col, n_rows, loss ? sums : nullptr, PosGrad{G, p.ldG, GT, p.ldT, dbias, pos});
+    KGE_LAUNCH_CHECK("bce_pos_kernel");
   }
-  if (loss) {
-    hipLaunchKernelGGL(bce_final_kernel, dim3(1), dim3(64), 0, st, sums, (double)B, (double)N, label_smoothing, loss);
+  const BceFinal fin{sums, (double)B, (double)N, label_smoothing, loss};
+  if (loss && p.k_splits == 1) {  // (else dQ's reduction does it)
+    hipLaunchKernelGGL(bce_final_kernel, dim3(1), dim3(64), 0, st, fin);
     KGE_LAUNCH_CHECK("bce_final_kernel");
   }
   // (2) the other operands with the summed index contiguous: ET [d, ldG], QT [d, ldT]
@@ -2128,7 +2170,7 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
     if (p.k_splits > 1) {
       const int64_t n = B * d;
       hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)((n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048)),
-                         dim3(256), 0, st, part, p.k_splits, n, dQ);
+                         dim3(256), 0, st, part, p.k_splits, n, dQ, fin);
       KGE_LAUNCH_CHECK("reduce_splits_kernel");
     }
   }

@@ -1298,132 +1298,6 @@ int build_query_backward_impl(int model, int p, int q, int r, const float* ent, 
 }  // namespace
 }  // namespace kge
 
-extern "C" size_t kge_batchnorm_workspace_bytes(int64_t B, int64_t d);
-
-namespace kge {
-namespace {
-int build_query_backward_impl(int model, int p, int q, int r, const float* ent, const float* rel, const float* coeff_p,
-                              const float* coeff_q, const float* coeff_r, int normalize_relation,
-                              const kge_norm_params* norm, const kge_norm_grads* dnorm, const int64_t* hr, int64_t B,
-                              int64_t d, int64_t N, int64_t R, const float* dQ, const float* dbias, float* d_ent,
-                              float* d_rel, float* d_coeff_p, float* d_coeff_q, float* d_coeff_r, void* stream,
-                              const kge_dropout_params* dropout = nullptr, bool batch_stats = false,
-                              void* workspace = nullptr, size_t workspace_bytes = 0) {
-  clear_error();
-  KGE_REQUIRE(B >= 0 && N > 0 && R > 0, KGE_ERR_INVALID, "kge_build_query_backward: B=%lld N=%lld R=%lld", (long long)B,
-              (long long)N, (long long)R);
-  if (B == 0) return KGE_OK;
-  KGE_REQUIRE(ent && rel && hr && dQ && d_ent && d_rel, KGE_ERR_INVALID, "kge_build_query_backward: null pointer argument");
-  KGE_REQUIRE(d >= 1 && d <= 8192, KGE_ERR_INVALID, "kge_build_query_backward: d=%lld outside [1, 8192]", (long long)d);
-  KGE_REQUIRE(B <= 0x7fffffff, KGE_ERR_INVALID, "kge_build_query_backward: B=%lld too large", (long long)B);
-  if (model != KGE_DECAL) r = 0;
-  switch (model) {
-    case KGE_DISTMULT: break;
-    case KGE_COMPLEX:
-      KGE_REQUIRE(d % 2 == 0, KGE_ERR_INVALID, "kge_build_query_backward: ComplEx needs even d, got %lld", (long long)d);
-      break;
-    case KGE_QMULT:
-      KGE_REQUIRE(d % 4 == 0, KGE_ERR_INVALID, "kge_build_query_backward: QMult needs d %% 4 == 0, got %lld", (long long)d);
-      break;
-    case KGE_OMULT:
-      KGE_REQUIRE(d % 8 == 0, KGE_ERR_INVALID, "kge_build_query_backward: OMult needs d %% 8 == 0, got %lld", (long long)d);
-      break;
-    case KGE_KECI:
-    case KGE_DECAL:
-      KGE_REQUIRE(p >= 0 && q >= 0 && r >= 0 && d % (p + q + r + 1) == 0, KGE_ERR_INVALID,
-                  "kge_build_query_backward: needs d / (p + q + r + 1) whole, got d=%lld p=%d q=%d r=%d", (long long)d, p,
-                  q, r);
-      KGE_REQUIRE((p == 0 || coeff_p) && (q == 0 || coeff_q) && (r == 0 || coeff_r), KGE_ERR_INVALID,
-                  "kge_build_query_backward: p=%d q=%d r=%d need their coefficient vectors", p, q, r);
-      break;
-    default: return set_error(KGE_ERR_INVALID, "kge_build_query_backward: unknown model %d", model);
-  }
-  QueryBwdArgs a;
-  a.ent = ent;
-  a.rel = rel;
-  a.coeff_p = coeff_p;
-  a.coeff_q = coeff_q;
-  a.coeff_r = coeff_r;
-  a.hr = hr;
-  a.dQ = dQ;
-  a.dbias = dbias;
-  a.d_ent = d_ent;
-  a.d_rel = d_rel;
-  a.d_coeff_p = d_coeff_p;
-  a.d_coeff_q = d_coeff_q;
-  a.d_coeff_r = d_coeff_r;
-  a.B = B;
-  a.N = N;
-  a.R = R;
-  a.d = (int)d;
-  a.p = p;
-  a.q = q;
-  a.r = r;
-  a.normalize_relation = normalize_relation;
-  a.norm.kind = KGE_NORM_NONE;
-  a.norm.eps = 0.f;
-  a.norm.h_a = a.norm.h_b = a.norm.r_a = a.norm.r_b = nullptr;
-  a.dn_h_a = a.dn_h_b = a.dn_r_a = a.dn_r_b = nullptr;
-  a.dy_h = a.dy_r = nullptr;
-  a.drop = kge_dropout_params{nullptr, nullptr, nullptr, 1.f, 1.f};
-  if (dropout) {
-    if (int rc = check_dropout("kge_build_query_backward", dropout, model)) return rc;
-    a.drop = *dropout;
-  }
-  hipStream_t st = (hipStream_t)stream;
-  if (batch_stats) {
-    KGE_REQUIRE(norm && norm->kind == KGE_NORM_BATCHNORM1D && norm->h_a && norm->h_b && norm->r_a && norm->r_b,
-                KGE_ERR_INVALID,
-                "kge_build_query_backward_batchnorm: norm must be BatchNorm1d with the batch's statistics");
-    KGE_REQUIRE(d <= 4096, KGE_ERR_UNSUPPORTED, "kge_build_query_backward_batchnorm: d=%lld exceeds 4096", (long long)d);
-    KGE_REQUIRE(B >= 2, KGE_ERR_INVALID, "kge_build_query_backward_batchnorm: batch statistics need B >= 2");
-    const size_t need = kge_batchnorm_workspace_bytes(B, d);
-    KGE_REQUIRE(workspace && workspace_bytes >= need, KGE_ERR_WORKSPACE,
-                "kge_build_query_backward_batchnorm: workspace of %zu bytes, need %zu", workspace_bytes, need);
-    KGE_REQUIRE(((uintptr_t)workspace & 15) == 0, KGE_ERR_WORKSPACE,
-                "kge_build_query_backward_batchnorm: workspace must be 16-byte aligned");
-    double* sums = (double*)workspace;
-    a.norm = *norm;
-    a.dy_h = (float*)(sums + 4 * d);
-    a.dy_r = a.dy_h + B * d;
-    hipLaunchKernelGGL(bn_zero_kernel, dim3((unsigned)((4 * d + 255) / 256)), dim3(256), 0, st, sums, (int)(4 * d));
-    KGE_LAUNCH_CHECK("bn_zero_kernel");
-    // (1) the gradients at the normalised rows, (2) their sums over the batch, (3) the gradients at the raw rows
-    if (int rc = launch_build_query_backward(a, model, true, st)) return rc;
-    BnSumArgs sa{ent, rel, hr, a.dy_h, a.dy_r, *norm, a.drop, sums, B, N, R, (int)d};
-    const unsigned slices = (unsigned)((B + 63) / 64 < 64 ? (B + 63) / 64 : 64);
-    dim3 grid((unsigned)((d + 63) / 64), slices);
-    hipLaunchKernelGGL(bn_sums_kernel<true>, grid, dim3(256), 0, st, sa);
-    KGE_LAUNCH_CHECK("bn_sums_kernel");
-    hipLaunchKernelGGL(bn_backward_apply_kernel, grid, dim3(256), 0, st, sa, d_ent, d_rel);
-    KGE_LAUNCH_CHECK("bn_backward_apply_kernel");
-    return KGE_OK;
-  }
-  if (norm && norm->kind != KGE_NORM_NONE) {
-    KGE_REQUIRE(norm->kind == KGE_NORM_LAYERNORM || norm->kind == KGE_NORM_BATCHNORM1D, KGE_ERR_INVALID,
-                "kge_build_query_backward_norm: unknown normalisation %d", norm->kind);
-    KGE_REQUIRE(norm->h_a && norm->h_b && norm->r_a && norm->r_b, KGE_ERR_INVALID,
-                "kge_build_query_backward_norm: normalisation parameters missing");
-    KGE_REQUIRE(d <= 4096, KGE_ERR_UNSUPPORTED,
-                "kge_build_query_backward_norm: d=%lld exceeds 4096 (five rows and a quarter per pair are kept in LDS)",
-                (long long)d);
-    a.norm = *norm;
-    if (dnorm) {
-      KGE_REQUIRE(norm->kind == KGE_NORM_LAYERNORM || !(dnorm->h_a || dnorm->h_b || dnorm->r_a || dnorm->r_b),
-                  KGE_ERR_INVALID,
-                  "kge_build_query_backward_norm: BatchNorm1d(affine=False) has no parameters to take a gradient");
-      a.dn_h_a = dnorm->h_a;
-      a.dn_h_b = dnorm->h_b;
-      a.dn_r_a = dnorm->r_a;
-      a.dn_r_b = dnorm->r_b;
-    }
-    return launch_build_query_backward(a, model, true, st);
-  }
-  return launch_build_query_backward(a, model, false, st);
-}
-}  // namespace
-}  // namespace kge
-
 namespace kge {
 namespace {
 struct ZeroList {

@@ -186,6 +186,10 @@ class BaseKGE(torch.nn.Module):
     def _query_kwargs(self):
         return {}
 
+    def _bias_varies(self):
+        """Does the per-query bias depend on any parameter?  (The sums over pairs of Clifford bases, alone.)"""
+        return any(getattr(self, n, 0) >= 2 for n in ("p", "q") + (("r",) if self.name == "DeCaL" else ()))
+
     def query(self, x, heads=False, norm=_FROM_MODEL, dropout=_FROM_MODEL):
         """(Q [B,d], bias [B]) for ``x`` [B,2]: gather + interaction
         (get_head_relation_representation, base_model.py:377-384, then the model's elementwise part).
@@ -304,17 +308,19 @@ class BaseKGE(torch.nn.Module):
         rows = csr.rows_for(x.to(device=E.device, dtype=torch.int64))
         return ops.bce_multihot(Q, bias, E, scale, rows, csr.row_ptr, csr.col, label_smoothing)[0]
 
-    def kvsall_bce_backward(self, x, csr, label_smoothing=0.0, grad_out=1.0, norm=_FROM_MODEL, dropout=_FROM_MODEL):
+    def kvsall_bce_backward(self, x, csr, label_smoothing=0.0, grad_out=1.0, norm=_FROM_MODEL, dropout=_FROM_MODEL,
+                            want_dbias=True):
         """The same step with its backward through the scores: ``(loss, dQ [B,d], dbias [B], dE [N,d])`` where
         ``dQ`` / ``dbias`` are the gradients at the query vectors and per-query biases of ``self.query(x)`` and ``dE``
         the gradient the contraction sends to the entity table (fp32 tables only).  What
-        ``loss_batch.backward()`` computes for the ``torch.mm`` / ``einsum`` and the loss of the reference's step."""
+        ``loss_batch.backward()`` computes for the ``torch.mm`` / ``einsum`` and the loss of the reference's step.  ``want_dbias=False``: None in its place."""
         Q, bias = self.query(x, norm=norm, dropout=dropout)
         E, scale = self.table()
         if scale is not None:
             raise TypeError("the backward needs an fp32 entity table")
         rows = csr.rows_for(x.to(device=E.device, dtype=torch.int64))
-        loss, dQ, dbias, dE = ops.bce_multihot_backward(Q, bias, E, rows, csr.row_ptr, csr.col, label_smoothing, grad_out)
+        loss, dQ, dbias, dE = ops.bce_multihot_backward(Q, bias, E, rows, csr.row_ptr, csr.col, label_smoothing, grad_out,
+                                                        want_dbias=want_dbias)
         return loss[0], dQ, dbias, dE
 
     def kvsall_bce_gradients(self, x, csr, label_smoothing=0.0):
@@ -333,15 +339,18 @@ class BaseKGE(torch.nn.Module):
         x = x.to(device=E.device, dtype=torch.int64).contiguous()
         dropout = self._draw_dropout(x.shape[0], E.device)
         norm = self._norm_params(x, dropout)
-        loss, dQ, dbias, dE = self.kvsall_bce_backward(x, csr, label_smoothing, norm=norm, dropout=dropout)
+        loss, dQ, dbias, dE = self.kvsall_bce_backward(x, csr, label_smoothing, norm=norm, dropout=dropout,
+                                                       want_dbias=self._bias_varies())
         rel = self._rel()
-        dR = torch.zeros_like(rel)
         name = self.name if self.name != "CKeci" else "Keci"
-        dnorm = None
-        if norm is not None and norm["kind"] == "LayerNorm":
-            dnorm = {k: torch.zeros_like(norm[k], dtype=torch.float32) for k in ("h_a", "h_b", "r_a", "r_b")}
+        kw = self._query_kwargs()
+        coeffs = [kw.get(c) for c in ("coeff_p", "coeff_q", "coeff_r")]
+        layer = ("h_a", "h_b", "r_a", "r_b") if norm is not None and norm["kind"] == "LayerNorm" else ()
+        dR, *rest = ops.zeros([rel.shape] + [None if c is None else c.shape for c in coeffs] + [norm[k].shape for k in layer],
+                              E.device)
+        dnorm = dict(zip(layer, rest[3:])) or None
         dcoeff = ops.build_query_backward(name, E, rel, x, dQ, dbias, dE, dR, norm=norm, dnorm=dnorm, dropout=dropout,
-                                          **self._query_kwargs())
+                                          dcoeff=rest[:3], **kw)
         grads = {"entity_embeddings.weight": dE, "relation_embeddings.weight": dR}
         if dnorm is not None:
             grads["normalize_head_entity_embeddings.weight"] = dnorm["h_a"]

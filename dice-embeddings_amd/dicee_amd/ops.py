@@ -166,10 +166,11 @@ def batchnorm_stats(ent, rel, hr, *, eps=1e-5, momentum=0.1, running=None, dropo
 
 
 def build_query_backward(model, ent, rel, hr, dQ, dbias, d_ent, d_rel, *, p=0, q=0, r=0, coeff_p=None, coeff_q=None,
-                         coeff_r=None, normalize_relation=True, norm=None, dnorm=None, dropout=None):
+                         coeff_r=None, normalize_relation=True, norm=None, dnorm=None, dropout=None, dcoeff=None):
     """Adds the gradients that ``dQ`` [B,d] / ``dbias`` [B] send back through ``build_query`` into ``d_ent`` [N,d]
     and ``d_rel`` [R,d] (fp32, caller-initialised); returns the gradients of the Clifford coefficients
-    ``(d_coeff_p, d_coeff_q, d_coeff_r)`` (None where the model has none).  ``norm``: the normalisation layer of
+    ``(d_coeff_p, d_coeff_q, d_coeff_r)`` (None where the model has none; ``dcoeff``: such a triple of zeroed tensors to
+    add them to).  ``dbias`` may be None where the bias is constant.  ``norm``: the normalisation layer of
     ``build_query``; ``dnorm``: for LayerNorm, a dict with any of ``h_a, h_b, r_a, r_b`` ([d] fp32,
     caller-initialised) that receive the gradients of the normalisers' weights and biases.  A ``norm`` that
     ``batchnorm_stats`` made for this batch (``norm["batch"]``) is differentiated as a function of the batch."""
@@ -179,7 +180,14 @@ def build_query_backward(model, ent, rel, hr, dQ, dbias, d_ent, d_rel, *, p=0, q
         if t.dtype != torch.float32 or not t.is_contiguous():
             raise TypeError("build_query_backward needs contiguous fp32 tensors")
     B, (N, d), R = hr.shape[0], ent.shape, rel.shape[0]
-    outs = [torch.zeros_like(c) if c is not None else None for c in (coeff_p, coeff_q, coeff_r)]
+    outs = dcoeff
+    if outs is None:
+        outs = [torch.zeros_like(c) if c is not None else None for c in (coeff_p, coeff_q, coeff_r)]
+    else:
+        for o, c in zip(outs, (coeff_p, coeff_q, coeff_r)):
+            if (o is None) != (c is None) or (o is not None and (o.dtype != torch.float32 or o.numel() != c.numel())):
+                raise ValueError("dcoeff must hold one float32 tensor per coefficient vector")
+        _require_gpu(*outs)
     ds, dkeep = _dropout_struct(dropout, B, d)
     dsp = ctypes.byref(ds) if ds is not None else None
     if norm is not None and norm.get("batch"):
@@ -279,6 +287,19 @@ def row_minmax(Q, bias, E, scale=None):
                             _ptr(hi), _stream())
     _lib.check(rc)
     return lo, hi
+
+
+def zeros(shapes, device):
+    """Zeroed fp32 tensors of the given shapes (None where the shape is None), cleared by one launch per eight."""
+    lib = _lib.load()
+    out = [None if s is None else torch.empty(s, dtype=torch.float32, device=device) for s in shapes]
+    todo = [t for t in out if t is not None and t.numel()]
+    for i in range(0, len(todo), 8):
+        part = todo[i:i + 8]
+        ptrs = (ctypes.c_void_p * len(part))(*[t.data_ptr() for t in part])
+        counts = (ctypes.c_int64 * len(part))(*[t.numel() for t in part])
+        _lib.check(lib.kge_fill_zero(ptrs, counts, len(part), _stream()))
+    return out
 
 
 def csr_lookup(hr, keys, num_relations):
@@ -459,9 +480,10 @@ def bce_multihot(Q, bias, E, scale, csr_row, row_ptr, col, label_smoothing=0.0):
     return loss
 
 
-def bce_multihot_backward(Q, bias, E, csr_row, row_ptr, col, label_smoothing=0.0, grad_out=1.0, want_loss=True):
+def bce_multihot_backward(Q, bias, E, csr_row, row_ptr, col, label_smoothing=0.0, grad_out=1.0, want_loss=True,
+                          want_dbias=True):
     """Gradients of ``bce_multihot`` with respect to ``Q`` [B,d], ``bias`` [B] and the fp32 table ``E`` [N,d]:
-    ``(loss or None, dQ, dbias, dE)``.  The [B,N] gradient of the scores lives only in the call's workspace."""
+    ``(loss or None, dQ, dbias or None, dE)``.  The [B,N] gradient of the scores lives only in the call's workspace."""
     lib = _lib.load()
     _require_gpu(Q, bias, E, csr_row, row_ptr, col)
     _check_qe(Q, E, None, bias)
@@ -471,7 +493,7 @@ def bce_multihot_backward(Q, bias, E, csr_row, row_ptr, col, label_smoothing=0.0
     N = E.shape[0]
     loss = torch.empty((1,), dtype=torch.float32, device=Q.device) if want_loss else None
     dQ = torch.empty((B, d), dtype=torch.float32, device=Q.device)
-    dbias = torch.empty((B,), dtype=torch.float32, device=Q.device)
+    dbias = torch.empty((B,), dtype=torch.float32, device=Q.device) if want_dbias else None
     dE = torch.empty((N, d), dtype=torch.float32, device=Q.device)
     ws_bytes = lib.kge_bce_backward_workspace_bytes(B, d, N)
     ws = torch.empty(((ws_bytes + 7) // 8,), dtype=torch.float64, device=Q.device)

@@ -177,6 +177,9 @@ int kge_build_query_backward(int model, int p, int q, int r, const float* ent, c
                              const float* dQ, const float* dbias, float* d_ent, float* d_rel, float* d_coeff_p,
                              float* d_coeff_q, float* d_coeff_r, void* stream);
 
+/* Clears n <= 8 fp32 buffers (counts[i] elements each) in one launch: the outputs that the backward adds to. */
+int kge_fill_zero(float* const* bufs, const int64_t* counts, int n, void* stream);
+
 /*
  * The same with the normalisation layer of kge_build_query between the lookups and the interaction
  * (dicee/models/base_model.py:283-294 applied at :381-383; norm as there, NULL or KGE_NORM_NONE: exactly

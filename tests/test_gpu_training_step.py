@@ -49,3 +49,43 @@ def test_query_backward_of_a_batch_is_the_sum_over_its_pairs(model, d, kw, layer
             m += g.double().abs()
     for g, w, m in zip(got, want, mass):
         assert ((g.double() - w).abs() <= B * EPS * m + 1e-30).all()
+
+
+@pytest.mark.parametrize("d", [4, 30, 64, 200])
+@pytest.mark.parametrize("eps", [0.0, 0.1])
+@pytest.mark.parametrize("want_dbias", [True, False])
+def test_bce_step_with_hub_rows_and_empty_rows(d, eps, want_dbias):
+    """Filter rows of 0, 1, 64, 65, 256, 257 and 3000 tails (a trip of the positives' kernel takes 4 per group, 64 groups per
+    query): loss, dQ, dbias, dE against float64 torch."""
+    from dicee_amd import ops
+    rng = np.random.default_rng(d)
+    N, lens = 5001, [0, 1, 64, 65, 256, 257, 3000]
+    B = len(lens) + 1
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    col = np.concatenate([np.sort(rng.choice(N, n, replace=False)) for n in lens]).astype(np.int32)
+    rows = torch.tensor(list(range(len(lens))) + [-1], device="cuda")          # the last query has no row
+    Q, E = (torch.from_numpy((rng.standard_normal(s) * 0.3).astype(np.float32)).cuda() for s in ((B, d), (N, d)))
+    bias = torch.from_numpy(rng.standard_normal(B).astype(np.float32)).cuda()
+    got = ops.bce_multihot_backward(Q, bias, E, rows, torch.from_numpy(ptr).cuda(), torch.from_numpy(col).cuda(), eps,
+                                    want_dbias=want_dbias)
+    y = torch.zeros(B, N, dtype=torch.float64, device="cuda")
+    for b, n in enumerate(lens):
+        y[b, torch.from_numpy(col[ptr[b]:ptr[b + 1]]).long().cuda()] = 1
+    if eps:
+        y = (1 - eps) * y + 1 / N
+    q, e, bb = (t.double().requires_grad_() for t in (Q, E, bias))
+    loss = torch.nn.functional.binary_cross_entropy_with_logits(q @ e.T + bb[:, None], y)
+    loss.backward()
+    assert abs(float(got[0]) - float(loss)) <= 2e-6 * abs(float(loss))
+    assert (got[2] is not None) == want_dbias
+    # each score gradient carries a few roundings of sigmoid and subtraction; a gradient is a sum of at most 5001 of them
+    for g, w in ((got[1], q.grad), (got[2], bb.grad), (got[3], e.grad)):
+        if g is not None:
+            assert float((g.double() - w).norm()) <= 1e-5 * float(w.norm())
+
+
+def test_zeros_clears_many_buffers():
+    from dicee_amd import ops
+    torch.full((3_000_000,), 7.0, device="cuda")            # (what the allocator hands out next is not zero already)
+    out = ops.zeros([(1,), None, (0, 3), (257, 3)] + [(n,) for n in range(1, 12)] + [(700001,)], "cuda")
+    assert out[1] is None and all(t is None or (t == 0).all() for t in out)
