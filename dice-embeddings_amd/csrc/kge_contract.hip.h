@@ -1682,10 +1682,18 @@ __global__ void __launch_bounds__(64 * I8_WG_WAVES, 2) qreg_i8_kernel(ContractAr
 }
 
 // ============================================================================================
-// ksplit_kernel: fp32 tables on the bf16 MFMA (split3_bf16x8).  256 entities x 128 queries per
-// workgroup of 8 waves (each wave 64 x 64), K in chunks of 32.  Both operands are loaded as fp32 into
-// registers while the previous chunk is multiplied, split into their three bf16 parts and stored as
-// three planes per operand in LDS; per 16-wide K step a wave reads 12 fragments and issues 24 MFMAs.
+// ksplit_kernel: fp32 tables on the bf16 MFMA (split3_bf16x8).  128 entities x 128 queries per workgroup of 4 waves (each
+// wave 64 x 64), two workgroups per CU, K in chunks of 32.  Both operands are loaded as fp32 into registers while the
+// previous chunk is multiplied, split into their three bf16 parts and stored as three planes per operand in LDS; per
+// 16-wide K step a wave reads 12 fragments and issues 24 MFMAs.  One LDS buffer (48 KB): a workgroup's split and store
+// stand between two barriers, and so do its first loads and its epilogue; what fills the matrix cores meanwhile is the
+// other workgroup of the CU, which is at another point of its walk.
+// Measured against 256 x 128 workgroups of 8 waves, one per CU, that split and stored the next chunk under the products
+// into a second buffer: 1000 x 40,943 scores, d = 256 157 -> 143 us; training step of 1000 x 14,541, d = 200 228 -> 220 us (the
+// score gradients 100 -> 60: half as many rows per tile, and the epilogue under another workgroup's products); at
+// 2048 x 40,943 the same within 3 %: power-limited matrix cores either way.  16-column chunks in two buffers, split under the
+// products, came out the same (step of 1000 217 us, scores 144, rank pass 1.4 % slower), and a branch around the column
+// masks slower (241): it parts the loads that should be in flight together.
 // Chain order per score: K steps of 16 ascending, inside a step the six products in SPLIT order.
 //
 // LDS plane layout: row r is 64 B = 4 pieces of 16 B (8 bf16); piece p sits in slot
@@ -1712,7 +1720,7 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
   using Epi = EpiT<KS_NQT>;
   static_assert(KMAJ == 0 || VEC, "K-major operands are loaded 16 bytes at a time");
   constexpr bool KE = (KMAJ & 1) != 0, KQ = (KMAJ & 2) != 0;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * KS_STAGE_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[KS_STAGE_BYTES];
 
   int qg;
   int64_t chunk;
@@ -1747,30 +1755,29 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
   const int n_it = n_et * nkc;
   const float* Ef = (const float*)a.E + (KE ? (int64_t)k_off * lde : (int64_t)k_off);
 
-  // Staging: a chunk is 384 rows (256 entity rows, then 128 query rows) of 128 B, taken in six passes of
-  // 64 rows; in pass g thread tid takes 16 B piece (tid & 7) of row 64 g + tid / 8, so eight neighbouring
-  // lanes read one whole 128 B line.  Loads are branch-free so that all six stay in flight: rows past the
+  // Staging: a chunk is 256 rows (128 entity rows, then 128 query rows) of 128 B, taken in eight passes of
+  // 32 rows; in pass g thread tid takes 16 B piece (tid & 7) of row 32 g + tid / 8, so eight neighbouring
+  // lanes read one whole 128 B line.  Loads are branch-free so that all eight stay in flight: rows past the
   // end repeat the last valid row (epilogues ignore them), columns past d are read from a clamped address
-  // and zeroed when stored.  Pass g of chunk i+2 is loaded right after pass g of chunk i+1 has been split
-  // and stored, both while chunk i is multiplied: one register set, and a whole iteration for a load to land.
+  // and zeroed when stored.  Chunk i+2 is loaded as soon as chunk i+1 has been split and stored, and has chunk i+1's
+  // multiplication to land.
   const int s_row = tid >> 3, s_piece = tid & 7;
   const int64_t q_last = a.B - 1, e_last = r1 - 1;
-  const float* q_ptr[2];
+  const float* q_ptr[4];
 #pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    int64_t qr = q_base + 64 * g + s_row;
+  for (int g = 0; g < 4; ++g) {
+    int64_t qr = q_base + 32 * g + s_row;
     qr = qr < q_last ? qr : q_last;
     q_ptr[g] = a.Q + k_off + qr * ldq;
   }
-  // K-major operands: pass g of the entity operand is k rows 8 g + wave of the chunk, lane l the four rows 4 l ..;
-  // pass g of the query operand k rows 16 (g - 4) + tid / 32, four rows 4 (tid % 32) ..  A quad of rows past the
-  // operand's end is read from the last quad inside the pitch instead (its scores are never stored).
-  const int ke_kk = wave, ke_mq = lane, kq_kk = tid >> 5, kq_mq = tid & 31;
+  // K-major operands: pass g of either operand is k rows 8 (g % 4) + tid / 32 of the chunk, four rows 4 (tid % 32) ..  A quad
+  // of rows past the operand's end is read from the last quad inside the pitch instead (its scores are never stored).
+  const int ke_kk = tid >> 5, ke_mq = tid & 31, kq_kk = ke_kk, kq_mq = ke_mq;
   int64_t kq_col = q_base + 4 * kq_mq;
   if (KQ) kq_col = (kq_col + 4 <= ldq) ? kq_col : ldq - 4;
   const float* Qk = a.Q + (int64_t)k_off * ldq;
   int st_k0 = 0, ld_k0 = 0;  // first k of the staged chunk, of the chunk being loaded
-  f32x4 staged[6];             // passes 0..3: entity rows, 4..5: query rows
+  f32x4 staged[8];             // passes 0..3: entity rows, 4..7: query rows
   int st_valid = 0;            // how many of this thread's four columns of the staged chunk are inside d
   int ld_valid = 0, ld_k = 0;  // the same, and the first column, for the chunk being loaded
   int ld_kc = 0;               // K chunk and first row of the tile the next loads fetch
@@ -1790,12 +1797,12 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
       return;
     }
     if (KQ && g >= 4) {
-      const int k = ld_k0 + 16 * (g - 4) + kq_kk;
+      const int k = ld_k0 + 8 * (g - 4) + kq_kk;
       staged[g] = *(const f32x4*)(Qk + (int64_t)(k < d ? k : 0) * ldq + kq_col);
       return;
     }
     if (g < 4) {
-      int64_t er = ld_row + 64 * g;
+      int64_t er = ld_row + 32 * g;
       er = er < e_last ? er : e_last;
       row_ptr = Ef + er * lde;
     } else {
@@ -1815,14 +1822,14 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
     st_valid = ld_valid;
     st_k0 = ld_k0;
   };
-  // 8-byte half (s_piece & 1) of 16-byte piece (s_piece >> 1); rows 64 g + s_row share the swizzle of s_row
+  // 8-byte half (s_piece & 1) of 16-byte piece (s_piece >> 1); rows 32 g + s_row share the swizzle of s_row
   const int st_off = s_row * 64 + ((((s_piece >> 1) ^ ((s_row >> 2) & 3)) << 4) | ((s_piece & 1) << 3));
-  auto store_pass = [&](int buf, int g) {
+  auto store_pass = [&](int g) {
     if ((KE && g < 4) || (KQ && g >= 4)) {
       const bool e_side = g < 4;
-      const int kk = e_side ? 8 * g + ke_kk : 16 * (g - 4) + kq_kk, mq = e_side ? ke_mq : kq_mq;
+      const int kk = e_side ? 8 * g + ke_kk : 8 * (g - 4) + kq_kk, mq = e_side ? ke_mq : kq_mq;
       const int pitch = e_side ? 2 * KS_TILE_ROWS : 2 * KS_WG_QUERIES, plane = e_side ? KS_E_PLANE : KS_Q_PLANE;
-      unsigned char* base = lds + buf * KS_STAGE_BYTES + (e_side ? 0 : 3 * KS_E_PLANE) + kk * pitch +
+      unsigned char* base = lds + (e_side ? 0 : 3 * KS_E_PLANE) + kk * pitch +
                             ((((mq >> 2) ^ (2 * (kk & 3))) << 5) | ((mq & 3) << 3));
       f32x4 v = staged[g];
       const bool live = st_k0 + kk < d;
@@ -1834,8 +1841,7 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
       for (int part = 0; part < 3; ++part) *(bf16x4*)(base + part * plane) = s[part];
       return;
     }
-    unsigned char* base = lds + buf * KS_STAGE_BYTES + st_off +
-                          (g < 4 ? g * 4096 : 3 * KS_E_PLANE + (g - 4) * 4096);
+    unsigned char* base = lds + st_off + (g < 4 ? g * 2048 : 3 * KS_E_PLANE + (g - 4) * 2048);
     const int plane = g < 4 ? KS_E_PLANE : KS_Q_PLANE;
     f32x4 v = staged[g];
 #pragma unroll
@@ -1873,63 +1879,47 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[te][tq][i] = 0.f;
 
-  if (n_it > 0) {
+  auto load_chunk = [&]() {  // past the last chunk the clamped addresses still point into the tables
     load_begin();
 #pragma unroll
-    for (int g = 0; g < 6; ++g) load_pass(g);
+    for (int g = 0; g < 8; ++g) load_pass(g);
     load_end();
-    load_begin();
-#pragma unroll
-    for (int g = 0; g < 6; ++g) {
-      store_pass(0, g);
-      load_pass(g);  // past the last chunk the clamped addresses still point into the tables
-    }
-    load_end();
-  }
-  __syncthreads();
+  };
+  if (n_it > 0) load_chunk();
   int kc = 0;
   int64_t et0 = r0;
+  const unsigned char* be = lds + (64 * we) * 64;
+  const unsigned char* bq = lds + 3 * KS_E_PLANE + (64 * wq) * 64;
   for (int it = 0; it < n_it; ++it) {
-    const int buf = it & 1;
-    const unsigned char* be = lds + buf * KS_STAGE_BYTES + (64 * we) * 64;
-    const unsigned char* bq = lds + buf * KS_STAGE_BYTES + 3 * KS_E_PLANE + (64 * wq) * 64;
-    bf16x8 fe[2][3][2], fq[2][3][2];
-    auto read_step = [&](int ks) {
+#pragma unroll
+    for (int g = 0; g < 8; ++g) store_pass(g);
+    __syncthreads();
+    load_chunk();
+#pragma unroll
+    for (int ks = 0; ks < KS_KC / 16; ++ks) {
+      bf16x8 fe[3][2], fq[3][2];
 #pragma unroll
       for (int part = 0; part < 3; ++part)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           if constexpr (KE)
-            fe[ks][part][t] = tr_fragment(lds + buf * KS_STAGE_BYTES + part * KS_E_PLANE, 2 * KS_TILE_ROWS, 64 * we + 32 * t, ks);
+            fe[part][t] = tr_fragment(lds + part * KS_E_PLANE, 2 * KS_TILE_ROWS, 64 * we + 32 * t, ks);
           else
-            fe[ks][part][t] = *(const bf16x8*)(be + part * KS_E_PLANE + t * 2048 + foff[ks]);
+            fe[part][t] = *(const bf16x8*)(be + part * KS_E_PLANE + t * 2048 + foff[ks]);
           if constexpr (KQ)
-            fq[ks][part][t] = tr_fragment(lds + buf * KS_STAGE_BYTES + 3 * KS_E_PLANE + part * KS_Q_PLANE,
-                                          2 * KS_WG_QUERIES, 64 * wq + 32 * t, ks);
+            fq[part][t] = tr_fragment(lds + 3 * KS_E_PLANE + part * KS_Q_PLANE, 2 * KS_WG_QUERIES, 64 * wq + 32 * t, ks);
           else
-            fq[ks][part][t] = *(const bf16x8*)(bq + part * KS_Q_PLANE + t * 2048 + foff[ks]);
+            fq[part][t] = *(const bf16x8*)(bq + part * KS_Q_PLANE + t * 2048 + foff[ks]);
         }
-    };
-    // The iteration in six slices, fenced so that each keeps its share of the work: eight of the chunk's
-    // 48 MFMAs, and the split + store of one staged pass of chunk it+1 followed by the load of that pass of
-    // chunk it+2.  Unconditional on purpose (no branches inside the iteration): after the last chunk this
-    // stores and loads a chunk nobody reads.
-    read_step(0);
-    load_begin();
 #pragma unroll
-    for (int sl = 0; sl < 6; ++sl) {
-      if (sl == 2) read_step(1);
-      store_pass(buf ^ 1, sl);
-      load_pass(sl);
+      for (int p = 0; p < SPLIT_PRODUCTS; ++p)
 #pragma unroll
-      for (int m = 8 * sl; m < 8 * sl + 8; ++m) {
-        const int ks = m / 24, p = (m % 24) / 4, te = (m >> 1) & 1, tq = m & 1;
-        acc[te][tq] = Epi::SWAP ? mfma_bf16(fq[ks][SPLIT_B[p]][tq], fe[ks][SPLIT_A[p]][te], acc[te][tq])
-                                : mfma_bf16(fe[ks][SPLIT_A[p]][te], fq[ks][SPLIT_B[p]][tq], acc[te][tq]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+        for (int te = 0; te < 2; ++te)
+#pragma unroll
+          for (int tq = 0; tq < 2; ++tq)
+            acc[te][tq] = Epi::SWAP ? mfma_bf16(fq[SPLIT_B[p]][tq], fe[SPLIT_A[p]][te], acc[te][tq])
+                                    : mfma_bf16(fe[SPLIT_A[p]][te], fq[SPLIT_B[p]][tq], acc[te][tq]);
     }
-    load_end();
     if (kc == nkc - 1) {  // this entity tile is complete
       float sc16[16];
 #pragma unroll
@@ -1951,19 +1941,19 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
       if (Epi::STAGE_HOOK) epi.stage_end();
     } else {
       ++kc;
-      __syncthreads();
+      __syncthreads();  // the buffer has been read
     }
   }
   epi.finish();
 }
 
 template <template <int> class EpiT, bool VEC>
-__global__ void __launch_bounds__(512, 2) ksplit_kernel(ContractArgs a, typename EpiT<KS_NQT>::Args ea) {
+__global__ void __launch_bounds__(256, 2) ksplit_kernel(ContractArgs a, typename EpiT<KS_NQT>::Args ea) {
   ksplit_body<EpiT, VEC, 0>(a, ea);
 }
 // the same with K-major operands (KMAJ = 1: the entity operand, 3: both)
 template <template <int> class EpiT, int KMAJ>
-__global__ void __launch_bounds__(512, 2) ksplit_kmajor_kernel(ContractArgs a, typename EpiT<KS_NQT>::Args ea) {
+__global__ void __launch_bounds__(256, 2) ksplit_kmajor_kernel(ContractArgs a, typename EpiT<KS_NQT>::Args ea) {
   ksplit_body<EpiT, true, KMAJ>(a, ea);
 }
 
@@ -1978,8 +1968,9 @@ __global__ void __launch_bounds__(512, 2) ksplit_kmajor_kernel(ContractArgs a, t
 //
 // LDS row: 128 B = 8 pieces of 16 B (8 bf16); piece p of row r sits in slot r*8 + (p ^ (r & 7)).
 // ============================================================================================
+using host::KB_TILE_ROWS;
 constexpr int KB_KC = 64;
-constexpr int KB_E_PLANE = KS_TILE_ROWS * 128;
+constexpr int KB_E_PLANE = KB_TILE_ROWS * 128;
 constexpr int KB_Q_PLANE = KS_WG_QUERIES * 128;
 constexpr int KB_STAGE_BYTES = KB_E_PLANE + KB_Q_PLANE;
 
@@ -2007,7 +1998,7 @@ __global__ void __launch_bounds__(512, 2) kchunk_kernel(ContractArgs a, typename
   const int64_t r0 = a.e_begin + chunk * a.chunk_rows;
   const int64_t r1 = (r0 + a.chunk_rows < a.e_end) ? r0 + a.chunk_rows : a.e_end;
   const int nkc = (d + KB_KC - 1) / KB_KC;
-  const int n_et = (int)((r1 - r0 + KS_TILE_ROWS - 1) / KS_TILE_ROWS);
+  const int n_et = (int)((r1 - r0 + KB_TILE_ROWS - 1) / KB_TILE_ROWS);
   const int n_it = n_et * nkc;
   const unsigned char* Eb = (const unsigned char*)a.E;
   constexpr int ESZ = I8 ? 1 : 2;  // bytes per table element
@@ -2062,7 +2053,7 @@ __global__ void __launch_bounds__(512, 2) kchunk_kernel(ContractArgs a, typename
     }
     if (ld_kc == nkc - 1) {  // (uniform)
       ld_kc = 0;
-      ld_row += KS_TILE_ROWS;
+      ld_row += KB_TILE_ROWS;
       tile_rows();
     } else {
       ++ld_kc;
@@ -2163,7 +2154,7 @@ __global__ void __launch_bounds__(512, 2) kchunk_kernel(ContractArgs a, typename
           for (int i = 0; i < 16; ++i) acc[te][tq][i] = 0.f;
       }
       kc = 0;
-      et0 += KS_TILE_ROWS;
+      et0 += KB_TILE_ROWS;
       if (Epi::STAGE_HOOK) epi.stage_mark();
       __syncthreads();
       if (Epi::STAGE_HOOK) epi.stage_end();

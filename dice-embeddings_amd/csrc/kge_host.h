@@ -36,7 +36,9 @@ constexpr int TOPK_MAX_K = 1024;
 constexpr int TOPK_FIRST_ROWS = 1024;    // first round takes everything: must not exceed TOPK_CAP
 constexpr int BCE_SLOTS = 128;
 constexpr int KS_WG_QUERIES = 128;       // workgroup shape of the fp32 contraction (also sizes the backward's K split)
-constexpr int KS_TILE_ROWS = 256;
+constexpr int KS_TILE_ROWS = 128;
+constexpr int KS_WGS = 512;              // workgroups of that shape the chip holds: two per CU
+constexpr int KB_TILE_ROWS = 256;        // entity rows of the bf16 / int8 contraction of wide rows, one workgroup per CU
 
 // Work decomposition of the four-tile filtered-rank main loop (bf16 tables, d == 128): 8-wave workgroups of
 // 4 x 32 queries per wave, one per CU; the workgroups resident on one XCD (32) are shared out among the query
@@ -292,9 +294,9 @@ inline BwdPlan bwd_plan(int64_t B, int64_t d, int64_t N) {
   BwdPlan p{};
   p.ldG = (N + 31) / 32 * 32;  // rows start on 128-byte lines: a wave's run of 32 gradients is one whole line
   p.ldT = (B + 3) / 4 * 4;
-  // dQ = G . E sums over N: split so that about 256 workgroups run
+  // dQ = G . E sums over N: split so that about KS_WGS workgroups run
   const int64_t tiles = ((B + KS_WG_QUERIES - 1) / KS_WG_QUERIES) * ((d + KS_TILE_ROWS - 1) / KS_TILE_ROWS);
-  int64_t splits = (256 + tiles - 1) / tiles;
+  int64_t splits = (KS_WGS + tiles - 1) / tiles;
   if (splits > 64) splits = 64;
   if (splits < 1) splits = 1;
   const int64_t len = ((N + splits - 1) / splits + 31) / 32 * 32;

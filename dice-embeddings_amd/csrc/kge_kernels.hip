@@ -1198,12 +1198,12 @@ ContractArgs make_args(const float* Q, const void* E, int dtype, const float* sc
     a.persistent = 1;
     return a;
   }
-  // non-persistent paths (the split kernel and kchunk_kernel: 8-wave workgroups of 256 entity rows, one per CU): one
+  // non-persistent paths (the split kernel: 128 entity rows, two workgroups per CU; kchunk_kernel: 256, one): one
   // workgroup per (query group, chunk), `resident` workgroups at a time; choose the chunk length whose last round of
   // workgroups is fullest, preferring longer chunks (less per-workgroup set-up) among near-equal candidates.
-  const int tile = KS_TILE_ROWS;
+  const int tile = dtype == KGE_F32 ? KS_TILE_ROWS : host::KB_TILE_ROWS;
   const int max_chunk = 1024;
-  const int64_t resident = 256;
+  const int64_t resident = dtype == KGE_F32 ? host::KS_WGS : 256;
   int64_t best_chunk = tile;
   double best_eff = -1.0;
   for (int64_t chunk = tile; chunk <= max_chunk; chunk += tile) {
@@ -1284,7 +1284,8 @@ int launch_contract(int dtype, const ContractArgs& a, const EArgs& ea, hipStream
   KGE_REQUIRE(nwg <= 0x7fffffffLL, KGE_ERR_INVALID, "%s: grid of %lld workgroups too large", name, (long long)nwg);
   const bool f32_split = (dtype == KGE_F32);
   const bool wide_bf16 = (dtype == KGE_BF16 || dtype == KGE_I8) && rc.lds_d == 0 && !wide_q;
-  dim3 grid((unsigned)nwg), block(fast_i8 ? 64 * I8_WG_WAVES : wide_q ? 64 * QW_WG_WAVES : persistent ? 64 * QA_WG_WAVES : 512);
+  dim3 grid((unsigned)nwg), block(fast_i8 ? 64 * I8_WG_WAVES : wide_q ? 64 * QW_WG_WAVES : persistent ? 64 * QA_WG_WAVES
+                                         : f32_split ? 256 : 512);
   LaunchTimer timer;
   if (int trc = timer.begin(st)) return trc;
   char kname[160];  // the kernel as dispatched below, for kge_profile_kernel()
@@ -1406,7 +1407,7 @@ int launch_ksplit(const ContractArgs& a, const EArgs& ea, unsigned k_splits, hip
   const int ldq = a.ldq ? a.ldq : a.d, lde = a.lde ? a.lde : a.d;
   const bool rows_aligned = (ldq % 4 == 0) && (lde % 4 == 0) && (((uintptr_t)a.E | (uintptr_t)a.Q) % 16 == 0) &&
                             (a.k_split_len % 4 == 0);
-  dim3 grid((unsigned)nwg, k_splits), block(512);
+  dim3 grid((unsigned)nwg, k_splits), block(256);
   LaunchTimer timer;
   if (int trc = timer.begin(st)) return trc;
   if constexpr (std::is_same<EpiT<KS_NQT>, StoreEpi<KS_NQT>>::value || std::is_same<EpiT<KS_NQT>, StoreTEpi<KS_NQT>>::value) {
