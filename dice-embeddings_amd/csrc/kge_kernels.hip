@@ -293,6 +293,59 @@ constexpr int FIX_ITEMS = 16;  // work items a workgroup resolves side by side
 // streams them, 16 lanes per row straight into LDS (whole 128-byte lines per request) in the swizzled stage
 // layout, and the MFMA fragments are read from there; the generic path reads every row 16 bytes per lane at
 // a stride, which costs four requests per line.
+// A work item of at most 32 entities whose members all hold one query vector, by one wave: the entities' scores stay in
+// its registers (every column of the result tile holds the query), and column c counts for member c.
+constexpr int FIX_SMALL = 32;
+template <int EDT>
+__device__ __forceinline__ void filter_fix_small(const ContractArgs& a, const FixPlan& plan, int64_t b0, const int32_t* col,
+                                                 const int64_t* target, const float* thr, int32_t* n_gt, int32_t* n_eq,
+                                                 int32_t* n_eql, int i0, int m, int64_t z0, int n, int c, int hf) {
+  int32_t e = c < n ? col[z0 + c] : -1;
+  if (e < 0 || (int64_t)e >= a.N) e = -1;
+  const int64_t bq = b0 + (int64_t)host::plan_key_pos(plan.skey[i0]);
+  // the first members' thresholds and targets travel beside the rows
+  int64_t b = 0, t = 0;
+  float th = 0.f;
+  auto member = [&](int mi) {
+    if (mi < m) {
+      b = b0 + (int64_t)host::plan_key_pos(plan.skey[i0 + mi]);
+      th = thr[b];
+      t = target[b];
+    }
+  };
+  member(c);
+  float sc = 1.f;
+  if (EDT == KGE_I8 && e >= 0) sc = a.scale[e];
+  const f32x16 acc = chain_direct<EDT>(a.E, a.d, e, a.Q, bq, hf);
+  for (int m0 = 0; m0 < m; m0 += 32) {
+    const int mi = m0 + c;
+    if (m0) member(mi);
+    int g = 0, eq = 0, eql = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = row_of(i, hf);
+      const int32_t er = __shfl(e, r, 64);
+      float s = acc[i];
+      if (EDT == KGE_I8) s *= __shfl(sc, r, 64);
+      if (er >= 0 && (int64_t)er != t) {
+        g += (s > th) ? 1 : 0;
+        if (s == th) {
+          eq += 1;
+          eql += ((int64_t)er < t) ? 1 : 0;
+        }
+      }
+    }
+    g += __shfl_xor(g, 32, 64);
+    eq += __shfl_xor(eq, 32, 64);
+    eql += __shfl_xor(eql, 32, 64);
+    if (hf == 0 && mi < m) {
+      if (g) atomicSub(&n_gt[b], g);
+      if (eq) atomicSub(&n_eq[b], eq);
+      if (eql) atomicSub(&n_eql[b], eql);
+    }
+  }
+}
+
 template <int EDT, bool ROWS256>
 __global__ void __launch_bounds__(256) filter_fix_kernel(ContractArgs a, FixPlan plan, int64_t b0,
                                                         const int64_t* row_ptr, const int32_t* col,
@@ -353,7 +406,22 @@ __global__ void __launch_bounds__(256) filter_fix_kernel(ContractArgs a, FixPlan
       }
     }
     __syncthreads();
+    // Most groups are a few queries on a row of a few entities (4827 groups of 16 entries on average for 8192 queries of
+    // a 14.5k graph): an item is then one chain of dependent loads and one tile, and the workgroup's four waves take
+    // such items side by side instead of waiting for one of them in turn (that batch, ComplEx d = 200: 119 -> 87 us; a
+    // pass of 20,000 queries 1394 -> 1323; heads and tails of 5000 triples, int8 d = 240, 1265 -> 1258).
+    // (Not where rows are gathered through LDS, bf16 d = 128: there the second set of registers costs more.)
+    auto small = [&](int kk) {
+      return !ROWS256 && it_z1[kk] - it_z0[kk] <= FIX_SMALL && (it_m[kk] == 1 || it_mixed[kk] == 0);
+    };
+    if constexpr (!ROWS256) {
+      for (int kk = wave; kk < FIX_ITEMS && blockIdx.x + (int64_t)(k0 + kk) * gridDim.x < n_work; kk += 4)
+        if (small(kk))
+          filter_fix_small<EDT>(a, plan, b0, col, target, thr, n_gt, n_eq, n_eql, it_i0[kk], it_m[kk], it_z0[kk],
+                                (int)(it_z1[kk] - it_z0[kk]), c, hf);
+    }
   for (int kk = 0; kk < FIX_ITEMS && blockIdx.x + (int64_t)(k0 + kk) * gridDim.x < n_work; ++kk) {
+    if (small(kk)) continue;  // (the same for the workgroup)
     const int i0 = it_i0[kk];
     const int m = it_m[kk];
     const int64_t z0 = it_z0[kk], z1 = it_z1[kk];
