@@ -13,7 +13,7 @@ import numpy as np
 import torch
 
 from .csr import FilterCSR
-from .evaluator import rank_in_batches
+from .evaluator import check_triple_ids, rank_in_batches
 
 
 def _as_csr(vocab, key_mult, device):
@@ -53,16 +53,14 @@ def evaluate_lp(model, triple_idx, num_entities=None, er_vocab=None, re_vocab=No
     if triple_idx.ndim != 2 or triple_idx.shape[1] != 3:
         raise ValueError("triple_idx must have shape [n, 3]")
     n = len(triple_idx)
-    if n and (triple_idx[:, [0, 2]].min() < 0 or triple_idx[:, [0, 2]].max() >= N or triple_idx[:, 1].min() < 0
-              or triple_idx[:, 1].max() >= R):
-        raise IndexError("triple_idx holds an entity or relation id outside the model's tables")
+    ids = check_triple_ids(triple_idx, N, R)
     if info:
         print(info)
         print(f"Num of triples {n}")
     dev = model.entity_embeddings.weight.device
     er = _as_csr(er_vocab, R, dev)
     re = _as_csr(re_vocab, N, dev)
-    trip = torch.from_numpy(np.ascontiguousarray(triple_idx.astype(np.int64))).to(dev)
+    trip = torch.from_numpy(ids).to(dev)
     tail_ranks = rank_in_batches(model, trip[:, :2], trip[:, 2], er, batch_size, tie, streams)
     head_ranks = rank_in_batches(model, trip[:, 1:], trip[:, 0], re, batch_size, tie, streams, heads=True)
     hr_, tr_ = head_ranks.cpu().numpy(), tail_ranks.cpu().numpy()
