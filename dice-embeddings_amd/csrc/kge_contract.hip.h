@@ -207,6 +207,100 @@ __device__ __forceinline__ f32x16 chain_direct(const void* E, int d, int64_t e_r
   return acc;
 }
 
+// The same tile for ONE query in all 32 columns, its row kept in LDS as MFMA fragments by the whole workgroup (a lane's
+// fragment depends on its half alone: [K step][part][half] of 16 bytes): rescoring the rows of a list for one query then
+// neither loads nor splits the query again for every tile, which is half the work of a tile of fp32 rows.
+constexpr int QUERY_LDS_MAX_D = 1024;
+constexpr int query_lds_bytes(int edt, int d) { return (d + 15) / 16 * (edt == KGE_F32 ? 3 : 1) * 32; }
+template <int EDT>
+__device__ __forceinline__ void query_to_lds(const float* q_row, int d, unsigned char* lds, int tid, int threads) {
+  const int n = (d + 15) / 16 * 2;
+  for (int i = tid; i < n; i += threads) {
+    const int s = i >> 1, k = 16 * s + 8 * (i & 1);
+    f32x4 lo, hi;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      lo[j] = k + j < d ? q_row[k + j] : 0.f;
+      hi[j] = k + 4 + j < d ? q_row[k + 4 + j] : 0.f;
+    }
+    if constexpr (EDT == KGE_F32) {
+      bf16x8 p[3];
+      split3_bf16x8(lo, hi, p);
+#pragma unroll
+      for (int part = 0; part < 3; ++part) *(bf16x8*)(lds + ((s * 3 + part) * 2 + (i & 1)) * 16) = p[part];
+    } else {
+      *(bf16x8*)(lds + i * 16) = cvt_bf16x8(lo, hi);
+    }
+  }
+}
+template <int EDT>
+__device__ __forceinline__ f32x16 chain_one_query(const void* E, int d, int64_t e_row, const unsigned char* lds, int hf) {
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  const bool ok = e_row >= 0;
+  const int64_t row = ok ? e_row : 0;
+  const int nks = (d + 15) >> 4;
+  if (EDT == KGE_F32) {
+    const float* p = (const float*)E + row * d;
+    const bool vec_ok = (d & 3) == 0;
+    for (int ks0 = 0; ks0 < nks; ks0 += 4) {
+      f32x4 fe[4][2];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = (ks0 + u) * 16 + 8 * hf + 4 * h;
+          if (vec_ok) {
+            fe[u][h] = *(const f32x4*)(p + (k < d ? k : 0));
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) fe[u][h][j] = p[k + j < d ? k + j : 0];
+          }
+        }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (ks0 + u < nks) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int k = (ks0 + u) * 16 + 8 * hf + 4 * h;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) fe[u][h][j] = (ok && k + j < d) ? fe[u][h][j] : 0.f;
+          }
+          bf16x8 se[3], sq[3];
+          split3_bf16x8(fe[u][0], fe[u][1], se);
+#pragma unroll
+          for (int part = 0; part < 3; ++part) sq[part] = *(const bf16x8*)(lds + (((ks0 + u) * 3 + part) * 2 + hf) * 16);
+#pragma unroll
+          for (int q = 0; q < SPLIT_PRODUCTS; ++q) acc = mfma_bf16(se[SPLIT_A[q]], sq[SPLIT_B[q]], acc);
+        }
+      }
+    }
+  } else {
+    for (int s0 = 0; s0 < nks; s0 += 8) {
+      u32x4 ev[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int k = 16 * (s0 + u) + 8 * hf;
+        ev[u] = u32x4{0u, 0u, 0u, 0u};
+        if (ok && k < d) {
+          if (EDT == KGE_BF16) {
+            ev[u] = *(const u32x4*)((const uint16_t*)E + row * d + k);
+          } else {
+            const u32x2 w = *(const u32x2*)((const int8_t*)E + row * d + k);
+            ev[u] = i8x8_to_bf16x8(w[0], w[1]);
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (s0 + u < nks)
+          acc = mfma_bf16(__builtin_bit_cast(bf16x8, ev[u]), *(const bf16x8*)(lds + ((s0 + u) * 2 + hf) * 16), acc);
+    }
+  }
+  return acc;
+}
+
 // XCD-aware decomposition of a flat workgroup id: hardware deals consecutive ids round-robin over
 // the 8 XCDs, so ids with the same (id % 8) share an L2.  Consecutive slots on one XCD walk the
 // query groups of ONE entity chunk, which keeps that chunk's rows hot in that XCD's L2.

@@ -27,22 +27,35 @@ struct FewArgs {
   const float* Q;
   const void* E;
   const float* scale;
-  const float* bias;  // STORE only
-  float* out;         // STORE: scores [B, ldo]; else the maximum over every 32-row tile [B, ldo]
-  int64_t ldo, N, n_tiles;
+  const float* bias;  // FEW_STORE only
+  float* out;         // FEW_STORE: scores [B, ldo]; else the maximum over every 32-row tile [B, ldo]
+  float* runs;        // FEW_MAX with tpw = 8: the maximum over every run of eight tiles [B, ldo / 8]
+  float* raw;         // FEW_MAX_RAW: the scores themselves too, without a bias [B, ldr], whole tiles
+  int64_t ldo, ldr, N, n_tiles;
   int B, d, nks;
   int tpw;  // consecutive tiles a wave takes at a time
 };
 
-// One wave at a time: 32-row tiles, their rows as MFMA operands straight from memory (lane (c, hf) reads its 16 or 32
-// bytes of row c; four K steps of a bf16 row, two of an fp32 row make a 128-byte line, requested back to back), the
-// loads of one chunk of K steps in flight while the chunk before is multiplied, across tiles.
-template <int EDT, int QT, bool STORE>
+// One wave at a time: chunks of a 32-row tile, 128 (bf16: 256) bytes of every row, loaded as whole lines into registers
+// (eight or sixteen lanes per row), put into the wave's own LDS (16-byte piece p of row r at p ^ (r & 7 or 15)) and read back as MFMA
+// operands; the next chunk's loads are in flight while a chunk is multiplied, across tiles, and no wave waits for another.
+// (Operands loaded straight from memory, each lane its 16 or 32 bytes of a row: every request touches 32 lines, four
+// requests share them, and a CU's waves push each other's lines out of the L1 in between: bf16 d = 128, N = 2.5M 152 us against 143, int8 N = 10M
+// whole calls of 32 queries 507 against 382.)
+constexpr int few_stage_bytes(int edt) { return edt == KGE_BF16 ? 8192 : 4096; }
+enum FewMode { FEW_MAX, FEW_MAX_RAW, FEW_STORE };
+constexpr int FEW_RUN = 8;  // tiles of a run whose maxima go out together
+template <int EDT, int QT, int MODE>
 __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_scan_kernel(FewArgs a) {
   constexpr int PARTS = EDT == KGE_F32 ? 3 : 1;
-  constexpr int CH = EDT == KGE_F32 ? 4 : 8;  // K steps per chunk: eight 16-byte loads (int8: eight of 8 bytes)
+  constexpr int CH = EDT == KGE_F32 ? 2 : 8;            // K steps per chunk: a line of an fp32 or int8 row, two of a bf16 row
+  constexpr int PIECES = EDT == KGE_BF16 ? 16 : 8;       // 16-byte pieces of a row's chunk
+  constexpr int RPL = 64 / PIECES, NLD = 32 / RPL;       // rows per wave-wide load, loads per chunk
+  constexpr int PER_PIECE = EDT == KGE_F32 ? 4 : EDT == KGE_BF16 ? 8 : 16;  // elements
+  constexpr bool STORE = MODE == FEW_STORE;
   extern __shared__ __attribute__((aligned(16))) unsigned char fq_lds[];
-  __shared__ float s_bias[32 * QT];
+  __shared__ float s_bias[STORE ? 32 * QT : 1];
+  __shared__ __attribute__((aligned(16))) float s_max[MODE == FEW_MAX ? 4 * 32 * QT * FEW_RUN : 4];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q0 = (int)blockIdx.y * (32 * QT);
@@ -71,10 +84,10 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
   }
   __syncthreads();
 
-  struct Chunk {
-    u32x4 v[CH * (EDT == KGE_F32 ? 2 : 1)];  // (int8: the low halves)
-    f32x4 sc[EDT == KGE_I8 ? 4 : 1];
-  };
+  unsigned char* stage = fq_lds + (size_t)QT * nks * PARTS * 1024 + wave * few_stage_bytes(EDT);
+  u32x4 staged[NLD];
+  f32x4 next_sc[EDT == KGE_I8 ? 4 : 1], sc[EDT == KGE_I8 ? 4 : 1];  // int8: row scales of the chunk loaded, multiplied
+  const int l_row = lane / PIECES, l_piece = lane % PIECES;
   const int nch = (nks + CH - 1) / CH;
   int64_t unit = blockIdx.x, tile = (unit * 4 + wave) * a.tpw;
   int ch = 0, in_unit = 0;
@@ -89,39 +102,47 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
       tile = (unit * 4 + wave) * a.tpw;
     }
   };
-  auto load = [&](Chunk& x) {
-    int64_t row = tile * 32 + c;
-    row = row < a.N ? row : a.N - 1;  // rows past the end repeat the last one; the epilogues ignore them
+  constexpr int64_t ELEM = EDT == KGE_F32 ? 4 : EDT == KGE_BF16 ? 2 : 1;
+  auto load = [&]() {
+    int k = ch * CH * 16 + l_piece * PER_PIECE;
+    k = k < d ? k : 0;  // (pieces past the row's end: any valid address, their columns are zeroed below)
+    const unsigned char* base = (const unsigned char*)a.E + k * ELEM;
 #pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const int k = (ch * CH + u) * 16 + 8 * hf;
-      if constexpr (EDT == KGE_F32) {
-        const float* p = (const float*)a.E + row * d;
-        x.v[2 * u] = *(const u32x4*)(p + (k < d ? k : 0));
-        x.v[2 * u + 1] = *(const u32x4*)(p + (k + 4 < d ? k + 4 : 0));
-      } else if constexpr (EDT == KGE_BF16) {
-        x.v[u] = *(const u32x4*)((const uint16_t*)a.E + row * d + (k < d ? k : 0));
-      } else {
-        const u32x2 w = *(const u32x2*)((const int8_t*)a.E + row * d + (k < d ? k : 0));
-        x.v[u][0] = w[0];
-        x.v[u][1] = w[1];
-      }
+    for (int i = 0; i < NLD; ++i) {
+      int64_t row = tile * 32 + i * RPL + l_row;
+      row = row < a.N ? row : a.N - 1;  // rows past the end repeat the last one; the epilogues ignore them
+      staged[i] = *(const u32x4*)(base + row * d * ELEM);
     }
     if constexpr (EDT == KGE_I8) {
-      if (STORE) {
-        x.sc[0][0] = a.scale[row];
-      } else if (ch == nch - 1) {
+      if (ch == nch - 1) {
+        if (STORE) {
+          next_sc[0][0] = a.scale[tile * 32 + c < a.N ? tile * 32 + c : a.N - 1];
+        } else {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int64_t e = tile * 32 + 8 * g + 4 * hf;
+          for (int g = 0; g < 4; ++g) {
+            const int64_t e = tile * 32 + 8 * g + 4 * hf;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) x.sc[g][j] = a.scale[e + j < a.N ? e + j : a.N - 1];
+            for (int j = 0; j < 4; ++j) next_sc[g][j] = a.scale[e + j < a.N ? e + j : a.N - 1];
+          }
         }
       }
     }
   };
+  auto store = [&]() {
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const int row = i * RPL + l_row;
+      *(u32x4*)(stage + (row * PIECES + (l_piece ^ (row & (PIECES - 1)))) * 16) = staged[i];
+    }
+    if constexpr (EDT == KGE_I8) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) sc[g] = next_sc[g];
+    }
+  };
+  auto piece = [&](int p) -> const unsigned char* { return stage + (c * PIECES + (p ^ (c & (PIECES - 1)))) * 16; };
   f32x16 acc[QT];
-  auto multiply = [&](Chunk& x, int64_t t_tile, int t_ch) {
+  float run_max[QT];  // FEW_MAX with tpw = FEW_RUN
+  auto multiply = [&](int64_t t_tile, int t_ch) {
     if (t_ch == 0) {
 #pragma unroll
       for (int t = 0; t < QT; ++t)
@@ -135,7 +156,7 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
         const int k = 16 * s + 8 * hf;
         bf16x8 fe[PARTS];
         if constexpr (EDT == KGE_F32) {
-          f32x4 lo = __builtin_bit_cast(f32x4, x.v[2 * u]), hi = __builtin_bit_cast(f32x4, x.v[2 * u + 1]);
+          f32x4 lo = *(const f32x4*)piece(4 * u + 2 * hf), hi = *(const f32x4*)piece(4 * u + 2 * hf + 1);
           if (16 * s + 16 > d) {  // the row's last, partial step: its columns past d are zeros, whatever was read
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -148,8 +169,13 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
 #pragma unroll
           for (int part = 0; part < 3; ++part) fe[part] = p[part];
         } else {
-          u32x4 w = x.v[u];
-          if constexpr (EDT == KGE_I8) w = i8x8_to_bf16x8(w[0], w[1]);
+          u32x4 w;
+          if constexpr (EDT == KGE_I8) {
+            const u32x2 b = *(const u32x2*)(piece(u) + 8 * hf);
+            w = i8x8_to_bf16x8(b[0], b[1]);
+          } else {
+            w = *(const u32x4*)piece(2 * u + hf);
+          }
           if (16 * s + 16 > d && k >= d) w = u32x4{0u, 0u, 0u, 0u};
           fe[0] = __builtin_bit_cast(bf16x8, w);
         }
@@ -180,47 +206,73 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
           for (int i = 0; i < 16; ++i) {
             const int r = 32 * t + row_of(i, hf);
             if (q0 + r < a.B) {
-              const float v = EDT == KGE_I8 ? acc[t][i] * x.sc[0][0] : acc[t][i];
+              const float v = EDT == KGE_I8 ? acc[t][i] * sc[0][0] : acc[t][i];
               a.out[(int64_t)(q0 + r) * a.ldo + e] = v + s_bias[r];
             }
           }
       }
     } else {
       const bool whole = t_tile * 32 + 32 <= a.N;
+      const bool in_runs = MODE == FEW_MAX && a.tpw == FEW_RUN;
+      const int at = (int)(t_tile & (FEW_RUN - 1));
 #pragma unroll
       for (int t = 0; t < QT; ++t) {
         float m = __uint_as_float(0xff800000u);  // (a NaN score never becomes the maximum)
+        const int q = q0 + 32 * t + c;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          float v = acc[t][i];
-          if constexpr (EDT == KGE_I8) v *= x.sc[i >> 2][i & 3];
-          if (!whole && t_tile * 32 + row_of(i, hf) >= a.N) v = __uint_as_float(0xff800000u);
-          m = __builtin_fmaxf(m, v);
+        for (int g = 0; g < 4; ++g) {
+          f32x4 v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            v[r] = acc[t][4 * g + r];
+            if constexpr (EDT == KGE_I8) v[r] *= sc[g][r];
+            if (!whole && t_tile * 32 + 8 * g + 4 * hf + r >= a.N) v[r] = __uint_as_float(0xff800000u);
+            m = __builtin_fmaxf(m, v[r]);
+          }
+          if constexpr (MODE == FEW_MAX_RAW) {
+            if (q < a.B) *(f32x4*)(a.raw + (int64_t)q * a.ldr + t_tile * 32 + 8 * g + 4 * hf) = v;
+          }
         }
         m = __builtin_fmaxf(m, __shfl_xor(m, 32, 64));
-        const int q = q0 + 32 * t + c;
-        if (hf == 0 && q < a.B) a.out[(int64_t)q * a.ldo + t_tile] = m;
+        if (in_runs) {
+          if (hf == 0) s_max[(wave * 32 * QT + 32 * t + c) * FEW_RUN + at] = m;
+          run_max[t] = at == 0 ? m : __builtin_fmaxf(run_max[t], m);
+        } else if (hf == 0 && q < a.B) {
+          a.out[(int64_t)q * a.ldo + t_tile] = m;
+        }
+      }
+      if constexpr (MODE == FEW_MAX) {
+        // a run's maxima together, 32 bytes per query (one by one, 4 bytes to each of 32 rows, they cost a sixth of the
+        // scan); what lies past the last tile is never read
+        if (in_runs && (at == FEW_RUN - 1 || t_tile == a.n_tiles - 1)) {
+          wave_sync();
+          const int64_t run = t_tile / FEW_RUN;
+          for (int i = lane; i < 32 * QT * 2; i += 64) {
+            const int q = q0 + (i >> 1);
+            const f32x4 v = *(const f32x4*)(s_max + (wave * 32 * QT + (i >> 1)) * FEW_RUN + 4 * (i & 1));
+            if (q < a.B) *(f32x4*)(a.out + (int64_t)q * a.ldo + run * FEW_RUN + 4 * (i & 1)) = v;
+          }
+#pragma unroll
+          for (int t = 0; t < QT; ++t)
+            if (hf == 0 && q0 + 32 * t + c < a.B) a.runs[(int64_t)(q0 + 32 * t + c) * (a.ldo / FEW_RUN) + run] = run_max[t];
+          wave_sync();
+        }
       }
     }
   };
   if (tile >= a.n_tiles) return;
-  Chunk x0, x1;
-  load(x0);
+  load();
   for (;;) {
-    int64_t t_tile = tile;
-    int t_ch = ch;
+    store();
+    wave_sync();
+    const int64_t t_tile = tile;
+    const int t_ch = ch;
     advance();
-    const bool more1 = tile < a.n_tiles;
-    if (more1) load(x1);
-    multiply(x0, t_tile, t_ch);
-    if (!more1) break;
-    t_tile = tile;
-    t_ch = ch;
-    advance();
-    const bool more0 = tile < a.n_tiles;
-    if (more0) load(x0);
-    multiply(x1, t_tile, t_ch);
-    if (!more0) break;
+    const bool more = tile < a.n_tiles;
+    if (more) load();
+    multiply(t_tile, t_ch);
+    wave_sync();
+    if (!more) break;
   }
 }
 
@@ -243,20 +295,17 @@ __device__ __forceinline__ uint32_t score_key(float v) {
 // The positions of the k largest of vals[0 .. M) (ties: the lower positions; zeros never), ascending, into pos; returns
 // how many.  M <= 16 * FEW_THREADS.  The k-th largest value is found two bits at a time, three counts per step, by the
 // whole workgroup; a step that splits off exactly k ends the search.
-__device__ int block_select(const uint32_t* vals, int M, int k, int* pos, SelectShared& sh) {
+template <int V>
+__device__ int block_select_of(const uint32_t* vals, int M, int k, int* pos, SelectShared& sh) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int V = (M + FEW_THREADS - 1) / FEW_THREADS;
   __syncthreads();  // vals is complete; sh and pos are free
   if (tid < 16) sh.cnt[tid] = 0;
-  uint32_t v[16];
+  uint32_t v[V];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    v[j] = 0;
-    if (j < V) {
-      const int p = j * FEW_THREADS + tid;
-      if (p < M) v[j] = vals[p];
-    }
+  for (int j = 0; j < V; ++j) {
+    const int p = j * FEW_THREADS + tid;
+    v[j] = p < M ? vals[p] : 0u;
   }
   __syncthreads();
   uint32_t th = 0;
@@ -265,8 +314,7 @@ __device__ int block_select(const uint32_t* vals, int M, int k, int* pos, Select
     const uint32_t t1 = th | (1u << b), t2 = th | (2u << b), t3 = th | (3u << b);
     int c1 = 0, c2 = 0, c3 = 0;
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
-      if (j < V) {
+    for (int j = 0; j < V; ++j) {
         c1 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] >= t1));
         c2 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] >= t2));
         c3 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] >= t3));
@@ -291,8 +339,7 @@ __device__ int block_select(const uint32_t* vals, int M, int k, int* pos, Select
   const uint32_t above = exact ? th - 1 : th;  // (exact only with th > 0)
   const uint32_t at = exact ? 0u : th;         // 0: none
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
-    if (j < V) {
+  for (int j = 0; j < V; ++j) {
       const int ng = __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] > above));
       const int ne = __builtin_popcountll(__builtin_amdgcn_ballot_w64(at != 0 && v[j] == at));
       if (lane == 0) sh.scan[j * 16 + wave] = (uint32_t)ng | ((uint32_t)ne << 16);
@@ -327,8 +374,7 @@ __device__ int block_select(const uint32_t* vals, int M, int k, int* pos, Select
   const int need = n_eq < k - n_gt ? n_eq : k - n_gt;
   const unsigned long long below_lane = (1ull << lane) - 1;
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
-    if (j < V) {
+  for (int j = 0; j < V; ++j) {
       const unsigned long long bg = __builtin_amdgcn_ballot_w64(v[j] > above);
       const unsigned long long be = __builtin_amdgcn_ballot_w64(at != 0 && v[j] == at);
       const uint32_t base = sh.scan[j * 16 + wave];
@@ -339,6 +385,11 @@ __device__ int block_select(const uint32_t* vals, int M, int k, int* pos, Select
   __syncthreads();
   return n_gt + need;
 }
+__device__ __forceinline__ int block_select(const uint32_t* vals, int M, int k, int* pos, SelectShared& sh) {
+  if (M <= 2 * FEW_THREADS) return block_select_of<2>(vals, M, k, pos, sh);
+  if (M <= 4 * FEW_THREADS) return block_select_of<4>(vals, M, k, pos, sh);
+  return block_select_of<16>(vals, M, k, pos, sh);
+}
 
 struct FewFinishArgs {
   const float* Q;
@@ -346,7 +397,9 @@ struct FewFinishArgs {
   const float* scale;
   const float* bias;
   const float* maxima;  // [B, ldm]
-  int64_t ldm, N, n_tiles;
+  const float* runs;    // [B, ldm / FEW_RUN], where there are more tiles than one workgroup selects from
+  const float* raw;     // [B, ldr] the scores, or null: formed again
+  int64_t ldm, ldr, N, n_tiles;
   int d, k, sigmoid;
   float* out_scores;
   int64_t* out_idx;
@@ -354,102 +407,145 @@ struct FewFinishArgs {
 
 template <int EDT>
 __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a) {
-  __shared__ uint32_t vals[16 * FEW_THREADS];
+  __shared__ __attribute__((aligned(16))) uint32_t vals[16 * FEW_THREADS];
   __shared__ int pos[FEW_MAX_K], groups[FEW_MAX_K];
   __shared__ int64_t tiles[FEW_MAX_K];
   __shared__ unsigned long long keys[FEW_MAX_K];
   __shared__ SelectShared sh;
+  __shared__ __attribute__((aligned(16))) unsigned char s_query[query_lds_bytes(EDT, QUERY_LDS_MAX_D)];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t q = blockIdx.x;
   const float* mx = a.maxima + q * a.ldm;
   const int T = (int)a.n_tiles, k = a.k;
-  int n;
-  if (T <= FEW_TILES_DIRECT) {
-    for (int t = tid; t < T; t += FEW_THREADS) vals[t] = score_key(mx[t]);
-    n = block_select(vals, T, k, pos, sh);
-    for (int j = tid; j < n; j += FEW_THREADS) tiles[j] = pos[j];
-  } else {
-    const int G = (T + 31) / 32;
-    for (int g = tid; g < G; g += FEW_THREADS) {
-      float m = __uint_as_float(0xff800000u);
-      if (32 * g + 32 <= T) {
+  // Three levels, groups of 32 tiles (where there are too many tiles), tiles, entities: the candidates' keys into vals, the
+  // best k of them picked.  (One loop, so that the selection is in the code once: the kernel runs a few microseconds, and
+  // every copy of it would be fetched cold.)
+  const bool grouped = T > FEW_TILES_DIRECT;
+  int n = 0;
+  bool direct_rank = false;  // the entities are few enough to be ranked without being picked first
+  for (int level = grouped ? 0 : 1; level < 3; ++level) {
+    int M;
+    if (level == 0) {
+      M = (T + 31) / 32;
+      for (int g = tid; g < M; g += FEW_THREADS) {
+        const f32x4 x = *(const f32x4*)(a.runs + q * (a.ldm / FEW_RUN) + 4 * (int64_t)g);  // 4 runs: 32 tiles
+        float m = x[0];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const f32x4 x = *(const f32x4*)(mx + 32 * (int64_t)g + 4 * i);
-          m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(m, x[0]), __builtin_fmaxf(x[1], x[2])), x[3]);
-        }
-      } else {
-        for (int t = 32 * g; t < T; ++t) m = __builtin_fmaxf(m, mx[t]);
+        for (int i = 1; i < 4; ++i)
+          if (FEW_RUN * (4 * g + i) < T) m = __builtin_fmaxf(m, x[i]);
+        vals[g] = score_key(m);
       }
-      vals[g] = score_key(m);
-    }
-    const int ng = block_select(vals, G, k, groups, sh);
-    for (int i = tid; i < 32 * ng; i += FEW_THREADS) {
-      const int t = 32 * groups[i >> 5] + (i & 31);
-      vals[i] = t < T ? score_key(mx[t]) : 0u;
-    }
-    n = block_select(vals, 32 * ng, k, pos, sh);
-    for (int j = tid; j < n; j += FEW_THREADS) tiles[j] = 32 * (int64_t)groups[pos[j] >> 5] + (pos[j] & 31);
-  }
-  __syncthreads();
-  // the tiles' scores again: every column of the result tile holds this query, lane c < 16 keeps accumulator c
-  for (int j = wave; j < n; j += FEW_THREADS / 64) {
-    const int64_t row = tiles[j] * 32 + c;
-    const f32x16 acc = chain_direct<EDT>(a.E, a.d, row < a.N ? row : -1, a.Q, q, hf);
-    float v = 0.f;
+    } else if (level == 1) {
+      M = grouped ? 32 * n : T;
+      for (int i = tid; i < M; i += FEW_THREADS) {
+        const int t = grouped ? 32 * groups[i >> 5] + (i & 31) : i;
+        vals[i] = t < T ? score_key(mx[t]) : 0u;
+      }
+    } else {
+      // the tiles' scores: kept by the scan, or formed again (every column of the result tile holds this query, lane
+      // c < 16 keeps accumulator c)
+      M = 32 * n;
+      if (a.raw) {
+        for (int i = tid; i < M; i += FEW_THREADS)
+          vals[i] = score_key(a.raw[q * a.ldr + tiles[i >> 5] * 32 + (i & 31)]);  // (rows past the end: -inf)
+      } else {
+        query_to_lds<EDT>(a.Q + q * a.d, a.d, s_query, tid, FEW_THREADS);
+        __syncthreads();
+        for (int j = wave; j < n; j += FEW_THREADS / 64) {
+          const int64_t row = tiles[j] * 32 + c;
+          const f32x16 acc = chain_one_query<EDT>(a.E, a.d, row < a.N ? row : -1, s_query, hf);
+          float v = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (i == c) v = acc[i];
-    if (c < 16) {
-      const int r = row_of(c, hf);
-      const int64_t e = tiles[j] * 32 + r;
-      if constexpr (EDT == KGE_I8) v *= a.scale[e < a.N ? e : a.N - 1];
-      vals[32 * j + r] = e < a.N ? score_key(v) : 0u;
+          for (int i = 0; i < 16; ++i)
+            if (i == c) v = acc[i];
+          if (c < 16) {
+            const int r = row_of(c, hf);
+            const int64_t e = tiles[j] * 32 + r;
+            if constexpr (EDT == KGE_I8) v *= a.scale[e < a.N ? e : a.N - 1];
+            vals[32 * j + r] = e < a.N ? score_key(v) : 0u;
+          }
+        }
+      }
+      direct_rank = M <= FEW_THREADS;
+      if (direct_rank) break;
     }
+    n = block_select(vals, M, k, pos, sh);
+    if (level == 0) {
+      for (int j = tid; j < n; j += FEW_THREADS) groups[j] = pos[j];
+    } else if (level == 1) {
+      for (int j = tid; j < n; j += FEW_THREADS)
+        tiles[j] = grouped ? 32 * (int64_t)groups[pos[j] >> 5] + (pos[j] & 31) : (int64_t)pos[j];
+    } else {
+      break;
+    }
+    __syncthreads();
   }
-  n = block_select(vals, 32 * n, k, pos, sh);
-  for (int j = tid; j < n; j += FEW_THREADS)
-    keys[j] = ((unsigned long long)vals[pos[j]] << 32) | (0xffffffffull - (unsigned long long)(tiles[pos[j] >> 5] * 32 + (pos[j] & 31)));
-  __syncthreads();
-  for (int j = tid; j < k; j += FEW_THREADS) {
-    int at = j;
+  auto put = [&](int at, uint32_t key, int64_t e) {  // key 0: fewer than k could be ranked
     float s = __uint_as_float(0x7fc00000u);
-    int64_t e = -1;
-    if (j < n) {
-      const unsigned long long key = keys[j];
-      at = 0;
-      for (int i = 0; i < n; ++i) at += keys[i] > key ? 1 : 0;
-      s = ordered_to_f32((uint32_t)(key >> 32));
-      e = (int64_t)(0xffffffffu - (uint32_t)(key & 0xffffffffull));
+    if (key) {
+      s = ordered_to_f32(key);
       if (a.bias) s += a.bias[q];
       if (a.sigmoid) s = 1.0f / (1.0f + expf(-s));
     }
     a.out_scores[q * k + at] = s;
-    a.out_idx[q * k + at] = e;
+    a.out_idx[q * k + at] = key ? e : -1;
+  };
+  if (direct_rank) {
+    // one value per thread: its rank is the number of values above it (equal ones at lower positions count as above)
+    const int M = 32 * n;
+    __syncthreads();
+    const uint32_t mine = tid < M ? vals[tid] : 0u;
+    int at = 0;
+    if (wave * 64 < M) {
+      for (int j = 0; j < M; j += 4) {
+        const u32x4 v = *(const u32x4*)(vals + j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) at += (v[i] > mine || (v[i] == mine && j + i < tid)) ? 1 : 0;
+      }
+    }
+    const int ranked = __syncthreads_count(mine != 0);
+    if (mine != 0 && at < k) put(at, mine, tiles[tid >> 5] * 32 + (tid & 31));
+    for (int j = ranked + tid; j < k; j += FEW_THREADS) put(j, 0u, 0);
+    return;
+  }
+  for (int j = tid; j < n; j += FEW_THREADS)
+    keys[j] = ((unsigned long long)vals[pos[j]] << 32) | (0xffffffffull - (unsigned long long)(tiles[pos[j] >> 5] * 32 + (pos[j] & 31)));
+  __syncthreads();
+  for (int j = tid; j < k; j += FEW_THREADS) {
+    if (j >= n) {
+      put(j, 0u, 0);
+      continue;
+    }
+    const unsigned long long key = keys[j];
+    int at = 0;
+    for (int i = 0; i < n; ++i) at += keys[i] > key ? 1 : 0;
+    put(at, (uint32_t)(key >> 32), (int64_t)(0xffffffffu - (uint32_t)(key & 0xffffffffull)));
   }
 }
 
-template <bool STORE>
+template <int MODE>
 int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
   const int parts = dtype == KGE_F32 ? 3 : 1;
   a.nks = (a.d + 15) / 16;
   a.n_tiles = (a.N + 31) / 32;
   // as many query tiles per wave as the batch has and LDS holds fragments of: every tile reads the table's rows once
   int qt = 1;
-  while (qt < (STORE ? 2 : 4) && 32 * qt < a.B && 2 * qt * a.nks * parts <= FEW_LDS_KB) qt *= 2;
+  while (qt < (MODE == FEW_STORE ? 2 : 4) && 32 * qt < a.B && 2 * qt * a.nks * parts <= FEW_LDS_KB) qt *= 2;
   const int n_qg = (a.B + 32 * qt - 1) / (32 * qt);
-  // four workgroups per CU walk units of 4 * tpw tiles; the longest runs that leave each of them four units
-  a.tpw = 8;
-  while (a.tpw > 1 && a.n_tiles < (int64_t)4 * a.tpw * 4096) a.tpw /= 2;
-  const int64_t units = (a.n_tiles + 4 * a.tpw - 1) / (4 * a.tpw);
-  const dim3 grid((unsigned)std::min<int64_t>(units, 1024), (unsigned)n_qg), block(256);
-  const size_t lds = (size_t)qt * a.nks * parts * 1024;
+  // one round of workgroups (as many per CU as registers and LDS allow) walks units of 4 * tpw tiles, each the same number
+  // of them; runs of eight tiles where there are more tiles than the selection reads one by one
+  a.tpw = a.n_tiles > FEW_TILES_DIRECT ? FEW_RUN : 1;
+  const size_t lds = (size_t)qt * a.nks * parts * 1024 + 4 * few_stage_bytes(dtype);
+  const size_t room = 163840 / (lds + (MODE == FEW_MAX ? 4096 * qt : 0) + 512);
+  const int64_t slots = 256 * std::max<int64_t>(1, std::min<int64_t>(room, qt > 1 ? 2 : dtype == KGE_F32 ? 3 : 4));
+  const int64_t units = (a.n_tiles + 4 * a.tpw - 1) / (4 * a.tpw), each = (units + slots - 1) / slots;
+  const dim3 grid((unsigned)((units + each - 1) / each), (unsigned)n_qg), block(256);
   auto go = [&](auto edt) {
     constexpr int EDT = decltype(edt)::value;
-    if (qt == 1) hipLaunchKernelGGL((few_scan_kernel<EDT, 1, STORE>), grid, block, lds, st, a);
-    else if (qt == 2) hipLaunchKernelGGL((few_scan_kernel<EDT, 2, STORE>), grid, block, lds, st, a);
-    else if constexpr (!STORE) hipLaunchKernelGGL((few_scan_kernel<EDT, 4, STORE>), grid, block, lds, st, a);
+    if (qt == 1) hipLaunchKernelGGL((few_scan_kernel<EDT, 1, MODE>), grid, block, lds, st, a);
+    else if (qt == 2) hipLaunchKernelGGL((few_scan_kernel<EDT, 2, MODE>), grid, block, lds, st, a);
+    else if constexpr (MODE != FEW_STORE) hipLaunchKernelGGL((few_scan_kernel<EDT, 4, MODE>), grid, block, lds, st, a);
   };
   if (dtype == KGE_F32) go(std::integral_constant<int, KGE_F32>{});
   else if (dtype == KGE_BF16) go(std::integral_constant<int, KGE_BF16>{});
@@ -461,18 +557,21 @@ int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
 
 int few_scores_launch(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
                       int64_t N, float* out, int64_t ldo, hipStream_t st) {
-  FewArgs a{Q, E, scale, bias, out, ldo, N, 0, (int)B, (int)d, 0, 0};
-  return launch_few_scan<true>(dtype, a, st);
+  FewArgs a{Q, E, scale, bias, out, nullptr, nullptr, ldo, 0, N, 0, (int)B, (int)d, 0, 0};
+  return launch_few_scan<FEW_STORE>(dtype, a, st);
 }
 
 int few_topk_launch(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
                     int64_t N, int64_t k, float* out_scores, int64_t* out_idx, int apply_sigmoid, void* workspace,
                     hipStream_t st) {
-  const int64_t ldm = host::few_maxima_pitch(N);
-  FewArgs a{Q, E, scale, nullptr, (float*)workspace, ldm, N, 0, (int)B, (int)d, 0, 0};
-  int rc = launch_few_scan<false>(dtype, a, st);
+  const host::FewTopkWs w = host::few_topk_ws(B, N);
+  float* maxima = (float*)workspace;
+  float* runs = w.runs ? maxima + w.runs : nullptr;
+  float* raw = w.raw ? maxima + w.raw : nullptr;
+  FewArgs a{Q, E, scale, nullptr, maxima, runs, raw, w.ldm, w.ldr, N, 0, (int)B, (int)d, 0, 0};
+  const int rc = raw ? launch_few_scan<FEW_MAX_RAW>(dtype, a, st) : launch_few_scan<FEW_MAX>(dtype, a, st);
   if (rc) return rc;
-  FewFinishArgs f{Q, E, scale, bias, (const float*)workspace, ldm, N, (N + 31) / 32, (int)d, (int)k, apply_sigmoid,
+  FewFinishArgs f{Q, E, scale, bias, maxima, runs, raw, w.ldm, w.ldr, N, (N + 31) / 32, (int)d, (int)k, apply_sigmoid,
                   out_scores, out_idx};
   const dim3 grid((unsigned)B), block(FEW_THREADS);
   if (dtype == KGE_F32) hipLaunchKernelGGL((few_finish_kernel<KGE_F32>), grid, block, 0, st, f);

@@ -240,7 +240,28 @@ constexpr int FEW_MAX_K = 128;            // tiles scored again per query: one w
 constexpr int FEW_TILES_DIRECT = 16384;   // tile maxima one workgroup selects from; more go through maxima of 32 tiles
 constexpr int64_t FEW_MAX_N = (int64_t)FEW_TILES_DIRECT * 32 * 32;
 constexpr int FEW_LDS_KB = 64;            // LDS for the query fragments: 1 KB per K step of 16, bf16 part and query tile
-inline int64_t few_maxima_pitch(int64_t N) { return ((N + 31) / 32 + 31) / 32 * 32; }
+// The workspace in floats: the tile maxima [B, ldm], then the maxima of runs of eight tiles [B, ldm / 8] (tables of more than
+// FEW_TILES_DIRECT tiles) or the scores themselves [B, ldr] (up to FEW_RAW_BYTES of them: writing them costs less than
+// forming the best tiles' scores again, 16 us for a trip of sixteen fp32 d = 256 tiles).
+constexpr int64_t FEW_RAW_BYTES = 32 << 20;
+struct FewTopkWs {
+  int64_t ldm, ldr, runs, raw, total;  // pitches; offsets of the second and third part (0: absent); floats in all
+};
+inline FewTopkWs few_topk_ws(int64_t B, int64_t N) {
+  FewTopkWs w{};
+  const int64_t tiles = (N + 31) / 32;
+  w.ldm = (tiles + 31) / 32 * 32;
+  w.ldr = tiles * 32;
+  w.total = B * w.ldm;
+  if (tiles > FEW_TILES_DIRECT) {
+    w.runs = w.total;
+    w.total += B * (w.ldm / 8);
+  } else if (B * w.ldr * 4 <= FEW_RAW_BYTES) {
+    w.raw = w.total;
+    w.total += B * w.ldr;
+  }
+  return w;
+}
 inline bool few_rows_ok(int dtype, int64_t d) {
   return (d + 15) / 16 * (dtype == KGE_F32 ? 3 : 1) <= FEW_LDS_KB && (dtype != KGE_F32 || d % 4 == 0);
 }
@@ -251,7 +272,7 @@ inline bool few_scores_applies(int dtype, int64_t B, int64_t d) {
   return B >= 1 && B <= FEW_SCORES_MAX_B && few_rows_ok(dtype, d);
 }
 inline size_t few_topk_ws_bytes(int64_t B, int64_t N, int64_t k) {
-  return (B <= FEW_MAX_B && k <= FEW_MAX_K && N <= FEW_MAX_N) ? (size_t)B * (size_t)few_maxima_pitch(N) * 4 : 0;
+  return (B <= FEW_MAX_B && k <= FEW_MAX_K && N <= FEW_MAX_N) ? (size_t)few_topk_ws(B, N).total * 4 : 0;
 }
 
 // The threshold a scan of `n_next` more rows may use once `ranked` rows are ranked: the j-th best score so far, j as

@@ -52,6 +52,14 @@ int few_scores_launch(const float* Q, const float* bias, const void* E, int dtyp
 // acc[i] of lane l holds output (row_of(i, l / 32), l % 32).
 __device__ __forceinline__ int row_of(int i, int hf) { return ((i >> 2) << 3) + (hf << 2) + (i & 3); }
 
+// The lanes of one wave see each other's LDS writes from here on (a wave's LDS accesses complete in order, so that only the
+// compiler has to be told): for kernels whose waves work on LDS rows of their own.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // Order-preserving map float -> uint32 (larger float <=> larger key); NaN is not handled.
 __device__ __forceinline__ uint32_t f32_to_ordered(float f) {
   uint32_t u = __float_as_uint(f);

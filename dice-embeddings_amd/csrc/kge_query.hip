@@ -299,14 +299,6 @@ __global__ void __launch_bounds__(64) build_query_kernel(QueryArgs a, int model)
   if (lane == 0) a.bias[b] = bias;
 }
 
-// The lanes of one wave see each other's LDS writes from here on (a wave's LDS accesses complete in order, so that only the
-// compiler has to be told): for kernels whose waves work on LDS rows of their own.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-}
-
 // ---- backward of the query builder ---------------------------------------------------------------
 // Given dL/dQ[b, :] and dL/dbias[b], add dL/d(head row) to d_ent[h], dL/d(relation row) to d_rel[r] and, for
 // the Clifford models, dL/d(coefficients) to d_coeff_*.  One wavefront per pair; rows that several pairs share
