@@ -524,6 +524,56 @@ __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a
   }
 }
 
+// ---- the best k of a vector of values (descending, equal values by position, NaN first: a stable descending sort cut at k) --
+__device__ __forceinline__ uint32_t value_key(float v) {
+  return v != v ? 0xffffffffu : f32_to_ordered(v + 0.f);  // (-0 and 0 are equal); never 0
+}
+// the largest key of every 32 values
+__global__ void __launch_bounds__(256) value_tiles_kernel(const float* values, int N, uint32_t* tiles, int n_tiles) {
+  const int t = blockIdx.x * 8 + (threadIdx.x >> 5), i = 32 * t + (threadIdx.x & 31);
+  uint32_t k = i < N ? value_key(values[i]) : 0u;
+#pragma unroll
+  for (int o = 16; o >= 1; o >>= 1) {
+    const uint32_t y = __shfl_xor(k, o, 64);
+    k = y > k ? y : k;
+  }
+  if ((threadIdx.x & 31) == 0 && t < n_tiles) tiles[t] = k;
+}
+// One workgroup: latency, not work, is what this costs.  tiles: null where the workgroup selects from the values
+// themselves.  (The hop of a query answered by the library's device sort was seven launches for ten values.)
+__global__ void __launch_bounds__(FEW_THREADS) topk_values_kernel(const float* values, int N, const uint32_t* tiles,
+                                                                  int n_tiles, int k, float* out_values, int64_t* out_idx) {
+  __shared__ __attribute__((aligned(16))) uint32_t vals[16 * FEW_THREADS];
+  __shared__ int pos[FEW_MAX_K], best[FEW_MAX_K];
+  __shared__ unsigned long long keys[FEW_MAX_K];
+  __shared__ SelectShared sh;
+  const int tid = threadIdx.x;
+  int M = N, n = 0;
+  if (tiles) {
+    for (int t = tid; t < n_tiles; t += FEW_THREADS) vals[t] = tiles[t];
+    n = block_select(vals, n_tiles, k, best, sh);
+    M = 32 * n;
+  }
+  for (int i = tid; i < M; i += FEW_THREADS) {
+    const int at = tiles ? 32 * best[i >> 5] + (i & 31) : i;
+    vals[i] = at < N ? value_key(values[at]) : 0u;
+  }
+  n = block_select(vals, M, k, pos, sh);  // k <= N: there are k
+  for (int j = tid; j < n; j += FEW_THREADS) {
+    const int at = tiles ? 32 * best[pos[j] >> 5] + (pos[j] & 31) : pos[j];
+    keys[j] = ((unsigned long long)vals[pos[j]] << 32) | (0xffffffffu - (uint32_t)at);
+  }
+  __syncthreads();
+  for (int j = tid; j < n; j += FEW_THREADS) {
+    const unsigned long long key = keys[j];
+    int rank = 0;
+    for (int i = 0; i < n; ++i) rank += keys[i] > key ? 1 : 0;
+    const uint32_t at = 0xffffffffu - (uint32_t)(key & 0xffffffffull);
+    out_values[rank] = values[at];
+    out_idx[rank] = (int64_t)at;
+  }
+}
+
 template <int MODE>
 int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
   const int parts = dtype == KGE_F32 ? 3 : 1;
@@ -581,3 +631,32 @@ int few_topk_launch(const float* Q, const float* bias, const void* E, int dtype,
   return KGE_OK;
 }
 }  // namespace kge
+
+extern "C" size_t kge_topk_values_workspace_bytes(int64_t N) {
+  return N > kge::host::FEW_TILES_DIRECT ? (size_t)((N + 31) / 32) * 4 : 0;
+}
+
+extern "C" int kge_topk_values(const float* values, int64_t N, int64_t k, float* out_values, int64_t* out_idx,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace kge;
+  clear_error();
+  KGE_REQUIRE(N >= 1 && N <= 32LL * FEW_TILES_DIRECT, KGE_ERR_UNSUPPORTED, "kge_topk_values: N=%lld outside [1, %lld]",
+              (long long)N, 32LL * FEW_TILES_DIRECT);
+  KGE_REQUIRE(k >= 1 && k <= N && k <= FEW_MAX_K, KGE_ERR_UNSUPPORTED, "kge_topk_values: k=%lld outside [1, min(N, %d)]",
+              (long long)k, FEW_MAX_K);
+  KGE_REQUIRE(values && out_values && out_idx, KGE_ERR_INVALID, "kge_topk_values: null pointer argument");
+  const size_t need = kge_topk_values_workspace_bytes(N);
+  KGE_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 3) == 0), KGE_ERR_WORKSPACE,
+              "kge_topk_values: workspace of %zu bytes, need %zu, 4-byte aligned", workspace_bytes, need);
+  hipStream_t st = (hipStream_t)stream;
+  const int n_tiles = (int)((N + 31) / 32);
+  uint32_t* tiles = need ? (uint32_t*)workspace : nullptr;
+  if (tiles) {
+    hipLaunchKernelGGL(value_tiles_kernel, dim3((unsigned)((n_tiles + 7) / 8)), dim3(256), 0, st, values, (int)N, tiles, n_tiles);
+    KGE_LAUNCH_CHECK("value_tiles_kernel");
+  }
+  hipLaunchKernelGGL(topk_values_kernel, dim3(1), dim3(FEW_THREADS), 0, st, values, (int)N, tiles, n_tiles, (int)k, out_values,
+                     out_idx);
+  KGE_LAUNCH_CHECK("topk_values_kernel");
+  return KGE_OK;
+}

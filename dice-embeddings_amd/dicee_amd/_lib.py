@@ -49,6 +49,8 @@ SIGNATURES = {
                                                ctypes.POINTER(NormParams), ctypes.POINTER(NormGrads),
                                                ctypes.POINTER(DropoutParams), _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp,
                                                _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "kge_topk_values_workspace_bytes": (_sz, [_c_i64]),
+    "kge_topk_values": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _vp, _sz, _vp]),
     "kge_fill_zero": (_c_int, [_vp, _vp, _c_int, _vp]),
     "kge_batchnorm_workspace_bytes": (_sz, [_c_i64, _c_i64]),
     "kge_batchnorm_stats": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(DropoutParams), _c_f,

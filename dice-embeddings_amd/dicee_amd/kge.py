@@ -278,14 +278,24 @@ class KGE:
         with torch.no_grad():
             return self.model.forward_k_vs_all(torch.stack([head_ids, rel], dim=1).contiguous())
 
+    @staticmethod
+    def _best(scores, k):
+        """(values, positions) of the k best of a vector of scores, as a stable descending sort orders them."""
+        from . import ops
+        if (scores.is_cuda and scores.dtype == torch.float32 and 1 <= k <= min(scores.numel(), ops.TOPK_VALUES_MAX_K)
+                and scores.numel() <= ops.TOPK_VALUES_MAX_N and not scores.requires_grad):
+            return ops.topk_values(scores.contiguous(), k)
+        s, idx = torch.sort(scores, descending=True, stable=True)
+        return s[:k], idx[:k]
+
     def _multi_hop_scores(self, query_type, query, tnorm, neg_norm, lambda_, k):
         """[N] GPU tensor: score of every entity as the answer (the norms act on logits, as in the reference,
         whose ``predict`` defaults to ``logits=True``)."""
         one = lambda e, r: self._atom([self.entity_to_idx[e]], r)[0]
 
         def hop(prev, r):          # keep the k best substitutions of the variable, then the best t-norm per answer
-            s, idx = torch.sort(prev, descending=True, stable=True)
-            return torch.max(self.t_norm(s[:k, None], self._atom(idx[:k], r), tnorm), dim=0)[0]
+            s, idx = self._best(prev, k)
+            return torch.max(self.t_norm(s[:, None], self._atom(idx, r), tnorm), dim=0)[0]
         if query_type == "1p":
             e, (r1,) = query
             return one(e, r1)
@@ -310,11 +320,11 @@ class KGE:
             return hop(self._multi_hop_scores(inner_type, inner, tnorm, neg_norm, lambda_, k), r)
         if query_type in ("pi", "pin", "pni"):
             (e1, rels), (e3, rel3) = query
-            s, idx = torch.sort(one(e1, rels[0]), descending=True, stable=True)
-            a2 = self._atom(idx[:k], rels[1])
+            s, idx = self._best(one(e1, rels[0]), k)
+            a2 = self._atom(idx, rels[1])
             if query_type == "pni":
                 a2 = self.negnorm(a2, lambda_, neg_norm)
-            two_p = torch.max(self.t_norm(s[:k, None], a2, tnorm), dim=0)[0]
+            two_p = torch.max(self.t_norm(s[:, None], a2, tnorm), dim=0)[0]
             last = one(e3, rel3[0])
             if query_type == "pin":
                 last = self.negnorm(last, lambda_, neg_norm)

@@ -462,6 +462,25 @@ def topk(Q, bias, E, scale, k, sigmoid=False, prepared=None):
     return out_s, out_i
 
 
+TOPK_VALUES_MAX_K, TOPK_VALUES_MAX_N = 128, 524288
+
+
+def topk_values(values, k):
+    """(values [k], positions int64 [k]): the first k of ``torch.sort(values, descending=True, stable=True)`` of a
+    contiguous fp32 vector of up to 524,288 values, k up to 128."""
+    lib = _lib.load()
+    _require_gpu(values)
+    if values.dtype != torch.float32 or values.dim() != 1:
+        raise TypeError("values must be a float32 vector")
+    n = values.numel()
+    out_v = torch.empty((k,), dtype=torch.float32, device=values.device)
+    out_i = torch.empty((k,), dtype=torch.int64, device=values.device)
+    nbytes = lib.kge_topk_values_workspace_bytes(n)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=values.device) if nbytes else None
+    _lib.check(lib.kge_topk_values(_ptr(values), n, int(k), _ptr(out_v), _ptr(out_i), _ptr(ws), nbytes, _stream()))
+    return out_v, out_i
+
+
 def bce_multihot(Q, bias, E, scale, csr_row, row_ptr, col, label_smoothing=0.0):
     """Mean BCE-with-logits of the [B,N] scores against the multi-hot of the CSR rows: [1] fp32 tensor."""
     lib = _lib.load()

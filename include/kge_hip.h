@@ -177,6 +177,15 @@ int kge_build_query_backward(int model, int p, int q, int r, const float* ent, c
                              const float* dQ, const float* dbias, float* d_ent, float* d_rel, float* d_coeff_p,
                              float* d_coeff_q, float* d_coeff_r, void* stream);
 
+/*
+ * The k largest of a vector of values with their positions, descending, equal values by position, NaN before everything:
+ * the first k of a stable descending sort (the substitutions a multi-hop query goes on with,
+ * dicee/knowledge_graph_embeddings.py answer_multi_hop_query).  1 <= k <= min(N, 128), N <= 524288.
+ */
+size_t kge_topk_values_workspace_bytes(int64_t N);
+int kge_topk_values(const float* values, int64_t N, int64_t k, float* out_values, int64_t* out_idx, void* workspace,
+                    size_t workspace_bytes, void* stream);
+
 /* Clears n <= 8 fp32 buffers (counts[i] elements each) in one launch: the outputs that the backward adds to. */
 int kge_fill_zero(float* const* bufs, const int64_t* counts, int n, void* stream);
 

@@ -85,3 +85,26 @@ def test_topk_of_few_queries_ranks_no_nan_and_is_capturable(storage, d):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(gi, idx) and torch.equal(torch.nan_to_num(gv), torch.nan_to_num(vals))
+
+
+@pytest.mark.parametrize("n", [1, 31, 135, 2048, 2049, 14541, 16384, 16385, 100003, 524288])
+@pytest.mark.parametrize("pattern", ["random", "ties", "special"])
+def test_topk_values_is_the_head_of_a_stable_sort(n, pattern):
+    """Edges of the selection's register classes and of the direct form; massive ties, signed zeros, infinities, NaN."""
+    from dicee_amd import ops
+    rng = np.random.default_rng(n)
+    v = rng.standard_normal(n).astype(np.float32)
+    if pattern != "random":
+        v = np.round(v * 1.5) / 2 * np.where(rng.random(n) < 0.5, 1, -1).astype(np.float32)      # holds 0.0 and -0.0
+    if pattern == "special":
+        v[rng.random(n) < 0.2] = -np.inf
+        v[rng.random(n) < 0.001] = np.inf
+        v[rng.random(n) < 0.0005] = np.nan
+    t = torch.from_numpy(v.astype(np.float32)).cuda()
+    s, i = torch.sort(t, descending=True, stable=True)
+    for k in {1, min(3, n), min(10, n), min(64, n), min(128, n)}:
+        got, at = ops.topk_values(t, k)
+        assert torch.equal(at, i[:k])
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(s[:k])) and torch.equal(got.isnan(), s[:k].isnan())
+    with pytest.raises(Exception):
+        ops.topk_values(t, min(n, 128) + 1)
