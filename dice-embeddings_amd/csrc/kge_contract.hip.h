@@ -1950,7 +1950,7 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
   int foff[KS_KC / 16];
 #pragma unroll
   for (int ks = 0; ks < KS_KC / 16; ++ks) foff[ks] = c * 64 + (((2 * ks + hf) ^ ((c >> 2) & 3)) << 4);
-  // K-major planes: this lane's address inside a 32-row tile for the transposing reads of K step 0, first half (k rows
+  // K-major planes: this lane's address inside a 32-row tile for the transposing reads of a K step, first half (k rows
   // 8 hf + (lane % 16) / 4, rows 16 ((lane / 16) % 2) + 4 (lane % 4) ..); per row pitch: the tile's first segment is
   // added before the swizzle, so the two parts are kept apart
   const int tr_k = 8 * hf + ((lane & 15) >> 2);
@@ -2054,7 +2054,7 @@ __global__ void __launch_bounds__(256, 2) ksplit_kmajor_kernel(ContractArgs a, t
 // ============================================================================================
 // kchunk_kernel: bf16 or per-row int8 table of any width (d % 8 == 0); used for d > 256, where the queries no
 // longer fit the register file of the persistent kernels.  int8 rows are widened to bf16 (exactly) on the way into
-// LDS and a finished tile's scores are multiplied by the row scales, as in the other int8 kernels.  The shape of ksplit_kernel with one part per operand:
+// LDS and a finished tile's scores are multiplied by the row scales, as in the other int8 kernels.  One part per operand,
 // 256 entities x 128 queries per workgroup of 8 waves (64 x 64 per wave), K in chunks of 64, both operands
 // staged through registers into double-buffered LDS (the fp32 queries are rounded to bf16 on the way, as in
 // the other bf16 kernels), one MFMA per 32 x 32 x 16 block.  Reduction order per score: K ascending in steps of

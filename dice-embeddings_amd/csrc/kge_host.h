@@ -234,8 +234,10 @@ inline TopkWsOffsets topk_ws_offsets(int64_t B, int64_t N, int64_t k, bool with_
 // Few queries (kge_few.hip): every wave holds the same queries and the rows are shared out, so the table is read once per
 // 32 .. 128 queries at the rate of memory.  The top-k form keeps the maximum of every 32-row tile per query in the
 // workspace: 4 N / 32 bytes per query.
-constexpr int FEW_MAX_B = 128;            // top-k
-constexpr int FEW_SCORES_MAX_B = 64;
+constexpr int FEW_MAX_B = 128;            // top-k: four query tiles in one pass over the table.  There, k = 10, against the
+                                          // rounds (whose cost is flat up to 512 queries): bf16 2.5M x 128 228 us / 425,
+                                          // int8 10M x 128 660 / 1029, fp32 41k x 256 60 / 196; 500k x 128 200 / 298
+constexpr int FEW_SCORES_MAX_B = 64;      // scores: fp32 41k x 256 24 us / 26 at 64 queries, 27 / 27 at 96
 constexpr int FEW_MAX_K = 128;            // tiles scored again per query: one workgroup's work
 constexpr int FEW_TILES_DIRECT = 16384;   // tile maxima one workgroup selects from; more go through maxima of 32 tiles
 constexpr int64_t FEW_MAX_N = (int64_t)FEW_TILES_DIRECT * 32 * 32;

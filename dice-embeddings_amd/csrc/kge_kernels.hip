@@ -2247,7 +2247,7 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
   {
     if (kmajor) {
       // the rows of Q as the "queries", the rows of G (N of them, read up to the padded pitch) as the "entities": a
-      // workgroup's share of G is 256 neighbouring columns (1 KB of every row), and the result is stored transposed
+      // workgroup's share of G is 128 neighbouring columns (512 bytes of every row), and the result is stored transposed
       ContractArgs b = make_args(Q, G, KGE_F32, nullptr, d, B, p.ldG, 0, p.ldG);
       b.ldq = (int)d;
       b.lde = (int)p.ldG;

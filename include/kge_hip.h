@@ -383,7 +383,8 @@ int kge_rank_filtered_static(const float* Q, const float* bias, const void* E, i
  *   the order of their unbiased scores.
  * This call (and kge_topk_prepared) synchronises `stream`: once before returning to read back one overflow
  * counter, and once more per repair scan when a candidate buffer overflowed (at most 16 scans; still overflowing
- * after those: KGE_ERR_OVERFLOW).  Neither can be captured into a HIP graph.
+ * after those: KGE_ERR_OVERFLOW).  Neither can be captured into a HIP graph.  Calls of at most 128 queries with k <= 128,
+ * N <= 2^24 and rows of at most 336 fp32 (a multiple of 4) or 1024 bf16 / int8 elements read nothing back and can be.
  */
 size_t kge_topk_workspace_bytes(int64_t B, int64_t N, int64_t k);
 int kge_topk(const float* Q, const float* bias, const void* E, int dtype, const float* scale,
