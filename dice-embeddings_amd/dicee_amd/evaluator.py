@@ -48,6 +48,8 @@ def check_triple_ids(triples, num_entities, num_relations):
     """``triples`` [n,3] of an integer type as contiguous int64, or ``IndexError`` where an id is outside the model's
     tables.  (One maximum per column: a negative id is a huge unsigned one.  Minima and maxima of picked columns, and the
     copies they imply, were a tenth of an evaluation of 20,000 triples, with the GPU waiting.)"""
+    if triples.dtype.kind not in "iub" and triples.size and triples.min() < 0:      # (-0.5 is not the id 0)
+        raise IndexError("triple_idx holds an entity or relation id outside the model's tables")
     ids = np.ascontiguousarray(triples, dtype=np.int64)
     if len(ids):
         top = ids.view(np.uint64)
