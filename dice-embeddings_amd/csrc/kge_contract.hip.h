@@ -38,6 +38,7 @@ struct ContractArgs {
   // ksplit_kernel only: 0, or the number of K ranges (a multiple of 8) of a launch whose grid is flat: range y is
   // dealt to XCD y % 8, so that the workgroups that read one range of a K-major operand share an L2
   int k_split_xcd;
+  int ks_rows;     // host side, fp32 tables: the form of the split kernel (0: not planned yet)
   int persistent;  // host side: the decomposition above is that of a persistent kernel (checked at launch)
 };
 
@@ -1776,18 +1777,21 @@ __global__ void __launch_bounds__(64 * I8_WG_WAVES, 2) qreg_i8_kernel(ContractAr
 }
 
 // ============================================================================================
-// ksplit_kernel: fp32 tables on the bf16 MFMA (split3_bf16x8).  128 entities x 128 queries per workgroup of 4 waves (each
-// wave 64 x 64), two workgroups per CU, K in chunks of 32.  Both operands are loaded as fp32 into registers while the
-// previous chunk is multiplied, split into their three bf16 parts and stored as three planes per operand in LDS; per
-// 16-wide K step a wave reads 12 fragments and issues 24 MFMAs.  One LDS buffer (48 KB): a workgroup's split and store
-// stand between two barriers, and so do its first loads and its epilogue; what fills the matrix cores meanwhile is the
-// other workgroup of the CU, which is at another point of its walk.
-// Measured against 256 x 128 workgroups of 8 waves, one per CU, that split and stored the next chunk under the products
-// into a second buffer: 1000 x 40,943 scores, d = 256 157 -> 143 us; training step of 1000 x 14,541, d = 200 228 -> 220 us (the
-// score gradients 100 -> 60: half as many rows per tile, and the epilogue under another workgroup's products); at
-// 2048 x 40,943 the same within 3 %: power-limited matrix cores either way.  16-column chunks in two buffers, split under the
-// products, came out the same (step of 1000 217 us, scores 144, rank pass 1.4 % slower), and a branch around the column
-// masks slower (241): it parts the loads that should be in flight together.
+// ksplit_kernel: fp32 tables on the bf16 MFMA (split3_bf16x8).  64 x 64 scores per wave, K in chunks of 32; both operands go
+// as fp32 through registers, are split into their three bf16 parts and stored as three planes per operand in LDS; per
+// 16-wide K step a wave reads 12 fragments and issues 24 MFMAs.  Two workgroup forms (host::ks_plan chooses, per launch):
+// * wide, ROWS = 256: 256 entities x 128 queries, 8 waves, one workgroup per CU, two LDS buffers: a chunk is split and
+//   stored under the products of the chunk before, in slices between them, so the matrix cores wait for neither; what they
+//   wait for is the first loads and the epilogue, and a CU whose neighbours have a tile more.
+// * narrow, ROWS = 128: 128 x 128, 4 waves, one buffer, two or three workgroups per CU: split and store stand between two
+//   barriers, and what fills the matrix cores meanwhile is the CU's other workgroups, at another point of their walk.  It
+//   multiplies 5 - 10 % more slowly once every CU is full, but it hides epilogues that write, and halves the tile that a
+//   last round, or a launch smaller than the chip, waits for.
+// Wide against narrow, us: scores 1000 x 40,943, d = 256 157 / 143; the score gradients of a training step of 1000 x 14,541,
+// d = 200 100 / 60; scores of 128 queries, N = 500k, d = 256 207 / 235; ranks of 1000 queries, N = 41k, d = 512 238 / 273, of
+// 5000 queries, N = 1000, d = 200 32 / 39, of 2048 queries, N = 5000, d = 256 58 / 49.
+// (16-column chunks in two buffers in the narrow form came out the same, and a branch around the column masks slower, 241
+// for 220 us of a training step: it parts the loads that should be in flight together.)
 // Chain order per score: K steps of 16 ascending, inside a step the six products in SPLIT order.
 //
 // LDS plane layout: row r is 64 B = 4 pieces of 16 B (8 bf16); piece p sits in slot
@@ -1795,11 +1799,11 @@ __global__ void __launch_bounds__(64 * I8_WG_WAVES, 2) qreg_i8_kernel(ContractAr
 // ============================================================================================
 constexpr int KS_NQT = 2;
 using host::KS_WG_QUERIES;
-using host::KS_TILE_ROWS;
+using host::KS_NARROW_ROWS;
+using host::KS_WIDE_ROWS;
 constexpr int KS_KC = 32;
-constexpr int KS_E_PLANE = KS_TILE_ROWS * 64;
 constexpr int KS_Q_PLANE = KS_WG_QUERIES * 64;
-constexpr int KS_STAGE_BYTES = 3 * KS_E_PLANE + 3 * KS_Q_PLANE;
+constexpr int ks_threads(int rows) { return 2 * rows; }  // a wave per 64 x 64 scores
 
 // KMAJ (bit 0: the entity operand, bit 1: the query operand; VEC only): that operand is given K-MAJOR, X[k][row] with
 // the rows contiguous (row pitch lde / ldq), as the backward of a contraction meets its operands (dQ = G E sums over
@@ -1809,12 +1813,17 @@ constexpr int KS_STAGE_BYTES = 3 * KS_E_PLANE + 3 * KS_Q_PLANE;
 // (ds_read_b64_tr_b16: within 16 lanes, lane j receives element j % 4 of the 8 bytes that lanes j / 4 + 4 i
 // addressed, i = 0..3), each giving a lane its row at four consecutive k.  Same products in the same order as the
 // row-major form.  The K-major operand's row count and pitch must be multiples of 4 and its base 16-byte aligned.
-template <template <int> class EpiT, bool VEC, int KMAJ>
+template <template <int> class EpiT, bool VEC, int KMAJ, int ROWS>
 __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typename EpiT<KS_NQT>::Args& ea) {
   using Epi = EpiT<KS_NQT>;
+  constexpr bool WIDE = ROWS == KS_WIDE_ROWS;
+  constexpr int KS_E_PLANE = ROWS * 64, KS_STAGE_BYTES = 3 * KS_E_PLANE + 3 * KS_Q_PLANE;
+  constexpr int PASS = ks_threads(ROWS) / 8;                  // rows of a staging pass
+  constexpr int QP = KS_WG_QUERIES / PASS, NP = 4 + QP;       // passes of the query rows, of both operands
+  constexpr int KE_STEP = 4 * ks_threads(ROWS) / ROWS, KQ_STEP = ks_threads(ROWS) / 32;  // K-major: k rows of a pass
   static_assert(KMAJ == 0 || VEC, "K-major operands are loaded 16 bytes at a time");
   constexpr bool KE = (KMAJ & 1) != 0, KQ = (KMAJ & 2) != 0;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[KS_STAGE_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[(WIDE ? 2 : 1) * KS_STAGE_BYTES];
 
   int qg;
   int64_t chunk;
@@ -1845,33 +1854,35 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
   const int64_t r0 = a.e_begin + chunk * a.chunk_rows;
   const int64_t r1 = (r0 + a.chunk_rows < a.e_end) ? r0 + a.chunk_rows : a.e_end;
   const int nkc = (d + KS_KC - 1) / KS_KC;
-  const int n_et = (int)((r1 - r0 + KS_TILE_ROWS - 1) / KS_TILE_ROWS);
+  const int n_et = (int)((r1 - r0 + ROWS - 1) / ROWS);
   const int n_it = n_et * nkc;
   const float* Ef = (const float*)a.E + (KE ? (int64_t)k_off * lde : (int64_t)k_off);
 
-  // Staging: a chunk is 256 rows (128 entity rows, then 128 query rows) of 128 B, taken in eight passes of
-  // 32 rows; in pass g thread tid takes 16 B piece (tid & 7) of row 32 g + tid / 8, so eight neighbouring
-  // lanes read one whole 128 B line.  Loads are branch-free so that all eight stay in flight: rows past the
+  // Staging: a chunk is ROWS entity rows, then 128 query rows, of 128 B, taken in NP passes of PASS rows (wide: six of 64,
+  // narrow: eight of 32); in pass g thread tid takes 16 B piece (tid & 7) of row PASS g + tid / 8, so eight neighbouring
+  // lanes read one whole 128 B line.  Loads are branch-free so that all of them stay in flight: rows past the
   // end repeat the last valid row (epilogues ignore them), columns past d are read from a clamped address
-  // and zeroed when stored.  Chunk i+2 is loaded as soon as chunk i+1 has been split and stored, and has chunk i+1's
-  // multiplication to land.
+  // and zeroed when stored.  Wide: pass g of chunk i+2 is loaded right after pass g of chunk i+1 has been split and stored,
+  // both while chunk i is multiplied: one register set, and a whole iteration for a load to land.  Narrow: chunk i+2 is
+  // loaded as soon as chunk i+1 has been split and stored, and has chunk i+1's multiplication to land.
   const int s_row = tid >> 3, s_piece = tid & 7;
   const int64_t q_last = a.B - 1, e_last = r1 - 1;
-  const float* q_ptr[4];
+  const float* q_ptr[QP];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    int64_t qr = q_base + 32 * g + s_row;
+  for (int g = 0; g < QP; ++g) {
+    int64_t qr = q_base + PASS * g + s_row;
     qr = qr < q_last ? qr : q_last;
     q_ptr[g] = a.Q + k_off + qr * ldq;
   }
-  // K-major operands: pass g of either operand is k rows 8 (g % 4) + tid / 32 of the chunk, four rows 4 (tid % 32) ..  A quad
-  // of rows past the operand's end is read from the last quad inside the pitch instead (its scores are never stored).
-  const int ke_kk = tid >> 5, ke_mq = tid & 31, kq_kk = ke_kk, kq_mq = ke_mq;
+  // K-major operands: pass g of the entity operand is k rows KE_STEP g + tid / (ROWS / 4) of the chunk, four rows
+  // 4 (tid % (ROWS / 4)) ..; pass g of the query operand k rows KQ_STEP (g - 4) + tid / 32, four rows 4 (tid % 32) ..  A quad of
+  // rows past the operand's end is read from the last quad inside the pitch instead (its scores are never stored).
+  const int ke_kk = WIDE ? wave : tid >> 5, ke_mq = tid & (ROWS / 4 - 1), kq_kk = tid >> 5, kq_mq = tid & 31;
   int64_t kq_col = q_base + 4 * kq_mq;
   if (KQ) kq_col = (kq_col + 4 <= ldq) ? kq_col : ldq - 4;
   const float* Qk = a.Q + (int64_t)k_off * ldq;
   int st_k0 = 0, ld_k0 = 0;  // first k of the staged chunk, of the chunk being loaded
-  f32x4 staged[8];             // passes 0..3: entity rows, 4..7: query rows
+  f32x4 staged[NP];            // passes 0..3: entity rows, then query rows
   int st_valid = 0;            // how many of this thread's four columns of the staged chunk are inside d
   int ld_valid = 0, ld_k = 0;  // the same, and the first column, for the chunk being loaded
   int ld_kc = 0;               // K chunk and first row of the tile the next loads fetch
@@ -1884,19 +1895,19 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
   auto load_pass = [&](int g) {
     const float* row_ptr;
     if (KE && g < 4) {
-      const int k = ld_k0 + 8 * g + ke_kk;
+      const int k = ld_k0 + KE_STEP * g + ke_kk;
       int64_t col = ld_row + 4 * ke_mq;
       col = (col + 4 <= r1) ? col : r1 - 4;
       staged[g] = *(const f32x4*)(Ef + (int64_t)(k < d ? k : 0) * lde + col);
       return;
     }
     if (KQ && g >= 4) {
-      const int k = ld_k0 + 8 * (g - 4) + kq_kk;
+      const int k = ld_k0 + KQ_STEP * (g - 4) + kq_kk;
       staged[g] = *(const f32x4*)(Qk + (int64_t)(k < d ? k : 0) * ldq + kq_col);
       return;
     }
     if (g < 4) {
-      int64_t er = ld_row + 32 * g;
+      int64_t er = ld_row + PASS * g;
       er = er < e_last ? er : e_last;
       row_ptr = Ef + er * lde;
     } else {
@@ -1912,18 +1923,18 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
   auto load_end = [&]() {
     const bool wrap = (ld_kc == nkc - 1);
     ld_kc = wrap ? 0 : ld_kc + 1;
-    ld_row += wrap ? KS_TILE_ROWS : 0;
+    ld_row += wrap ? ROWS : 0;
     st_valid = ld_valid;
     st_k0 = ld_k0;
   };
-  // 8-byte half (s_piece & 1) of 16-byte piece (s_piece >> 1); rows 32 g + s_row share the swizzle of s_row
+  // 8-byte half (s_piece & 1) of 16-byte piece (s_piece >> 1); rows PASS g + s_row share the swizzle of s_row
   const int st_off = s_row * 64 + ((((s_piece >> 1) ^ ((s_row >> 2) & 3)) << 4) | ((s_piece & 1) << 3));
-  auto store_pass = [&](int g) {
+  auto store_pass = [&](unsigned char* to, int g) {  // to: the buffer
     if ((KE && g < 4) || (KQ && g >= 4)) {
       const bool e_side = g < 4;
-      const int kk = e_side ? 8 * g + ke_kk : 8 * (g - 4) + kq_kk, mq = e_side ? ke_mq : kq_mq;
-      const int pitch = e_side ? 2 * KS_TILE_ROWS : 2 * KS_WG_QUERIES, plane = e_side ? KS_E_PLANE : KS_Q_PLANE;
-      unsigned char* base = lds + (e_side ? 0 : 3 * KS_E_PLANE) + kk * pitch +
+      const int kk = e_side ? KE_STEP * g + ke_kk : KQ_STEP * (g - 4) + kq_kk, mq = e_side ? ke_mq : kq_mq;
+      const int pitch = e_side ? 2 * ROWS : 2 * KS_WG_QUERIES, plane = e_side ? KS_E_PLANE : KS_Q_PLANE;
+      unsigned char* base = to + (e_side ? 0 : 3 * KS_E_PLANE) + kk * pitch +
                             ((((mq >> 2) ^ (2 * (kk & 3))) << 5) | ((mq & 3) << 3));
       f32x4 v = staged[g];
       const bool live = st_k0 + kk < d;
@@ -1935,7 +1946,7 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
       for (int part = 0; part < 3; ++part) *(bf16x4*)(base + part * plane) = s[part];
       return;
     }
-    unsigned char* base = lds + st_off + (g < 4 ? g * 2048 : 3 * KS_E_PLANE + (g - 4) * 2048);
+    unsigned char* base = to + st_off + (g < 4 ? g * (64 * PASS) : 3 * KS_E_PLANE + (g - 4) * (64 * PASS));
     const int plane = g < 4 ? KS_E_PLANE : KS_Q_PLANE;
     f32x4 v = staged[g];
 #pragma unroll
@@ -1973,46 +1984,85 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[te][tq][i] = 0.f;
 
+  // One K step of 16 of a buffer: its fragments, and products m0 .. m1 of its 24 (in order, four tiles each)
+  struct Step {
+    bf16x8 e[3][2], q[3][2];
+  };
+  auto read_step = [&](const unsigned char* from, int ks, Step& f) {
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        if constexpr (KE)
+          f.e[part][t] = tr_fragment(from + part * KS_E_PLANE, 2 * ROWS, 64 * we + 32 * t, ks);
+        else
+          f.e[part][t] = *(const bf16x8*)(from + 64 * we * 64 + part * KS_E_PLANE + t * 2048 + foff[ks]);
+        if constexpr (KQ)
+          f.q[part][t] = tr_fragment(from + 3 * KS_E_PLANE + part * KS_Q_PLANE, 2 * KS_WG_QUERIES, 64 * wq + 32 * t, ks);
+        else
+          f.q[part][t] = *(const bf16x8*)(from + 3 * KS_E_PLANE + 64 * wq * 64 + part * KS_Q_PLANE + t * 2048 + foff[ks]);
+      }
+  };
+  auto multiply = [&](const Step& f, int m0, int m1) {
+#pragma unroll
+    for (int m = m0; m < m1; ++m) {
+      const int p = m / 4, te = (m >> 1) & 1, tq = m & 1;
+      acc[te][tq] = Epi::SWAP ? mfma_bf16(f.q[SPLIT_B[p]][tq], f.e[SPLIT_A[p]][te], acc[te][tq])
+                              : mfma_bf16(f.e[SPLIT_A[p]][te], f.q[SPLIT_B[p]][tq], acc[te][tq]);
+    }
+  };
   auto load_chunk = [&]() {  // past the last chunk the clamped addresses still point into the tables
     load_begin();
 #pragma unroll
-    for (int g = 0; g < 8; ++g) load_pass(g);
+    for (int g = 0; g < NP; ++g) load_pass(g);
     load_end();
   };
-  if (n_it > 0) load_chunk();
+  if (n_it > 0) {
+    load_chunk();
+    if constexpr (WIDE) {
+      load_begin();
+#pragma unroll
+      for (int g = 0; g < NP; ++g) {
+        store_pass(lds, g);
+        load_pass(g);
+      }
+      load_end();
+    }
+  }
+  if constexpr (WIDE) __syncthreads();
   int kc = 0;
   int64_t et0 = r0;
-  const unsigned char* be = lds + (64 * we) * 64;
-  const unsigned char* bq = lds + 3 * KS_E_PLANE + (64 * wq) * 64;
   for (int it = 0; it < n_it; ++it) {
+    if constexpr (WIDE) {
+      // The iteration in six slices, fenced so that each keeps its share of the work: eight of the chunk's
+      // 48 MFMAs, and the split + store of one staged pass of chunk it+1 followed by the load of that pass of
+      // chunk it+2.  Unconditional on purpose (no branches inside the iteration): after the last chunk this
+      // stores and loads a chunk nobody reads.
+      const unsigned char* cur = lds + (it & 1) * KS_STAGE_BYTES;
+      unsigned char* next = lds + ((it & 1) ^ 1) * KS_STAGE_BYTES;
+      Step f[2];
+      read_step(cur, 0, f[0]);
+      load_begin();
 #pragma unroll
-    for (int g = 0; g < 8; ++g) store_pass(g);
-    __syncthreads();
-    load_chunk();
+      for (int sl = 0; sl < 6; ++sl) {
+        if (sl == 2) read_step(cur, 1, f[1]);
+        store_pass(next, sl);
+        load_pass(sl);
+        multiply(f[sl / 3], 8 * (sl % 3), 8 * (sl % 3) + 8);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      load_end();
+    } else {
 #pragma unroll
-    for (int ks = 0; ks < KS_KC / 16; ++ks) {
-      bf16x8 fe[3][2], fq[3][2];
+      for (int g = 0; g < NP; ++g) store_pass(lds, g);
+      __syncthreads();
+      load_chunk();
 #pragma unroll
-      for (int part = 0; part < 3; ++part)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          if constexpr (KE)
-            fe[part][t] = tr_fragment(lds + part * KS_E_PLANE, 2 * KS_TILE_ROWS, 64 * we + 32 * t, ks);
-          else
-            fe[part][t] = *(const bf16x8*)(be + part * KS_E_PLANE + t * 2048 + foff[ks]);
-          if constexpr (KQ)
-            fq[part][t] = tr_fragment(lds + 3 * KS_E_PLANE + part * KS_Q_PLANE, 2 * KS_WG_QUERIES, 64 * wq + 32 * t, ks);
-          else
-            fq[part][t] = *(const bf16x8*)(bq + part * KS_Q_PLANE + t * 2048 + foff[ks]);
-        }
-#pragma unroll
-      for (int p = 0; p < SPLIT_PRODUCTS; ++p)
-#pragma unroll
-        for (int te = 0; te < 2; ++te)
-#pragma unroll
-          for (int tq = 0; tq < 2; ++tq)
-            acc[te][tq] = Epi::SWAP ? mfma_bf16(fq[SPLIT_B[p]][tq], fe[SPLIT_A[p]][te], acc[te][tq])
-                                    : mfma_bf16(fe[SPLIT_A[p]][te], fq[SPLIT_B[p]][tq], acc[te][tq]);
+      for (int ks = 0; ks < KS_KC / 16; ++ks) {
+        Step f;
+        read_step(lds, ks, f);
+        multiply(f, 0, 24);
+      }
     }
     if (kc == nkc - 1) {  // this entity tile is complete
       float sc16[16];
@@ -2029,7 +2079,7 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
           for (int i = 0; i < 16; ++i) acc[te][tq][i] = 0.f;
       }
       kc = 0;
-      et0 += KS_TILE_ROWS;
+      et0 += ROWS;
       if (Epi::STAGE_HOOK) epi.stage_mark();
       __syncthreads();
       if (Epi::STAGE_HOOK) epi.stage_end();
@@ -2041,14 +2091,14 @@ __device__ __forceinline__ void ksplit_body(const ContractArgs& a, const typenam
   epi.finish();
 }
 
-template <template <int> class EpiT, bool VEC>
-__global__ void __launch_bounds__(256, 2) ksplit_kernel(ContractArgs a, typename EpiT<KS_NQT>::Args ea) {
-  ksplit_body<EpiT, VEC, 0>(a, ea);
+template <template <int> class EpiT, bool VEC, int ROWS>
+__global__ void __launch_bounds__(ks_threads(ROWS), 2) ksplit_kernel(ContractArgs a, typename EpiT<KS_NQT>::Args ea) {
+  ksplit_body<EpiT, VEC, 0, ROWS>(a, ea);
 }
 // the same with K-major operands (KMAJ = 1: the entity operand, 3: both)
-template <template <int> class EpiT, int KMAJ>
-__global__ void __launch_bounds__(256, 2) ksplit_kmajor_kernel(ContractArgs a, typename EpiT<KS_NQT>::Args ea) {
-  ksplit_body<EpiT, true, KMAJ>(a, ea);
+template <template <int> class EpiT, int KMAJ, int ROWS>
+__global__ void __launch_bounds__(ks_threads(ROWS), 2) ksplit_kmajor_kernel(ContractArgs a, typename EpiT<KS_NQT>::Args ea) {
+  ksplit_body<EpiT, true, KMAJ, ROWS>(a, ea);
 }
 
 // ============================================================================================

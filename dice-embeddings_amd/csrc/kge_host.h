@@ -36,8 +36,8 @@ constexpr int TOPK_MAX_K = 1024;
 constexpr int TOPK_FIRST_ROWS = 1024;    // first round takes everything: must not exceed TOPK_CAP
 constexpr int BCE_SLOTS = 128;
 constexpr int KS_WG_QUERIES = 128;       // workgroup shape of the fp32 contraction (also sizes the backward's K split)
-constexpr int KS_TILE_ROWS = 128;
-constexpr int KS_WGS = 512;              // workgroups of that shape the chip holds: two per CU
+constexpr int KS_NARROW_ROWS = 128;      // entity rows of its narrow form, two or three workgroups per CU,
+constexpr int KS_WIDE_ROWS = 256;        // and of its wide form, one per CU
 constexpr int KB_TILE_ROWS = 256;        // entity rows of the bf16 / int8 contraction of wide rows, one workgroup per CU
 
 // Work decomposition of the four-tile filtered-rank main loop (bf16 tables, d == 128): 8-wave workgroups of
@@ -93,6 +93,61 @@ inline void flat_walk(int groups, int64_t rows, int stage_rows, int max_chunk, i
 // workgroups of a persistent launch of either form
 inline int64_t walk_grid(int groups, int n_lanes, int lanes_flat) {
   return lanes_flat ? ((int64_t)groups * lanes_flat + 7) / 8 * 8 : 8 * (int64_t)groups * n_lanes;
+}
+
+// ---- work decomposition of the tiled contractions (decompose_wg) -----------------------------------------------------
+inline int64_t contract_wgs(int64_t n_chunks, int n_qgroups) {  // workgroups of a launch
+  return (n_chunks < 8 ? n_chunks : (n_chunks + 7) / 8 * 8) * n_qgroups;
+}
+// The chunk length whose last round of `resident` workgroups is fullest, preferring longer chunks (less per-workgroup
+// set-up) among near-equal candidates.
+inline int fullest_chunk(int64_t rows, int n_qgroups, int tile, int64_t resident) {
+  int best_chunk = tile;
+  double best_eff = -1.0;
+  for (int chunk = tile; chunk <= 1024; chunk += tile) {
+    const int64_t rounds = (contract_wgs((rows + chunk - 1) / chunk, n_qgroups) + resident - 1) / resident;
+    const double eff = (double)rows * n_qgroups / ((double)rounds * (double)resident * (double)chunk);
+    if (eff > best_eff + 0.02) {
+      best_eff = eff;
+      best_chunk = chunk;
+    } else if (eff > best_eff - 0.02 && rounds >= 2) {
+      best_chunk = chunk;  // about as full, fewer and longer workgroups
+      if (eff > best_eff) best_eff = eff;
+    }
+  }
+  return best_chunk;
+}
+
+// Which form of the fp32 contraction a launch takes, and its chunk length.  Time is counted in K chunks of 32 columns of one
+// 256 x 128 tile on a CU of its own.  A wide workgroup takes wide_wg for its first loads and its end, and per tile its K
+// chunks and wide_tile for the epilogue; the busiest CU runs ceil(workgroups / 256) of them in turn.  Of the narrow
+// workgroups a CU holds three: the busiest one takes together[m] times as long for m of them as a wide workgroup's K chunks
+// over the same number of tiles would.  The constants are fits, per epilogue, over 11 widths, 10 table sizes and 12 batches,
+// both forms timed on one card.  Against always taking the faster form the choice costs 0.3 % on average, more than 4 % for
+// one shape in forty (always narrow 2 %, one in six; always wide 8 %, one in two); the largest losses, 8 - 17 %, are scores
+// of a few hundred to thousands of queries at d <= 64, whose time is their store's.
+constexpr int KS_NARROW_PER_CU = 3;
+struct KsCost {
+  double wide_tile, wide_wg, narrow_tile, narrow_wg;
+  double together[KS_NARROW_PER_CU + 1];
+};
+struct KsPlan {
+  int tile_rows, chunk_rows;
+  int64_t n_chunks;
+};
+// narrow_factor: what the narrow form loses besides
+inline KsPlan ks_plan(const KsCost& c, int64_t rows, int n_qgroups, int64_t d, double narrow_factor) {
+  const double k_chunks = (double)((d + 31) / 32);
+  auto chunks = [&](int chunk) { return (rows + chunk - 1) / chunk; };
+  auto busiest = [&](int chunk) { return (contract_wgs(chunks(chunk), n_qgroups) + 255) / 256; };  // workgroups of a CU
+  const int wide = fullest_chunk(rows, n_qgroups, KS_WIDE_ROWS, 256);
+  const int narrow = fullest_chunk(rows, n_qgroups, KS_NARROW_ROWS, 512);
+  const double t_wide = (double)busiest(wide) * (wide / KS_WIDE_ROWS * (k_chunks + c.wide_tile) + c.wide_wg);
+  const int64_t m = busiest(narrow);
+  const double t_narrow = ((double)(m / KS_NARROW_PER_CU) * c.together[KS_NARROW_PER_CU] + c.together[m % KS_NARROW_PER_CU]) *
+                          narrow_factor * (narrow / KS_NARROW_ROWS * (k_chunks + c.narrow_tile) + c.narrow_wg);
+  if (t_narrow < t_wide) return KsPlan{KS_NARROW_ROWS, narrow, chunks(narrow)};
+  return KsPlan{KS_WIDE_ROWS, wide, chunks(wide)};
 }
 
 struct Status {
@@ -310,6 +365,7 @@ inline size_t bce_ws_bytes() { return (2 * BCE_SLOTS + BCE_POS_SLOTS) * sizeof(d
 struct BwdPlan {
   int64_t ldG, ldT;  // row strides of G [B, ldG] (a multiple of 32) and GT [N, ldT] (a multiple of 4)
   int k_splits, k_split_len;
+  int dq_rows;  // dQ's form of the contraction
   bool kmajor;  // d a multiple of 4: the gradient contractions read G, E and Q where they lie (no GT, ET, QT)
   size_t off_G, off_GT, off_ET, off_QT, off_part, total;
 };
@@ -317,9 +373,14 @@ inline BwdPlan bwd_plan(int64_t B, int64_t d, int64_t N) {
   BwdPlan p{};
   p.ldG = (N + 31) / 32 * 32;  // rows start on 128-byte lines: a wave's run of 32 gradients is one whole line
   p.ldT = (B + 3) / 4 * 4;
-  // dQ = G . E sums over N: split so that about KS_WGS workgroups run
-  const int64_t tiles = ((B + KS_WG_QUERIES - 1) / KS_WG_QUERIES) * ((d + KS_TILE_ROWS - 1) / KS_TILE_ROWS);
-  int64_t splits = (KS_WGS + tiles - 1) / tiles;
+  // dQ = G . E sums over N, at most 64 ways: split so that every CU gets a wide workgroup or two narrow ones.  Narrow where
+  // half a wide tile of d would be padding (d = 128, B = 1000, N = 41k 104 -> 66 us), where 64 splits leave CUs without a wide
+  // workgroup (d = 256, B = 128, N = 41k 47 -> 42 us), and where a workgroup's sum is short (d = 256, B = 500, N = 1000 14.3 -> 12.0 us); elsewhere
+  // wide (d = 256, N = 41k, B = 1000 111 us for 118, B = 2048 211 for 228).
+  const int64_t groups = (B + KS_WG_QUERIES - 1) / KS_WG_QUERIES;
+  const int64_t wide = groups * ((d + KS_WIDE_ROWS - 1) / KS_WIDE_ROWS), narrow = groups * ((d + KS_NARROW_ROWS - 1) / KS_NARROW_ROWS);
+  p.dq_rows = (narrow < 2 * wide || wide * 64 < 256 || N * wide < 65536) ? KS_NARROW_ROWS : KS_WIDE_ROWS;
+  int64_t splits = p.dq_rows == KS_WIDE_ROWS ? (256 + wide - 1) / wide : (512 + narrow - 1) / narrow;
   if (splits > 64) splits = 64;
   if (splits < 1) splits = 1;
   const int64_t len = ((N + splits - 1) / splits + 31) / 32 * 32;

@@ -1240,11 +1240,14 @@ ContractArgs make_args(const float* Q, const void* E, int dtype, const float* sc
   a.k_split_len = 0;
   a.k_split_xcd = 0;
   a.persistent = 0;
+  a.ks_rows = 0;
+  a.chunk_rows = 0;
+  a.n_chunks = 0;
   const RowClass rc = row_class(d);
   const bool fast_bf16 = dtype == KGE_BF16 && rc.lds_d != 0;  // (persistent whatever the epilogue)
   const bool fast_i8 = dtype == KGE_I8 && rc.lds_d != 0;
   const bool wide_q = wide_query_rows(dtype, d);  // qwide_kernel: persistent, one 32-query tile per wave
-  const bool wide_bf16 = (dtype == KGE_BF16 || dtype == KGE_I8) && rc.lds_d == 0 && !wide_q;  // kchunk_kernel: the workgroup shape of the split kernel
+  const bool wide_bf16 = (dtype == KGE_BF16 || dtype == KGE_I8) && rc.lds_d == 0 && !wide_q;  // kchunk_kernel: the queries per workgroup of the split kernel
   const int wgq = (dtype == KGE_F32 || wide_bf16) ? KS_WG_QUERIES : wide_q ? QW_WG_QUERIES : rc.lds_d == 256 ? QS256_WG_QUERIES
                   : fast_bf16 ? QA_WG_QUERIES : I8_WG_QUERIES;
   a.n_qgroups = (int)((B + wgq - 1) / wgq);
@@ -1266,35 +1269,40 @@ ContractArgs make_args(const float* Q, const void* E, int dtype, const float* sc
     a.persistent = 1;
     return a;
   }
-  // non-persistent paths (the split kernel: 128 entity rows, two workgroups per CU; kchunk_kernel: 256, one): one
-  // workgroup per (query group, chunk), `resident` workgroups at a time; choose the chunk length whose last round of
-  // workgroups is fullest, preferring longer chunks (less per-workgroup set-up) among near-equal candidates.
-  const int tile = dtype == KGE_F32 ? KS_TILE_ROWS : host::KB_TILE_ROWS;
-  const int max_chunk = 1024;
-  const int64_t resident = dtype == KGE_F32 ? host::KS_WGS : 256;
-  int64_t best_chunk = tile;
-  double best_eff = -1.0;
-  for (int64_t chunk = tile; chunk <= max_chunk; chunk += tile) {
-    const int64_t n_chunks = (rows + chunk - 1) / chunk;
-    const int64_t wgs = (n_chunks < 8) ? n_chunks * a.n_qgroups : (n_chunks + 7) / 8 * 8 * a.n_qgroups;
-    const int64_t rounds = (wgs + resident - 1) / resident;
-    const double eff = (double)rows * a.n_qgroups / ((double)rounds * (double)resident * (double)chunk);
-    if (eff > best_eff + 0.02) {
-      best_eff = eff;
-      best_chunk = chunk;
-    } else if (eff > best_eff - 0.02 && rounds >= 2) {
-      best_chunk = chunk;  // about as full, fewer and longer workgroups
-      if (eff > best_eff) best_eff = eff;
-    }
-  }
-  a.chunk_rows = (int)best_chunk;
-  a.n_chunks = (rows + best_chunk - 1) / best_chunk;
+  // tiled paths: one workgroup per (query group, chunk); the split kernel's chunks depend on the epilogue and are planned
+  // where it is launched
+  if (dtype == KGE_F32) return a;
+  a.chunk_rows = host::fullest_chunk(rows, a.n_qgroups, host::KB_TILE_ROWS, 256);
+  a.n_chunks = (rows + a.chunk_rows - 1) / a.chunk_rows;
   return a;
 }
 
-// workgroups of a non-persistent contraction launch: what decompose_wg() expects
-static int64_t contract_grid_wgs(const ContractArgs& a) {
-  return (a.n_chunks < 8) ? a.n_chunks * a.n_qgroups : (a.n_chunks + 7) / 8 * 8 * a.n_qgroups;
+// workgroups of a tiled contraction launch: what decompose_wg() expects
+static int64_t contract_grid_wgs(const ContractArgs& a) { return host::contract_wgs(a.n_chunks, a.n_qgroups); }
+
+// The split kernel's decomposition under an epilogue (host::ks_plan; forced: this form whatever the plan says).
+template <template <int> class EpiT>
+void plan_ksplit(ContractArgs& a, bool rows_aligned, int forced = 0) {
+  using E = EpiT<2>;
+  constexpr bool store = std::is_same<E, StoreEpi<2>>::value, store_t = std::is_same<E, StoreTEpi<2>>::value;
+  constexpr host::KsCost cost = store     ? host::KsCost{2.2, 1.2, 1.7, 0.2, {0, 0.74, 1.2, 1.56}}
+                                : store_t ? host::KsCost{1.7, 2.0, 1.1, 0.6, {0, 0.83, 1.25, 1.75}}
+                                          : host::KsCost{0.4, 1.0, 0.0, 0.65, {0, 0.82, 1.12, 1.6}};
+  const int64_t rows = a.e_end - a.e_begin;
+  // the score gradients (sigmoids and a store per score) are always faster narrow: N = 41k, d = 256, B = 2048 375 -> 345 us
+  if (std::is_same<E, GradEpi<2>>::value && !forced) forced = KS_NARROW_ROWS;
+  if (forced) {
+    a.ks_rows = forced;
+    a.chunk_rows = host::fullest_chunk(rows, a.n_qgroups, forced, forced == KS_NARROW_ROWS ? 512 : 256);
+    a.n_chunks = (rows + a.chunk_rows - 1) / a.chunk_rows;
+    return;
+  }
+  // (rows that cannot be loaded 16 bytes at a time take four loads for one, which the narrow form waits for between its
+  // barriers: ranks of 1000 queries, N = 41k, d = 201 157 us wide, 203 narrow)
+  const host::KsPlan p = host::ks_plan(cost, rows, a.n_qgroups, a.d, rows_aligned ? 1.0 : 1.15);
+  a.ks_rows = p.tile_rows;
+  a.chunk_rows = p.chunk_rows;
+  a.n_chunks = p.n_chunks;
 }
 
 // HIP events around a main-loop launch while kge_profile_begin() is in effect (the bench's per-launch timing)
@@ -1337,8 +1345,24 @@ constexpr const char* epilogue_name() {
 }
 
 template <template <int> class EpiT, class EArgs>
-int launch_contract(int dtype, const ContractArgs& a, const EArgs& ea, hipStream_t st, const char* name) {
+void ksplit_go(bool rows_aligned, dim3 grid, dim3 block, hipStream_t st, const ContractArgs& a, const EArgs& ea) {
+  constexpr bool narrow_only = std::is_same<EpiT<2>, GradEpi<2>>::value;
+  if constexpr (!narrow_only) {
+    if (a.ks_rows == KS_WIDE_ROWS) {
+      if (rows_aligned) hipLaunchKernelGGL((ksplit_kernel<EpiT, true, KS_WIDE_ROWS>), grid, block, 0, st, a, ea);
+      else hipLaunchKernelGGL((ksplit_kernel<EpiT, false, KS_WIDE_ROWS>), grid, block, 0, st, a, ea);
+      return;
+    }
+  }
+  if (rows_aligned) hipLaunchKernelGGL((ksplit_kernel<EpiT, true, KS_NARROW_ROWS>), grid, block, 0, st, a, ea);
+  else hipLaunchKernelGGL((ksplit_kernel<EpiT, false, KS_NARROW_ROWS>), grid, block, 0, st, a, ea);
+}
+
+template <template <int> class EpiT, class EArgs>
+int launch_contract(int dtype, ContractArgs a, const EArgs& ea, hipStream_t st, const char* name) {
   if (a.B == 0 || a.e_end <= a.e_begin) return KGE_OK;
+  const bool rows_aligned = (a.d % 4 == 0) && (((uintptr_t)a.E | (uintptr_t)a.Q) % 16 == 0);
+  if (dtype == KGE_F32) plan_ksplit<EpiT>(a, rows_aligned);
   const RowClass rc = row_class(a.d);
   const bool fast_bf16 = dtype == KGE_BF16 && rc.lds_d != 0;
   const bool fast_i8 = dtype == KGE_I8 && rc.lds_d != 0;
@@ -1353,18 +1377,15 @@ int launch_contract(int dtype, const ContractArgs& a, const EArgs& ea, hipStream
   const bool f32_split = (dtype == KGE_F32);
   const bool wide_bf16 = (dtype == KGE_BF16 || dtype == KGE_I8) && rc.lds_d == 0 && !wide_q;
   dim3 grid((unsigned)nwg), block(fast_i8 ? 64 * I8_WG_WAVES : wide_q ? 64 * QW_WG_WAVES : persistent ? 64 * QA_WG_WAVES
-                                         : f32_split ? 256 : 512);
+                                         : f32_split ? ks_threads(a.ks_rows) : 512);
   LaunchTimer timer;
   if (int trc = timer.begin(st)) return trc;
   char kname[160];  // the kernel as dispatched below, for kge_profile_kernel()
   const char* epi = epilogue_name<EpiT>();
-  const bool rows_aligned = (a.d % 4 == 0) && (((uintptr_t)a.E | (uintptr_t)a.Q) % 16 == 0);
-  if (f32_split) snprintf(kname, sizeof(kname), "ksplit_kernel<%s, %s>", epi, rows_aligned ? "true" : "false");
+  if (f32_split) snprintf(kname, sizeof(kname), "ksplit_kernel<%s, %s, %d>", epi, rows_aligned ? "true" : "false", a.ks_rows);
   else if (wide_bf16) snprintf(kname, sizeof(kname), "kchunk_kernel<%s, %s>", dtype == KGE_BF16 ? "KGE_BF16" : "KGE_I8", epi);
-  if (f32_split && rows_aligned)
-    hipLaunchKernelGGL((ksplit_kernel<EpiT, true>), grid, block, 0, st, a, ea);
-  else if (f32_split)
-    hipLaunchKernelGGL((ksplit_kernel<EpiT, false>), grid, block, 0, st, a, ea);
+  if (f32_split)
+    ksplit_go<EpiT>(rows_aligned, grid, block, st, a, ea);
   else if (wide_bf16 && dtype == KGE_BF16)
     hipLaunchKernelGGL((kchunk_kernel<KGE_BF16, EpiT>), grid, block, 0, st, a, ea);
   else if (wide_bf16)
@@ -1464,50 +1485,48 @@ int launch_rank128(const ContractArgs& base, const RankArgs& ea, hipStream_t st,
 }
 
 // ksplit_kernel alone (fp32 operands), with row strides and an optional split of K over grid.y.
-// kmaj (StoreEpi only): bit 0 / bit 1: the entity / query operand is K-major (ksplit_kmajor_kernel).
+// kmaj (StoreEpi / StoreTEpi only): bit 0 / bit 1: the entity / query operand is K-major (ksplit_kmajor_kernel).
 template <template <int> class EpiT, class EArgs>
-int launch_ksplit(const ContractArgs& a, const EArgs& ea, unsigned k_splits, hipStream_t st, const char* name,
-                  int kmaj = 0) {
+int launch_ksplit(ContractArgs a, const EArgs& ea, unsigned k_splits, hipStream_t st, const char* name, int kmaj = 0,
+                  int form = 0) {
   if (a.B == 0 || a.e_end <= a.e_begin) return KGE_OK;
-  const int64_t nwg = contract_grid_wgs(a);
-  KGE_REQUIRE(nwg <= 0x7fffffffLL && k_splits >= 1 && k_splits <= 65535, KGE_ERR_INVALID,
-              "%s: grid of %lld x %u workgroups too large", name, (long long)nwg, k_splits);
   const int ldq = a.ldq ? a.ldq : a.d, lde = a.lde ? a.lde : a.d;
   const bool rows_aligned = (ldq % 4 == 0) && (lde % 4 == 0) && (((uintptr_t)a.E | (uintptr_t)a.Q) % 16 == 0) &&
                             (a.k_split_len % 4 == 0);
-  dim3 grid((unsigned)nwg, k_splits), block(256);
+  plan_ksplit<EpiT>(a, rows_aligned, form);
+  const int64_t nwg = contract_grid_wgs(a);
+  KGE_REQUIRE(nwg <= 0x7fffffffLL && k_splits >= 1 && k_splits <= 65535, KGE_ERR_INVALID,
+              "%s: grid of %lld x %u workgroups too large", name, (long long)nwg, k_splits);
+  dim3 grid((unsigned)nwg, k_splits), block(ks_threads(a.ks_rows));
   LaunchTimer timer;
   if (int trc = timer.begin(st)) return trc;
-  if constexpr (std::is_same<EpiT<KS_NQT>, StoreEpi<KS_NQT>>::value || std::is_same<EpiT<KS_NQT>, StoreTEpi<KS_NQT>>::value) {
+  char kname[160];
+  constexpr bool store = std::is_same<EpiT<KS_NQT>, StoreEpi<KS_NQT>>::value;
+  constexpr bool store_t = std::is_same<EpiT<KS_NQT>, StoreTEpi<KS_NQT>>::value;
+  if constexpr (store || store_t) {
     if (kmaj) {
       // a K-major operand: whole quads of rows, 16-byte aligned (the caller chooses this form only then)
-      KGE_REQUIRE(rows_aligned && (a.e_end - a.e_begin) % 4 == 0 && a.e_begin % 4 == 0 && (kmaj == 1 || kmaj == 3),
-                  KGE_ERR_INVALID, "%s: K-major operands need aligned quads of rows", name);
+      constexpr int KMAJ = store ? 1 : 3;
+      KGE_REQUIRE(rows_aligned && (a.e_end - a.e_begin) % 4 == 0 && a.e_begin % 4 == 0 && kmaj == KMAJ, KGE_ERR_INVALID,
+                  "%s: K-major operands need aligned quads of rows", name);
       // K ranges in eights with few entity chunks: a flat grid that keeps every range on one XCD (the workgroups of
       // a range read the same rows of the K-major entity operand)
-      ContractArgs ax = a;
       if (k_splits % 8 == 0 && a.n_chunks < 8 && nwg * k_splits <= 0x7fffffffLL) {
-        ax.k_split_xcd = (int)k_splits;
+        a.k_split_xcd = (int)k_splits;
         grid = dim3((unsigned)(nwg * k_splits), 1);
       }
-      if (kmaj == 1) hipLaunchKernelGGL((ksplit_kmajor_kernel<EpiT, 1>), grid, block, 0, st, ax, ea);
-      else hipLaunchKernelGGL((ksplit_kmajor_kernel<EpiT, 3>), grid, block, 0, st, ax, ea);
+      if (a.ks_rows == KS_WIDE_ROWS) hipLaunchKernelGGL((ksplit_kmajor_kernel<EpiT, KMAJ, KS_WIDE_ROWS>), grid, block, 0, st, a, ea);
+      else hipLaunchKernelGGL((ksplit_kmajor_kernel<EpiT, KMAJ, KS_NARROW_ROWS>), grid, block, 0, st, a, ea);
       KGE_LAUNCH_CHECK(name);
-      char kname[160];
-      snprintf(kname, sizeof(kname), "ksplit_kmajor_kernel<%s, %d>", epilogue_name<EpiT>(), kmaj);
-      if (int trc = timer.end(kname)) return trc;
-      return KGE_OK;
+      snprintf(kname, sizeof(kname), "ksplit_kmajor_kernel<%s, %d, %d>", epilogue_name<EpiT>(), kmaj, a.ks_rows);
+      return timer.end(kname);
     }
   }
-  if (rows_aligned)
-    hipLaunchKernelGGL((ksplit_kernel<EpiT, true>), grid, block, 0, st, a, ea);
-  else
-    hipLaunchKernelGGL((ksplit_kernel<EpiT, false>), grid, block, 0, st, a, ea);
+  if constexpr (store_t) return set_error(KGE_ERR_INVALID, "%s: a transposed store takes K-major operands", name);
+  else ksplit_go<EpiT>(rows_aligned, grid, block, st, a, ea);
   KGE_LAUNCH_CHECK(name);
-  char kname[160];
-  snprintf(kname, sizeof(kname), "ksplit_kernel<%s, %s>", epilogue_name<EpiT>(), rows_aligned ? "true" : "false");
-  if (int trc = timer.end(kname)) return trc;
-  return KGE_OK;
+  snprintf(kname, sizeof(kname), "ksplit_kernel<%s, %s, %d>", epilogue_name<EpiT>(), rows_aligned ? "true" : "false", a.ks_rows);
+  return timer.end(kname);
 }
 
 #define KGE_DISPATCH_DTYPE(dtype, KERNEL, grid, block, shmem, st, ...)                       \
@@ -2234,7 +2253,8 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
     b.lde = kmajor ? (int)d : (int)p.ldG;
     b.k_split_len = p.k_split_len;
     StoreArgs sa{p.k_splits > 1 ? part : dQ, nullptr, d, (int64_t)B * d};
-    rc = launch_ksplit<StoreEpi>(b, sa, (unsigned)p.k_splits, st, "kge_bce_multihot_backward: dQ", kmajor ? 1 : 0);
+    rc = launch_ksplit<StoreEpi>(b, sa, (unsigned)p.k_splits, st, "kge_bce_multihot_backward: dQ", kmajor ? 1 : 0,
+                                 p.dq_rows);
     if (rc) return rc;
     if (p.k_splits > 1) {
       const int64_t n = B * d;
@@ -2247,7 +2267,7 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
   {
     if (kmajor) {
       // the rows of Q as the "queries", the rows of G (N of them, read up to the padded pitch) as the "entities": a
-      // workgroup's share of G is 128 neighbouring columns (512 bytes of every row), and the result is stored transposed
+      // workgroup's share of G is 256 or 128 neighbouring columns of every row, and the result is stored transposed
       ContractArgs b = make_args(Q, G, KGE_F32, nullptr, d, B, p.ldG, 0, p.ldG);
       b.ldq = (int)d;
       b.lde = (int)p.ldG;

@@ -287,8 +287,36 @@ static void test_flat_walk() {
     }
 }
 
+// the fp32 contraction's plans: whole tiles of their form, every row in exactly one chunk; and dQ's split of the summed index
+static void test_ks_plan() {
+  const KsCost store{2.2, 1.2, 1.7, 0.2, {0, 0.74, 1.2, 1.56}}, rank{0.4, 1.0, 0.0, 0.65, {0, 0.82, 1.12, 1.6}};
+  int narrow = 0, wide = 0;
+  for (const KsCost& c : {store, rank})
+    for (int64_t rows : {1LL, 127LL, 128LL, 129LL, 257LL, 1000LL, 14541LL, 100003LL, 2500000LL, 2147483647LL})
+      for (int groups : {1, 2, 7, 40, 131072})
+        for (int64_t d : {1, 32, 33, 200, 256, 512, 65536})
+          for (double f : {1.0, 1.15}) {
+            const KsPlan p = ks_plan(c, rows, groups, d, f);
+            CHECK(p.tile_rows == KS_NARROW_ROWS || p.tile_rows == KS_WIDE_ROWS);
+            CHECK(p.chunk_rows >= p.tile_rows && p.chunk_rows <= 1024 && p.chunk_rows % p.tile_rows == 0);
+            CHECK(p.n_chunks * p.chunk_rows >= rows && (p.n_chunks - 1) * p.chunk_rows < rows);
+            CHECK(contract_wgs(p.n_chunks, groups) >= p.n_chunks * groups);
+            ++(p.tile_rows == KS_WIDE_ROWS ? wide : narrow);
+          }
+  CHECK(narrow > 0 && wide > 0);
+  for (int64_t N : {1, 31, 135, 8191, 40943, 16777216})
+    for (int64_t B : {1, 128, 129, 2048, 100000})
+      for (int64_t d : {1, 4, 128, 132, 256, 400}) {
+        const BwdPlan p = bwd_plan(B, d, N);
+        CHECK(p.dq_rows == KS_NARROW_ROWS || p.dq_rows == KS_WIDE_ROWS);
+        CHECK(p.k_splits >= 1 && p.k_splits <= 64 && p.k_split_len % 32 == 0);
+        CHECK((int64_t)p.k_splits * p.k_split_len >= N && (int64_t)(p.k_splits - 1) * p.k_split_len < N);
+      }
+}
+
 int main() {
   test_flat_walk();
+  test_ks_plan();
   test_contract_rules();
   test_layouts();
   test_csr_keys();
