@@ -332,6 +332,12 @@ inline size_t few_topk_ws_bytes(int64_t B, int64_t N, int64_t k) {
   return (B <= FEW_MAX_B && k <= FEW_MAX_K && N <= FEW_MAX_N) ? (size_t)few_topk_ws(B, N).total * 4 : 0;
 }
 
+// What a call is offered; topk_ws_offsets().total, which grows with B, N and k, is what it takes at least.
+inline size_t topk_ws_bytes(int64_t B, int64_t N, int64_t k, bool with_table) {
+  const size_t rounds = topk_ws_offsets(B, N, k, with_table).total, few = few_topk_ws_bytes(B, N, k);
+  return rounds > few ? rounds : few;
+}
+
 // The threshold a scan of `n_next` more rows may use once `ranked` rows are ranked: the j-th best score so far, j as
 // small as the order statistics allow.  Of the best k of all ranked + n_next rows, the number X that are among
 // the rows already ranked is hypergeometric (rows in exchangeable order), mean k rho, variance below

@@ -1896,8 +1896,7 @@ extern "C" size_t kge_topk_workspace_bytes(int64_t B, int64_t N, int64_t k) {
   if (N < 1) N = 1;
   if (k < 1) k = 1;
   if (k > TOPK_MAX_K) k = TOPK_MAX_K;
-  const size_t rounds = topk_ws_layout(B, N, k, nullptr, nullptr), few = host::few_topk_ws_bytes(B, N, k);
-  return rounds > few ? rounds : few;
+  return host::topk_ws_bytes(B, N, k, true);
 }
 
 namespace {
@@ -1915,7 +1914,7 @@ int topk_prepare_launch(const void* E, const float* scale, int64_t N, unsigned c
 
 int topk_impl(const char* who, const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B,
               int64_t d, int64_t N, int64_t k, float* out_scores, int64_t* out_idx, int apply_sigmoid,
-              const void* prepared, void* workspace, hipStream_t st);
+              const void* prepared, void* workspace, size_t workspace_bytes, hipStream_t st);
 }  // namespace
 
 extern "C" size_t kge_topk_prepared_bytes(int dtype, int64_t d, int64_t N) {
@@ -1945,8 +1944,7 @@ extern "C" size_t kge_topk_prepared_workspace_bytes(int64_t B, int64_t N, int64_
   if (N < 1) N = 1;
   if (k < 1) k = 1;
   if (k > TOPK_MAX_K) k = TOPK_MAX_K;
-  const size_t rounds = topk_ws_layout(B, N, k, nullptr, nullptr, nullptr, false), few = host::few_topk_ws_bytes(B, N, k);
-  return rounds > few ? rounds : few;
+  return host::topk_ws_bytes(B, N, k, false);
 }
 
 extern "C" int kge_topk(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B,
@@ -1960,11 +1958,12 @@ extern "C" int kge_topk(const float* Q, const float* bias, const void* E, int dt
               TOPK_MAX_K);
   if (B == 0) return KGE_OK;
   KGE_REQUIRE(out_scores && out_idx, KGE_ERR_INVALID, "kge_topk: null output pointer");
-  KGE_REQUIRE(workspace && workspace_bytes >= kge_topk_workspace_bytes(B, N, k), KGE_ERR_WORKSPACE,
-              "kge_topk: workspace of %zu bytes, need %zu", workspace_bytes, kge_topk_workspace_bytes(B, N, k));
+  const size_t need = host::topk_ws_offsets(B, N, k).total;
+  KGE_REQUIRE(workspace && workspace_bytes >= need, KGE_ERR_WORKSPACE, "kge_topk: workspace of %zu bytes, need %zu",
+              workspace_bytes, need);
   KGE_REQUIRE(((uintptr_t)workspace & 15) == 0, KGE_ERR_WORKSPACE, "kge_topk: workspace must be 16-byte aligned");
   return topk_impl("kge_topk", Q, bias, E, dtype, scale, B, d, N, k, out_scores, out_idx, apply_sigmoid, nullptr,
-                   workspace, (hipStream_t)stream);
+                   workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 extern "C" int kge_topk_prepared(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B,
@@ -1986,20 +1985,21 @@ extern "C" int kge_topk_prepared(const float* Q, const float* bias, const void* 
   KGE_REQUIRE(((uintptr_t)prepared & 15) == 0, KGE_ERR_INVALID, "kge_topk_prepared: prepared must be 16-byte aligned");
   if (B == 0) return KGE_OK;
   KGE_REQUIRE(out_scores && out_idx, KGE_ERR_INVALID, "kge_topk_prepared: null output pointer");
-  KGE_REQUIRE(workspace && workspace_bytes >= kge_topk_prepared_workspace_bytes(B, N, k), KGE_ERR_WORKSPACE,
-              "kge_topk_prepared: workspace of %zu bytes, need %zu", workspace_bytes,
-              kge_topk_prepared_workspace_bytes(B, N, k));
+  const size_t need = host::topk_ws_offsets(B, N, k, false).total;
+  KGE_REQUIRE(workspace && workspace_bytes >= need, KGE_ERR_WORKSPACE,
+              "kge_topk_prepared: workspace of %zu bytes, need %zu", workspace_bytes, need);
   KGE_REQUIRE(((uintptr_t)workspace & 15) == 0, KGE_ERR_WORKSPACE, "kge_topk_prepared: workspace must be 16-byte aligned");
   return topk_impl("kge_topk_prepared", Q, bias, E, dtype, scale, B, d, N, k, out_scores, out_idx, apply_sigmoid, prepared,
-                   workspace, (hipStream_t)stream);
+                   workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 namespace {
 int topk_impl(const char* who, const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B,
               int64_t d, int64_t N, int64_t k, float* out_scores, int64_t* out_idx, int apply_sigmoid,
-              const void* prepared, void* workspace, hipStream_t st) {
+              const void* prepared, void* workspace, size_t workspace_bytes, hipStream_t st) {
   int rc = KGE_OK;
-  if (host::few_topk_applies(dtype, B, d, N, k)) {
+  // (a workspace made for a larger batch may hold the rounds and not the few-query form)
+  if (host::few_topk_applies(dtype, B, d, N, k) && workspace_bytes >= host::few_topk_ws_bytes(B, N, k)) {
     LaunchTimer timer;
     if ((rc = timer.begin(st))) return rc;
     if ((rc = few_topk_launch(Q, bias, E, dtype, scale, B, d, N, k, out_scores, out_idx, apply_sigmoid, workspace, st))) return rc;

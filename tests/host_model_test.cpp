@@ -96,6 +96,17 @@ static void test_layouts() {
       }
     }
   }
+  // a workspace that was offered to a larger call holds every smaller one: what a call takes at least grows with B, N and k
+  for (bool table : {true, false})
+    for (int64_t N : {1000LL, 65536LL, 100000LL, 10000000LL})
+      for (int64_t k : {1LL, 10LL, 128LL, 129LL, 1024LL})
+        for (int64_t B : {1LL, 32LL, 100LL, 128LL, 129LL, 512LL, 1024LL}) {
+          const size_t offered = topk_ws_bytes(B, N, k, table);
+          for (int64_t b : {1LL, 31LL, 100LL, 128LL, 129LL, 512LL})
+            for (int64_t j : {1LL, 10LL, 100LL, 128LL, 129LL, 1000LL})
+              if (b <= B && j <= k) CHECK(topk_ws_offsets(b, N, j, table).total <= offered);
+          if (B <= FEW_MAX_B && k <= FEW_MAX_K) CHECK(few_topk_ws_bytes(B, N, k) <= offered);
+        }
   // the rank whose score a scan may use as its threshold: between the expected number of survivors and k
   for (int64_t k : {1LL, 10LL, 100LL, 1000LL}) {
     CHECK(topk_speculative_rank(k, 0, 1000) == k && topk_speculative_rank(k, 1000, 0) == k);

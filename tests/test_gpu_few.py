@@ -108,3 +108,33 @@ def test_topk_values_is_the_head_of_a_stable_sort(n, pattern):
         assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(s[:k])) and torch.equal(got.isnan(), s[:k].isnan())
     with pytest.raises(Exception):
         ops.topk_values(t, min(n, 128) + 1)
+
+
+@pytest.mark.parametrize("storage,N,d", [("fp32", 65536, 32), ("bf16", 65500, 64), ("int8", 2000001, 128)])
+def test_a_workspace_of_a_larger_batch_holds_a_smaller_one(storage, N, d):
+    """The workspace of the largest batch (512) handed to shorter ones, as a C caller does on the last batch: accepted, and
+    the same answers, by the few-query form where it fits and by the general one where it does not."""
+    from dicee_amd import _lib, ops
+    lib = _lib.load()
+    rng = np.random.default_rng(N)
+    E, sc = _table(rng, storage, N, d, "random")
+    Q = torch.from_numpy((rng.standard_normal((512, d)) * 0.3).astype(np.float32)).cuda()
+    k, p = 10, ops._ptr
+    dtype = {"fp32": 0, "bf16": 1, "int8": 2}[storage]
+    prepared = ops.topk_prepare(E, sc) if storage == "int8" else None
+    size = lib.kge_topk_workspace_bytes if prepared is None else lib.kge_topk_prepared_workspace_bytes
+    full = size(512, N, k)
+    ws = torch.empty(full, dtype=torch.uint8, device="cuda")
+    too_big = 0
+    for B in (512, 300, 129, 128, 100, 33, 1):
+        too_big += size(B, N, k) > full
+        vals, idx = torch.empty(B, k, device="cuda"), torch.empty(B, k, dtype=torch.int64, device="cuda")
+        if prepared is None:
+            rc = lib.kge_topk(p(Q), None, p(E), dtype, p(sc), B, d, N, k, p(vals), p(idx), 0, p(ws), full, ops._stream())
+        else:
+            rc = lib.kge_topk_prepared(p(Q), None, p(E), dtype, p(sc), B, d, N, k, p(vals), p(idx), 0, p(prepared),
+                                       prepared.numel(), p(ws), full, ops._stream())
+        _lib.check(rc)
+        want_v, want_i = ops.topk(Q[:B].contiguous(), None, E, sc, k, prepared=prepared)
+        assert torch.equal(vals, want_v) and torch.equal(idx, want_i)
+    assert too_big                                            # (a batch whose own form would not have fitted was among them)
