@@ -9,6 +9,8 @@
 // the coefficient of head part i is sum_j sign[j][i] * r^_(i xor j) * t_j.
 #include "kge_internal.h"
 
+#include <type_traits>
+
 namespace kge {
 namespace {
 
@@ -367,12 +369,19 @@ __device__ __forceinline__ void normalise_row_backward(const float* x, const flo
       s2 += g * ((x[k] - mu) * inv);
     }
     const float m1 = wave_sum(s1) / (float)d, m2 = wave_sum(s2) / (float)d;
-    for (int k = lane; k < d; k += 64) {
-      const float xh = (x[k] - mu) * inv, g = dy[k] * a[k];
-      if (dw) atomicAdd(&dw[k], dy[k] * xh);
-      if (db) atomicAdd(&db[k], dy[k]);
-      emit(k, inv * (g - m1 - xh * m2) * drop_factor(keep, k, keep_scale));
-    }
+    // (the row first while the parameters' addresses are not crowded: d = 64, 16 pairs 6.4 us for 7.1; d = 512, 1024 pairs, one
+    // per workgroup, 104 us for 80)
+    auto add = [&](auto row_first) {
+      for (int k = lane; k < d; k += 64) {
+        const float xh = (x[k] - mu) * inv, g = dy[k] * a[k];
+        if constexpr (row_first) emit(k, inv * (g - m1 - xh * m2) * drop_factor(keep, k, keep_scale));
+        if (dw) atomicAdd(&dw[k], dy[k] * xh);
+        if (db) atomicAdd(&db[k], dy[k]);
+        if constexpr (!row_first) emit(k, inv * (g - m1 - xh * m2) * drop_factor(keep, k, keep_scale));
+      }
+    };
+    if (!IN_LDS && gridDim.x < 512) add(std::integral_constant<bool, !IN_LDS>{});
+    else add(std::false_type{});
   } else {  // BatchNorm1d with running statistics: an elementwise affine map
     for (int k = lane; k < d; k += 64) emit(k, dy[k] / sqrtf(b[k] + eps) * drop_factor(keep, k, keep_scale));
   }
@@ -383,9 +392,8 @@ __device__ __forceinline__ void normalise_row_backward(const float* x, const flo
 // normalisers' parameters, of which there are few (18 relations, one coefficient: 2048 additions to one address).  With
 // W > 1 those sums are formed in LDS first: the gradients at the relation rows stay there, pairs of the workgroup that
 // share a relation are added up, and each distinct row, coefficient and parameter is added to memory once per workgroup.
-// W = 1 is left for rows too long for eight sets of LDS rows and for the batch-statistics form, which writes rows.
 // Measured: 2048 pairs, Keci (0, 1), d = 256, 18 relations 39 -> 16 us; 1000 pairs, ComplEx d = 200 behind LayerNorm
-// 66 -> 26 us.
+// 66 -> 26 us.  W = 1 elsewhere (bq_eight_pairs).
 constexpr int BQ_COEFFS = 64;  // coefficients combined in LDS; bases past that go to memory one by one
 template <bool NORM, int W>
 __global__ void __launch_bounds__(64 * W) build_query_backward_kernel(QueryBwdArgs a, int model) {
@@ -393,7 +401,7 @@ __global__ void __launch_bounds__(64 * W) build_query_backward_kernel(QueryBwdAr
   constexpr bool COMBINE = W > 1;
   const int d = a.d;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int set = NORM ? 5 * d + (d + 3) / 4 : COMBINE ? 4 * d : 3 * d;  // floats of LDS per wave (bq_bwd_lds)
+  const int set = NORM ? 5 * d + (d + 3) / 4 : COMBINE ? 4 * d : 3 * d;  // floats of LDS per wave
   float* lds = lds_all + wave * set;
   float* sh = lds;          // head row
   float* sr = lds + d;      // relation row
@@ -710,12 +718,25 @@ __global__ void __launch_bounds__(64 * W) build_query_backward_kernel(QueryBwdAr
   }
 }
 
-// One launch of it: eight pairs per workgroup where their LDS rows fit 64 KB.
+// Eight pairs per workgroup or one?  Eight waves wait for one another and for the sums' passes over LDS, and 32 pairs are
+// four workgroups, so that they pay only where enough additions meet at one address (us, one / eight): every pair adds to a
+// LayerNorm's parameters (d = 200: 256 pairs 18.8 / 20.9, 512 pairs 29.7 / 21.7) and to the Clifford coefficients (d = 256,
+// (p, q) = (0, 1): 128 pairs 8.0 / 10.0, 256 9.5 / 10.1, 512 13.1 / 10.2; (1, 2): 256 14.8 / 12.3), B / R of them to a relation's
+// row (d = 256, 18 relations: 1024 pairs 5.2 / 5.4, 2048 7.6 / 7.2; 1000 relations: 4096 10.5 / 10.8; QMult, two passes over that
+// row: 18 relations, d = 200: 256 5.6 / 6.4, 512 8.2 / 6.6; 1000 relations: 1024 d = 64 4.9 / 5.5, d = 200 7.8 / 7.2).
+bool bq_eight_pairs(const QueryBwdArgs& a, int model, size_t lds_bytes) {
+  if (a.dy_h || lds_bytes > 65536) return false;  // the batch-statistics form writes rows; eight sets of long rows
+  if (a.norm.kind == KGE_NORM_LAYERNORM && (a.dn_h_a || a.dn_h_b || a.dn_r_a || a.dn_r_b)) return a.B >= 300;
+  if ((model == KGE_KECI || model == KGE_DECAL) && (a.d_coeff_p || a.d_coeff_q || a.d_coeff_r))
+    return a.B * (a.p + a.q + a.r) >= 512;
+  if (model == KGE_QMULT) return (a.B >= 512 && a.B >= 16 * a.R) || (a.B >= 1024 && a.d >= 128);
+  return a.B >= 2048 && a.B >= 16 * a.R;
+}
 int launch_build_query_backward(const QueryBwdArgs& a, int model, bool norm, hipStream_t st) {
   const size_t d = (size_t)a.d, set = norm ? 5 * d + (d + 3) / 4 : 4 * d;
   constexpr int W = 8;
   const size_t wide = (W * set + (norm ? 4 * d : 0)) * sizeof(float);
-  if (a.dy_h == nullptr && wide <= 65536) {
+  if (bq_eight_pairs(a, model, wide)) {
     const dim3 grid((unsigned)((a.B + W - 1) / W)), block(64 * W);
     if (norm) hipLaunchKernelGGL((build_query_backward_kernel<true, W>), grid, block, wide, st, a, model);
     else hipLaunchKernelGGL((build_query_backward_kernel<false, W>), grid, block, wide, st, a, model);

@@ -8,13 +8,14 @@ pytestmark = pytest.mark.gpu
 EPS = float(np.finfo(np.float32).eps)
 
 
-# one, a partial and several workgroups of eight pairs; rows of the widest eight-pair form and of the one-pair form past it
-# (4 rows of d floats per pair, with a layer 5.25 and 4 more, in 64 KB); more coefficients than are combined in LDS
+# batches that go one pair per workgroup, and one (2051: a partial last workgroup) that goes eight; rows of the widest
+# eight-pair form and past it (4 rows of d floats per pair, with a layer 5.25 and 4 more, in 64 KB); more coefficients than are
+# combined in LDS
 @pytest.mark.parametrize("model,d,kw,layer", [
     ("DistMult", 512, {}, False), ("DistMult", 513, {}, False), ("ComplEx", 200, {}, True), ("QMult", 356, {}, True),
     ("QMult", 364, {}, True), ("OMult", 24, {}, False), ("Keci", 256, {"p": 0, "q": 1}, False),
     ("Keci", 201, {"p": 30, "q": 36}, False), ("DeCaL", 28, {"p": 2, "q": 2, "r": 2}, True)])
-@pytest.mark.parametrize("B", [1, 13, 203])
+@pytest.mark.parametrize("B", [1, 13, 203, 2051])
 def test_query_backward_of_a_batch_is_the_sum_over_its_pairs(model, d, kw, layer, B):
     """Pairs that share heads, relations, coefficients and a layer's parameters: the batch's gradients against the
     float64 sum of those of the pairs alone.  A sum of n fp32 terms in any order is within n eps of the sum of their
