@@ -23,11 +23,12 @@ def _table(rng, storage, N, d, pattern):
 
 # (scores kept by the scan up to 32 MB, formed again past that)
 # edges: one row, a partial tile, whole tiles, one past; one and several query tiles; a partial last K step; every k range;
-# 16384 tiles (the longest table selected from directly) and one more row
+# 16384 tiles (the longest table selected from directly) and one more row; as many tiles as k
 CASES = [("fp32", 1, 4, 1, 1), ("fp32", 33, 20, 2, 33), ("fp32", 4096, 200, 33, 100), ("fp32", 5003, 256, 128, 10),
          ("fp32", 3001, 340, 5, 7), ("bf16", 31, 8, 3, 31), ("bf16", 4097, 128, 32, 128), ("bf16", 2000, 1024, 65, 10),
          ("bf16", 524288, 32, 2, 50), ("bf16", 524289, 32, 40, 128), ("int8", 1000, 16, 1, 10), ("int8", 7777, 240, 128, 100),
-         ("int8", 70001, 128, 64, 3), ("fp32", 140000, 64, 65, 40), ("int8", 150000, 32, 128, 5), ("int8", 600011, 16, 1, 5)]
+         ("int8", 70001, 128, 64, 3), ("fp32", 140000, 64, 65, 40), ("int8", 150000, 32, 128, 5), ("int8", 600011, 16, 1, 5),
+         ("fp32", 4096, 32, 3, 128)]
 
 
 @pytest.mark.parametrize("storage,N,d,B,k", CASES)
