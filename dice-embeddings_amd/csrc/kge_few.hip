@@ -33,7 +33,9 @@ struct FewArgs {
   float* raw;         // FEW_MAX_RAW: the scores themselves too, without a bias [B, ldr], whole tiles
   int64_t ldo, ldr, N, n_tiles;
   int B, d, nks;
-  int tpw;  // consecutive tiles a wave takes at a time
+  int tpw;   // consecutive tiles a wave takes at a time
+  int n_qg;  // query groups: 32 * QT queries each, as many as LDS holds fragments of
+  int n_wg;  // workgroups of a group, a multiple of 8
 };
 
 // One wave at a time: chunks of a 32-row tile, 128 (bf16: 256) bytes of every row, loaded as whole lines into registers
@@ -58,7 +60,11 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
   __shared__ __attribute__((aligned(16))) float s_max[MODE == FEW_MAX ? 4 * 32 * QT * FEW_RUN : 4];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q0 = (int)blockIdx.y * (32 * QT);
+  // The query groups of a batch walk the table side by side, a row's groups on one XCD (ids go round the eight of them): the
+  // first to come loads it, the others find it in that L2.  (One group after the other, each reads the whole table: fp32
+  // d = 256, N = 2M, 128 queries 1565 us; side by side 1196.)
+  const int slot = (int)blockIdx.x >> 3, qg = slot % a.n_qg, wg = slot / a.n_qg * 8 + ((int)blockIdx.x & 7);
+  const int q0 = qg * (32 * QT);
   const int nks = a.nks, d = a.d;
   for (int i = tid; i < QT * nks * 64; i += 256) {
     const int l = i & 63, s = (i >> 6) % nks, t = (i >> 6) / nks;
@@ -89,7 +95,7 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
   f32x4 next_sc[EDT == KGE_I8 ? 4 : 1], sc[EDT == KGE_I8 ? 4 : 1];  // int8: row scales of the chunk loaded, multiplied
   const int l_row = lane / PIECES, l_piece = lane % PIECES;
   const int nch = (nks + CH - 1) / CH;
-  int64_t unit = blockIdx.x, tile = (unit * 4 + wave) * a.tpw;
+  int64_t unit = wg, tile = (unit * 4 + wave) * a.tpw;
   int ch = 0, in_unit = 0;
   // the position after (tile, ch); past the end: tile >= n_tiles
   auto advance = [&]() {
@@ -98,7 +104,7 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
     ++tile;
     if (++in_unit == a.tpw) {
       in_unit = 0;
-      unit += gridDim.x;
+      unit += a.n_wg;
       tile = (unit * 4 + wave) * a.tpw;
     }
   };
@@ -425,7 +431,7 @@ __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a
   int n = 0;
   bool direct_rank = false;  // the entities are few enough to be ranked without being picked first
   // Every tile is among the best k: nothing to pick (a step of the selection is a barrier, sixteen of them 8 us: k = 100,
-  // N = 1000, d = 32 71 us a call, 63 without, 64 by the rounds).
+  // N = 1000, d = 32, 64 queries 72 us a call, 62 without, 66 by the rounds).
   const bool all = T <= k;
   if (all) {
     n = T;
@@ -587,18 +593,28 @@ int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
   const int parts = dtype == KGE_F32 ? 3 : 1;
   a.nks = (a.d + 15) / 16;
   a.n_tiles = (a.N + 31) / 32;
-  // as many query tiles per wave as the batch has and LDS holds fragments of: every tile reads the table's rows once
-  int qt = 1;
-  while (qt < (MODE == FEW_STORE ? 2 : 4) && 32 * qt < a.B && 2 * qt * a.nks * parts <= FEW_LDS_KB) qt *= 2;
-  const int n_qg = (a.B + 32 * qt - 1) / (32 * qt);
-  // one round of workgroups (as many per CU as registers and LDS allow) walks units of 4 * tpw tiles, each the same number
-  // of them; runs of eight tiles where there are more tiles than the selection reads one by one
+  const int qt = host::few_query_tiles(dtype, a.B, a.d, MODE == FEW_STORE ? 2 : 4);
+  a.n_qg = (a.B + 32 * qt - 1) / (32 * qt);
+  // workgroups, as many per CU as registers and LDS allow, walk units of 4 * tpw tiles, each the same number of them; runs of
+  // eight tiles where there are more tiles than the selection reads one by one
   a.tpw = a.n_tiles > FEW_TILES_DIRECT ? FEW_RUN : 1;
   const size_t lds = (size_t)qt * a.nks * parts * 1024 + 4 * few_stage_bytes(dtype);
-  const size_t room = 163840 / (lds + (MODE == FEW_MAX ? 4096 * qt : 0) + 512);
+  const size_t own = (lds + (MODE == FEW_MAX ? 4096 * qt : MODE == FEW_STORE ? 128 * qt : 0) + 1279) / 1280 * 1280;  // (granules of 1280)
+  const size_t room = 163840 / own;
   const int64_t slots = 256 * std::max<int64_t>(1, std::min<int64_t>(room, qt > 1 ? 2 : dtype == KGE_F32 ? 3 : 4));
-  const int64_t units = (a.n_tiles + 4 * a.tpw - 1) / (4 * a.tpw), each = (units + slots - 1) / slots;
-  const dim3 grid((unsigned)((units + each - 1) / each), (unsigned)n_qg), block(256);
+  const int64_t units = (a.n_tiles + 4 * a.tpw - 1) / (4 * a.tpw);
+  // one to four rounds of them: the fewest units in turn on a slot, a workgroup's start counted as one (several query groups
+  // rarely divide one round: int8 d = 1024, N = 41k, 96 queries, one round 89 us, the best of four 65)
+  int64_t best = -1;
+  for (int64_t r = 1; r <= (a.n_qg > 1 ? 4 : 1); ++r) {
+    const int64_t share = slots * r / a.n_qg / 8 * 8, each = (units + share - 1) / share;
+    const int64_t n_wg = ((units + each - 1) / each + 7) / 8 * 8, rounds = (n_wg * a.n_qg + slots - 1) / slots;
+    if (best < 0 || rounds * (each + 1) < best) {
+      best = rounds * (each + 1);
+      a.n_wg = (int)n_wg;
+    }
+  }
+  const dim3 grid((unsigned)(a.n_wg * a.n_qg)), block(256);
   auto go = [&](auto edt) {
     constexpr int EDT = decltype(edt)::value;
     if (qt == 1) hipLaunchKernelGGL((few_scan_kernel<EDT, 1, MODE>), grid, block, lds, st, a);
@@ -615,7 +631,7 @@ int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
 
 int few_scores_launch(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
                       int64_t N, float* out, int64_t ldo, hipStream_t st) {
-  FewArgs a{Q, E, scale, bias, out, nullptr, nullptr, ldo, 0, N, 0, (int)B, (int)d, 0, 0};
+  FewArgs a{Q, E, scale, bias, out, nullptr, nullptr, ldo, 0, N, 0, (int)B, (int)d, 0, 0, 0, 0};
   return launch_few_scan<FEW_STORE>(dtype, a, st);
 }
 
@@ -626,7 +642,7 @@ int few_topk_launch(const float* Q, const float* bias, const void* E, int dtype,
   float* maxima = (float*)workspace;
   float* runs = w.runs ? maxima + w.runs : nullptr;
   float* raw = w.raw ? maxima + w.raw : nullptr;
-  FewArgs a{Q, E, scale, nullptr, maxima, runs, raw, w.ldm, w.ldr, N, 0, (int)B, (int)d, 0, 0};
+  FewArgs a{Q, E, scale, nullptr, maxima, runs, raw, w.ldm, w.ldr, N, 0, (int)B, (int)d, 0, 0, 0, 0};
   const int rc = raw ? launch_few_scan<FEW_MAX_RAW>(dtype, a, st) : launch_few_scan<FEW_MAX>(dtype, a, st);
   if (rc) return rc;
   FewFinishArgs f{Q, E, scale, bias, maxima, runs, raw, w.ldm, w.ldr, N, (N + 31) / 32, (int)d, (int)k, apply_sigmoid,

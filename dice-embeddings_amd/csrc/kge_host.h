@@ -289,9 +289,9 @@ inline TopkWsOffsets topk_ws_offsets(int64_t B, int64_t N, int64_t k, bool with_
 // Few queries (kge_few.hip): every wave holds the same queries and the rows are shared out, so the table is read once per
 // 32 .. 128 queries at the rate of memory.  The top-k form keeps the maximum of every 32-row tile per query in the
 // workspace: 4 N / 32 bytes per query.
-constexpr int FEW_MAX_B = 128;            // top-k: four query tiles in one pass over the table.  There, k = 10, against the
-                                          // rounds (whose cost is flat up to 512 queries): bf16 2.5M x 128 228 us / 425,
-                                          // int8 10M x 128 660 / 1029, fp32 41k x 256 60 / 196; 500k x 128 200 / 298
+constexpr int FEW_MAX_B = 128;            // top-k: four query tiles.  128 queries, k = 10, against the rounds (whose cost is
+                                          // flat up to 512 queries): bf16 2.5M x 128 228 us / 425, int8 10M x 128
+                                          // 660 / 1029, fp32 41k x 256 60 / 196, 500k x 128 200 / 298 (few_topk_pays)
 constexpr int FEW_SCORES_MAX_B = 64;      // scores: fp32 41k x 256 24 us / 26 at 64 queries, 27 / 27 at 96
 constexpr int FEW_MAX_K = 128;            // tiles scored again per query: one workgroup's work
 constexpr int FEW_TILES_DIRECT = 16384;   // tile maxima one workgroup selects from; more go through maxima of 32 tiles
@@ -325,7 +325,28 @@ inline bool few_rows_ok(int dtype, int64_t d) {
 inline bool few_topk_applies(int dtype, int64_t B, int64_t d, int64_t N, int64_t k) {
   return B >= 1 && B <= FEW_MAX_B && k <= FEW_MAX_K && N <= FEW_MAX_N && few_rows_ok(dtype, d);
 }
-inline bool few_scores_applies(int dtype, int64_t B, int64_t d) {
+// Query tiles of 32 per wave: as many as the batch has and LDS holds fragments of
+inline int few_query_tiles(int dtype, int64_t B, int64_t d, int most) {
+  const int64_t kb = (d + 15) / 16 * (dtype == KGE_F32 ? 3 : 1);
+  int qt = 1;
+  while (qt < most && 32 * qt < B && 2 * qt * kb <= FEW_LDS_KB) qt *= 2;
+  return qt;
+}
+// Is it faster than the rounds?  Wherever the batch's tiles go together, and up to two of them.  Several query groups split
+// and multiply the table once each, where the rounds' main loops do it once for 128 queries or more: k = 10, few / rounds
+// in us, fp32 d = 256 N = 500k 96 queries 291 / 394, 128 356 / 406; N = 2M 96 944 / 889, 128 1196 / 913; two groups of two
+// tiles, N = 2M, 128 queries d = 128 534 / 563, d = 160 750 / 657; bf16 d = 768 N = 500k 96 373 / 387, 128 448 / 400; int8 d = 1024 N = 500k 96 561 / 459, N = 100k 128 188 / 268.
+inline bool few_topk_pays(int dtype, int64_t B, int64_t d, int64_t N) {
+  const int qt = few_query_tiles(dtype, B, d, 4);
+  const int64_t groups = (B + 32 * qt - 1) / (32 * qt);
+  if (groups * qt <= 2 || groups == 1) return true;
+  const int64_t millions = N * d / 1000000;
+  return millions <= (groups <= 3 ? (dtype == KGE_F32 ? 300 : 450) : (dtype == KGE_F32 ? 140 : 300));
+}
+inline bool few_scores_applies(int dtype, int64_t B, int64_t d, int64_t N) {
+  // (bf16 and int8 rows past 512 elements leave LDS for 32 queries' fragments, and for one workgroup per CU: 64 queries of
+  // bf16 d = 1024 few / kchunk_kernel N = 14.5k 20 us / 25, N = 41k 34 / 27)
+  if (dtype != KGE_F32 && d > 512 && B > 32 && N * d > 20000000) return false;
   return B >= 1 && B <= FEW_SCORES_MAX_B && few_rows_ok(dtype, d);
 }
 inline size_t few_topk_ws_bytes(int64_t B, int64_t N, int64_t k) {

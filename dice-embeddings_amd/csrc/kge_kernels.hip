@@ -1619,7 +1619,7 @@ extern "C" int kge_scores(const float* Q, const float* bias, const void* E, int 
   if (B == 0) return KGE_OK;
   KGE_REQUIRE(S && ldS >= N, KGE_ERR_INVALID, "kge_scores: S is null or ldS=%lld < N=%lld", (long long)ldS,
               (long long)N);
-  if (host::few_scores_applies(dtype, B, d)) {
+  if (host::few_scores_applies(dtype, B, d, N)) {
     LaunchTimer timer;
     if ((rc = timer.begin((hipStream_t)stream))) return rc;
     if ((rc = few_scores_launch(Q, bias, E, dtype, scale, B, d, N, S, ldS, (hipStream_t)stream))) return rc;
@@ -1998,8 +1998,18 @@ int topk_impl(const char* who, const float* Q, const float* bias, const void* E,
               int64_t d, int64_t N, int64_t k, float* out_scores, int64_t* out_idx, int apply_sigmoid,
               const void* prepared, void* workspace, size_t workspace_bytes, hipStream_t st) {
   int rc = KGE_OK;
-  // (a workspace made for a larger batch may hold the rounds and not the few-query form)
-  if (host::few_topk_applies(dtype, B, d, N, k) && workspace_bytes >= host::few_topk_ws_bytes(B, N, k)) {
+  // (a workspace made for a larger batch may hold the rounds and not the few-query form; and the rounds read back, so that a
+  // call that is being captured takes the other form whatever it costs)
+  auto captured = [&]() {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return status != hipStreamCaptureStatusNone;
+  };
+  if (host::few_topk_applies(dtype, B, d, N, k) && workspace_bytes >= host::few_topk_ws_bytes(B, N, k) &&
+      (host::few_topk_pays(dtype, B, d, N) || captured())) {
     LaunchTimer timer;
     if ((rc = timer.begin(st))) return rc;
     if ((rc = few_topk_launch(Q, bias, E, dtype, scale, B, d, N, k, out_scores, out_idx, apply_sigmoid, workspace, st))) return rc;

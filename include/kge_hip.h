@@ -384,8 +384,10 @@ int kge_rank_filtered_static(const float* Q, const float* bias, const void* E, i
  * This call (and kge_topk_prepared) synchronises `stream`: once before returning to read back one overflow
  * counter, and once more per repair scan when a candidate buffer overflowed (at most 16 scans; still overflowing
  * after those: KGE_ERR_OVERFLOW).  Neither can be captured into a HIP graph.  Calls of at most 128 queries with k <= 128,
- * N <= 2^24 and rows of at most 336 fp32 (a multiple of 4) or 1024 bf16 / int8 elements read nothing back and can be,
- * if their workspace has the kge_topk[_prepared]_workspace_bytes of the call itself.
+ * N <= 2^24 and rows of at most 336 fp32 (a multiple of 4) or 1024 bf16 / int8 elements, in a workspace of the
+ * kge_topk[_prepared]_workspace_bytes of the call itself, have a form that reads nothing back: they can be captured, and
+ * outside a capture they take it too, but for more than 64 queries on wide rows of a long table, where the general form is
+ * faster.
  * Workspace: the bytes of the call itself, or of any call with a batch and a k at least as large on a table at least as
  * long, are enough.  (The few-query form above takes more per query than the general one, up to 180 MB at N = 10M; a call
  * whose workspace does not hold it, because it was made for a batch past 128, say, goes the general way.)

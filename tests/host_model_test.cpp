@@ -299,6 +299,23 @@ static void test_flat_walk() {
 }
 
 // the fp32 contraction's plans: whole tiles of their form, every row in exactly one chunk; and dQ's split of the summed index
+static void test_few_rules() {
+  for (int dtype : {KGE_F32, KGE_BF16, KGE_I8})
+    for (int64_t d : {16, 80, 96, 160, 176, 256, 336, 512, 528, 1024})
+      for (int64_t B : {1, 32, 33, 64, 65, 96, 97, 128}) {
+        if (!few_rows_ok(dtype, d)) continue;
+        const int qt = few_query_tiles(dtype, B, d, 4);
+        CHECK((qt == 1 || qt == 2 || qt == 4) && qt * ((d + 15) / 16) * (dtype == KGE_F32 ? 3 : 1) <= FEW_LDS_KB);
+        CHECK(qt == 1 || 16 * qt < B);                                         // never a tile more than twice what is needed
+        CHECK(few_topk_pays(dtype, B, d, 14541));                              // tables in the caches
+        if (B <= 64) CHECK(few_topk_pays(dtype, B, d, FEW_MAX_N));             // two tiles
+        if (few_topk_pays(dtype, B, d, 2000000)) CHECK(few_topk_pays(dtype, B, d, 1000000));
+      }
+  CHECK(few_topk_pays(KGE_BF16, 128, 256, FEW_MAX_N) && few_topk_pays(KGE_F32, 128, 80, FEW_MAX_N));   // four tiles together
+  CHECK(!few_topk_pays(KGE_F32, 128, 256, 2000000) && !few_topk_pays(KGE_I8, 65, 1024, 500000));
+  CHECK(few_scores_applies(KGE_BF16, 64, 1024, 14541) && !few_scores_applies(KGE_BF16, 33, 1024, 41000));
+  CHECK(few_scores_applies(KGE_BF16, 32, 1024, 41000) && few_scores_applies(KGE_F32, 64, 336, 41000));
+}
 static void test_ks_plan() {
   const KsCost store{2.2, 1.2, 1.7, 0.2, {0, 0.74, 1.2, 1.56}}, rank{0.4, 1.0, 0.0, 0.65, {0, 0.82, 1.12, 1.6}};
   int narrow = 0, wide = 0;
@@ -328,6 +345,7 @@ static void test_ks_plan() {
 int main() {
   test_flat_walk();
   test_ks_plan();
+  test_few_rules();
   test_contract_rules();
   test_layouts();
   test_csr_keys();

@@ -139,3 +139,27 @@ def test_a_workspace_of_a_larger_batch_holds_a_smaller_one(storage, N, d):
         want_v, want_i = ops.topk(Q[:B].contiguous(), None, E, sc, k, prepared=prepared)
         assert torch.equal(vals, want_v) and torch.equal(idx, want_i)
     assert too_big                                            # (a batch whose own form would not have fitted was among them)
+
+
+@pytest.mark.parametrize("storage,N,d,B", [("fp32", 450000, 336, 128), ("bf16", 300001, 1024, 100)])
+def test_many_query_groups_on_a_long_table_go_the_general_way_unless_captured(storage, N, d, B):
+    """The same answers by the rounds (three or four query groups on a long table: the faster form) and by the few-query
+    form, which a captured call takes since it reads nothing back."""
+    from dicee_amd import ops
+    E = torch.randn(N, d, device="cuda") * 0.1
+    E[N - 3] = float("nan")                                   # (in the last, partial tile)
+    if storage == "bf16":
+        E = E.to(torch.bfloat16)
+    Q = torch.randn(B, d, device="cuda") * 0.3
+    ops.profile_begin()
+    vals, idx = ops.topk(Q, None, E, None, 10)
+    ops.profile_end()
+    assert ops.profile_kernel() != "few_scan_kernel"
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gv, gi = ops.topk(Q, None, E, None, 10)
+    for _ in range(2):
+        gv.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(gv, vals) and torch.equal(gi, idx)
