@@ -45,17 +45,19 @@ def compute_metrics_from_ranks_simple(ranks, num_triples, hits_dict):
 
 
 def check_triple_ids(triples, num_entities, num_relations):
-    """``triples`` [n,3] of an integer type as contiguous int64, or ``IndexError`` where an id is outside the model's
-    tables.  (One maximum per column: a negative id is a huge unsigned one.  Minima and maxima of picked columns, and the
-    copies they imply, were a tenth of an evaluation of 20,000 triples, with the GPU waiting.)"""
+    """``triples`` [n,3] as contiguous, writable int64 (the caller's own array where it is that already), or
+    ``IndexError`` where an id is outside the model's tables.  (One maximum per column: a negative id is a huge unsigned
+    one.  Minima and maxima of picked columns, and the copies they imply, were a tenth of an evaluation of 20,000 triples,
+    with the GPU waiting.)"""
+    outside = IndexError("triple_idx holds an entity or relation id outside the model's tables")
     if triples.dtype.kind not in "iub" and triples.size and triples.min() < 0:      # (-0.5 is not the id 0)
-        raise IndexError("triple_idx holds an entity or relation id outside the model's tables")
+        raise outside
     ids = np.ascontiguousarray(triples, dtype=np.int64)
     if len(ids):
         top = ids.view(np.uint64)
         if top[:, 0].max() >= num_entities or top[:, 2].max() >= num_entities or top[:, 1].max() >= num_relations:
-            raise IndexError("triple_idx holds an entity or relation id outside the model's tables")
-    return ids
+            raise outside
+    return ids if ids.flags.writeable else ids.copy()           # (torch.from_numpy warns of a read-only array)
 
 
 def ranks_from_counts(n_greater, n_equal, n_equal_lower, tie="stable"):
