@@ -50,8 +50,9 @@ def check_triple_ids(triples, num_entities, num_relations):
     one.  Minima and maxima of picked columns, and the copies they imply, were a tenth of an evaluation of 20,000 triples,
     with the GPU waiting.)"""
     outside = IndexError("triple_idx holds an entity or relation id outside the model's tables")
-    if triples.dtype.kind not in "iub" and triples.size and triples.min() < 0:      # (-0.5 is not the id 0)
-        raise outside
+    if triples.dtype.kind not in "iub" and len(triples):        # (-0.5 is not the id 0, and 2**70 no int64)
+        if triples.min() < 0 or triples[:, [0, 2]].max() >= num_entities or triples[:, 1].max() >= num_relations:
+            raise outside
     ids = np.ascontiguousarray(triples, dtype=np.int64)
     if len(ids):
         top = ids.view(np.uint64)

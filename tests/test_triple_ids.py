@@ -26,6 +26,10 @@ def test_ids_outside_their_table_are_refused(bad):
         check_triple_ids(t, 10, 3)
     with pytest.raises(IndexError):
         check_triple_ids(np.array([[-0.5, 0, 1]]), 10, 3)
+    with pytest.raises(IndexError):
+        check_triple_ids(np.array([[0, 0, 2**70]], dtype=object), 10, 3)
+    with pytest.raises(IndexError):
+        check_triple_ids(np.array([[0, 0, -2**70]], dtype=object), 10, 3)
 
 
 def test_a_read_only_test_set_goes_to_torch_without_a_warning(tmp_path):
