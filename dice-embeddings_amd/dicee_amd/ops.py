@@ -1,5 +1,6 @@
 """Tensor-level wrappers of the C ABI.  torch is used for device memory and streams only."""
 import ctypes
+import operator
 
 import torch
 
@@ -468,6 +469,7 @@ TOPK_VALUES_MAX_K, TOPK_VALUES_MAX_N = 128, 524288
 def topk_values(values, k):
     """(values [k], positions int64 [k]): the first k of ``torch.sort(values, descending=True, stable=True)`` of a
     contiguous fp32 vector of up to 524,288 values, k up to 128."""
+    k = operator.index(k)                                     # (2.5 is no number of values, as for a slice)
     lib = _lib.load()
     _require_gpu(values)
     if values.dtype != torch.float32 or values.dim() != 1:
@@ -477,7 +479,7 @@ def topk_values(values, k):
     out_i = torch.empty((k,), dtype=torch.int64, device=values.device)
     nbytes = lib.kge_topk_values_workspace_bytes(n)
     ws = torch.empty((nbytes,), dtype=torch.uint8, device=values.device) if nbytes else None
-    _lib.check(lib.kge_topk_values(_ptr(values), n, int(k), _ptr(out_v), _ptr(out_i), _ptr(ws), nbytes, _stream()))
+    _lib.check(lib.kge_topk_values(_ptr(values), n, k, _ptr(out_v), _ptr(out_i), _ptr(ws), nbytes, _stream()))
     return out_v, out_i
 
 

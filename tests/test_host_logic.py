@@ -344,3 +344,13 @@ def test_host_logic_builds_and_runs_under_address_and_ub_sanitizers(tmp_path):
     run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert run.returncode == 0, (run.stdout + run.stderr)[-3000:]
     assert "host logic ok" in run.stdout
+
+
+def test_a_fractional_number_of_substitutions_is_refused():
+    """As by the slice that cut the sorted scores before the k best were picked by a kernel; the check comes first."""
+    from dicee_amd import ops
+    for k in (2.0, 2.5, np.float32(3)):
+        with pytest.raises(TypeError):
+            ops.topk_values(torch.zeros(8), k)
+    with pytest.raises(RuntimeError):                      # a whole one gets as far as the tensor, which is on the CPU
+        ops.topk_values(torch.zeros(8), np.int64(2))
