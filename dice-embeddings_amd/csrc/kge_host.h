@@ -67,8 +67,9 @@ inline void rank128_plan(int64_t B, int64_t rows, int* n_qgroups, int* n_lanes, 
 // 20 of the 32 workgroups an XCD holds (5000 queries, heads and tails, on an int8 d = 240 table of 123k rows: 1554 us a pass
 // with the main loop on 160 CUs, 1265 us on 240), one of 33
 // groups a second round for the thirty-third; a group's rows are then read behind fewer L2s, which is why the per-XCD
-// form stays wherever it fills the chip to within a tenth as well.  The chunk length is the one whose busiest lane has
-// the fewest rows (longer chunks among equals).
+// form stays wherever it fills the chip to within a tenth as well, and where a table is so short that its lanes of that form
+// have a stage each already (bf16 d = 192, N = 1000, 2700 queries: scores 15.3 us per XCD, 17.8 flat).  The chunk length is
+// the one whose busiest lane has the fewest rows (longer chunks among equals).
 inline void flat_walk(int groups, int64_t rows, int stage_rows, int max_chunk, int* lanes_flat, int* chunk_rows,
                       int64_t* n_chunks) {
   *lanes_flat = 0;
@@ -78,6 +79,7 @@ inline void flat_walk(int groups, int64_t rows, int stage_rows, int max_chunk, i
   const double fill = (double)wgs / (256.0 * ((wgs + 255) / 256));
   const int lanes = 256 / groups;
   if (lanes * groups / 256.0 < 1.1 * fill) return;
+  if (wgs <= 256 && (rows + stage_rows - 1) / stage_rows <= 8 * per_xcd) return;
   int64_t best = -1;
   for (int chunk = max_chunk; chunk >= stage_rows; chunk -= stage_rows) {
     const int64_t n = (rows + chunk - 1) / chunk;

@@ -1246,7 +1246,7 @@ constexpr bool stream256_epilogue() {
   return std::is_same<EpiT<2>, RankEpi<2>>::value || std::is_same<EpiT<2>, StoreEpi<2>>::value;
 }
 ContractArgs make_args(const float* Q, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
-                       int64_t N, int64_t e_begin, int64_t e_end) {
+                       int64_t N, int64_t e_begin, int64_t e_end, bool may_be_flat = true) {
   ContractArgs a;
   a.Q = Q;
   a.E = E;
@@ -1285,7 +1285,7 @@ ContractArgs make_args(const float* Q, const void* E, int dtype, const float* sc
     if (chunk > 1024) chunk = 1024;
     a.chunk_rows = (int)chunk;
     a.n_chunks = (rows + chunk - 1) / chunk;
-    host::flat_walk(a.n_qgroups, rows, QA_STAGE_ROWS, 1024, &a.lanes_flat, &a.chunk_rows, &a.n_chunks);
+    if (may_be_flat) host::flat_walk(a.n_qgroups, rows, QA_STAGE_ROWS, 1024, &a.lanes_flat, &a.chunk_rows, &a.n_chunks);
     a.persistent = 1;
     return a;
   }
@@ -1645,7 +1645,12 @@ extern "C" int kge_scores(const float* Q, const float* bias, const void* E, int 
     if ((rc = few_scores_launch(Q, bias, E, dtype, scale, B, d, N, S, ldS, (hipStream_t)stream))) return rc;
     return timer.end("few_scan_kernel");
   }
-  ContractArgs a = make_args(Q, E, dtype, scale, B, d, N, 0, N);
+  // Where a score is written for few products, more workgroups side by side only crowd the stores (the per-XCD form of 5600
+  // queries, N = 123k, d = 64 1135 us, flat 1276; 8400, N = 41k, d = 128 480 / 550; 5000, N = 123k, int8 d = 240 837 / 933): flat
+  // up to 256 elements only past 128 and while the scores fit the caches, start on lines (2700, N = 100k, d = 192 flat 0.67 of the
+  // other), or a group would wait for a second round (8400, N = 41k, d = 192 0.78).
+  const bool flat = d > 256 || (d > 128 && ((double)B * N * 4 <= 3.4e8 || ldS % 32 == 0 || B > 32 * QS256_WG_QUERIES));
+  ContractArgs a = make_args(Q, E, dtype, scale, B, d, N, 0, N, flat);
   StoreArgs ea{S, bias, ldS, 0};
   return launch_contract<StoreEpi>(dtype, a, ea, (hipStream_t)stream, "kge_scores");
 }

@@ -287,6 +287,7 @@ static void test_flat_walk() {
       CHECK(chunk >= 128 && chunk <= 1024 && chunk % 128 == 0 && n == (rows + chunk - 1) / chunk);
       const int per_xcd = 32 / groups > 1 ? 32 / groups : 1, wgs = 8 * groups * per_xcd, rounds = (wgs + 255) / 256;
       CHECK(lanes * groups <= 256 && lanes * groups * rounds > wgs);
+      CHECK(wgs > 256 || rows > 128 * 8 * per_xcd);      // (a table that gives every lane of the other form a stage)
       const int64_t grid = walk_grid(groups, per_xcd, lanes);
       CHECK(grid % 8 == 0 && grid <= 256 && grid >= (int64_t)groups * lanes);
       std::vector<int> seen((size_t)groups * lanes, 0);
@@ -295,6 +296,14 @@ static void test_flat_walk() {
         if (idx / groups < lanes) ++seen[(size_t)((idx % groups) * lanes + idx / groups)];
       }
       for (int v : seen) CHECK(v == 1);
+    }
+  // the group counts that the GPU tests of the walk stand on are flat ones, at the row counts where they say so
+  for (int groups : {11, 17, 20, 33})
+    for (int64_t rows : {5003LL, 16000LL, 40001LL}) {
+      int lanes = 0, chunk = 0;
+      int64_t n = 0;
+      flat_walk(groups, rows, 128, 1024, &lanes, &chunk, &n);
+      CHECK(lanes > 0);
     }
 }
 
