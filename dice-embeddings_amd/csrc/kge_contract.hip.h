@@ -326,16 +326,21 @@ __device__ __forceinline__ bool decompose_wg(const ContractArgs& a, int& qg, int
 //   behind the same L2.  The host takes it where 32 workgroups per XCD do not divide evenly by the query groups
 //   (host::flat_walk).
 // (rank128_kernel and topk_i8_filter_kernel, 1024 queries per workgroup, keep the first form: at most a ninth of the chip
-// is idle up to 8192 queries, and the hand-allocated kernel ran 2.5 % slower with the choice in its prologue.)
+// is idle up to 8192 queries, and the hand-allocated kernel ran 2.5 % slower with the choice in its prologue.  qstream_kernel is
+// compiled for either form: with the choice inside, its registers fell out worse for both, ranks of 32 queries, bf16 d = 256,
+// N = 500k 60 -> 67 us.)
 // Ids past the last lane get a first chunk past the end.
+enum WalkForm { WALK_PER_XCD, WALK_FLAT, WALK_EITHER };
+template <WalkForm FORM = WALK_EITHER>
 __device__ __forceinline__ void walk_of_wg(const ContractArgs& a, int64_t wg, int& qg, int64_t& c_first, int64_t& c_stride) {
+  const bool flat = FORM == WALK_EITHER ? a.lanes_flat != 0 : FORM == WALK_FLAT;
   const int xcd = (int)(wg & 7);
   const int64_t slot = wg >> 3;
-  const int64_t idx = a.lanes_flat ? (int64_t)xcd * (gridDim.x >> 3) + slot : slot;
+  const int64_t idx = flat ? (int64_t)xcd * (gridDim.x >> 3) + slot : slot;
   qg = (int)(idx % a.n_qgroups);
   const int64_t wlane = idx / a.n_qgroups;
-  c_first = a.lanes_flat ? (wlane < a.lanes_flat ? wlane : a.n_chunks) : xcd + 8 * wlane;
-  c_stride = a.lanes_flat ? (int64_t)a.lanes_flat : 8 * (int64_t)a.n_lanes;
+  c_first = flat ? (wlane < a.lanes_flat ? wlane : a.n_chunks) : xcd + 8 * wlane;
+  c_stride = flat ? (int64_t)a.lanes_flat : 8 * (int64_t)a.n_lanes;
 }
 
 // ============================================================================================
@@ -1366,7 +1371,8 @@ constexpr int QS_VALU_PER_MFMA = 5;
 
 // KSTEPS: K steps of 16 per score (8: d == 128; 16: d == 256, rows of 512 bytes, one query tile per wave; 4: d == 64).
 // PAD: rows narrower than the LDS rows, as in qreg_async_kernel.
-template <template <int> class EpiT, int NQT, int W, int OCC, int KSTEPS = 8, bool PAD = false>
+// WALK: the form of the walk the launch was planned for.
+template <template <int> class EpiT, int NQT, int W, int OCC, int KSTEPS, bool PAD, WalkForm WALK>
 __global__ void __launch_bounds__(64 * W, OCC) qstream_kernel(ContractArgs a, typename EpiT<NQT>::Args ea) {
   using Epi = EpiT<NQT>;
   constexpr int d = 16 * KSTEPS;
@@ -1380,7 +1386,7 @@ __global__ void __launch_bounds__(64 * W, OCC) qstream_kernel(ContractArgs a, ty
   const int64_t wg = blockIdx.x;
   int qg;
   int64_t c_first, c_stride;
-  walk_of_wg(a, wg, qg, c_first, c_stride);
+  walk_of_wg<WALK>(a, wg, qg, c_first, c_stride);
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t q0 = (int64_t)qg * (W * 32 * NQT) + wave * (32 * NQT);

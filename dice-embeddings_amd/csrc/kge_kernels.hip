@@ -1436,10 +1436,17 @@ int launch_contract(int dtype, ContractArgs a, const EArgs& ea, hipStream_t st, 
                  QA_WAVES_PER_SIMD, KS, PAD ? "true" : "false");
       else
         snprintf(kname, sizeof(kname), "qreg_async_kernel<%s, %d, %d, %s>", epi, NQT, KS, PAD ? "true" : "false");
-      if constexpr (is_rank)
-        hipLaunchKernelGGL((qstream_kernel<RankFastEpi, NQT, QA_WG_WAVES, QA_WAVES_PER_SIMD, KS, PAD>), grid, block, 0, st, a, ea);
-      else if constexpr (STREAMED)
-        hipLaunchKernelGGL((qstream_kernel<EpiT, NQT, QA_WG_WAVES, QA_WAVES_PER_SIMD, KS, PAD>), grid, block, 0, st, a, ea);
+      auto stream = [&](auto walk) {
+        constexpr WalkForm WALK = decltype(walk)::value;
+        if constexpr (is_rank)
+          hipLaunchKernelGGL((qstream_kernel<RankFastEpi, NQT, QA_WG_WAVES, QA_WAVES_PER_SIMD, KS, PAD, WALK>), grid, block, 0, st, a, ea);
+        else
+          hipLaunchKernelGGL((qstream_kernel<EpiT, NQT, QA_WG_WAVES, QA_WAVES_PER_SIMD, KS, PAD, WALK>), grid, block, 0, st, a, ea);
+      };
+      if constexpr (is_rank || STREAMED) {
+        if (a.lanes_flat) stream(std::integral_constant<WalkForm, WALK_FLAT>{});
+        else stream(std::integral_constant<WalkForm, WALK_PER_XCD>{});
+      }
       else
         hipLaunchKernelGGL((qreg_async_kernel<EpiT, NQT, KS, PAD>), grid, block, 0, st, a, ea);
     };
