@@ -163,3 +163,32 @@ def test_many_query_groups_on_a_long_table_go_the_general_way_unless_captured(st
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(gv, vals) and torch.equal(gi, idx)
+
+
+@pytest.mark.parametrize("storage,N,d,B", [("fp32", 140005, 64, 65), ("bf16", 524300, 32, 9), ("int8", 600011, 16, 5),
+                                           ("fp32", 524289, 32, 3)])
+def test_nan_rows_and_queries_where_scores_are_formed_again(storage, N, d, B):
+    """Past 32 MB of scores the best tiles' are formed again, past 16,384 tiles after a pick among runs of tiles: NaN rows in
+    the first tile, the last, partial tile and its run, and a NaN query, and negative scores against padding."""
+    from dicee_amd import ops
+    rng = np.random.default_rng(N)
+    E, sc = _table(rng, storage, N, d, "random")
+    Q = -torch.rand(B, d, device="cuda")
+    Q[B // 2] = float("nan")
+    if storage != "int8":
+        E[-40:] = E[-40:].abs()                               # the last rows' scores are all negative
+    bad = torch.tensor([3, N // 2, N - 33, N - 2, N - 1], device="cuda")
+    if storage == "int8":
+        sc[bad] = float("nan")
+    else:
+        E[bad] = float("nan")
+    k = 60
+    vals, idx = ops.topk(Q, None, E, sc, k)
+    S = ops.scores(Q.repeat(-(-130 // B), 1), None, E, sc)[:B]
+    assert S[0, bad].isnan().all()
+    want_v, want_i = torch.sort(torch.nan_to_num(S, nan=-float("inf")), dim=1, descending=True, stable=True)
+    for b in range(B):
+        if b == B // 2:
+            assert (idx[b] == -1).all() and vals[b].isnan().all()
+        else:
+            assert torch.equal(idx[b], want_i[b, :k]) and torch.equal(vals[b], want_v[b, :k])
