@@ -938,9 +938,10 @@ struct BceEpi {
   }
 };
 
-// x / y for y in [1, 2] and x in [0, 1]: the hardware reciprocal (one unit in the last place) and one residual step, which
-// leaves the rounding of a division (nothing here can overflow or lose the residual, which is what the general division's
-// scaling and fix-up instructions, two thirds of it, are for).
+// x / y for y in [1, 2] and x in [0, 1]: the hardware reciprocal (one unit in the last place) and one residual step.  Within
+// one unit of the division's result, and equal to it for all but a few in a million; the general division's scaling and
+// fix-up instructions, two thirds of it, are for operands that do not occur here (a tiny x may lose its residual: its
+// quotient is off by less than the smallest normal number).
 __device__ __forceinline__ float quotient_1_2(float x, float y) {
   const float r = __builtin_amdgcn_rcpf(y), q = x * r;
   return __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);

@@ -85,6 +85,22 @@ def test_bce_step_with_hub_rows_and_empty_rows(d, eps, want_dbias):
             assert float((g.double() - w).norm()) <= 1e-5 * float(w.norm())
 
 
+def test_score_gradients_are_sigmoids_to_the_last_places():
+    """One query (1, 0, 0, 0) and grad_out = N: dE[:, 0] are the sigmoids of E[:, 0].  With u the unit roundoff 2^-24: exp(v) is
+    2 to the product v log2(e), which is rounded (u |v|) and whose constant is 0.22 u off, by an instruction good to one unit
+    in the last place (2 u): (1.22 |v| + 2) u relative, which moves the sigmoid s by that times s (1 - s).  The sum 1 + exp
+    moves it by u s more, the quotient, good to one unit, by 2 u s."""
+    from dicee_amd import ops
+    v = torch.linspace(-80, 80, 400001, device="cuda")
+    E = torch.zeros(v.numel(), 4, device="cuda")
+    E[:, 0] = v
+    Q = torch.tensor([[1.0, 0.0, 0.0, 0.0]], device="cuda")
+    rows, ptr = torch.tensor([-1], device="cuda"), torch.zeros(2, dtype=torch.int64, device="cuda")
+    dE = ops.bce_multihot_backward(Q, None, E, rows, ptr, rows.int(), grad_out=float(v.numel()))[3]
+    s, u = torch.sigmoid(v.double()), 2.0 ** -24
+    assert ((dE[:, 0].double() - s).abs() <= u * s * ((1.22 * v.double().abs() + 2) * (1 - s) + 3) + 2.0 ** -126).all()
+
+
 def test_zeros_clears_many_buffers():
     from dicee_amd import ops
     torch.full((3_000_000,), 7.0, device="cuda")            # (what the allocator hands out next is not zero already)
