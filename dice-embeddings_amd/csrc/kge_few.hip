@@ -4,10 +4,10 @@
 // The main loops of kge_contract.hip.h give every wave its own queries and every workgroup all of a chunk's rows: 512
 // queries (256 / 128) per workgroup, so that a batch of 32 multiplies sixteen times the rows it needs, for padding
 // queries, and runs at the matrix rate of the padding (bf16 d = 128, N = 2.5M, B = 32: 2.9 TB/s of table).  Here all waves
-// hold the SAME queries, as MFMA fragments in LDS, and share out the entity rows, which go from global memory straight
-// into fragment registers: what bounds the scan is the table's bytes.
-// Measured, whole calls: top-10 of 32 queries, bf16 d = 128, N = 2.5M 408 -> 193 us; top-10 of one question by name, fp32
-// d = 256, N = 41k 284 -> 141 us (the rounds of the large-batch form were four to seven scans and selections, and a
+// hold the SAME queries, as MFMA fragments in LDS, and share out the entity rows, which go as whole lines through
+// registers and a wave's own LDS into operands (few_scan_kernel): what bounds the scan is the table's bytes.
+// Measured, whole calls: top-10 of 32 queries, bf16 d = 128, N = 2.5M 408 -> 180 us; top-10 of one question by name, fp32
+// d = 256, N = 41k 284 -> 131 us (the rounds of the large-batch form were four to seven scans and selections, and a
 // read-back).
 //
 // Scores are formed by the chain every kernel uses (K steps of 16 ascending; fp32 operands as three bf16 parts, six

@@ -123,7 +123,7 @@ inline int fullest_chunk(int64_t rows, int n_qgroups, int tile, int64_t resident
 // Which form of the fp32 contraction a launch takes, and its chunk length.  Time is counted in K chunks of 32 columns of one
 // 256 x 128 tile on a CU of its own.  A wide workgroup takes wide_wg for its first loads and its end, and per tile its K
 // chunks and wide_tile for the epilogue; the busiest CU runs ceil(workgroups / 256) of them in turn.  Of the narrow
-// workgroups a CU holds three: the busiest one takes together[m] times as long for m of them as a wide workgroup's K chunks
+// workgroups a CU holds up to three: the busiest one takes together[m] times as long for m of them as a wide workgroup's K chunks
 // over the same number of tiles would.  The constants are fits, per epilogue, over 11 widths, 10 table sizes and 12 batches,
 // both forms timed on one card.  Against always taking the faster form the choice costs 0.3 % on average, more than 4 % for
 // one shape in forty (always narrow 2 %, one in six; always wide 8 %, one in two); the largest losses, 8 - 17 %, are scores
@@ -288,8 +288,8 @@ inline TopkWsOffsets topk_ws_offsets(int64_t B, int64_t N, int64_t k, bool with_
   return o;
 }
 
-// Few queries (kge_few.hip): every wave holds the same queries and the rows are shared out, so the table is read once per
-// 32 .. 128 queries at the rate of memory.  The top-k form keeps the maximum of every 32-row tile per query in the
+// Few queries (kge_few.hip): every wave holds the same queries and the rows are shared out, so the table is read at the rate
+// of memory and multiplied once per group of 32 .. 128 queries.  The top-k form keeps the maximum of every 32-row tile per query in the
 // workspace: 4 N / 32 bytes per query.
 constexpr int FEW_MAX_B = 128;            // top-k: four query tiles.  128 queries, k = 10, against the rounds (whose cost is
                                           // flat up to 512 queries): bf16 2.5M x 128 228 us / 425, int8 10M x 128
