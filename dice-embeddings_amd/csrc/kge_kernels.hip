@@ -294,8 +294,11 @@ constexpr int FIX_ITEMS = 16;  // work items a workgroup resolves side by side
 // layout, and the MFMA fragments are read from there; the generic path reads every row 16 bytes per lane at
 // a stride, which costs four requests per line.
 // A work item of at most 32 entities whose members all hold one query vector, by one wave: the entities' scores stay in
-// its registers (every column of the result tile holds the query), and column c counts for member c.
+// its registers (every column of the result tile holds the query), and column c counts for members c and 32 + c.  More members
+// than two rounds of columns go to the workgroup: 4000 queries on four rows of 16, fp32 d = 32, N = 135 43 us, 85 by waves; 64
+// members a row 2 % more, 32 as many.
 constexpr int FIX_SMALL = 32;
+constexpr int FIX_SMALL_MEMBERS = 64;
 template <int EDT>
 __device__ __forceinline__ void filter_fix_small(const ContractArgs& a, const FixPlan& plan, int64_t b0, const int32_t* col,
                                                  const int64_t* target, const float* thr, int32_t* n_gt, int32_t* n_eq,
@@ -366,7 +369,7 @@ __global__ void __launch_bounds__(256) filter_fix_kernel(ContractArgs a, FixPlan
   // This workgroup's work items are w = blockIdx.x + k * gridDim.x.  Up to FIX_ITEMS of them at a time are
   // resolved by one thread each, side by side (group by binary search, then the group's row and extent),
   // so that their chains of dependent loads overlap instead of running once per item.
-  __shared__ int32_t it_i0[FIX_ITEMS], it_m[FIX_ITEMS], it_mixed[FIX_ITEMS];
+  __shared__ int32_t it_i0[FIX_ITEMS], it_m[FIX_ITEMS], it_mixed[FIX_ITEMS], it_small[FIX_ITEMS];
   __shared__ int64_t it_z0[FIX_ITEMS], it_z1[FIX_ITEMS];
   for (int k0 = 0; blockIdx.x + (int64_t)k0 * gridDim.x < n_work; k0 += FIX_ITEMS) {
     __syncthreads();
@@ -403,6 +406,7 @@ __global__ void __launch_bounds__(256) filter_fix_kernel(ContractArgs a, FixPlan
         it_mixed[tid] = plan.mixed[b0 + host::plan_key_pos(key)];
         it_z0[tid] = z0;
         it_z1[tid] = (z0 + slice < L1) ? z0 + slice : L1;
+        it_small[tid] = it_z1[tid] - z0 <= FIX_SMALL && it_m[tid] <= FIX_SMALL_MEMBERS && (it_m[tid] == 1 || it_mixed[tid] == 0);
       }
     }
     __syncthreads();
@@ -411,9 +415,7 @@ __global__ void __launch_bounds__(256) filter_fix_kernel(ContractArgs a, FixPlan
     // such items side by side instead of waiting for one of them in turn (that batch, ComplEx d = 200: 119 -> 87 us; a
     // pass of 20,000 queries 1394 -> 1323; heads and tails of 5000 triples, int8 d = 240, 1265 -> 1258).
     // (Not where rows are gathered through LDS, bf16 d = 128: there the second set of registers costs more.)
-    auto small = [&](int kk) {
-      return !ROWS256 && it_z1[kk] - it_z0[kk] <= FIX_SMALL && (it_m[kk] == 1 || it_mixed[kk] == 0);
-    };
+    auto small = [&](int kk) { return !ROWS256 && it_small[kk] != 0; };
     if constexpr (!ROWS256) {
       for (int kk = wave; kk < FIX_ITEMS && blockIdx.x + (int64_t)(k0 + kk) * gridDim.x < n_work; kk += 4)
         if (small(kk))

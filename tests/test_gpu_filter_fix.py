@@ -9,11 +9,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("storage,d", [("fp32", 200), ("fp32", 30), ("bf16", 64), ("bf16", 128), ("int8", 240)])
 @pytest.mark.parametrize("same_vector", [True, False])
 def test_rows_of_up_to_a_tile_and_past_it(storage, d, same_vector):
-    """Rows of 0, 1, 31, 32, 33, 64, 65 and 300 entries, shared by 1, 31, 32, 33 and 70 queries that hold one vector or
+    """Rows of 0, 1, 31, 32, 33, 64, 65 and 300 entries, shared by 1, 31, 32, 33, 64, 65 and 70 queries that hold one vector or
     different ones; tied entities, the target in and out of its row.  Counters against the library's own scores."""
     from dicee_amd import ops
     rng = np.random.default_rng(d)
-    N, lens, members = 2003, [0, 1, 31, 32, 33, 64, 65, 300], [1, 31, 32, 33, 70]
+    N, lens, members = 2003, [0, 1, 31, 32, 33, 64, 65, 300], [1, 31, 32, 33, 64, 65, 70]
     ints = rng.integers(-90, 91, (N, d)).astype(np.int8)
     ints[500:900] = ints[rng.integers(0, 20, 400)]                       # exact ties
     E = torch.from_numpy(ints).cuda()
