@@ -230,6 +230,31 @@ inline RankWsOffsets rank_ws_offsets(int64_t B) {
   return o;
 }
 
+// workspace of kge_rank_pass
+struct RankPassOffsets {
+  size_t Q, bias, pairs, targets, rows, counts, thr, score, rank, total;
+};
+inline RankPassOffsets rank_pass_offsets(int64_t n, int64_t d) {
+  RankPassOffsets o{};
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off = align_up(off + bytes, 256);
+    return at;
+  };
+  o.Q = take((size_t)n * d * 4);
+  o.bias = take((size_t)n * 4);
+  o.pairs = take((size_t)n * 16);
+  o.targets = take((size_t)n * 8);
+  o.rows = take((size_t)n * 8);
+  o.counts = take((size_t)n * 12);
+  o.thr = take((size_t)n * 4);
+  o.score = take((size_t)n * 4);
+  o.rank = take(rank_ws_offsets(n).total);
+  o.total = off;
+  return o;
+}
+
 // tau: k-th best score per query (kth: the k-th best as a packed key, 0 while fewer than k are known); tau_scan: the threshold the next scan admits candidates with (tau, or a tighter
 // guess that the selection verifies); list: the best k so far as packed keys; cand: this round's candidates as packed
 // keys; cand_id: this round's candidates as entity ids (int8 filter scan, scored exactly before they are ranked);

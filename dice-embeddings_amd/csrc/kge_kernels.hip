@@ -129,17 +129,45 @@ __global__ void __launch_bounds__(256) triple_score_kernel(ContractArgs a, const
 }
 
 // ---- (head, relation) -> filter row: binary search in the sorted key array -----------------------
-__global__ void csr_lookup_kernel(const int64_t* hr, int64_t B, const int64_t* keys, int64_t n_rows,
-                                  int64_t num_relations, int64_t* csr_row) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  const int64_t key = hr[2 * b] * num_relations + hr[2 * b + 1];
+__device__ __forceinline__ int64_t filter_row(int64_t first, int64_t second, const int64_t* keys, int64_t n_rows,
+                                              int64_t num_relations) {
+  const int64_t key = first * num_relations + second;
   int64_t lo = 0, hi = n_rows;
   while (lo < hi) {
     const int64_t mid = (lo + hi) >> 1;
     if (keys[mid] < key) lo = mid + 1; else hi = mid;
   }
-  csr_row[b] = (lo < n_rows && keys[lo] == key) ? lo : -1;
+  return (lo < n_rows && keys[lo] == key) ? lo : -1;
+}
+__global__ void csr_lookup_kernel(const int64_t* hr, int64_t B, const int64_t* keys, int64_t n_rows,
+                                  int64_t num_relations, int64_t* csr_row) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < B) csr_row[b] = filter_row(hr[2 * b], hr[2 * b + 1], keys, n_rows, num_relations);
+}
+
+// ---- the two ends of an evaluation pass: its queries out of a matrix of ids, its ranks out of the counters --------------
+// pairs [B, 2], targets [B] and filter rows [B] (null: no filter) from ids that lie at any strides
+struct PassIds {
+  const int64_t *pair, *target;
+  int64_t pair_row, pair_col, target_row;  // strides in elements
+};
+__global__ void rank_pass_ids_kernel(PassIds ids, int64_t B, const int64_t* keys, int64_t n_rows, int64_t num_relations,
+                                     int64_t* pairs, int64_t* targets, int64_t* csr_row) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= B) return;
+  const int64_t first = ids.pair[b * ids.pair_row], second = ids.pair[b * ids.pair_row + ids.pair_col];
+  pairs[2 * b] = first;
+  pairs[2 * b + 1] = second;
+  targets[b] = ids.target[b * ids.target_row];
+  if (csr_row) csr_row[b] = filter_row(first, second, keys, n_rows, num_relations);
+}
+// rank = 1 + greater, and of the entities that tie: those of lower ids, none, all, or half of them (rounded down)
+__global__ void ranks_kernel(const int32_t* n_gt, const int32_t* n_eq, const int32_t* n_eql, int64_t B, int tie, int64_t* ranks) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= B) return;
+  const int64_t eq = n_eq[b], ties = tie == KGE_TIE_STABLE ? (int64_t)n_eql[b] : tie == KGE_TIE_OPTIMISTIC ? 0
+                                     : tie == KGE_TIE_PESSIMISTIC ? eq : eq >> 1;
+  ranks[b] = 1 + (int64_t)n_gt[b] + ties;
 }
 
 // ---- group the queries of one sub-batch by filter row and plan the correction work -----------
@@ -164,8 +192,21 @@ struct FixPlan {
   int32_t* mixed;            // [B] per leader: set when some member of its group holds another query vector
 };
 
-__global__ void __launch_bounds__(1024) plan_fix_kernel(const int64_t* csr_row, int64_t b0, int nb, int64_t n_rows,
-                                                       const int64_t* row_ptr, FixPlan plan) {
+// the plan of sub-batch `sub` (the workspace holds one per sub-batch, `stride` bytes apart; lead and mixed are the batch's)
+__device__ __forceinline__ FixPlan plan_of(FixPlan p, int64_t stride, int64_t sub) {
+  p.skey = (unsigned long long*)((char*)p.skey + sub * stride);
+  p.gend = (int32_t*)((char*)p.gend + sub * stride);
+  p.work = (int32_t*)((char*)p.work + sub * stride);
+  p.meta = (int32_t*)((char*)p.meta + sub * stride);
+  return p;
+}
+
+// One workgroup per sub-batch, side by side (the chain of steps of one workgroup is the kernel's time: 25 us for 8192 queries).
+__global__ void __launch_bounds__(1024) plan_fix_kernel(const int64_t* csr_row, int64_t B, int64_t n_rows,
+                                                       const int64_t* row_ptr, FixPlan first_plan, int64_t plan_stride) {
+  const int64_t b0 = (int64_t)blockIdx.x * SORT_MAX;
+  const int nb = (int)((B - b0 < SORT_MAX) ? B - b0 : SORT_MAX);
+  const FixPlan plan = plan_of(first_plan, plan_stride, blockIdx.x);
   __shared__ int32_t tab_row[PLAN_SLOTS];  // filter row + 1 that owns the slot, 0 = free
   __shared__ int32_t tab_cnt[PLAN_SLOTS];  // members of the slot's group; later: position of its first member
   __shared__ unsigned long long part[1024];
@@ -351,10 +392,13 @@ __device__ __forceinline__ void filter_fix_small(const ContractArgs& a, const Fi
 }
 
 template <int EDT, bool ROWS256>
-__global__ void __launch_bounds__(256) filter_fix_kernel(ContractArgs a, FixPlan plan, int64_t b0,
+__global__ void __launch_bounds__(256) filter_fix_kernel(ContractArgs a, FixPlan first_plan, int64_t plan_stride,
                                                         const int64_t* row_ptr, const int32_t* col,
                                                         const int64_t* target, const float* thr, int32_t* n_gt,
                                                         int32_t* n_eq, int32_t* n_eql) {
+  // grid.y: the sub-batches, side by side
+  const FixPlan plan = plan_of(first_plan, plan_stride, blockIdx.y);
+  const int64_t b0 = (int64_t)blockIdx.y * SORT_MAX;
   constexpr int CAP = ROWS256 ? 512 : FIX_CAP;  // entities per pass (the staged rows leave less LDS for the scores)
   __shared__ float s_s[CAP];
   __shared__ float s_sc[EDT == KGE_I8 ? CAP : 1];
@@ -1803,9 +1847,30 @@ int check_rank_args(const char* who, const float* Q, const void* E, int dtype, c
   return KGE_OK;
 }
 
+int rank_main_loop(const char* who, const float* Q, const void* E, int dtype, const float* scale, int64_t B, int64_t d, int64_t N,
+                   const RankArgs& ea, hipStream_t st) {
+  const ContractArgs a = make_args(Q, E, dtype, scale, B, d, N, 0, N);
+  return rank128_applies(dtype, d, B) ? launch_rank128(a, ea, st, who) : launch_contract<RankEpi>(dtype, a, ea, st, who);
+}
+int launch_filter_fix(int dtype, const ContractArgs& a, const FixPlan& plan, int64_t plan_stride, unsigned n_subs,
+                      const int64_t* row_ptr, const int32_t* col, const int64_t* target, const float* thr, int32_t* n_greater,
+                      int32_t* n_equal, int32_t* n_equal_lower, hipStream_t st) {
+  dim3 grid(2048, n_subs), block(256);
+  auto go = [&](auto edt, auto rows256) {
+    hipLaunchKernelGGL((filter_fix_kernel<decltype(edt)::value, decltype(rows256)::value>), grid, block, 0, st, a, plan, plan_stride,
+                       row_ptr, col, target, thr, n_greater, n_equal, n_equal_lower);
+  };
+  if (dtype == KGE_F32) go(std::integral_constant<int, KGE_F32>{}, std::false_type{});
+  else if (dtype == KGE_BF16 && a.d == 128) go(std::integral_constant<int, KGE_BF16>{}, std::true_type{});
+  else if (dtype == KGE_BF16) go(std::integral_constant<int, KGE_BF16>{}, std::false_type{});
+  else go(std::integral_constant<int, KGE_I8>{}, std::false_type{});
+  KGE_LAUNCH_CHECK("filter_fix_kernel");
+  return KGE_OK;
+}
+
 // the launches of a filtered-rank call; `ws_base` is a caller's workspace or the library's static scratch.
-// Order: the plan of every sub-batch (it only needs the filter rows, and tells every query its group's leader),
-// thresholds + counters + the one-vector-per-group check, the main loop, the filter correction of every sub-batch.
+// Order: the plans of all sub-batches (they only need the filter rows, and tell every query its group's leader),
+// thresholds + counters + the one-vector-per-group check, the main loop, the filter correction of all sub-batches.
 int rank_filtered_launch(const char* who, const float* Q, const float* bias, const void* E, int dtype, const float* scale,
                          int64_t B, int64_t d, int64_t N, const int64_t* target, const int64_t* csr_row,
                          const int64_t* row_ptr, const int32_t* col, int64_t n_rows, int32_t* n_greater, int32_t* n_equal,
@@ -1816,14 +1881,12 @@ int rank_filtered_launch(const char* who, const float* Q, const float* bias, con
   RankWs ws;
   rank_ws_layout(B, ws_base, &ws);
   if (thr_in) ws.thr = const_cast<float*>(thr_in);  // formed (and the counters initialised) by kge_rank_thresholds
+  const unsigned n_subs = (unsigned)((B + SORT_MAX - 1) / SORT_MAX);
+  const int64_t plan_stride = (int64_t)host::rank_ws_offsets(B).plan_stride;
   if (filtered) {
-    for (int64_t b0 = 0, sub = 0; b0 < B; b0 += SORT_MAX, ++sub) {
-      const int nb = (int)((B - b0 < SORT_MAX) ? B - b0 : SORT_MAX);
-      RankWs wsub;
-      rank_ws_layout(B, ws_base, &wsub, sub);
-      hipLaunchKernelGGL(plan_fix_kernel, dim3(1), dim3(1024), 0, st, csr_row, b0, nb, n_rows, row_ptr, wsub.plan);
-      KGE_LAUNCH_CHECK("plan_fix_kernel");
-    }
+    KGE_REQUIRE(n_subs <= 65535, KGE_ERR_INVALID, "%s: B=%lld too large", who, (long long)B);
+    hipLaunchKernelGGL(plan_fix_kernel, dim3(n_subs), dim3(1024), 0, st, csr_row, B, n_rows, row_ptr, ws.plan, plan_stride);
+    KGE_LAUNCH_CHECK("plan_fix_kernel");
   }
   if (!thr_in) {
     dim3 grid((unsigned)((B + 127) / 128 * (filtered ? 2 : 1))), block(256);  // (second half: the group check)
@@ -1836,30 +1899,11 @@ int rank_filtered_launch(const char* who, const float* Q, const float* bias, con
                        (const int32_t*)ws.plan.lead, ws.plan.mixed);
     KGE_LAUNCH_CHECK("group_check_kernel");
   }
-  RankArgs ea{ws.thr, target, n_greater, n_equal, n_equal_lower};
-  int rc = rank128_applies(dtype, d, B) ? launch_rank128(a, ea, st, who) : launch_contract<RankEpi>(dtype, a, ea, st, who);
+  int rc = rank_main_loop(who, Q, E, dtype, scale, B, d, N, RankArgs{ws.thr, target, n_greater, n_equal, n_equal_lower}, st);
   if (rc) return rc;
-  if (filtered) {
-    for (int64_t b0 = 0, sub = 0; b0 < B; b0 += SORT_MAX, ++sub) {
-      RankWs wsub;
-      rank_ws_layout(B, ws_base, &wsub, sub);
-      dim3 grid(2048), block(256);
-      if (dtype == KGE_F32)
-        hipLaunchKernelGGL((filter_fix_kernel<KGE_F32, false>), grid, block, 0, st, a, wsub.plan, b0, row_ptr, col, target,
-                           ws.thr, n_greater, n_equal, n_equal_lower);
-      else if (dtype == KGE_BF16 && d == 128)
-        hipLaunchKernelGGL((filter_fix_kernel<KGE_BF16, true>), grid, block, 0, st, a, wsub.plan, b0, row_ptr, col, target,
-                           ws.thr, n_greater, n_equal, n_equal_lower);
-      else if (dtype == KGE_BF16)
-        hipLaunchKernelGGL((filter_fix_kernel<KGE_BF16, false>), grid, block, 0, st, a, wsub.plan, b0, row_ptr, col, target,
-                           ws.thr, n_greater, n_equal, n_equal_lower);
-      else
-        hipLaunchKernelGGL((filter_fix_kernel<KGE_I8, false>), grid, block, 0, st, a, wsub.plan, b0, row_ptr, col, target,
-                           ws.thr, n_greater, n_equal, n_equal_lower);
-      KGE_LAUNCH_CHECK("filter_fix_kernel");
-    }
-  }
-  return KGE_OK;
+  return filtered ? launch_filter_fix(dtype, a, ws.plan, plan_stride, n_subs, row_ptr, col, target, ws.thr, n_greater, n_equal,
+                                      n_equal_lower, st)
+                  : KGE_OK;
 }
 }  // namespace
 
@@ -1923,6 +1967,84 @@ extern "C" int kge_rank_filtered_with_thresholds(const float* Q, const void* E, 
                               row_ptr, col, n_rows, n_greater, n_equal, n_equal_lower, nullptr, workspace,
                               (hipStream_t)stream, thr, one_vector_per_row != 0);
 }
+
+// ---- a whole evaluation pass ------------------------------------------------------------------------------
+extern "C" size_t kge_rank_pass_workspace_bytes(int64_t n, int64_t d) {
+  return n < 1 || d < 1 ? 0 : host::rank_pass_offsets(n, d).total;
+}
+
+extern "C" int kge_rank_pass(const kge_rank_pass_params* p, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  KGE_REQUIRE(p, KGE_ERR_INVALID, "kge_rank_pass: null parameters");
+  const int64_t n = p->n, d = p->d;
+  KGE_REQUIRE(n >= 0 && d >= 1, KGE_ERR_INVALID, "kge_rank_pass: n=%lld d=%lld", (long long)n, (long long)d);
+  KGE_REQUIRE(p->tie >= KGE_TIE_STABLE && p->tie <= KGE_TIE_MEAN, KGE_ERR_INVALID, "kge_rank_pass: tie=%d", p->tie);
+  if (n == 0) return KGE_OK;
+  KGE_REQUIRE(p->pairs && p->targets && p->ranks, KGE_ERR_INVALID, "kge_rank_pass: null ids or ranks");
+  KGE_REQUIRE(!p->keys == !p->row_ptr && !p->keys == !p->col, KGE_ERR_INVALID, "kge_rank_pass: a filter is keys, row_ptr and col");
+  KGE_REQUIRE(p->n_rows >= 0 && (!p->keys || p->key_mult >= 1), KGE_ERR_INVALID, "kge_rank_pass: n_rows=%lld key_mult=%lld",
+              (long long)p->n_rows, (long long)p->key_mult);
+  const host::RankPassOffsets o = host::rank_pass_offsets(n, d);
+  KGE_REQUIRE(workspace && workspace_bytes >= o.total, KGE_ERR_WORKSPACE, "kge_rank_pass: workspace of %zu bytes, need %zu",
+              workspace_bytes, o.total);
+  KGE_REQUIRE(((uintptr_t)workspace & 255) == 0, KGE_ERR_WORKSPACE, "kge_rank_pass: workspace must be 256-byte aligned");
+  char* ws = (char*)workspace;
+  float* Q = (float*)(ws + o.Q);
+  float* bias = (float*)(ws + o.bias);
+  int64_t *pairs = (int64_t*)(ws + o.pairs), *targets = (int64_t*)(ws + o.targets), *rows = (int64_t*)(ws + o.rows);
+  int32_t *gt = (int32_t*)(ws + o.counts), *eq = gt + n, *eql = eq + n;
+  float *thr = (float*)(ws + o.thr), *score = (float*)(ws + o.score);
+  hipStream_t st = (hipStream_t)stream;
+  const bool filtered = p->keys && p->n_rows > 0;
+  const unsigned blocks = (unsigned)((n + 255) / 256);
+  // (checked before anything is launched: the rules of the calls below)
+  int rc = check_rank_args("kge_rank_pass", Q, p->ent, p->ent_dtype, p->ent_scale, n, d, p->N, targets, filtered ? rows : nullptr,
+                           p->row_ptr, p->col, p->n_rows, gt, eq, eql, score);
+  if (rc) return rc;
+  hipLaunchKernelGGL(rank_pass_ids_kernel, dim3(blocks), dim3(256), 0, st,
+                     PassIds{p->pairs, p->targets, p->pair_row, p->pair_col, p->target_row}, n, p->keys, p->n_rows, p->key_mult,
+                     pairs, targets, filtered ? rows : nullptr);
+  KGE_LAUNCH_CHECK("rank_pass_ids_kernel");
+  if (p->model == KGE_DECAL)
+    rc = kge_build_query_decal(p->head, p->p, p->q, p->r, p->ent, p->ent_dtype, p->ent_scale, p->rel, p->rel_dtype, p->coeff_p,
+                               p->coeff_q, p->coeff_r, p->norm, pairs, n, d, p->N, p->R, Q, bias, stream);
+  else
+    rc = (p->head ? kge_build_query_head : kge_build_query)(p->model, p->p, p->q, p->ent, p->ent_dtype, p->ent_scale, p->rel,
+                                                           p->rel_dtype, p->coeff_p, p->coeff_q, p->normalize_relation, p->norm,
+                                                           pairs, n, d, p->N, p->R, Q, bias, stream);
+  if (rc) return rc;
+  rc = kge_rank_thresholds(Q, bias, p->ent, p->ent_dtype, p->ent_scale, n, d, p->N, targets, thr, gt, eq, eql, score, stream);
+  if (rc) return rc;
+  // The plans and the correction of the whole pass in one launch each; the main loop of 16-bit and 8-bit tables in launches of
+  // 8192 queries (their persistent workgroups share table rows through an XCD's L2 while a launch holds few query groups).
+  RankWs rws;
+  rank_ws_layout(n, ws + o.rank, &rws);
+  const unsigned n_subs = (unsigned)((n + SORT_MAX - 1) / SORT_MAX);
+  KGE_REQUIRE(n_subs <= 65535, KGE_ERR_INVALID, "kge_rank_pass: n=%lld too large", (long long)n);
+  const int64_t plan_stride = (int64_t)host::rank_ws_offsets(n).plan_stride;
+  if (filtered) {
+    hipLaunchKernelGGL(plan_fix_kernel, dim3(n_subs), dim3(1024), 0, st, (const int64_t*)rows, n, p->n_rows, p->row_ptr, rws.plan,
+                       plan_stride);
+    KGE_LAUNCH_CHECK("plan_fix_kernel");
+  }
+  const int64_t slice = p->ent_dtype == KGE_F32 ? n : SORT_MAX;
+  for (int64_t b = 0; b < n; b += slice) {
+    const int64_t nb = n - b < slice ? n - b : slice;
+    rc = rank_main_loop("kge_rank_pass", Q + b * d, p->ent, p->ent_dtype, p->ent_scale, nb, d, p->N,
+                        RankArgs{thr + b, targets + b, gt + b, eq + b, eql + b}, st);
+    if (rc) return rc;
+  }
+  if (filtered) {
+    const ContractArgs a = make_args(Q, p->ent, p->ent_dtype, p->ent_scale, n, d, p->N, 0, p->N);
+    rc = launch_filter_fix(p->ent_dtype, a, rws.plan, plan_stride, n_subs, p->row_ptr, p->col, targets, thr, gt, eq, eql, st);
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL(ranks_kernel, dim3(blocks), dim3(256), 0, st, (const int32_t*)gt, (const int32_t*)eq, (const int32_t*)eql, n,
+                     p->tie, p->ranks);
+  KGE_LAUNCH_CHECK("ranks_kernel");
+  return KGE_OK;
+}
+
 
 // ---- the same call for callers that cannot allocate ---------------------------------------------------
 // The workspace of kge_rank_filtered (thresholds, the plan of the filter correction) lives in a file-scope

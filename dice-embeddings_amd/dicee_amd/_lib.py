@@ -31,6 +31,18 @@ class NormGrads(ctypes.Structure):
     _fields_ = [("h_a", _vp), ("h_b", _vp), ("r_a", _vp), ("r_b", _vp)]
 
 
+class RankPassParams(ctypes.Structure):
+    _fields_ = ([(k, ctypes.c_int32) for k in ("model", "p", "q", "r", "ent_dtype", "rel_dtype", "normalize_relation",
+                                               "head", "tie")]
+                + [(k, _vp) for k in ("ent", "ent_scale", "rel", "coeff_p", "coeff_q", "coeff_r")]
+                + [("norm", ctypes.POINTER(NormParams)), ("pairs", _vp), ("targets", _vp)]
+                + [(k, _c_i64) for k in ("pair_row", "pair_col", "target_row", "n", "d", "N", "R")]
+                + [("keys", _vp), ("n_rows", _c_i64), ("key_mult", _c_i64), ("row_ptr", _vp), ("col", _vp),
+                   ("ranks", _vp)])
+
+
+TIES = {"stable": 0, "optimistic": 1, "pessimistic": 2, "mean": 3}
+
 SIGNATURES = {
     "kge_last_error": (ctypes.c_char_p, []),
     "kge_abi_version": (_c_int, []),
@@ -72,6 +84,8 @@ SIGNATURES = {
     "kge_rank_thresholds": (_c_int, [_vp, _vp, _vp, _c_int, _vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "kge_rank_filtered_with_thresholds": (_c_int, [_vp, _vp, _c_int, _vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _vp, _vp, _vp,
                                                    _c_i64, _c_int, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "kge_rank_pass_workspace_bytes": (_sz, [_c_i64, _c_i64]),
+    "kge_rank_pass": (_c_int, [ctypes.POINTER(RankPassParams), _vp, _sz, _vp]),
     "kge_rank_static_init": (_c_int, []),
     "kge_rank_filtered_static": (_c_int, [_vp, _vp, _vp, _c_int, _vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _vp, _vp, _c_i64,
                                           _vp, _vp, _vp, _vp, _vp]),

@@ -131,14 +131,37 @@ class _BatchStreams:
             self.cur.wait_stream(s)
 
 
+def eval_mode(model):
+    """``model.eval()``, which walks and writes to every module, where some module is not in that mode yet."""
+    if any(m.training for m in model.modules()):
+        model.eval()
+
+
+def _plain_queries(model, x_all, target_all):
+    """Does ``ops.rank_pass`` form these queries?  (A model with a query builder of its own, dropout or batch statistics: no.)"""
+    from .models import BaseKGE
+    if type(model).query is not BaseKGE.query or type(model).table is not BaseKGE.table:
+        return False
+    if model.training and (model.input_dropout_rate > 0.0
+                           or isinstance(model.normalize_head_entity_embeddings, torch.nn.BatchNorm1d)):
+        return False
+    dev = model.entity_embeddings.weight.device
+    return (dev.type == "cuda" and all(t.device == dev and t.dtype == torch.int64 for t in (x_all, target_all))
+            and x_all.dim() == 2 and x_all.shape[1] == 2)
+
+
 def rank_in_batches(model, x_all, target_all, csr, batch_size, tie="stable", streams=2, heads=False,
-                    call_queries=8192):
-    """Ranks (int64 tensor [n] on the model's device) of ``target_all`` [n] for the queries ``x_all`` [n,2]: one fused
-    rank call per batch of ``batch_size`` queries, or per run of whole batches that together hold at least
-    ``call_queries`` queries (the reference's batch size bounds the B x N score matrix it materialises,
-    evaluator.py:484-508; the fused call forms no such matrix, a query's counters do not depend on what else is in
-    its call, and a call's fixed cost (the plan of its correction, launches, the last round of workgroups) is paid
-    once per call: ``call_queries=0`` keeps one call per batch).  What does not depend on the batching is done for many batches at a
+                    call_queries=8192, out=None):
+    """Ranks (int64 tensor [n] on the model's device; ``out``: where to write them) of ``target_all`` [n] for the queries
+    ``x_all`` [n,2].  The reference's batch size bounds the B x N score matrix it materialises (evaluator.py:484-508); the
+    fused call forms no such matrix and a query's counters do not depend on what else is in its call, so that the pass is
+    one call (``ops.rank_pass``; one per 256 MB of query vectors): seven launches, one behind the other.  (Alternating whole
+    batches over two streams around calls per batch: 20,000 queries of a 14.5k graph 994 us on two streams and 1060 on one
+    against about 1000; 2 x 5000 queries of an int8 table 1005 and 925.)
+
+    ``call_queries=0``, and models that build their queries otherwise: one fused rank call per batch of ``batch_size``
+    queries (or, with ``call_queries``, per run of whole batches that together hold at least that many).  What does not
+    depend on the batching is done for many batches at a
     time: the query vectors and the filter rows of a group of batches (at most 64 batches or 256 MB of vectors; every
     row is a function of its own (h, r) pair alone, so the numbers are those of batch-wise calls) and the thresholds
     (the raw scores of the targets) come from one launch each, and a batch is then nothing but the plan of its filter
@@ -146,6 +169,18 @@ def rank_in_batches(model, x_all, target_all, csr, batch_size, tie="stable", str
     from . import ops
     n = int(x_all.shape[0])
     dev = x_all.device
+    if call_queries and n and _plain_queries(model, x_all, target_all):
+        with torch.no_grad():
+            E, scale = model.table()
+            rel, norm = model._rel(), model._norm_params()
+            name = model.name if model.name != "CKeci" else "Keci"
+            if out is None:
+                out = torch.empty((n,), dtype=torch.int64, device=dev)
+            group = max(1, int(batch_size), (1 << 28) // (4 * E.shape[1]))
+            for g in range(0, n, group):
+                ops.rank_pass(name, E, rel, x_all[g:g + group], target_all[g:g + group], csr, ent_scale=scale, norm=norm,
+                              head=heads, tie=tie, out=out[g:g + group], **model._query_kwargs())
+        return out
     x_all = x_all.contiguous()
     target_all = target_all.to(dtype=torch.int64).contiguous()
     counts = {k: torch.empty((n,), dtype=dt, device=dev) for k, dt in ops._RANK_OUT}
@@ -181,7 +216,8 @@ def rank_in_batches(model, x_all, target_all, csr, batch_size, tie="stable", str
                 lanes.join()    # before the group's vectors are released to the allocator of the caller's stream
     finally:
         lanes.join()
-    return ranks_from_counts(counts["n_greater"], counts["n_equal"], counts["n_equal_lower"], tie)
+    ranks = ranks_from_counts(counts["n_greater"], counts["n_equal"], counts["n_equal_lower"], tie)
+    return ranks if out is None else out.copy_(ranks)
 
 
 class Evaluator:
@@ -343,7 +379,7 @@ class Evaluator:
 
     def evaluate_lp_k_vs_all(self, model, triple_idx, info=None, form_of_labelling=None):
         """Filtered link prediction with KvsAll scoring -> ``{'H@1','H@3','H@10','MRR'}``."""
-        model.eval()
+        eval_mode(model)
         num_triples = len(triple_idx)
         if info and not self.during_training:
             print(info + ":", end=" ")

@@ -13,7 +13,7 @@ import numpy as np
 import torch
 
 from .csr import FilterCSR
-from .evaluator import check_triple_ids, rank_in_batches
+from .evaluator import check_triple_ids, eval_mode, rank_in_batches
 
 
 def _as_csr(vocab, key_mult, device):
@@ -40,7 +40,7 @@ def evaluate_lp(model, triple_idx, num_entities=None, er_vocab=None, re_vocab=No
     assert triple_idx is not None, "triple_idx must be provided"
     assert er_vocab is not None, "er_vocab must be provided"
     assert re_vocab is not None, "re_vocab must be provided"
-    model.eval()
+    eval_mode(model)
     from .models import IdentityClass
     if not isinstance(getattr(model, "normalize_tail_entity_embeddings", IdentityClass()), IdentityClass):
         # the reference scores every candidate through forward_triples here, i.e. against NORMALISED tail rows
@@ -61,9 +61,10 @@ def evaluate_lp(model, triple_idx, num_entities=None, er_vocab=None, re_vocab=No
     er = _as_csr(er_vocab, R, dev)
     re = _as_csr(re_vocab, N, dev)
     trip = torch.from_numpy(ids).to(dev)
-    tail_ranks = rank_in_batches(model, trip[:, :2], trip[:, 2], er, batch_size, tie, streams)
-    head_ranks = rank_in_batches(model, trip[:, 1:], trip[:, 0], re, batch_size, tie, streams, heads=True)
-    hr_, tr_ = head_ranks.cpu().numpy(), tail_ranks.cpu().numpy()
+    ranks = torch.empty((2, n), dtype=torch.int64, device=dev)           # heads, tails: one copy to the host for both
+    rank_in_batches(model, trip[:, :2], trip[:, 2], er, batch_size, tie, streams, out=ranks[1])
+    rank_in_batches(model, trip[:, 1:], trip[:, 0], re, batch_size, tie, streams, heads=True, out=ranks[0])
+    hr_, tr_ = ranks.cpu().numpy()
     divisor = float(2 * n) if n else 1.0
     results = {f"H@{k}": float((np.count_nonzero(hr_ <= k) + np.count_nonzero(tr_ <= k)) / divisor) for k in (1, 3, 10)}
     results["MRR"] = float((1.0 / hr_ + 1.0 / tr_).sum() / divisor)

@@ -419,6 +419,60 @@ def rank_filtered(Q, bias, E, scale, target, csr_row=None, row_ptr=None, col=Non
     return out
 
 
+def rank_pass(model, ent, rel, pairs, targets, csr=None, *, ent_scale=None, p=0, q=0, r=0, coeff_p=None, coeff_q=None,
+              coeff_r=None, normalize_relation=True, norm=None, head=False, tie="stable", out=None):
+    """Ranks (int64 [n]) of ``targets`` [n] for the queries ``pairs`` [n,2] in one call: ``build_query``, ``csr_lookup``,
+    ``rank_thresholds``, ``rank_filtered(one_vector_per_row=True)`` and 1 + greater + ties, for queries whose vectors and
+    filter rows both come from their pair.  ``pairs`` / ``targets``: int64 GPU tensors of any strides (columns of a matrix of
+    triples); ``csr``: a ``FilterCSR`` on the GPU, or None; ``out``: a contiguous int64 [n] tensor to write into."""
+    lib = _lib.load()
+    _require_gpu(ent, rel, ent_scale, coeff_p, coeff_q, coeff_r, out)
+    if not pairs.is_cuda or not targets.is_cuda:
+        raise RuntimeError("dicee_amd ops need tensors on the GPU (there is no CPU path)")
+    n, (N, d) = pairs.shape[0], ent.shape
+    if pairs.dtype != torch.int64 or pairs.dim() != 2 or pairs.shape[1] != 2:
+        raise ValueError("pairs must be an int64 tensor of shape [n, 2]")
+    if targets.dtype != torch.int64 or targets.shape != (n,):
+        raise ValueError("targets must be an int64 tensor of shape [n]")
+    if rel.shape[1] != d:
+        raise ValueError("entity and relation tables must have the same embedding dim")
+    if ent.dtype == torch.int8 and ent_scale is None:
+        raise ValueError("int8 tables need per-row scales")
+    if tie not in _lib.TIES:
+        raise ValueError(tie)
+    if out is None:
+        out = torch.empty((n,), dtype=torch.int64, device=ent.device)
+    elif out.dtype != torch.int64 or out.shape != (n,):
+        raise ValueError("out must be an int64 tensor of shape [n]")
+    keys = row_ptr = col = None
+    n_rows, mult = 0, 1
+    if csr is not None and csr.keys.numel():
+        _require_gpu(csr.keys, csr.row_ptr, csr.col)
+        if csr.keys.dtype != torch.int64 or csr.row_ptr.dtype != torch.int64 or csr.col.dtype != torch.int32:
+            raise TypeError("the filter's keys / row_ptr must be int64 and col int32")
+        keys, row_ptr, col = csr.keys.data_ptr(), csr.row_ptr.data_ptr(), csr.col.data_ptr()
+        n_rows, mult = csr.row_ptr.numel() - 1, int(csr.num_relations)
+        if csr.keys.numel() != n_rows:
+            raise ValueError("a filter has one key per row")
+        if col == 0:                                    # (every row empty: nothing to filter)
+            keys = row_ptr = col = None
+    ns, keep = _norm_struct(norm)
+
+    def at(t):
+        return None if t is None else t.data_ptr()
+    s = _lib.RankPassParams(MODEL_IDS[model], int(p), int(q), int(r), _table_dtype(ent), _table_dtype(rel),
+                            int(bool(normalize_relation)), int(bool(head)), _lib.TIES[tie], ent.data_ptr(), at(ent_scale),
+                            rel.data_ptr(), at(coeff_p), at(coeff_q), at(coeff_r),
+                            ctypes.pointer(ns) if ns is not None else None, pairs.data_ptr(), targets.data_ptr(),
+                            pairs.stride(0), pairs.stride(1), targets.stride(0), n, d, N, rel.shape[0], keys, n_rows, mult,
+                            row_ptr, col, out.data_ptr())
+    nbytes = lib.kge_rank_pass_workspace_bytes(n, d)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=ent.device)
+    _lib.check(lib.kge_rank_pass(ctypes.byref(s), ws.data_ptr(), nbytes, _stream()))
+    del keep
+    return out
+
+
 def topk_prepare(E, scale):
     """The derived form of a table that ``topk`` scans (made once per table and handed to every call as
     ``prepared=``), or None where the storage has none (every storage but per-row int8 with d = 128)."""

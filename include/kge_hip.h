@@ -349,6 +349,36 @@ int kge_rank_filtered_with_thresholds(const float* Q, const void* E, int dtype, 
                                       size_t workspace_bytes, void* stream);
 
 /*
+ * A whole evaluation pass in one call: the loop of evaluate_lp_k_vs_all (dicee/evaluation/evaluator.py:473-510) over n queries,
+ * or one direction of evaluate_lp (link_prediction.py:351-473) with head != 0.  From id matrices at any strides to int64 ranks:
+ * what kge_csr_lookup, kge_build_query (_head, _decal), kge_rank_thresholds and kge_rank_filtered_with_thresholds
+ * (one_vector_per_row) give in a row, and 1 + greater + the share of the ties that `tie` names.  No filter: keys, row_ptr and
+ * col NULL.  Ranks do not depend on how the queries are divided over calls.
+ */
+enum kge_tie { KGE_TIE_STABLE = 0, KGE_TIE_OPTIMISTIC = 1, KGE_TIE_PESSIMISTIC = 2, KGE_TIE_MEAN = 3 };
+typedef struct kge_rank_pass_params {
+  int32_t model, p, q, r, ent_dtype, rel_dtype, normalize_relation, head, tie;
+  const void* ent;
+  const float* ent_scale;
+  const void* rel;
+  const float* coeff_p;
+  const float* coeff_q;
+  const float* coeff_r;
+  const kge_norm_params* norm;
+  const int64_t* pairs;   /* pair b: pairs[b * pair_row], pairs[b * pair_row + pair_col] */
+  const int64_t* targets; /* target b: targets[b * target_row] */
+  int64_t pair_row, pair_col, target_row;
+  int64_t n, d, N, R;
+  const int64_t* keys; /* [n_rows] sorted: first * key_mult + second */
+  int64_t n_rows, key_mult;
+  const int64_t* row_ptr;
+  const int32_t* col;
+  int64_t* ranks; /* [n] */
+} kge_rank_pass_params;
+size_t kge_rank_pass_workspace_bytes(int64_t n, int64_t d);
+int kge_rank_pass(const kge_rank_pass_params* params, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * kge_rank_filtered without a workspace argument and without any allocation.  No counterpart in the reference:
  * it exists for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  The thresholds and the plan of the filter correction live in a

@@ -123,6 +123,15 @@ static void test_layouts() {
   // the static scratch array of kge_rank_filtered_static holds the layout of its largest batch
   CHECK(rank_ws_offsets(KGE_RANK_STATIC_MAX_B).total <= KGE_RANK_STATIC_SCRATCH_BYTES);
   CHECK(TOPK_FIRST_ROWS <= TOPK_CAP);
+  for (int64_t n : {1, 8191, 8192, 8193, 20000})
+    for (int64_t d : {1, 32, 201}) {
+      const RankPassOffsets o = rank_pass_offsets(n, d);
+      const size_t m = (size_t)n;
+      check_disjoint({{o.Q, m * d * 4}, {o.bias, m * 4}, {o.pairs, m * 16}, {o.targets, m * 8}, {o.rows, m * 8}, {o.counts, m * 12},
+                      {o.thr, m * 4}, {o.score, m * 4}, {o.rank, rank_ws_offsets(n).total}},
+                     o.total);
+      for (size_t at : {o.Q, o.pairs, o.rank}) CHECK(at % 256 == 0);
+    }
   for (auto bdn : {std::array<int64_t, 3>{1, 1, 1}, {2048, 256, 40943}, {5, 7, 3}, {4096, 128, 1 << 24}}) {
     const BwdPlan p = bwd_plan(bdn[0], bdn[1], bdn[2]);
     CHECK(p.ldG % 4 == 0 && p.ldG >= bdn[2] && p.ldT % 4 == 0 && p.ldT >= bdn[0]);
