@@ -288,43 +288,55 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
 // score at a lower id).  So one workgroup per query picks the k best tiles, forms their 32 k scores again and picks the
 // k best of those: no thresholds, no candidate buffers that could overflow, nothing read back.  Tables of more than
 // FEW_TILES_DIRECT tiles go through the maxima of 32 tiles first, by the same argument.
+constexpr int FEW_THREADS = 1024;
+constexpr int SELECT_GROUPS = FEW_THREADS / 4, SELECT_CAP = 512;
+// This many entities are ranked without being picked first (each against all: 320 of them cost 7 us more than their selection)
+constexpr int FEW_DIRECT = 160;
 struct SelectShared {
   unsigned long long cnt[16];
-  uint32_t scan[256];
+  union {
+    uint32_t scan[256];           // block_select_bits
+    __attribute__((aligned(16))) uint32_t top[SELECT_GROUPS];  // the largest value of every four threads (t, t + 256, ..)
+  };
+  int rank[SELECT_GROUPS];
+  __attribute__((aligned(16))) unsigned long long cand[SELECT_CAP];  // (value, then the lower position) as one key, zeros behind them
+  int picked[FEW_MAX_K];
+  int n_cand, n_above;
+  uint32_t bound, least;
 };
-constexpr int FEW_THREADS = 1024;
 
 __device__ __forceinline__ uint32_t score_key(float v) {
   return v > __uint_as_float(0xff800000u) ? f32_to_ordered(v) : 0u;  // NaN and -inf are never ranked
 }
 
 // The positions of the k largest of vals[0 .. M) (ties: the lower positions; zeros never), ascending, into pos; returns
-// how many.  M <= 16 * FEW_THREADS.  The k-th largest value is found two bits at a time, three counts per step, by the
-// whole workgroup; a step that splits off exactly k ends the search.
-template <int V>
-__device__ int block_select_of(const uint32_t* vals, int M, int k, int* pos, SelectShared& sh) {
+// how many.  M <= 16 * FEW_THREADS.  (Loops that are not unrolled: a launch is one pass of a few workgroups through the code, and
+// what the code's length costs in fetches is more than what its loops cost; selections of two, four and sixteen values per
+// thread in registers, the steps below otherwise alike, made the kernel 27.7 us where the bits alone took 24.8.)
+//
+// block_select_bits: the k-th largest value is found two bits at a time, three counts per step, by the whole workgroup; a step
+// that splits off exactly k ends the search.  known: it is that value, no search.
+__device__ __forceinline__ int block_select_bits(const uint32_t* vals, int M, int k, int* pos, SelectShared& sh, uint32_t known) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  __syncthreads();  // vals is complete; sh and pos are free
-  if (tid < 16) sh.cnt[tid] = 0;
-  uint32_t v[V];
-#pragma unroll
-  for (int j = 0; j < V; ++j) {
-    const int p = j * FEW_THREADS + tid;
-    v[j] = p < M ? vals[p] : 0u;
-  }
+  const int V = (M + FEW_THREADS - 1) / FEW_THREADS;
+  auto value = [&](int j) { return j * FEW_THREADS + tid < M ? vals[j * FEW_THREADS + tid] : 0u; };
   __syncthreads();
-  uint32_t th = 0;
+  if (tid < 16) sh.cnt[tid] = 0;
+  __syncthreads();
+  uint32_t th = known;
   bool exact = false;  // exactly k values are >= th
-  for (int b = 30; b >= 0 && !exact; b -= 2) {
+#pragma unroll 1
+  for (int b = 30; b >= 0 && !exact && !known; b -= 2) {
     const uint32_t t1 = th | (1u << b), t2 = th | (2u << b), t3 = th | (3u << b);
     int c1 = 0, c2 = 0, c3 = 0;
-#pragma unroll
+#pragma unroll 1
     for (int j = 0; j < V; ++j) {
-        c1 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] >= t1));
-        c2 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] >= t2));
-        c3 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] >= t3));
-      }
+      const uint32_t v = value(j);
+      c1 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v >= t1));
+      c2 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v >= t2));
+      c3 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v >= t3));
+    }
     if (lane == 0)
       atomicAdd(&sh.cnt[b >> 1], (unsigned long long)c1 | ((unsigned long long)c2 << 20) | ((unsigned long long)c3 << 40));
     __syncthreads();
@@ -344,12 +356,13 @@ __device__ int block_select_of(const uint32_t* vals, int M, int k, int* pos, Sel
   // above: selected whatever the ties do; at: values equal to the k-th largest, taken in order until there are k
   const uint32_t above = exact ? th - 1 : th;  // (exact only with th > 0)
   const uint32_t at = exact ? 0u : th;         // 0: none
-#pragma unroll
+#pragma unroll 1
   for (int j = 0; j < V; ++j) {
-      const int ng = __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] > above));
-      const int ne = __builtin_popcountll(__builtin_amdgcn_ballot_w64(at != 0 && v[j] == at));
-      if (lane == 0) sh.scan[j * 16 + wave] = (uint32_t)ng | ((uint32_t)ne << 16);
-    }
+    const uint32_t v = value(j);
+    const int ng = __builtin_popcountll(__builtin_amdgcn_ballot_w64(v > above));
+    const int ne = __builtin_popcountll(__builtin_amdgcn_ballot_w64(at != 0 && v == at));
+    if (lane == 0) sh.scan[j * 16 + wave] = (uint32_t)ng | ((uint32_t)ne << 16);
+  }
   __syncthreads();
   uint32_t total = 0;
   if (wave == 0) {
@@ -379,22 +392,115 @@ __device__ int block_select_of(const uint32_t* vals, int M, int k, int* pos, Sel
   const int n_gt = (int)(total & 0xffff), n_eq = (int)(total >> 16);
   const int need = n_eq < k - n_gt ? n_eq : k - n_gt;
   const unsigned long long below_lane = (1ull << lane) - 1;
-#pragma unroll
+#pragma unroll 1
   for (int j = 0; j < V; ++j) {
-      const unsigned long long bg = __builtin_amdgcn_ballot_w64(v[j] > above);
-      const unsigned long long be = __builtin_amdgcn_ballot_w64(at != 0 && v[j] == at);
-      const uint32_t base = sh.scan[j * 16 + wave];
-      const int g = (int)(base & 0xffff) + __builtin_popcountll(bg & below_lane);
-      const int e = (int)(base >> 16) + __builtin_popcountll(be & below_lane);
-      if (v[j] > above || (at != 0 && v[j] == at && e < need)) pos[g + (e < need ? e : need)] = j * FEW_THREADS + tid;
-    }
+    const uint32_t v = value(j);
+    const unsigned long long bg = __builtin_amdgcn_ballot_w64(v > above);
+    const unsigned long long be = __builtin_amdgcn_ballot_w64(at != 0 && v == at);
+    const uint32_t base = sh.scan[j * 16 + wave];
+    const int g = (int)(base & 0xffff) + __builtin_popcountll(bg & below_lane);
+    const int e = (int)(base >> 16) + __builtin_popcountll(be & below_lane);
+    if (v > above || (at != 0 && v == at && e < need)) pos[g + (e < need ? e : need)] = j * FEW_THREADS + tid;
+  }
   __syncthreads();
   return n_gt + need;
 }
+// block_select: what bounds it is its chain of steps, so it has few, and none waits for one LDS read at a time.  The k-th
+// largest of 256 maxima, of the values at every 256th position each, is a lower bound of the k-th largest value, and hardly more
+// than k values reach it; those are gathered and ranked by counting.  Where more than SELECT_CAP reach it, either one
+// value repeated is the k-th largest, or the bits decide.  Best 10 of 1280 and then of 320, with the loads: 24.9 -> 8.5 us; of 2442,
+// 320 and 320, with the scores formed again: 36.5 -> 19.6; of 14,541 values: 23.5 -> 8.2.
 __device__ __forceinline__ int block_select(const uint32_t* vals, int M, int k, int* pos, SelectShared& sh) {
-  if (M <= 2 * FEW_THREADS) return block_select_of<2>(vals, M, k, pos, sh);
-  if (M <= 4 * FEW_THREADS) return block_select_of<4>(vals, M, k, pos, sh);
-  return block_select_of<16>(vals, M, k, pos, sh);
+  const int tid = threadIdx.x, lane = tid & 63;
+  __syncthreads();  // sh and pos are free
+  if (tid < SELECT_CAP) sh.cand[tid] = 0;
+  if (tid < SELECT_GROUPS) {
+    sh.rank[tid] = 0;
+    sh.top[tid] = 0;
+  }
+  static_assert(SELECT_GROUPS == 256, "a group's number is a byte");
+  if (tid == 0) {
+    sh.n_cand = sh.n_above = 0;
+    sh.least = 0xffffffffu;
+    sh.bound = 1;  // (where fewer than k groups have a value: every value)
+  }
+  __syncthreads();  // vals is complete
+  uint32_t top = 0;
+#pragma unroll 2
+  for (int p = tid; p < M; p += FEW_THREADS) top = vals[p] > top ? vals[p] : top;
+  if (top) atomicMax(&sh.top[tid & (SELECT_GROUPS - 1)], (top & ~0xffu) | (uint32_t)(tid & (SELECT_GROUPS - 1)));
+  __syncthreads();
+  const int g = tid & (SELECT_GROUPS - 1), seg = tid / SELECT_GROUPS * 64;  // a quarter of the maxima against maximum g
+  // (the last byte gives way to the group's number: no two are equal, and one comparison orders them)
+  const uint32_t mine = sh.top[g];
+  int above = 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    u32x4 x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = *(const u32x4*)(sh.top + seg + 32 * h + 4 * i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) above += x[i][j] > mine ? 1 : 0;
+  }
+  if (above) atomicAdd(&sh.rank[g], above);
+  __syncthreads();
+  if (tid < SELECT_GROUPS && sh.rank[tid] == k - 1 && mine > 0xff) sh.bound = mine & ~0xffu;
+  __syncthreads();
+  const uint32_t bound = sh.bound;
+#pragma unroll 2
+  for (int p = tid; p < M; p += FEW_THREADS) {  // (lanes past the end sit out: a ballot counts the others)
+    const uint32_t v = vals[p];
+    const unsigned long long b = __builtin_amdgcn_ballot_w64(v >= bound);
+    if (v >= bound) {
+      int at = 0;
+      if (lane == __builtin_ctzll(b)) at = atomicAdd(&sh.n_cand, (int)__builtin_popcountll(b));
+      at = __builtin_amdgcn_readfirstlane(at) + __builtin_popcountll(b & ((1ull << lane) - 1));
+      if (at < SELECT_CAP) sh.cand[at] = ((unsigned long long)v << 32) | (0xffffffffu - (uint32_t)p);
+    }
+  }
+  __syncthreads();
+  const int C = sh.n_cand;
+  if (C > SELECT_CAP) {
+    // one value repeated?  The least of those that reach the bound, if fewer than k lie above it
+    uint32_t least = 0xffffffffu;
+#pragma unroll 2
+    for (int p = tid; p < M; p += FEW_THREADS) least = vals[p] >= bound && vals[p] < least ? vals[p] : least;
+    atomicMin(&sh.least, least);
+    __syncthreads();
+    least = sh.least;
+    int n_above = 0;
+#pragma unroll 2
+    for (int p = tid; p < M; p += FEW_THREADS) n_above += vals[p] > least ? 1 : 0;
+    if (n_above) atomicAdd(&sh.n_above, n_above);
+    __syncthreads();
+    return block_select_bits(vals, M, k, pos, sh, sh.n_above < k ? least : 0u);
+  }
+  const int n = C < k ? C : k;
+  if (tid < C) {
+    typedef __attribute__((ext_vector_type(2))) unsigned long long u64x2;
+    const unsigned long long key = sh.cand[tid];
+    int rank = 0;
+    for (int i = 0; i < C; i += 16) {
+      u64x2 x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = *(const u64x2*)(sh.cand + i + 2 * j);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) rank += (x[j][0] > key ? 1 : 0) + (x[j][1] > key ? 1 : 0);
+    }
+    if (rank < k) sh.picked[rank] = (int)(0xffffffffu - (uint32_t)key);
+  }
+  __syncthreads();
+  if (tid < n) {
+    const int p = sh.picked[tid];
+    int below = 0;
+#pragma unroll 8
+    for (int i = 0; i < n; ++i) below += sh.picked[i] < p ? 1 : 0;
+    pos[below] = p;
+  }
+  __syncthreads();
+  return n;
 }
 
 struct FewFinishArgs {
@@ -411,25 +517,38 @@ struct FewFinishArgs {
   int64_t* out_idx;
 };
 
-template <int EDT>
+// RAW: the scores are at hand (a form of its own: the code that forms scores again is not in a launch's way then)
+template <int EDT, bool RAW>
 __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a) {
   __shared__ __attribute__((aligned(16))) uint32_t vals[16 * FEW_THREADS];
   __shared__ int pos[FEW_MAX_K], groups[FEW_MAX_K];
   __shared__ int64_t tiles[FEW_MAX_K];
   __shared__ unsigned long long keys[FEW_MAX_K];
   __shared__ SelectShared sh;
-  __shared__ __attribute__((aligned(16))) unsigned char s_query[query_lds_bytes(EDT, QUERY_LDS_MAX_D)];
+  __shared__ __attribute__((aligned(16))) unsigned char s_query[RAW ? 16 : query_lds_bytes(EDT, QUERY_LDS_MAX_D)];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t q = blockIdx.x;
   const float* mx = a.maxima + q * a.ldm;
   const int T = (int)a.n_tiles, k = a.k;
+  const float bias = a.bias ? a.bias[q] : 0.f;  // (asked for long before it is needed)
+  // fill vals[0 .. M) from memory, four loads of a thread in flight
+  auto fill = [&](int M, auto load, auto key) {
+    for (int i0 = tid; i0 < M; i0 += 4 * FEW_THREADS) {
+      float x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = i0 + u * FEW_THREADS < M ? load(i0 + u * FEW_THREADS) : 0.f;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (i0 + u * FEW_THREADS < M) vals[i0 + u * FEW_THREADS] = key(i0 + u * FEW_THREADS, x[u]);
+    }
+  };
   // Three levels, groups of 32 tiles (where there are too many tiles), tiles, entities: the candidates' keys into vals, the
   // best k of them picked.  (One loop, so that the selection is in the code once: the kernel runs a few microseconds, and
   // every copy of it would be fetched cold.)
   const bool grouped = T > FEW_TILES_DIRECT;
   int n = 0;
-  bool direct_rank = false;  // the entities are few enough to be ranked without being picked first
+  bool picked = false;  // the entities: else they are few enough to be ranked all
   // Every tile is among the best k: nothing to pick (a step of the selection is a barrier, sixteen of them 8 us: k = 100,
   // N = 1000, d = 32, 64 queries 72 us a call, 62 without, 66 by the rounds).
   const bool all = T <= k;
@@ -442,27 +561,26 @@ __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a
     int M;
     if (level == 0) {
       M = (T + 31) / 32;
-      for (int g = tid; g < M; g += FEW_THREADS) {
+      fill(M, [&](int g) {
         const f32x4 x = *(const f32x4*)(a.runs + q * (a.ldm / FEW_RUN) + 4 * (int64_t)g);  // 4 runs: 32 tiles
         float m = x[0];
 #pragma unroll
         for (int i = 1; i < 4; ++i)
           if (FEW_RUN * (4 * g + i) < T) m = __builtin_fmaxf(m, x[i]);
-        vals[g] = score_key(m);
-      }
+        return m;
+      }, [&](int, float m) { return score_key(m); });
     } else if (level == 1) {
       M = grouped ? 32 * n : T;
-      for (int i = tid; i < M; i += FEW_THREADS) {
-        const int t = grouped ? 32 * groups[i >> 5] + (i & 31) : i;
-        vals[i] = t < T ? score_key(mx[t]) : 0u;
-      }
+      auto tile_at = [&](int i) { return grouped ? 32 * groups[i >> 5] + (i & 31) : i; };
+      fill(M, [&](int i) { return mx[tile_at(i) < T ? tile_at(i) : 0]; },
+           [&](int i, float m) { return tile_at(i) < T ? score_key(m) : 0u; });
     } else {
       // the tiles' scores: kept by the scan, or formed again (every column of the result tile holds this query, lane
       // c < 16 keeps accumulator c)
       M = 32 * n;
-      if (a.raw) {
-        for (int i = tid; i < M; i += FEW_THREADS)
-          vals[i] = score_key(a.raw[q * a.ldr + tiles[i >> 5] * 32 + (i & 31)]);  // (rows past the end: -inf)
+      if constexpr (RAW) {
+        fill(M, [&](int i) { return a.raw[q * a.ldr + tiles[i >> 5] * 32 + (i & 31)]; },  // (rows past the end: -inf)
+             [&](int, float x) { return score_key(x); });
       } else {
         query_to_lds<EDT>(a.Q + q * a.d, a.d, s_query, tid, FEW_THREADS);
         __syncthreads();
@@ -481,10 +599,10 @@ __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a
           }
         }
       }
-      direct_rank = M <= FEW_THREADS;
-      if (direct_rank) break;
     }
+    if (level == 2 && M <= FEW_DIRECT) break;
     n = block_select(vals, M, k, pos, sh);
+    picked = level == 2;
     if (level == 0) {
       for (int j = tid; j < n; j += FEW_THREADS) groups[j] = pos[j];
     } else if (level == 1) {
@@ -499,23 +617,27 @@ __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a
     float s = __uint_as_float(0x7fc00000u);
     if (key) {
       s = ordered_to_f32(key);
-      if (a.bias) s += a.bias[q];
+      if (a.bias) s += bias;
       if (a.sigmoid) s = 1.0f / (1.0f + expf(-s));
     }
     a.out_scores[q * k + at] = s;
     a.out_idx[q * k + at] = key ? e : -1;
   };
-  if (direct_rank) {
-    // one value per thread: its rank is the number of values above it (equal ones at lower positions count as above)
+  if (32 * n <= FEW_DIRECT && !picked) {
+    // few enough: one value per thread, whose rank is the number of values above it (equal ones at lower positions count as above)
     const int M = 32 * n;
     __syncthreads();
     const uint32_t mine = tid < M ? vals[tid] : 0u;
     int at = 0;
     if (wave * 64 < M) {
-      for (int j = 0; j < M; j += 4) {
-        const u32x4 v = *(const u32x4*)(vals + j);
+      for (int j = 0; j < M; j += 32) {
+        u32x4 v[8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) at += (v[i] > mine || (v[i] == mine && j + i < tid)) ? 1 : 0;
+        for (int u = 0; u < 8; ++u) v[u] = *(const u32x4*)(vals + j + 4 * u);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) at += (v[u][i] > mine || (v[u][i] == mine && j + 4 * u + i < tid)) ? 1 : 0;
       }
     }
     const int ranked = __syncthreads_count(mine != 0);
@@ -533,6 +655,7 @@ __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a
     }
     const unsigned long long key = keys[j];
     int at = 0;
+#pragma unroll 8
     for (int i = 0; i < n; ++i) at += keys[i] > key ? 1 : 0;
     put(at, (uint32_t)(key >> 32), (int64_t)(0xffffffffu - (uint32_t)(key & 0xffffffffull)));
   }
@@ -564,24 +687,42 @@ __global__ void __launch_bounds__(FEW_THREADS) topk_values_kernel(const float* v
   const int tid = threadIdx.x;
   int M = N, n = 0;
   if (tiles) {
+#pragma unroll 4
     for (int t = tid; t < n_tiles; t += FEW_THREADS) vals[t] = tiles[t];
     n = block_select(vals, n_tiles, k, best, sh);
     M = 32 * n;
   }
-  for (int i = tid; i < M; i += FEW_THREADS) {
-    const int at = tiles ? 32 * best[i >> 5] + (i & 31) : i;
-    vals[i] = at < N ? value_key(values[at]) : 0u;
+  for (int i0 = tid; i0 < M; i0 += 8 * FEW_THREADS) {  // (eight loads of a thread in flight)
+    float x[8];
+    int at[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = i0 + u * FEW_THREADS;
+      at[u] = i >= M ? N : tiles ? 32 * best[i >> 5] + (i & 31) : i;
+      x[u] = values[at[u] < N ? at[u] : 0];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i0 + u * FEW_THREADS < M) vals[i0 + u * FEW_THREADS] = at[u] < N ? value_key(x[u]) : 0u;
   }
-  n = block_select(vals, M, k, pos, sh);  // k <= N: there are k
+  const bool all = M <= FEW_MAX_K;  // few enough to be ranked without being picked first
+  if (all) {
+    __syncthreads();
+    n = M;
+  } else {
+    n = block_select(vals, M, k, pos, sh);  // k <= N: there are k
+  }
   for (int j = tid; j < n; j += FEW_THREADS) {
-    const int at = tiles ? 32 * best[pos[j] >> 5] + (pos[j] & 31) : pos[j];
-    keys[j] = ((unsigned long long)vals[pos[j]] << 32) | (0xffffffffu - (uint32_t)at);
+    const int p = all ? j : pos[j], at = tiles ? 32 * best[p >> 5] + (p & 31) : p;
+    keys[j] = ((unsigned long long)vals[p] << 32) | (0xffffffffu - (uint32_t)at);
   }
   __syncthreads();
   for (int j = tid; j < n; j += FEW_THREADS) {
     const unsigned long long key = keys[j];
     int rank = 0;
+#pragma unroll 8
     for (int i = 0; i < n; ++i) rank += keys[i] > key ? 1 : 0;
+    if (rank >= k) continue;
     const uint32_t at = 0xffffffffu - (uint32_t)(key & 0xffffffffull);
     out_values[rank] = values[at];
     out_idx[rank] = (int64_t)at;
@@ -648,9 +789,10 @@ int few_topk_launch(const float* Q, const float* bias, const void* E, int dtype,
   FewFinishArgs f{Q, E, scale, bias, maxima, runs, raw, w.ldm, w.ldr, N, (N + 31) / 32, (int)d, (int)k, apply_sigmoid,
                   out_scores, out_idx};
   const dim3 grid((unsigned)B), block(FEW_THREADS);
-  if (dtype == KGE_F32) hipLaunchKernelGGL((few_finish_kernel<KGE_F32>), grid, block, 0, st, f);
-  else if (dtype == KGE_BF16) hipLaunchKernelGGL((few_finish_kernel<KGE_BF16>), grid, block, 0, st, f);
-  else hipLaunchKernelGGL((few_finish_kernel<KGE_I8>), grid, block, 0, st, f);
+  if (raw) hipLaunchKernelGGL((few_finish_kernel<KGE_F32, true>), grid, block, 0, st, f);  // (whatever the table's type)
+  else if (dtype == KGE_F32) hipLaunchKernelGGL((few_finish_kernel<KGE_F32, false>), grid, block, 0, st, f);
+  else if (dtype == KGE_BF16) hipLaunchKernelGGL((few_finish_kernel<KGE_BF16, false>), grid, block, 0, st, f);
+  else hipLaunchKernelGGL((few_finish_kernel<KGE_I8, false>), grid, block, 0, st, f);
   KGE_LAUNCH_CHECK("few_finish_kernel");
   return KGE_OK;
 }
