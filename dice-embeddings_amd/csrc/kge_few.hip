@@ -679,7 +679,8 @@ __global__ void __launch_bounds__(256) value_tiles_kernel(const float* values, i
 // One workgroup: latency, not work, is what this costs.  tiles: null where the workgroup selects from the values
 // themselves.  (The hop of a query answered by the library's device sort was seven launches for ten values.)
 __global__ void __launch_bounds__(FEW_THREADS) topk_values_kernel(const float* values, int N, const uint32_t* tiles,
-                                                                  int n_tiles, int k, float* out_values, int64_t* out_idx) {
+                                                                  int n_tiles, int k, float* out_values, int64_t* out_idx,
+                                                                  int64_t idx_stride, int64_t relation) {
   __shared__ __attribute__((aligned(16))) uint32_t vals[16 * FEW_THREADS];
   __shared__ int pos[FEW_MAX_K], best[FEW_MAX_K];
   __shared__ unsigned long long keys[FEW_MAX_K];
@@ -725,7 +726,8 @@ __global__ void __launch_bounds__(FEW_THREADS) topk_values_kernel(const float* v
     if (rank >= k) continue;
     const uint32_t at = 0xffffffffu - (uint32_t)(key & 0xffffffffull);
     out_values[rank] = values[at];
-    out_idx[rank] = (int64_t)at;
+    out_idx[rank * idx_stride] = (int64_t)at;
+    if (idx_stride == 2) out_idx[rank * 2 + 1] = relation;  // (the pairs of the next hop's queries)
   }
 }
 
@@ -802,16 +804,17 @@ extern "C" size_t kge_topk_values_workspace_bytes(int64_t N) {
   return N > kge::host::FEW_TILES_DIRECT ? (size_t)((N + 31) / 32) * 4 : 0;
 }
 
-extern "C" int kge_topk_values(const float* values, int64_t N, int64_t k, float* out_values, int64_t* out_idx,
-                               void* workspace, size_t workspace_bytes, void* stream) {
-  using namespace kge;
+namespace kge {
+namespace {
+int topk_values_impl(const float* values, int64_t N, int64_t k, float* out_values, int64_t* out_idx, int64_t idx_stride,
+                     int64_t relation, void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
   KGE_REQUIRE(N >= 1 && N <= 32LL * FEW_TILES_DIRECT, KGE_ERR_UNSUPPORTED, "kge_topk_values: N=%lld outside [1, %lld]",
               (long long)N, 32LL * FEW_TILES_DIRECT);
   KGE_REQUIRE(k >= 1 && k <= N && k <= FEW_MAX_K, KGE_ERR_UNSUPPORTED, "kge_topk_values: k=%lld outside [1, min(N, %d)]",
               (long long)k, FEW_MAX_K);
   KGE_REQUIRE(values && out_values && out_idx, KGE_ERR_INVALID, "kge_topk_values: null pointer argument");
-  const size_t need = kge_topk_values_workspace_bytes(N);
+  const size_t need = ::kge_topk_values_workspace_bytes(N);
   KGE_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 3) == 0), KGE_ERR_WORKSPACE,
               "kge_topk_values: workspace of %zu bytes, need %zu, 4-byte aligned", workspace_bytes, need);
   hipStream_t st = (hipStream_t)stream;
@@ -822,7 +825,48 @@ extern "C" int kge_topk_values(const float* values, int64_t N, int64_t k, float*
     KGE_LAUNCH_CHECK("value_tiles_kernel");
   }
   hipLaunchKernelGGL(topk_values_kernel, dim3(1), dim3(FEW_THREADS), 0, st, values, (int)N, tiles, n_tiles, (int)k, out_values,
-                     out_idx);
+                     out_idx, idx_stride, relation);
   KGE_LAUNCH_CHECK("topk_values_kernel");
+  return KGE_OK;
+}
+
+// out[n] = the largest of t(weight[j], S[j, n]) over the substitutions j: a thread per entity, four rows' loads in flight
+template <bool MIN>
+__global__ void __launch_bounds__(256) hop_scores_kernel(const float* weight, const float* S, int k, int64_t N, int64_t ldS, float* out) {
+  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (n >= N) return;
+  float best = 0.f;
+#pragma unroll 4
+  for (int j = 0; j < k; ++j) {
+    const float w = weight[j], s = S[j * ldS + n];
+    const float v = MIN ? (w != w ? w : s < w || s != s ? s : w) : w * s;
+    best = j == 0 || v > best || v != v ? v : best;  // (a NaN stays: nothing is greater)
+  }
+  out[n] = best;
+}
+}  // namespace
+}  // namespace kge
+
+extern "C" int kge_topk_values(const float* values, int64_t N, int64_t k, float* out_values, int64_t* out_idx,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  return kge::topk_values_impl(values, N, k, out_values, out_idx, 1, 0, workspace, workspace_bytes, stream);
+}
+
+extern "C" int kge_topk_values_pairs(const float* values, int64_t N, int64_t k, int64_t relation, float* out_values,
+                                     int64_t* out_pairs, void* workspace, size_t workspace_bytes, void* stream) {
+  return kge::topk_values_impl(values, N, k, out_values, out_pairs, 2, relation, workspace, workspace_bytes, stream);
+}
+
+extern "C" int kge_hop_scores(const float* weight, const float* S, int64_t k, int64_t N, int64_t ldS, int tnorm, float* out,
+                              void* stream) {
+  using namespace kge;
+  clear_error();
+  KGE_REQUIRE(k >= 1 && k <= 0x7fffffff && N >= 1 && N <= 0x7fffffffLL * 256 && ldS >= N && (tnorm == 0 || tnorm == 1), KGE_ERR_INVALID,
+              "kge_hop_scores: k=%lld N=%lld ldS=%lld tnorm=%d", (long long)k, (long long)N, (long long)ldS, tnorm);
+  KGE_REQUIRE(weight && S && out, KGE_ERR_INVALID, "kge_hop_scores: null pointer argument");
+  const dim3 grid((unsigned)((N + 255) / 256)), block(256);
+  if (tnorm) hipLaunchKernelGGL((hop_scores_kernel<true>), grid, block, 0, (hipStream_t)stream, weight, S, (int)k, N, ldS, out);
+  else hipLaunchKernelGGL((hop_scores_kernel<false>), grid, block, 0, (hipStream_t)stream, weight, S, (int)k, N, ldS, out);
+  KGE_LAUNCH_CHECK("hop_scores_kernel");
   return KGE_OK;
 }

@@ -527,6 +527,28 @@ inline BwdPlan bwd_plan(int64_t B, int64_t d, int64_t N) {
   return p;
 }
 
+// workspace of kge_kvsall_step
+struct StepOffsets {
+  size_t Q, bias, rows, dQ, dbias, bwd, total;
+};
+inline StepOffsets step_offsets(int64_t B, int64_t d, int64_t N) {
+  StepOffsets o{};
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off = align_up(off + bytes, 256);
+    return at;
+  };
+  o.Q = take((size_t)B * d * 4);
+  o.bias = take((size_t)B * 4);
+  o.rows = take((size_t)B * 8);
+  o.dQ = take((size_t)B * d * 4);
+  o.dbias = take((size_t)B * 4);
+  o.bwd = take(bwd_plan(B, d, N).total);
+  o.total = off;
+  return o;
+}
+
 // ---- vocabulary keys: ((a * range_b + b) << vbits) | v ----------------------------------------------------
 KGE_HD inline int bits_for(int64_t range) {  // bits needed for values in [0, range)
   int b = 1;

@@ -170,6 +170,26 @@ __global__ void ranks_kernel(const int32_t* n_gt, const int32_t* n_eq, const int
   ranks[b] = 1 + (int64_t)n_gt[b] + ties;
 }
 
+// ---- what a training step needs before its contractions: the filter rows of its pairs, and its outputs that are added to cleared
+struct StepPrepare {
+  const int64_t* hr;
+  int64_t B;
+  const int64_t* keys;
+  int64_t n_rows, key_mult;
+  int64_t* rows;
+  float* clear[8];
+  int64_t counts[8];
+};
+__global__ void __launch_bounds__(256) step_prepare_kernel(StepPrepare s) {  // grid.y: 0 the rows, then the buffers
+  const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+  if (blockIdx.y == 0) {
+    for (int64_t b = i0; b < s.B; b += stride) s.rows[b] = filter_row(s.hr[2 * b], s.hr[2 * b + 1], s.keys, s.n_rows, s.key_mult);
+    return;
+  }
+  float* p = s.clear[blockIdx.y - 1];
+  for (int64_t i = i0; i < s.counts[blockIdx.y - 1]; i += stride) p[i] = 0.f;
+}
+
 // ---- group the queries of one sub-batch by filter row and plan the correction work -----------
 // One workgroup, no sort: (1) every query claims the slot of its filter row in an LDS hash table
 // (compare-and-swap on the row number) and takes a ticket from the slot's counter; the query with
@@ -2583,4 +2603,62 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
     KGE_LAUNCH_CHECK("reduce_splits_kernel");
   }
   return KGE_OK;
+}
+
+extern "C" size_t kge_kvsall_step_workspace_bytes(int64_t B, int64_t d, int64_t N) {
+  return B < 1 || d < 1 || N < 1 ? 0 : host::step_offsets(B, d, N).total;
+}
+
+extern "C" int kge_kvsall_step(const kge_step_params* p, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  KGE_REQUIRE(p, KGE_ERR_INVALID, "kge_kvsall_step: null parameters");
+  const int64_t B = p->B, d = p->d, N = p->N;
+  KGE_REQUIRE(B >= 1 && d >= 1 && N >= 1 && p->R >= 1, KGE_ERR_INVALID, "kge_kvsall_step: B=%lld d=%lld N=%lld R=%lld", (long long)B,
+              (long long)d, (long long)N, (long long)p->R);
+  KGE_REQUIRE(p->ent && p->rel && p->hr && p->loss && p->d_ent && p->d_rel, KGE_ERR_INVALID, "kge_kvsall_step: null pointer argument");
+  KGE_REQUIRE(!p->keys == !p->row_ptr && !p->keys == !p->col, KGE_ERR_INVALID, "kge_kvsall_step: a filter is keys, row_ptr and col");
+  KGE_REQUIRE(p->n_rows >= 0 && (!p->keys || p->key_mult >= 1), KGE_ERR_INVALID, "kge_kvsall_step: n_rows=%lld key_mult=%lld",
+              (long long)p->n_rows, (long long)p->key_mult);
+  const host::StepOffsets o = host::step_offsets(B, d, N);
+  KGE_REQUIRE(workspace && workspace_bytes >= o.total, KGE_ERR_WORKSPACE, "kge_kvsall_step: workspace of %zu bytes, need %zu",
+              workspace_bytes, o.total);
+  KGE_REQUIRE(((uintptr_t)workspace & 255) == 0, KGE_ERR_WORKSPACE, "kge_kvsall_step: workspace must be 256-byte aligned");
+  char* ws = (char*)workspace;
+  float *Q = (float*)(ws + o.Q), *bias = (float*)(ws + o.bias), *dQ = (float*)(ws + o.dQ);
+  float* dbias = p->bias_varies ? (float*)(ws + o.dbias) : nullptr;
+  int64_t* rows = (int64_t*)(ws + o.rows);
+  const bool filtered = p->keys && p->n_rows > 0;
+  StepPrepare sp{p->hr, filtered ? B : 0, p->keys, p->n_rows, p->key_mult, rows, {}, {}};
+  int n = 0;
+  int64_t most = filtered ? B : 0;
+  auto clear = [&](float* buf, int64_t count) {
+    if (!buf || count == 0) return;
+    sp.clear[n] = buf;
+    sp.counts[n++] = count;
+    most = count > most ? count : most;
+  };
+  clear(p->d_rel, p->R * d);
+  clear(p->d_coeff_p, p->coeff_p ? p->p : 0);
+  clear(p->d_coeff_q, p->coeff_q ? p->q : 0);
+  clear(p->d_coeff_r, p->coeff_r ? p->r : 0);
+  clear(p->d_norm.h_a, d);
+  clear(p->d_norm.h_b, d);
+  clear(p->d_norm.r_a, d);
+  clear(p->d_norm.r_b, d);
+  int rc = p->model == KGE_DECAL
+               ? kge_build_query_decal(0, p->p, p->q, p->r, p->ent, KGE_F32, nullptr, p->rel, KGE_F32, p->coeff_p, p->coeff_q,
+                                       p->coeff_r, p->norm, p->hr, B, d, N, p->R, Q, bias, stream)
+               : kge_build_query(p->model, p->p, p->q, p->ent, KGE_F32, nullptr, p->rel, KGE_F32, p->coeff_p, p->coeff_q,
+                                 p->normalize_relation, p->norm, p->hr, B, d, N, p->R, Q, bias, stream);
+  if (rc) return rc;
+  const int64_t blocks = (most + 255) / 256;
+  hipLaunchKernelGGL(step_prepare_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024), (unsigned)(n + 1)), dim3(256), 0,
+                     (hipStream_t)stream, sp);
+  KGE_LAUNCH_CHECK("step_prepare_kernel");
+  rc = kge_bce_multihot_backward(Q, bias, p->ent, KGE_F32, B, d, N, filtered ? rows : nullptr, p->row_ptr, p->col, p->n_rows,
+                                 p->label_smoothing, 1.0f, p->loss, dQ, dbias, p->d_ent, ws + o.bwd, workspace_bytes - o.bwd, stream);
+  if (rc) return rc;
+  return kge_build_query_backward_norm(p->model, p->p, p->q, p->r, p->ent, p->rel, p->coeff_p, p->coeff_q, p->coeff_r,
+                                       p->normalize_relation, p->norm, p->norm ? &p->d_norm : nullptr, nullptr, p->hr, B, d, N, p->R,
+                                       dQ, dbias, p->d_ent, p->d_rel, p->d_coeff_p, p->d_coeff_q, p->d_coeff_r, stream);
 }

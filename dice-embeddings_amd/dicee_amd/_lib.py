@@ -41,6 +41,17 @@ class RankPassParams(ctypes.Structure):
                    ("ranks", _vp)])
 
 
+class StepParams(ctypes.Structure):
+    _fields_ = ([(k, ctypes.c_int32) for k in ("model", "p", "q", "r", "normalize_relation", "bias_varies")]
+                + [("label_smoothing", _c_f)]
+                + [(k, _vp) for k in ("ent", "rel", "coeff_p", "coeff_q", "coeff_r")]
+                + [("norm", ctypes.POINTER(NormParams)), ("hr", _vp)]
+                + [(k, _c_i64) for k in ("B", "d", "N", "R")]
+                + [("keys", _vp), ("n_rows", _c_i64), ("key_mult", _c_i64), ("row_ptr", _vp), ("col", _vp)]
+                + [(k, _vp) for k in ("loss", "d_ent", "d_rel", "d_coeff_p", "d_coeff_q", "d_coeff_r")]
+                + [("d_norm", NormGrads)])
+
+
 TIES = {"stable": 0, "optimistic": 1, "pessimistic": 2, "mean": 3}
 
 SIGNATURES = {
@@ -63,6 +74,10 @@ SIGNATURES = {
                                                _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "kge_topk_values_workspace_bytes": (_sz, [_c_i64]),
     "kge_topk_values": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _vp, _sz, _vp]),
+    "kge_topk_values_pairs": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _vp, _sz, _vp]),
+    "kge_hop_scores": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp, _vp]),
+    "kge_kvsall_step_workspace_bytes": (_sz, [_c_i64, _c_i64, _c_i64]),
+    "kge_kvsall_step": (_c_int, [ctypes.POINTER(StepParams), _vp, _sz, _vp]),
     "kge_fill_zero": (_c_int, [_vp, _vp, _c_int, _vp]),
     "kge_batchnorm_workspace_bytes": (_sz, [_c_i64, _c_i64]),
     "kge_batchnorm_stats": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(DropoutParams), _c_f,

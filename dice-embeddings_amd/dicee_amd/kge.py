@@ -11,6 +11,8 @@ from typing import List, Union
 
 import torch
 
+from .models import BaseKGE
+
 
 def _call_size(batch_size, fused_topk):
     """Queries per library call.  The reference's batch size bounds the B x N score matrix of a batch
@@ -64,6 +66,28 @@ class KGE:
             rel = torch.LongTensor([self.relation_to_idx[relation]])
         return torch.cartesian_prod(head, rel).view(-1, 2)          # heads-major, as the reference
 
+    def _best_of_batch(self, pairs, topk, heads=False):
+        """``model.topk`` of pairs that are on the host, its scores and ids back on the host by one copy."""
+        dev = self.model.entity_embeddings.weight.device
+        P = pairs.size(0)
+        if dev.type != "cuda" or not isinstance(topk, int) or topk < 1 or type(self.model).topk is not BaseKGE.topk:
+            s, idx = self.model.topk(pairs.to(dev), topk, **({"heads": True} if heads else {}))
+            return s.cpu(), idx.cpu()
+        n = P * topk
+        buf = torch.empty((3 * n,), dtype=torch.int32, device=dev)
+        self.model.topk(pairs.to(dev), topk, heads=heads,
+                        out=(buf[2 * n:].view(torch.float32).view(P, topk), buf[:2 * n].view(torch.int64).view(P, topk)))
+        host = buf.cpu()
+        return host[2 * n:].view(torch.float32).view(P, topk), host[:2 * n].view(torch.int64).view(P, topk)
+
+    def _best(self, pairs, topk, batch_size, heads=False):
+        """(scores, ids) of the ``topk`` best entities per pair, flat, on the host (fused: no [B,N] matrix)."""
+        parts = [self._best_of_batch(pairs[i:i + batch_size], topk, heads) for i in range(0, pairs.size(0), batch_size)]
+        if len(parts) == 1:
+            return parts[0][0].flatten(), parts[0][1].flatten()
+        return (torch.cat([torch.zeros(0)] + [s.flatten() for s, _ in parts]),
+                torch.cat([torch.zeros(0, dtype=torch.long)] + [idx.flatten() for _, idx in parts]))
+
     def predict_missing_tail_entity(self, head_entity: Union[List[str], str], relation: Union[List[str], str],
                                     within: List[str] = None, batch_size=2, topk=1, return_indices=False):
         if within is not None:
@@ -72,24 +96,15 @@ class KGE:
         P = hr_pairs.size(0)
         T = self.num_entities
         dev = self.model.entity_embeddings.weight.device
-        if return_indices:
-            scores = torch.zeros(P, topk)
-            indices = torch.zeros(P, topk, dtype=torch.long)
-        else:
-            scores = torch.zeros(P * T)
         batch_size = _call_size(batch_size, return_indices)
+        if return_indices:
+            return self._best(hr_pairs, topk, batch_size)
+        scores = torch.zeros(P * T)
         for i in range(0, P, batch_size):
             batch_hr = hr_pairs[i:i + batch_size].to(dev)
             B = batch_hr.size(0)
-            if return_indices:
-                s, idx = self.model.topk(batch_hr, topk)          # fused: no [B,N] matrix
-                scores[i:i + batch_size, :] = s.cpu()
-                indices[i:i + batch_size, :] = idx.cpu()
-            else:
-                batch_scores = self.model(batch_hr).view(B, T)
-                scores[i * T:i * T + B * T] = batch_scores.flatten().cpu()
-        if return_indices:
-            return scores.flatten(), indices.flatten()
+            batch_scores = self.model(batch_hr).view(B, T)
+            scores[i * T:i * T + B * T] = batch_scores.flatten().cpu()
         return scores
 
     def predict_missing_head_entity(self, relation: Union[List[str], str], tail_entity: Union[List[str], str],
@@ -108,24 +123,15 @@ class KGE:
         tr_pairs = torch.cartesian_prod(tail, rel).view(-1, 2)
         P, H = tr_pairs.size(0), self.num_entities
         dev = self.model.entity_embeddings.weight.device
-        if return_indices:
-            scores = torch.zeros(P, topk)
-            indices = torch.zeros(P, topk, dtype=torch.long)
-        else:
-            scores = torch.zeros(P * H)
         batch_size = _call_size(batch_size, return_indices)
-        for i in range(0, P, batch_size):
-            batch = tr_pairs[i:i + batch_size]
-            rt = torch.stack([batch[:, 1], batch[:, 0]], dim=1).to(dev)      # the kernels take (relation, tail)
-            B = rt.size(0)
-            if return_indices:
-                s, idx = self.model.topk(rt, topk, heads=True)
-                scores[i:i + batch_size, :] = s.cpu()
-                indices[i:i + batch_size, :] = idx.cpu()
-            else:
-                scores[i * H:i * H + B * H] = self.model.forward_all_heads(rt).flatten().cpu()
+        rt_pairs = torch.stack([tr_pairs[:, 1], tr_pairs[:, 0]], dim=1)      # the kernels take (relation, tail)
         if return_indices:
-            return scores.flatten(), indices.flatten()
+            return self._best(rt_pairs, topk, batch_size, heads=True)
+        scores = torch.zeros(P * H)
+        for i in range(0, P, batch_size):
+            rt = rt_pairs[i:i + batch_size].to(dev)
+            B = rt.size(0)
+            scores[i * H:i * H + B * H] = self.model.forward_all_heads(rt).flatten().cpu()
         return scores
 
     def predict_missing_relations(self, head_entity: Union[List[str], str], tail_entity: Union[List[str], str],
@@ -273,20 +279,34 @@ class KGE:
         """[len(head_ids), N] logits of (head, relation, ?) on the GPU: ONE batched KvsAll call where the
         reference calls ``predict`` once per substitution."""
         dev = self.model.entity_embeddings.weight.device
+        if isinstance(head_ids, list):                      # (one copy to the device)
+            rel = self.relation_to_idx[relation]
+            with torch.no_grad():
+                return self.model.forward_k_vs_all(torch.tensor([[h, rel] for h in head_ids], dtype=torch.int64, device=dev))
         head_ids = torch.as_tensor(head_ids, dtype=torch.int64, device=dev).reshape(-1)
         rel = torch.full_like(head_ids, self.relation_to_idx[relation])
         with torch.no_grad():
             return self.model.forward_k_vs_all(torch.stack([head_ids, rel], dim=1).contiguous())
 
-    @staticmethod
-    def _best(scores, k):
-        """(values, positions) of the k best of a vector of scores, as a stable descending sort orders them."""
+    def _hop(self, scores, k, relation):
+        """The k best substitutions of a variable, as a stable descending sort of its ``scores`` orders them, and the logits
+        of every entity behind each: (values [k], [k, N])."""
         from . import ops
         if (scores.is_cuda and scores.dtype == torch.float32 and 1 <= k <= min(scores.numel(), ops.TOPK_VALUES_MAX_K)
                 and scores.numel() <= ops.TOPK_VALUES_MAX_N and not scores.requires_grad):
-            return ops.topk_values(scores.contiguous(), k)
+            s, pairs = ops.topk_values(scores.contiguous(), k, relation=self.relation_to_idx[relation])
+            with torch.no_grad():
+                return s, self.model.forward_k_vs_all(pairs)
         s, idx = torch.sort(scores, descending=True, stable=True)
-        return s[:k], idx[:k]
+        return s[:k], self._atom(idx[:k], relation)
+
+    def _best_path(self, s, logits, tnorm):
+        """[N]: the best t-norm over the substitutions, ``max(t_norm(s[:, None], logits), dim=0)``."""
+        from . import ops
+        if (logits.is_cuda and logits.dtype == s.dtype == torch.float32 and logits.shape[0] and logits.is_contiguous()
+                and type(self).t_norm is KGE.t_norm and ("min" in tnorm or "prod" in tnorm)):
+            return ops.hop_scores(s, logits, minimum="min" in tnorm)
+        return torch.max(self.t_norm(s[:, None], logits, tnorm), dim=0)[0]
 
     def _multi_hop_scores(self, query_type, query, tnorm, neg_norm, lambda_, k):
         """[N] GPU tensor: score of every entity as the answer (the norms act on logits, as in the reference,
@@ -294,8 +314,7 @@ class KGE:
         one = lambda e, r: self._atom([self.entity_to_idx[e]], r)[0]
 
         def hop(prev, r):          # keep the k best substitutions of the variable, then the best t-norm per answer
-            s, idx = self._best(prev, k)
-            return torch.max(self.t_norm(s[:, None], self._atom(idx, r), tnorm), dim=0)[0]
+            return self._best_path(*self._hop(prev, k, r), tnorm)
         if query_type == "1p":
             e, (r1,) = query
             return one(e, r1)
@@ -320,11 +339,10 @@ class KGE:
             return hop(self._multi_hop_scores(inner_type, inner, tnorm, neg_norm, lambda_, k), r)
         if query_type in ("pi", "pin", "pni"):
             (e1, rels), (e3, rel3) = query
-            s, idx = self._best(one(e1, rels[0]), k)
-            a2 = self._atom(idx, rels[1])
+            s, a2 = self._hop(one(e1, rels[0]), k, rels[1])
             if query_type == "pni":
                 a2 = self.negnorm(a2, lambda_, neg_norm)
-            two_p = torch.max(self.t_norm(s[:, None], a2, tnorm), dim=0)[0]
+            two_p = self._best_path(s, a2, tnorm)
             last = one(e3, rel3[0])
             if query_type == "pin":
                 last = self.negnorm(last, lambda_, neg_norm)

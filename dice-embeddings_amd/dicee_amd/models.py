@@ -289,7 +289,7 @@ class BaseKGE(torch.nn.Module):
         rows = csr.rows_for(x.to(device=E.device, dtype=torch.int64))
         return ops.rank_filtered(Q, bias, E, scale, target, rows, csr.row_ptr, csr.col, out=out)
 
-    def topk(self, x, k, sigmoid=False, heads=False):
+    def topk(self, x, k, sigmoid=False, heads=False, out=None):
         Q, bias = self.query(x, heads=heads)
         E, scale = self.table()
         # the quantised table's derived form for the scan lives and dies with the quantised table itself
@@ -298,7 +298,7 @@ class BaseKGE(torch.nn.Module):
             if self._topk_prepared is None or self._topk_prepared[0] != E.data_ptr():
                 self._topk_prepared = (E.data_ptr(), ops.topk_prepare(E, scale))
             prepared = self._topk_prepared[1]
-        return ops.topk(Q, bias, E, scale, k, sigmoid=sigmoid, prepared=prepared)
+        return ops.topk(Q, bias, E, scale, k, sigmoid=sigmoid, prepared=prepared, out=out)
 
     def kvsall_bce_loss(self, x, csr, label_smoothing=0.0):
         """Forward + loss of training_step (base_model.py:25-46) for a KvsAll batch whose multi-hot
@@ -339,6 +339,13 @@ class BaseKGE(torch.nn.Module):
         x = x.to(device=E.device, dtype=torch.int64).contiguous()
         dropout = self._draw_dropout(x.shape[0], E.device)
         norm = self._norm_params(x, dropout)
+        cls = type(self)
+        if (dropout is None and not (norm and norm.get("batch")) and cls.query is BaseKGE.query and cls.table is BaseKGE.table
+                and cls.kvsall_bce_backward is BaseKGE.kvsall_bce_backward):
+            loss, dE, dR, dcoeff, dnorm = ops.kvsall_step(
+                self.name if self.name != "CKeci" else "Keci", E, self._rel(), x, csr, label_smoothing, norm=norm,
+                bias_varies=self._bias_varies(), **self._query_kwargs())
+            return loss[0], self._named_gradients(dE, dR, dcoeff, dnorm)
         loss, dQ, dbias, dE = self.kvsall_bce_backward(x, csr, label_smoothing, norm=norm, dropout=dropout,
                                                        want_dbias=self._bias_varies())
         rel = self._rel()
@@ -351,6 +358,10 @@ class BaseKGE(torch.nn.Module):
         dnorm = dict(zip(layer, rest[3:])) or None
         dcoeff = ops.build_query_backward(name, E, rel, x, dQ, dbias, dE, dR, norm=norm, dnorm=dnorm, dropout=dropout,
                                           dcoeff=rest[:3], **kw)
+        return loss, self._named_gradients(dE, dR, dcoeff, dnorm)
+
+    @staticmethod
+    def _named_gradients(dE, dR, dcoeff, dnorm):
         grads = {"entity_embeddings.weight": dE, "relation_embeddings.weight": dR}
         if dnorm is not None:
             grads["normalize_head_entity_embeddings.weight"] = dnorm["h_a"]
@@ -360,16 +371,16 @@ class BaseKGE(torch.nn.Module):
         for key, g in zip(("p_coefficients.weight", "q_coefficients.weight", "r_coefficients.weight"), dcoeff):
             if g is not None:
                 grads[key] = g.reshape(1, -1)
-        return loss, grads
+        return grads
 
     def kvsall_training_step(self, x, csr, label_smoothing=0.0):
         """``training_step`` followed by ``loss.backward()`` (base_model.py:25-46) for one KvsAll batch: returns the
         loss (detached) and ACCUMULATES the gradients into ``.grad`` of the parameters the step reads, as
         autograd would, so that any ``torch.optim`` optimizer can take the step."""
         loss, grads = self.kvsall_bce_gradients(x, csr, label_smoothing)
-        params = dict(self.named_parameters())
         for name, g in grads.items():
-            prm = params[name]
+            layer, attr = name.split(".")
+            prm = getattr(getattr(self, layer), attr)
             if not prm.requires_grad:
                 continue
             prm.grad = g if prm.grad is None else prm.grad + g

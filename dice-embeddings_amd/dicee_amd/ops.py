@@ -419,6 +419,25 @@ def rank_filtered(Q, bias, E, scale, target, csr_row=None, row_ptr=None, col=Non
     return out
 
 
+def _at(t):
+    return None if t is None else t.data_ptr()
+
+
+def _filter_args(csr):
+    """(keys, rows, key multiplier, row_ptr, col) of a ``FilterCSR`` on the GPU, addresses None where it has no rows."""
+    if csr is None or not csr.keys.numel():
+        return None, 0, 1, None, None
+    _require_gpu(csr.keys, csr.row_ptr, csr.col)
+    if csr.keys.dtype != torch.int64 or csr.row_ptr.dtype != torch.int64 or csr.col.dtype != torch.int32:
+        raise TypeError("the filter's keys / row_ptr must be int64 and col int32")
+    n_rows, col = csr.row_ptr.numel() - 1, csr.col.data_ptr()
+    if csr.keys.numel() != n_rows:
+        raise ValueError("a filter has one key per row")
+    if col == 0:                                        # (every row is empty)
+        return None, 0, 1, None, None
+    return csr.keys.data_ptr(), n_rows, int(csr.num_relations), csr.row_ptr.data_ptr(), col
+
+
 def rank_pass(model, ent, rel, pairs, targets, csr=None, *, ent_scale=None, p=0, q=0, r=0, coeff_p=None, coeff_q=None,
               coeff_r=None, normalize_relation=True, norm=None, head=False, tie="stable", out=None):
     """Ranks (int64 [n]) of ``targets`` [n] for the queries ``pairs`` [n,2] in one call: ``build_query``, ``csr_lookup``,
@@ -444,22 +463,9 @@ def rank_pass(model, ent, rel, pairs, targets, csr=None, *, ent_scale=None, p=0,
         out = torch.empty((n,), dtype=torch.int64, device=ent.device)
     elif out.dtype != torch.int64 or out.shape != (n,):
         raise ValueError("out must be an int64 tensor of shape [n]")
-    keys = row_ptr = col = None
-    n_rows, mult = 0, 1
-    if csr is not None and csr.keys.numel():
-        _require_gpu(csr.keys, csr.row_ptr, csr.col)
-        if csr.keys.dtype != torch.int64 or csr.row_ptr.dtype != torch.int64 or csr.col.dtype != torch.int32:
-            raise TypeError("the filter's keys / row_ptr must be int64 and col int32")
-        keys, row_ptr, col = csr.keys.data_ptr(), csr.row_ptr.data_ptr(), csr.col.data_ptr()
-        n_rows, mult = csr.row_ptr.numel() - 1, int(csr.num_relations)
-        if csr.keys.numel() != n_rows:
-            raise ValueError("a filter has one key per row")
-        if col == 0:                                    # (every row empty: nothing to filter)
-            keys = row_ptr = col = None
+    keys, n_rows, mult, row_ptr, col = _filter_args(csr)
     ns, keep = _norm_struct(norm)
-
-    def at(t):
-        return None if t is None else t.data_ptr()
+    at = _at
     s = _lib.RankPassParams(MODEL_IDS[model], int(p), int(q), int(r), _table_dtype(ent), _table_dtype(rel),
                             int(bool(normalize_relation)), int(bool(head)), _lib.TIES[tie], ent.data_ptr(), at(ent_scale),
                             rel.data_ptr(), at(coeff_p), at(coeff_q), at(coeff_r),
@@ -490,17 +496,24 @@ def topk_prepare(E, scale):
     return buf
 
 
-def topk(Q, bias, E, scale, k, sigmoid=False, prepared=None):
+def topk(Q, bias, E, scale, k, sigmoid=False, prepared=None, out=None):
     """Fused top-k over all entities: ([B,k] fp32 descending, [B,k] int64).  ``prepared``: what ``topk_prepare``
-    returned for this very table (same results, without deriving it again in every call)."""
+    returned for this very table (same results, without deriving it again in every call).  ``out``: such a pair of
+    contiguous tensors to write into."""
     lib = _lib.load()
     _require_gpu(Q, bias, E, scale)
     _check_qe(Q, E, scale, bias)
     B, d = Q.shape
     N = E.shape[0]
     dev = Q.device
-    out_s = torch.empty((B, k), dtype=torch.float32, device=dev)
-    out_i = torch.empty((B, k), dtype=torch.int64, device=dev)
+    if out is None:
+        out_s = torch.empty((B, k), dtype=torch.float32, device=dev)
+        out_i = torch.empty((B, k), dtype=torch.int64, device=dev)
+    else:
+        out_s, out_i = out
+        _require_gpu(out_s, out_i)
+        if out_s.dtype != torch.float32 or out_i.dtype != torch.int64 or out_s.shape != (B, k) or out_i.shape != (B, k):
+            raise ValueError("out must be float32 and int64 tensors of shape [B, k]")
     if prepared is not None:
         _require_gpu(prepared)
         ws_bytes = lib.kge_topk_prepared_workspace_bytes(B, N, k)
@@ -520,9 +533,10 @@ def topk(Q, bias, E, scale, k, sigmoid=False, prepared=None):
 TOPK_VALUES_MAX_K, TOPK_VALUES_MAX_N = 128, 524288
 
 
-def topk_values(values, k):
+def topk_values(values, k, relation=None):
     """(values [k], positions int64 [k]): the first k of ``torch.sort(values, descending=True, stable=True)`` of a
-    contiguous fp32 vector of up to 524,288 values, k up to 128."""
+    contiguous fp32 vector of up to 524,288 values, k up to 128.  ``relation``: the positions as pairs (position, relation)
+    [k,2] instead, the next hop's queries."""
     k = operator.index(k)                                     # (2.5 is no number of values, as for a slice)
     lib = _lib.load()
     _require_gpu(values)
@@ -530,11 +544,64 @@ def topk_values(values, k):
         raise TypeError("values must be a float32 vector")
     n = values.numel()
     out_v = torch.empty((k,), dtype=torch.float32, device=values.device)
-    out_i = torch.empty((k,), dtype=torch.int64, device=values.device)
+    out_i = torch.empty((k,) if relation is None else (k, 2), dtype=torch.int64, device=values.device)
     nbytes = lib.kge_topk_values_workspace_bytes(n)
     ws = torch.empty((nbytes,), dtype=torch.uint8, device=values.device) if nbytes else None
-    _lib.check(lib.kge_topk_values(_ptr(values), n, k, _ptr(out_v), _ptr(out_i), _ptr(ws), nbytes, _stream()))
+    if relation is None:
+        _lib.check(lib.kge_topk_values(_ptr(values), n, k, _ptr(out_v), _ptr(out_i), _ptr(ws), nbytes, _stream()))
+    else:
+        _lib.check(lib.kge_topk_values_pairs(_ptr(values), n, k, int(relation), _ptr(out_v), _ptr(out_i), _ptr(ws), nbytes,
+                                             _stream()))
     return out_v, out_i
+
+
+def hop_scores(weight, S, minimum=False):
+    """[N] fp32: the largest over j of ``weight[j] * S[j]`` (``minimum``: of the smaller of the two), the scores of a hop over
+    its k substitutions: ``torch.max(t_norm(weight[:, None], S), dim=0)[0]``."""
+    lib = _lib.load()
+    _require_gpu(weight, S)
+    if weight.dtype != torch.float32 or S.dtype != torch.float32 or S.dim() != 2 or weight.shape != S.shape[:1]:
+        raise TypeError("weight [k] and S [k, N] must be float32")
+    out = torch.empty((S.shape[1],), dtype=torch.float32, device=S.device)
+    _lib.check(lib.kge_hop_scores(_ptr(weight), _ptr(S), S.shape[0], S.shape[1], S.shape[1], int(bool(minimum)), _ptr(out),
+                                  _stream()))
+    return out
+
+
+def kvsall_step(model, ent, rel, hr, csr, label_smoothing=0.0, *, p=0, q=0, r=0, coeff_p=None, coeff_q=None, coeff_r=None,
+                normalize_relation=True, norm=None, bias_varies=True):
+    """One KvsAll training step, forward and backward, in one call: ``(loss [1], d_ent [N,d], d_rel [R,d], (d_coeff_p,
+    d_coeff_q, d_coeff_r), d_norm)``, None where the model has no such parameter; ``d_norm``: for LayerNorm the dict of
+    ``h_a, h_b, r_a, r_b``.  What ``csr_lookup``, ``build_query``, ``bce_multihot_backward`` and ``build_query_backward`` do in
+    a row, without dropout and batch statistics."""
+    lib = _lib.load()
+    _require_gpu(ent, rel, hr, coeff_p, coeff_q, coeff_r)
+    if ent.dtype != torch.float32 or rel.dtype != torch.float32:
+        raise TypeError("kvsall_step needs fp32 tables")
+    if hr.dtype != torch.int64 or hr.dim() != 2 or hr.shape[1] != 2:
+        raise ValueError("hr must be an int64 tensor of shape [B, 2]")
+    B, (N, d), (R, dr) = hr.shape[0], ent.shape, rel.shape
+    if dr != d:
+        raise ValueError("entity and relation tables must have the same embedding dim")
+
+    def new(*shape):
+        return torch.empty(shape, dtype=torch.float32, device=ent.device)
+    loss, d_ent, d_rel = new(1), new(N, d), new(R, d)
+    d_coeff = tuple(None if c is None else new(*c.shape) for c in (coeff_p, coeff_q, coeff_r))
+    d_norm = {k: new(d) for k in ("h_a", "h_b", "r_a", "r_b")} if norm is not None and norm["kind"] == "LayerNorm" else None
+    keys, n_rows, mult, row_ptr, col = _filter_args(csr)
+    ns, keep = _norm_struct(norm)
+    gs = _lib.NormGrads(*[t.data_ptr() for t in d_norm.values()]) if d_norm else _lib.NormGrads()
+    s = _lib.StepParams(MODEL_IDS[model], int(p), int(q), int(r), int(bool(normalize_relation)), int(bool(bias_varies)),
+                        float(label_smoothing), ent.data_ptr(), rel.data_ptr(), _at(coeff_p), _at(coeff_q), _at(coeff_r),
+                        ctypes.pointer(ns) if ns is not None else None, hr.data_ptr(), B, d, N, R, keys, n_rows, mult,
+                        row_ptr, col, loss.data_ptr(), d_ent.data_ptr(), d_rel.data_ptr(), _at(d_coeff[0]), _at(d_coeff[1]),
+                        _at(d_coeff[2]), gs)
+    nbytes = lib.kge_kvsall_step_workspace_bytes(B, d, N)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=ent.device)
+    _lib.check(lib.kge_kvsall_step(ctypes.byref(s), ws.data_ptr(), nbytes, _stream()))
+    del keep
+    return loss, d_ent, d_rel, d_coeff, d_norm
 
 
 def bce_multihot(Q, bias, E, scale, csr_row, row_ptr, col, label_smoothing=0.0):

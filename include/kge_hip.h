@@ -186,6 +186,15 @@ size_t kge_topk_values_workspace_bytes(int64_t N);
 int kge_topk_values(const float* values, int64_t N, int64_t k, float* out_values, int64_t* out_idx, void* workspace,
                     size_t workspace_bytes, void* stream);
 
+/*
+ * The same for a hop of a multi-hop query: positions written as the pairs [k,2] (position, relation) of the next query.
+ * kge_hop_scores is its other end: out[n] = max over the k substitutions of t(weight[j], S[j, n]), t the product (tnorm 0) or the
+ * minimum (tnorm 1); NaN as torch.max and torch.min have it.  S: rows of N values, ldS apart.
+ */
+int kge_topk_values_pairs(const float* values, int64_t N, int64_t k, int64_t relation, float* out_values, int64_t* out_pairs,
+                          void* workspace, size_t workspace_bytes, void* stream);
+int kge_hop_scores(const float* weight, const float* S, int64_t k, int64_t N, int64_t ldS, int tnorm, float* out, void* stream);
+
 /* Clears n <= 8 fp32 buffers (counts[i] elements each) in one launch: the outputs that the backward adds to. */
 int kge_fill_zero(float* const* bufs, const int64_t* counts, int n, void* stream);
 
@@ -492,6 +501,38 @@ int kge_bce_multihot_backward(const float* Q, const float* bias, const void* E, 
                               int64_t N, const int64_t* csr_row, const int64_t* row_ptr, const int32_t* col,
                               int64_t n_rows, float label_smoothing, float grad_out, float* loss, float* dQ,
                               float* dbias, float* dE, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * A KvsAll training step in one call: training_step and loss.backward() (dicee/models/base_model.py:25-46) for one batch, fp32
+ * tables.  What kge_csr_lookup, kge_build_query (_decal), kge_bce_multihot_backward and kge_build_query_backward(_norm) do in a
+ * row; the outputs are overwritten.  norm: none, LayerNorm, or BatchNorm1d with its running statistics.  d_coeff_p / _q / _r and
+ * the arrays of d_norm may be NULL.  bias_varies: the per-query bias depends on a parameter (else its gradient is not formed).
+ */
+typedef struct kge_step_params {
+  int32_t model, p, q, r, normalize_relation, bias_varies;
+  float label_smoothing;
+  const float* ent;
+  const float* rel;
+  const float* coeff_p;
+  const float* coeff_q;
+  const float* coeff_r;
+  const kge_norm_params* norm;
+  const int64_t* hr; /* [B,2] */
+  int64_t B, d, N, R;
+  const int64_t* keys; /* as in kge_rank_pass_params; NULL: no positives */
+  int64_t n_rows, key_mult;
+  const int64_t* row_ptr;
+  const int32_t* col;
+  float* loss;   /* [1] */
+  float* d_ent;  /* [N,d] */
+  float* d_rel;  /* [R,d] */
+  float* d_coeff_p;
+  float* d_coeff_q;
+  float* d_coeff_r;
+  kge_norm_grads d_norm;
+} kge_step_params;
+size_t kge_kvsall_step_workspace_bytes(int64_t B, int64_t d, int64_t N);
+int kge_kvsall_step(const kge_step_params* params, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Measurement aid; no counterpart in the reference.  Between kge_profile_begin() and

@@ -123,6 +123,14 @@ static void test_layouts() {
   // the static scratch array of kge_rank_filtered_static holds the layout of its largest batch
   CHECK(rank_ws_offsets(KGE_RANK_STATIC_MAX_B).total <= KGE_RANK_STATIC_SCRATCH_BYTES);
   CHECK(TOPK_FIRST_ROWS <= TOPK_CAP);
+  for (int64_t B : {1, 127, 2048})
+    for (int64_t d : {1, 64, 201}) {
+      const StepOffsets o = step_offsets(B, d, 14541);
+      const size_t m = (size_t)B;
+      check_disjoint({{o.Q, m * d * 4}, {o.bias, m * 4}, {o.rows, m * 8}, {o.dQ, m * d * 4}, {o.dbias, m * 4}, {o.bwd, bwd_plan(B, d, 14541).total}},
+                     o.total);
+      for (size_t at : {o.Q, o.rows, o.dQ, o.bwd}) CHECK(at % 256 == 0);
+    }
   for (int64_t n : {1, 8191, 8192, 8193, 20000})
     for (int64_t d : {1, 32, 201}) {
       const RankPassOffsets o = rank_pass_offsets(n, d);
