@@ -45,6 +45,7 @@ struct HalfArgs {
   int64_t tail_first, tail_chunk, tail_stride;
   int tail_splits, tail_len;
   float* tail;
+  int k_splits;  // StoreEpi: the ranges K is summed in
 };
 
 // h and l of one value x whose product with `up` = 2^s lies below 2^15 (up_2k: 2^(s + 11)); the residual and its factor 2^11
@@ -56,11 +57,16 @@ __device__ __forceinline__ void half_parts(float x, float up, float up_2k, _Floa
 
 // ---- before the contractions: the largest magnitudes, then the split rows --------------------------------------------
 // One slot per workgroup: the first HALF_SLOTS workgroups take E, the rest Q (rows are whole 16-byte pieces, values that are
-// not finite do not count); beside that what bce_init_kernel clears.
+// not finite do not count); beside that what bce_init_kernel clears, and in the workgroups
+// behind those a step's preparations.
 constexpr int HALF_MAX_THREADS = 512;
 __global__ void __launch_bounds__(HALF_MAX_THREADS) half_max_kernel(const float* E, int64_t n_e, const float* Q, int64_t n_q,
                                                                    uint32_t* slots, double* sums, int n_sums, float* dbias,
-                                                                   int64_t B) {
+                                                                   int64_t B, StepPrepare prep) {
+  if (blockIdx.x >= 2 * HALF_SLOTS) {
+    step_prepare(prep, blockIdx.x - 2 * HALF_SLOTS, gridDim.x - 2 * HALF_SLOTS);
+    return;
+  }
   const int64_t gid = (int64_t)blockIdx.x * HALF_MAX_THREADS + threadIdx.x;
   if (gid < n_sums) sums[gid] = 0.0;
   if (dbias)
@@ -332,7 +338,7 @@ __global__ void __launch_bounds__(HALF_THREADS, 2) half_kernel(ContractArgs a, H
   constexpr int EL = E_BYTES / 1024 / WAVES, QL = Q_BYTES / 1024 / WAVES;  // loads of a wave per chunk, 1 KB each
   __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * STAGE_BYTES];
 
-  int qg, k_range = 0, k_len = a.k_split_len;
+  int qg, k_range = 0, k_off = 0, k_end = a.d;  // this workgroup's columns of K
   int64_t chunk, wg_flat = blockIdx.x;
   constexpr bool STORE_T = std::is_same<Epi, StoreTEpi<KS_NQT>>::value;
   bool tail = false;
@@ -340,25 +346,28 @@ __global__ void __launch_bounds__(HALF_THREADS, 2) half_kernel(ContractArgs a, H
   if (tail) {
     const int64_t rest = wg_flat - hs.tail_first, tile = rest / hs.tail_splits;
     k_range = (int)(rest % hs.tail_splits);
-    k_len = hs.tail_len;
+    k_off = k_range * hs.tail_len;
+    k_end = a.d - k_off > hs.tail_len ? k_off + hs.tail_len : a.d;
     qg = (int)(tile % a.n_qgroups);
     chunk = a.n_chunks + tile / a.n_qgroups;
   } else {
-    if (a.k_split_len) {
+    if (hs.k_splits > 1) {
       k_range = (int)blockIdx.y;
       if (a.k_split_xcd) {  // flat grid: consecutive ids go round the XCDs, and an XCD keeps to its K ranges
         const int64_t per_range = a.n_chunks * a.n_qgroups, slot = wg_flat >> 3;
         k_range = (int)(wg_flat & 7) + 8 * (int)(slot / per_range);
         wg_flat = slot % per_range;
       }
+      const int64_t chunks = a.d / KS_KC;  // whole chunks, as equal as they go
+      k_off = (int)(chunks * k_range / hs.k_splits) * KS_KC;
+      k_end = (int)(chunks * (k_range + 1) / hs.k_splits) * KS_KC;
     }
     if (!decompose_wg(a, qg, chunk, wg_flat)) return;
   }
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int we = wave >> 1, wq = wave & 1;
-  const int k_off = k_range * k_len;
-  const int d = (k_len && a.d - k_off > k_len) ? k_len : a.d - k_off;  // K range of this workgroup
+  const int d = k_end - k_off;
   const int64_t q_base = (int64_t)qg * KS_WG_QUERIES;
   const int64_t r0 = a.e_begin + chunk * a.chunk_rows;
   const int64_t r1 = (r0 + a.chunk_rows < a.e_end) ? r0 + a.chunk_rows : a.e_end;

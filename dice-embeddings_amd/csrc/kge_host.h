@@ -428,6 +428,7 @@ struct HalfPlan {
   // dE: the chunks of 128 entities from tail_chunk on have their sum over the batch split tail_splits ways (0: none), tail_len each
   int64_t tail_chunk;
   int tail_splits, tail_len;
+  int dq_splits;  // ranges of N that dQ is summed in, as equal as whole chunks allow
   size_t off_max, off_E, off_Q, off_tail;
 };
 // Against the six bf16 products (the other form), a step's three contractions: 2048 x 40,943, d = 256 804 -> 512 us, 1024 x 3000,
@@ -460,6 +461,18 @@ inline void half_tail(int64_t N, int64_t d, HalfPlan& h) {
   h.tail_len = h.tail_splits ? (int)((k_chunks + best - 1) / best * 32) : 0;
   if (!h.tail_splits) h.tail_chunk = chunks;
   else h.tail_splits = (int)((h.rows_q + h.tail_len - 1) / h.tail_len);  // (none of them empty)
+}
+// dQ: two workgroups per CU, at most 64 ranges, none shorter than four chunks; in eights where there are that many, so that an XCD
+// keeps to its ranges (the workgroups of a range read the same rows of E: a step of 1000 x 14,541, d = 200, in 31 ranges 30 - 40 us, in 32
+// 32)
+inline int half_dq_splits(int64_t B, int64_t d, int64_t N) {
+  const int64_t tiles = (B + KS_WG_QUERIES - 1) / KS_WG_QUERIES * ((d + HALF_ROWS - 1) / HALF_ROWS), chunks = (N + 31) / 32;
+  int64_t s = (512 + tiles - 1) / tiles;
+  if (s > 64) s = 64;
+  if (s > chunks / 4) s = chunks / 4;
+  if (s >= 6) s = (s + 3) / 8 * 8 > 0 ? (s + 3) / 8 * 8 : 8;
+  if (s * 2 > chunks) s = chunks / 2;
+  return (int)(s < 1 ? 1 : s);
 }
 inline unsigned half_split_blocks(int64_t rows, int64_t cols) {  // 32 lines at a time, four times over
   const int64_t n = (rows * (cols / 32) + 127) / 128;
@@ -518,7 +531,8 @@ inline BwdPlan bwd_plan(int64_t B, int64_t d, int64_t N) {
   p.off_GT = off;    off += p.kmajor ? 0 : up((size_t)N * p.ldT * sizeof(float));
   p.off_ET = off;    off += p.kmajor ? 0 : up((size_t)d * p.ldG * sizeof(float));
   p.off_QT = off;    off += p.kmajor ? 0 : up((size_t)d * p.ldT * sizeof(float));
-  p.off_part = off;  off += up((size_t)p.k_splits * B * d * sizeof(float));
+  if (h.on) h.dq_splits = half_dq_splits(B, d, N);
+  p.off_part = off;  off += up((size_t)(h.on && h.dq_splits > p.k_splits ? h.dq_splits : p.k_splits) * B * d * sizeof(float));
   if (h.on) {
     half_tail(N, d, h);
     h.off_tail = off;  off += up((size_t)h.tail_splits * (N - h.tail_chunk * HALF_ROWS) * d * sizeof(float));

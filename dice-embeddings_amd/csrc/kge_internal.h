@@ -80,4 +80,40 @@ __device__ __forceinline__ float just_below(float x) {
   return ordered_to_f32(f32_to_ordered(x) - 1u);
 }
 
+// ---- (head, relation) -> filter row: binary search in the sorted key array -----------------------
+__device__ __forceinline__ int64_t filter_row(int64_t first, int64_t second, const int64_t* keys, int64_t n_rows,
+                                              int64_t num_relations) {
+  const int64_t key = first * num_relations + second;
+  int64_t lo = 0, hi = n_rows;
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (keys[mid] < key) lo = mid + 1; else hi = mid;
+  }
+  return (lo < n_rows && keys[lo] == key) ? lo : -1;
+}
+
+// ---- what a training step needs beside its contractions: the filter rows of its pairs, and the outputs that are added to
+// cleared.  Work for some workgroups of a launch that comes early anyway (a launch of its own: 4 us of a toy step's 63).
+struct StepPrepare {
+  const int64_t* hr;
+  int64_t B;  // 0: no filter rows
+  const int64_t* keys;
+  int64_t n_rows, key_mult;
+  int64_t* rows;
+  float* clear[8];
+  int64_t counts[8];  // 0: no such buffer
+};
+inline unsigned step_prepare_wgs(const StepPrepare& s) {
+  int64_t most = s.B;
+  for (int64_t n : s.counts) most = n > most ? n : most;
+  const int64_t wgs = (most + 255) / 256;
+  return (unsigned)(wgs < 256 ? wgs : 256);
+}
+__device__ __forceinline__ void step_prepare(const StepPrepare& s, unsigned wg, unsigned wgs) {
+  const int64_t i0 = (int64_t)wg * blockDim.x + threadIdx.x, stride = (int64_t)wgs * blockDim.x;
+  for (int64_t b = i0; b < s.B; b += stride) s.rows[b] = filter_row(s.hr[2 * b], s.hr[2 * b + 1], s.keys, s.n_rows, s.key_mult);
+  for (int j = 0; j < 8; ++j)
+    for (int64_t i = i0; i < s.counts[j]; i += stride) s.clear[j][i] = 0.f;
+}
+
 }  // namespace kge

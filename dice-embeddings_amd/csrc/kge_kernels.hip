@@ -128,17 +128,6 @@ __global__ void __launch_bounds__(256) triple_score_kernel(ContractArgs a, const
   }
 }
 
-// ---- (head, relation) -> filter row: binary search in the sorted key array -----------------------
-__device__ __forceinline__ int64_t filter_row(int64_t first, int64_t second, const int64_t* keys, int64_t n_rows,
-                                              int64_t num_relations) {
-  const int64_t key = first * num_relations + second;
-  int64_t lo = 0, hi = n_rows;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    if (keys[mid] < key) lo = mid + 1; else hi = mid;
-  }
-  return (lo < n_rows && keys[lo] == key) ? lo : -1;
-}
 __global__ void csr_lookup_kernel(const int64_t* hr, int64_t B, const int64_t* keys, int64_t n_rows,
                                   int64_t num_relations, int64_t* csr_row) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -168,26 +157,6 @@ __global__ void ranks_kernel(const int32_t* n_gt, const int32_t* n_eq, const int
   const int64_t eq = n_eq[b], ties = tie == KGE_TIE_STABLE ? (int64_t)n_eql[b] : tie == KGE_TIE_OPTIMISTIC ? 0
                                      : tie == KGE_TIE_PESSIMISTIC ? eq : eq >> 1;
   ranks[b] = 1 + (int64_t)n_gt[b] + ties;
-}
-
-// ---- what a training step needs before its contractions: the filter rows of its pairs, and its outputs that are added to cleared
-struct StepPrepare {
-  const int64_t* hr;
-  int64_t B;
-  const int64_t* keys;
-  int64_t n_rows, key_mult;
-  int64_t* rows;
-  float* clear[8];
-  int64_t counts[8];
-};
-__global__ void __launch_bounds__(256) step_prepare_kernel(StepPrepare s) {  // grid.y: 0 the rows, then the buffers
-  const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
-  if (blockIdx.y == 0) {
-    for (int64_t b = i0; b < s.B; b += stride) s.rows[b] = filter_row(s.hr[2 * b], s.hr[2 * b + 1], s.keys, s.n_rows, s.key_mult);
-    return;
-  }
-  float* p = s.clear[blockIdx.y - 1];
-  for (int64_t i = i0; i < s.counts[blockIdx.y - 1]; i += stride) p[i] = 0.f;
 }
 
 // ---- group the queries of one sub-batch by filter row and plan the correction work -----------
@@ -1069,7 +1038,12 @@ __global__ void minmax_final_kernel(uint32_t* kmin, uint32_t* kmax, const float*
 // ---- BCE helpers --------------------------------------------------------------------------------
 // accumulators: BCE_SLOTS partial sums of softplus(s), BCE_SLOTS of s, then BCE_POS_SLOTS of the sum over the positives
 using host::BCE_POS_SLOTS;
-__global__ void bce_init_kernel(double* sums, float* dbias, int64_t B) {  // dbias: a [B] vector to clear as well, or null
+// (the workgroups from init_wgs on take a step's preparations)
+__global__ void bce_init_kernel(double* sums, float* dbias, int64_t B, unsigned init_wgs, StepPrepare prep) {  // dbias: a [B] vector to clear as well, or null
+  if (blockIdx.x >= init_wgs) {
+    step_prepare(prep, blockIdx.x - init_wgs, gridDim.x - init_wgs);
+    return;
+  }
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < 2 * BCE_SLOTS + BCE_POS_SLOTS) sums[i] = 0.0;
   if (dbias && i < B) dbias[i] = 0.f;
@@ -1666,8 +1640,9 @@ int launch_half(ContractArgs a, HalfArgs hs, const EArgs& ea, unsigned k_splits,
   constexpr bool store_t = std::is_same<EpiT<KS_NQT>, StoreTEpi<KS_NQT>>::value;
   constexpr int KMAJ = store ? 1 : store_t ? 3 : 0;
   KGE_REQUIRE(a.ldq % 32 == 0 && a.lde % 32 == 0 && a.ldq > 0 && a.lde > 0 && (((uintptr_t)a.E | (uintptr_t)a.Q) % 128 == 0) &&
-                  a.d % 32 == 0 && a.k_split_len % 32 == 0,
+                  a.d % 32 == 0 && (k_splits == 1 || (store && (int64_t)k_splits <= a.d / 32)),
               KGE_ERR_INVALID, "%s: split rows are whole lines", name);
+  hs.k_splits = (int)k_splits;
   // (dE: a tile per workgroup, the tail's shared out; else as full a last round as whole tiles give)
   a.chunk_rows = store_t ? host::HALF_ROWS : host::fullest_chunk(a.e_end - a.e_begin, a.n_qgroups, host::HALF_ROWS, 512);
   a.n_chunks = (a.e_end - a.e_begin + a.chunk_rows - 1) / a.chunk_rows;
@@ -2417,7 +2392,8 @@ extern "C" int kge_bce_multihot(const float* Q, const float* bias, const void* E
   KGE_REQUIRE(((uintptr_t)workspace & 7) == 0, KGE_ERR_WORKSPACE, "kge_bce_multihot: workspace must be 8-byte aligned");
   hipStream_t st = (hipStream_t)stream;
   double* sums = (double*)workspace;
-  hipLaunchKernelGGL(bce_init_kernel, dim3(bce_init_blocks(B, nullptr)), dim3(BCE_INIT_THREADS), 0, st, sums, nullptr, B);
+  hipLaunchKernelGGL(bce_init_kernel, dim3(bce_init_blocks(B, nullptr)), dim3(BCE_INIT_THREADS), 0, st, sums, nullptr, B,
+                     bce_init_blocks(B, nullptr), StepPrepare{});
   KGE_LAUNCH_CHECK("bce_init_kernel");
   ContractArgs a = make_args(Q, E, dtype, scale, B, d, N, 0, N);
   BceArgs ea{bias, sums, label_smoothing != 0.f ? 1 : 0};
@@ -2442,11 +2418,12 @@ extern "C" size_t kge_bce_backward_workspace_bytes(int64_t B, int64_t d, int64_t
   return bwd_plan(B, d, N).total;
 }
 
-extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, const void* E, int dtype, int64_t B,
-                                         int64_t d, int64_t N, const int64_t* csr_row, const int64_t* row_ptr,
-                                         const int32_t* col, int64_t n_rows, float label_smoothing, float grad_out,
-                                         float* loss, float* dQ, float* dbias, float* dE, void* workspace,
-                                         size_t workspace_bytes, void* stream) {
+namespace {
+// prep: what a training step wants done before (the filter rows it names are read by this call's later launches), or empty
+int bce_backward_impl(const float* Q, const float* bias, const void* E, int dtype, int64_t B, int64_t d, int64_t N,
+                      const int64_t* csr_row, const int64_t* row_ptr, const int32_t* col, int64_t n_rows, float label_smoothing,
+                      float grad_out, float* loss, float* dQ, float* dbias, float* dE, void* workspace, size_t workspace_bytes,
+                      void* stream, const StepPrepare& prep) {
   clear_error();
   KGE_REQUIRE(dtype == KGE_F32, KGE_ERR_UNSUPPORTED, "kge_bce_multihot_backward: fp32 tables only (got dtype %d)", dtype);
   int rc = check_contract("kge_bce_multihot_backward", Q, E, dtype, nullptr, B, d, N);
@@ -2476,6 +2453,7 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
   float* part = (float*)(ws + p.off_part);
   const float inv_bn = grad_out / ((float)B * (float)N);
 
+  const unsigned prep_wgs = step_prepare_wgs(prep);
   const host::HalfPlan& hp = p.half;
   HalfArgs hs{};
   const uint32_t* maxima = (const uint32_t*)(ws + hp.off_max);
@@ -2483,8 +2461,8 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
   int exp_g = 0;
   if (hp.on) {
     exp_g = host::half_gradient_exponent(inv_bn, label_smoothing, N);
-    hipLaunchKernelGGL(half_max_kernel, dim3(2 * HALF_SLOTS), dim3(HALF_MAX_THREADS), 0, st, (const float*)E, N * d, Q, B * d,
-                       (uint32_t*)maxima, sums, BCE_INIT_THREADS, dbias, B);
+    hipLaunchKernelGGL(half_max_kernel, dim3(2 * HALF_SLOTS + prep_wgs), dim3(HALF_MAX_THREADS), 0, st, (const float*)E, N * d, Q,
+                       B * d, (uint32_t*)maxima, sums, BCE_INIT_THREADS, dbias, B, prep);
     KGE_LAUNCH_CHECK("half_max_kernel");
     const HalfSplit se{(const float*)E, (unsigned char*)(ws + hp.off_E), N, hp.rows_e, (int)d, (int)(hp.cols / 32)};
     const HalfSplit sq{Q, (unsigned char*)(ws + hp.off_Q), B, hp.rows_q, (int)d, (int)(hp.cols / 32)};
@@ -2492,7 +2470,8 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
     hipLaunchKernelGGL(half_split_kernel, dim3(be + bq), dim3(256), 0, st, se, sq, be, maxima, (int32_t*)exps);
     KGE_LAUNCH_CHECK("half_split_kernel");
   } else {
-    hipLaunchKernelGGL(bce_init_kernel, dim3(bce_init_blocks(B, dbias)), dim3(BCE_INIT_THREADS), 0, st, sums, dbias, B);
+    const unsigned init_wgs = bce_init_blocks(B, dbias);
+    hipLaunchKernelGGL(bce_init_kernel, dim3(init_wgs + prep_wgs), dim3(BCE_INIT_THREADS), 0, st, sums, dbias, B, init_wgs, prep);
     KGE_LAUNCH_CHECK("bce_init_kernel");
   }
   // (1) scores -> g = (sigmoid(s) - dense part of y') * inv_bn, both layouts, and the loss sums
@@ -2526,7 +2505,8 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
     KGE_LAUNCH_CHECK("bce_pos_kernel");
   }
   const BceFinal fin{sums, (double)B, (double)N, label_smoothing, loss};
-  if (loss && p.k_splits == 1 && hp.tail_splits < 2) {  // (else the reduction of partial sums does it)
+  const int dq_splits = hp.on ? hp.dq_splits : p.k_splits;
+  if (loss && dq_splits == 1 && hp.tail_splits < 2) {  // (else the reduction of partial sums does it)
     hipLaunchKernelGGL(bce_final_kernel, dim3(1), dim3(64), 0, st, fin);
     KGE_LAUNCH_CHECK("bce_final_kernel");
   }
@@ -2547,13 +2527,14 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
     b.ldq = (int)p.ldG;
     b.lde = kmajor ? (int)d : (int)p.ldG;
     b.k_split_len = p.k_split_len;
-    StoreArgs sa{p.k_splits > 1 ? part : dQ, nullptr, d, (int64_t)B * d};
+    StoreArgs sa{dq_splits > 1 ? part : dQ, nullptr, d, (int64_t)B * d};
     if (hp.on) {
       b.E = ws + hp.off_E;
       b.d = (int)p.ldG;
       b.lde = (int)hp.cols;
+      b.k_split_len = 0;
       hs = HalfArgs{exps, nullptr, 0, exp_g};
-      rc = launch_half<StoreEpi>(b, hs, sa, (unsigned)p.k_splits, st, "kge_bce_multihot_backward: dQ");
+      rc = launch_half<StoreEpi>(b, hs, sa, (unsigned)dq_splits, st, "kge_bce_multihot_backward: dQ");
     } else {
       rc = launch_ksplit<StoreEpi>(b, sa, (unsigned)p.k_splits, st, "kge_bce_multihot_backward: dQ", kmajor ? 1 : 0, p.dq_rows);
     }
@@ -2596,13 +2577,23 @@ extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, cons
     if (rc) return rc;
   }
   // (5) partial sums
-  const SplitSums dq_sums{part, dQ, B * d, p.k_splits};
+  const SplitSums dq_sums{part, dQ, B * d, dq_splits};
   const unsigned b0 = split_sums_blocks(dq_sums), b1 = split_sums_blocks(tail_sums);
   if (b0 + b1) {
     hipLaunchKernelGGL(reduce_splits_kernel, dim3(b0 + b1), dim3(256), 0, st, dq_sums, tail_sums, b0, fin);
     KGE_LAUNCH_CHECK("reduce_splits_kernel");
   }
   return KGE_OK;
+}
+}  // namespace
+
+extern "C" int kge_bce_multihot_backward(const float* Q, const float* bias, const void* E, int dtype, int64_t B,
+                                         int64_t d, int64_t N, const int64_t* csr_row, const int64_t* row_ptr,
+                                         const int32_t* col, int64_t n_rows, float label_smoothing, float grad_out,
+                                         float* loss, float* dQ, float* dbias, float* dE, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
+  return bce_backward_impl(Q, bias, E, dtype, B, d, N, csr_row, row_ptr, col, n_rows, label_smoothing, grad_out, loss, dQ, dbias, dE,
+                           workspace, workspace_bytes, stream, StepPrepare{});
 }
 
 extern "C" size_t kge_kvsall_step_workspace_bytes(int64_t B, int64_t d, int64_t N) {
@@ -2630,12 +2621,10 @@ extern "C" int kge_kvsall_step(const kge_step_params* p, void* workspace, size_t
   const bool filtered = p->keys && p->n_rows > 0;
   StepPrepare sp{p->hr, filtered ? B : 0, p->keys, p->n_rows, p->key_mult, rows, {}, {}};
   int n = 0;
-  int64_t most = filtered ? B : 0;
   auto clear = [&](float* buf, int64_t count) {
     if (!buf || count == 0) return;
     sp.clear[n] = buf;
     sp.counts[n++] = count;
-    most = count > most ? count : most;
   };
   clear(p->d_rel, p->R * d);
   clear(p->d_coeff_p, p->coeff_p ? p->p : 0);
@@ -2651,12 +2640,8 @@ extern "C" int kge_kvsall_step(const kge_step_params* p, void* workspace, size_t
                : kge_build_query(p->model, p->p, p->q, p->ent, KGE_F32, nullptr, p->rel, KGE_F32, p->coeff_p, p->coeff_q,
                                  p->normalize_relation, p->norm, p->hr, B, d, N, p->R, Q, bias, stream);
   if (rc) return rc;
-  const int64_t blocks = (most + 255) / 256;
-  hipLaunchKernelGGL(step_prepare_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024), (unsigned)(n + 1)), dim3(256), 0,
-                     (hipStream_t)stream, sp);
-  KGE_LAUNCH_CHECK("step_prepare_kernel");
-  rc = kge_bce_multihot_backward(Q, bias, p->ent, KGE_F32, B, d, N, filtered ? rows : nullptr, p->row_ptr, p->col, p->n_rows,
-                                 p->label_smoothing, 1.0f, p->loss, dQ, dbias, p->d_ent, ws + o.bwd, workspace_bytes - o.bwd, stream);
+  rc = bce_backward_impl(Q, bias, p->ent, KGE_F32, B, d, N, filtered ? rows : nullptr, p->row_ptr, p->col, p->n_rows,
+                         p->label_smoothing, 1.0f, p->loss, dQ, dbias, p->d_ent, ws + o.bwd, workspace_bytes - o.bwd, stream, sp);
   if (rc) return rc;
   return kge_build_query_backward_norm(p->model, p->p, p->q, p->r, p->ent, p->rel, p->coeff_p, p->coeff_q, p->coeff_r,
                                        p->normalize_relation, p->norm, p->norm ? &p->d_norm : nullptr, nullptr, p->hr, B, d, N, p->R,

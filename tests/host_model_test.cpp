@@ -173,9 +173,11 @@ static void test_layouts() {
         const int64_t end_G = std::max(rows_end(B, pg), kmaj_end(h.rows_q, pg, p.ldG));
         const int64_t tail_row = h.tail_chunk * HALF_ROWS;
         check_disjoint({{0, bce_ws_bytes()}, {h.off_max, (2 * HALF_SLOTS + 2) * 4}, {h.off_E, (size_t)end_E}, {h.off_Q, (size_t)end_Q},
-                        {p.off_G, (size_t)end_G}, {p.off_part, (size_t)p.k_splits * B * d * 4},
+                        {p.off_G, (size_t)end_G}, {p.off_part, (size_t)h.dq_splits * B * d * 4},
                         {h.off_tail, h.tail_splits ? (size_t)h.tail_splits * (N - tail_row) * d * 4 : 0}},
                        p.total);
+        CHECK(h.dq_splits >= 1 && h.dq_splits <= 64 && (h.dq_splits < 8 || h.dq_splits % 8 == 0 || h.dq_splits == p.ldG / 32 / 2));
+        CHECK(h.dq_splits <= p.ldG / 32);                                                  // no range of dQ is empty
         const int64_t groups = (d + 127) / 128, chunks = up(p.ldG, HALF_ROWS) / HALF_ROWS;
         CHECK(h.tail_chunk >= 0 && h.tail_chunk <= chunks && (h.tail_splits == 0 || (h.tail_splits >= 2 && h.tail_splits <= 8)));
         if (!h.tail_splits) CHECK(h.tail_chunk == chunks);
