@@ -549,8 +549,7 @@ __global__ void __launch_bounds__(FEW_THREADS) few_finish_kernel(FewFinishArgs a
   const bool grouped = T > FEW_TILES_DIRECT;
   int n = 0;
   bool picked = false;  // the entities: else they are few enough to be ranked all
-  // Every tile is among the best k: nothing to pick (a step of the selection is a barrier, sixteen of them 8 us: k = 100,
-  // N = 1000, d = 32, 64 queries 72 us a call, 62 without, 66 by the rounds).
+  // Every tile is among the best k: nothing to pick (k = 100, N = 1000, d = 32, 64 queries: 10 us of the call).
   const bool all = T <= k;
   if (all) {
     n = T;
@@ -738,7 +737,7 @@ int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
   a.n_tiles = (a.N + 31) / 32;
   const int qt = host::few_query_tiles(dtype, a.B, a.d, MODE == FEW_STORE ? 2 : 4);
   a.n_qg = (a.B + 32 * qt - 1) / (32 * qt);
-  // workgroups, as many per CU as registers and LDS allow, walk units of 4 * tpw tiles, each the same number of them; runs of
+  // workgroups, as many per CU as registers and LDS allow, walk units of 4 * tpw tiles, each about the same number of them; runs of
   // eight tiles where there are more tiles than the selection reads one by one
   a.tpw = a.n_tiles > FEW_TILES_DIRECT ? FEW_RUN : 1;
   const size_t lds = (size_t)qt * a.nks * parts * 1024 + 4 * few_stage_bytes(dtype);
@@ -746,12 +745,18 @@ int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
   const size_t room = 163840 / own;
   const int64_t slots = 256 * std::max<int64_t>(1, std::min<int64_t>(room, qt > 1 ? 2 : dtype == KGE_F32 ? 3 : 4));
   const int64_t units = (a.n_tiles + 4 * a.tpw - 1) / (4 * a.tpw);
+  // In a long scan every slot has a workgroup, also where fewer would take as many units each: CUs that hold three beside others
+  // with two end last (32 queries, k = 10, N = 2.5M, the call: bf16 d = 128 616 workgroups 160 us, 768 150; int8 d = 128 816
+  // workgroups 116, 1024 98).  In a short one the start of the others costs more (fp32 d = 256, N = 200k: 392 workgroups
+  // 53.5 us, 512 55.3).
+  const bool fill = MODE == FEW_MAX && a.tpw > 1;
   // one to four rounds of them: the fewest units in turn on a slot, a workgroup's start counted as one (several query groups
   // rarely divide one round: int8 d = 1024, N = 41k, 96 queries, one round 89 us, the best of four 65)
   int64_t best = -1;
   for (int64_t r = 1; r <= (a.n_qg > 1 ? 4 : 1); ++r) {
     const int64_t share = slots * r / a.n_qg / 8 * 8, each = (units + share - 1) / share;
-    const int64_t n_wg = ((units + each - 1) / each + 7) / 8 * 8, rounds = (n_wg * a.n_qg + slots - 1) / slots;
+    const int64_t n_wg = ((fill ? std::min(share, units) : (units + each - 1) / each) + 7) / 8 * 8;
+    const int64_t rounds = (n_wg * a.n_qg + slots - 1) / slots;
     if (best < 0 || rounds * (each + 1) < best) {
       best = rounds * (each + 1);
       a.n_wg = (int)n_wg;

@@ -28,7 +28,9 @@ CASES = [("fp32", 1, 4, 1, 1), ("fp32", 33, 20, 2, 33), ("fp32", 4096, 200, 33, 
          ("fp32", 3001, 340, 5, 7), ("bf16", 31, 8, 3, 31), ("bf16", 4097, 128, 32, 128), ("bf16", 2000, 1024, 65, 10),
          ("bf16", 524288, 32, 2, 50), ("bf16", 524289, 32, 40, 128), ("int8", 1000, 16, 1, 10), ("int8", 7777, 240, 128, 100),
          ("int8", 70001, 128, 64, 3), ("fp32", 140000, 64, 65, 40), ("int8", 150000, 32, 128, 5), ("int8", 600011, 16, 1, 5),
-         ("fp32", 4096, 32, 3, 128)]
+         ("fp32", 4096, 32, 3, 128),
+         # runs of eight tiles: a batch that fills no line of the maxima, four query tiles, the table's last run of one tile
+         ("bf16", 16392 * 32 + 7, 32, 33, 10), ("int8", 16385 * 32, 16, 128, 128), ("fp32", 16399 * 32 + 1, 32, 97, 20)]
 
 
 @pytest.mark.parametrize("storage,N,d,B,k", CASES)
