@@ -241,7 +241,7 @@ class Evaluator:
         self.report = {}
         self.during_training = False
         self.tie = tie
-        self.streams = streams   # batches of an evaluation alternate over this many streams (1: the caller's only)
+        self.streams = streams   # batches ranked one by one alternate over this many streams (1: the caller's only)
         self.last_ranks = None
 
     # ------------------------------------------------------------------ filter preparation

@@ -34,8 +34,8 @@ def evaluate_lp(model, triple_idx, num_entities=None, er_vocab=None, re_vocab=No
     ``er_vocab`` / ``re_vocab``: the reference's dicts ``(h, r) -> [t]`` / ``(r, t) -> [h]``, or ``FilterCSR``
     objects (``FilterCSR.from_triples_gpu(..., kind="er" | "re")``).  ``chunk_size`` is accepted for
     signature compatibility; nothing is chunked.  ``return_ranks``: also return (head_ranks, tail_ranks).
-    ``streams``: the rank calls (two per batch, independent of one another) alternate over this many streams,
-    joined before the ranks are read; 1 keeps all of them on the caller's stream."""
+    ``streams``: where batches are ranked one by one (models that build their queries otherwise) they alternate over this many
+    streams, joined before the ranks are read; a direction ranked in one call stays on the caller's stream."""
     assert model is not None, "Model must be provided"
     assert triple_idx is not None, "triple_idx must be provided"
     assert er_vocab is not None, "er_vocab must be provided"
