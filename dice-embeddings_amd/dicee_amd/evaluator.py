@@ -133,14 +133,17 @@ class _BatchStreams:
 
 def eval_mode(model):
     """``model.eval()``, which walks and writes to every module, where some module is not in that mode yet."""
-    if any(m.training for m in model.modules()):
+    from .models import BaseKGE, as_defined
+    if not as_defined(model, BaseKGE, "eval", "train", "modules") or any(m.training for m in model.modules()):
         model.eval()
 
 
-def _plain_queries(model, x_all, target_all):
-    """Does ``ops.rank_pass`` form these queries?  (A model with a query builder of its own, dropout or batch statistics: no.)"""
-    from .models import BaseKGE
-    if type(model).query is not BaseKGE.query or type(model).table is not BaseKGE.table:
+def _plain_queries(model, x_all, target_all, csr=None):
+    """Does ``ops.rank_pass`` form these queries?  (A model with a query builder of its own, dropout or batch statistics, or
+    filter rows that are looked up otherwise: no.)"""
+    from .csr import FilterCSR
+    from .models import BaseKGE, as_defined
+    if not as_defined(model, BaseKGE, "query", "table") or not (csr is None or as_defined(csr, FilterCSR, "rows_for")):
         return False
     if model.training and (model.input_dropout_rate > 0.0
                            or isinstance(model.normalize_head_entity_embeddings, torch.nn.BatchNorm1d)):
@@ -169,7 +172,7 @@ def rank_in_batches(model, x_all, target_all, csr, batch_size, tie="stable", str
     from . import ops
     n = int(x_all.shape[0])
     dev = x_all.device
-    if call_queries and n and _plain_queries(model, x_all, target_all):
+    if call_queries and n and _plain_queries(model, x_all, target_all, csr):
         with torch.no_grad():
             E, scale = model.table()
             rel, norm = model._rel(), model._norm_params()

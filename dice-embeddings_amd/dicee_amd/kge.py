@@ -11,7 +11,7 @@ from typing import List, Union
 
 import torch
 
-from .models import BaseKGE
+from .models import BaseKGE, as_defined
 
 
 def _call_size(batch_size, fused_topk):
@@ -70,7 +70,7 @@ class KGE:
         """``model.topk`` of pairs that are on the host, its scores and ids back on the host by one copy."""
         dev = self.model.entity_embeddings.weight.device
         P = pairs.size(0)
-        if dev.type != "cuda" or not isinstance(topk, int) or topk < 1 or type(self.model).topk is not BaseKGE.topk:
+        if dev.type != "cuda" or not isinstance(topk, int) or topk < 1 or not as_defined(self.model, BaseKGE, "topk", "query"):
             s, idx = self.model.topk(pairs.to(dev), topk, **({"heads": True} if heads else {}))
             return s.cpu(), idx.cpu()
         n = P * topk
@@ -304,7 +304,7 @@ class KGE:
         """[N]: the best t-norm over the substitutions, ``max(t_norm(s[:, None], logits), dim=0)``."""
         from . import ops
         if (logits.is_cuda and logits.dtype == s.dtype == torch.float32 and logits.shape[0] and logits.is_contiguous()
-                and type(self).t_norm is KGE.t_norm and ("min" in tnorm or "prod" in tnorm)):
+                and as_defined(self, KGE, "t_norm") and ("min" in tnorm or "prod" in tnorm)):
             return ops.hop_scores(s, logits, minimum="min" in tnorm)
         return torch.max(self.t_norm(s[:, None], logits, tnorm), dim=0)[0]
 

@@ -15,6 +15,14 @@ stream: no two implementations share that).
 import torch
 
 from . import ops
+from .csr import FilterCSR
+
+
+def as_defined(obj, cls, *methods):
+    """Is ``obj`` a ``cls`` whose ``methods`` are those of ``cls``, overridden neither by its class nor on the object?  What one
+    native call does in place of several methods holds for such objects only; others are asked method by method."""
+    return (isinstance(obj, cls) and not any(m in vars(obj) for m in methods)
+            and all(getattr(type(obj), m) is getattr(cls, m) for m in methods))
 
 
 class IdentityClass(torch.nn.Module):
@@ -339,9 +347,8 @@ class BaseKGE(torch.nn.Module):
         x = x.to(device=E.device, dtype=torch.int64).contiguous()
         dropout = self._draw_dropout(x.shape[0], E.device)
         norm = self._norm_params(x, dropout)
-        cls = type(self)
-        if (dropout is None and not (norm and norm.get("batch")) and cls.query is BaseKGE.query and cls.table is BaseKGE.table
-                and cls.kvsall_bce_backward is BaseKGE.kvsall_bce_backward):
+        if (dropout is None and not (norm and norm.get("batch")) and as_defined(self, BaseKGE, "query", "table", "kvsall_bce_backward")
+                and as_defined(csr, FilterCSR, "rows_for")):
             loss, dE, dR, dcoeff, dnorm = ops.kvsall_step(
                 self.name if self.name != "CKeci" else "Keci", E, self._rel(), x, csr, label_smoothing, norm=norm,
                 bias_varies=self._bias_varies(), **self._query_kwargs())

@@ -252,6 +252,50 @@ def test_evaluating_a_model_on_the_cpu_raises_what_the_ops_raise():
         evaluate_lp(m, tr, 50, er, re_, info=None, batch_size=16)
 
 
+def test_one_call_forms_stand_for_unchanged_methods_only():
+    """A model that overrides a method (on its class or on itself), one that only looks like a model, and a filter with a
+    lookup of its own are asked method by method."""
+    from dicee_amd import KGE, FilterCSR, evaluator, models
+    args = {"model": "DistMult", "embedding_dim": 32, "num_entities": 50, "num_relations": 5}
+    calls = []
+
+    class Own(models.DistMult):
+        def query(self, x, **kw):
+            return super().query(x, **kw)
+
+    class Wrapped:
+        def __init__(self, model):
+            self.inner = model
+
+        def eval(self):
+            calls.append("eval")
+            return self
+
+        def __getattr__(self, name):
+            return getattr(self.__dict__["inner"], name)
+
+    class Lookup(FilterCSR):
+        def rows_for(self, hr):
+            return super().rows_for(hr)
+
+    names = ("query", "table")
+    plain = models.DistMult(args)
+    assert models.as_defined(plain, models.BaseKGE, *names)
+    patched = models.DistMult(args)
+    patched.query = lambda x, **kw: None
+    for m in (Own(args), Wrapped(plain), patched, object()):
+        assert not models.as_defined(m, models.BaseKGE, *names)
+        assert not evaluator._plain_queries(m, torch.zeros(1, 2, dtype=torch.int64), torch.zeros(1, dtype=torch.int64))
+    assert not models.as_defined(Lookup.__new__(Lookup), FilterCSR, "rows_for")
+    assert models.as_defined(FilterCSR.__new__(FilterCSR), FilterCSR, "rows_for")
+    assert not models.as_defined(object(), KGE, "t_norm")
+    assert models.as_defined(KGE.__new__(KGE), KGE, "t_norm")          # (a static method)
+    evaluator.eval_mode(Wrapped(plain))
+    assert calls == ["eval"]
+    evaluator.eval_mode(plain.train())
+    assert not plain.training
+
+
 def test_synthetic_configs_small_scale():
     from dicee_amd import synthetic
     c1 = synthetic.make_config("c1")
