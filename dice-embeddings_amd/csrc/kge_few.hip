@@ -15,6 +15,7 @@
 #include "kge_contract.hip.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace kge {
 namespace {
@@ -36,6 +37,7 @@ struct FewArgs {
   int tpw;   // consecutive tiles a wave takes at a time
   int n_qg;  // query groups: 32 * QT queries each, as many as LDS holds fragments of
   int n_wg;  // workgroups of a group, a multiple of 8
+  GradArgs grad;  // FEW_GRAD only
 };
 
 // One wave at a time: chunks of a 32-row tile, 128 (bf16: 256) bytes of every row, loaded as whole lines into registers
@@ -45,7 +47,8 @@ struct FewArgs {
 // requests share them, and a CU's waves push each other's lines out of the L1 in between: bf16 d = 128, N = 2.5M 152 us against 143, int8 N = 10M
 // whole calls of 32 queries 507 against 382.)
 constexpr int few_stage_bytes(int edt) { return edt == KGE_BF16 ? 8192 : 4096; }
-enum FewMode { FEW_MAX, FEW_MAX_RAW, FEW_STORE };
+// FEW_GRAD: GradEpi's gradients, loss sums and bias gradient in the place of the scores (fp32 tables)
+enum FewMode { FEW_MAX, FEW_MAX_RAW, FEW_STORE, FEW_GRAD };
 constexpr int FEW_RUN = 8;  // tiles of a run whose maxima go out together
 template <int EDT, int QT, int MODE>
 __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_scan_kernel(FewArgs a) {
@@ -54,9 +57,10 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
   constexpr int PIECES = EDT == KGE_BF16 ? 16 : 8;       // 16-byte pieces of a row's chunk
   constexpr int RPL = 64 / PIECES, NLD = 32 / RPL;       // rows per wave-wide load, loads per chunk
   constexpr int PER_PIECE = EDT == KGE_F32 ? 4 : EDT == KGE_BF16 ? 8 : 16;  // elements
-  constexpr bool STORE = MODE == FEW_STORE;
+  constexpr bool GRAD = MODE == FEW_GRAD;
+  constexpr bool STORE = MODE == FEW_STORE || GRAD;  // accumulator columns are entities
   extern __shared__ __attribute__((aligned(16))) unsigned char fq_lds[];
-  __shared__ float s_bias[STORE ? 32 * QT : 1];
+  __shared__ __attribute__((aligned(16))) float s_bias[STORE ? 32 * QT : 1];
   __shared__ __attribute__((aligned(16))) float s_max[MODE == FEW_MAX ? 4 * 32 * QT * FEW_RUN : 4];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -148,6 +152,11 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
   auto piece = [&](int p) -> const unsigned char* { return stage + (c * PIECES + (p ^ (c & (PIECES - 1)))) * 16; };
   f32x16 acc[QT];
   float run_max[QT];  // FEW_MAX with tpw = FEW_RUN
+  std::conditional_t<GRAD, GradEpi<QT>, int> epi;
+  if constexpr (GRAD) {
+    epi.init(a.grad, q0, c, hf, a.B);
+    epi.lb = s_bias;
+  }
   auto multiply = [&](int64_t t_tile, int t_ch) {
     if (t_ch == 0) {
 #pragma unroll
@@ -203,7 +212,10 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
       }
     }
     if (t_ch != nch - 1) return;
-    if constexpr (STORE) {
+    if constexpr (GRAD) {
+#pragma unroll
+      for (int t = 0; t < QT; ++t) epi.template tile<false>(t, acc[t], nullptr, 1.f, t_tile * 32, a.N);
+    } else if constexpr (STORE) {
       const int64_t e = t_tile * 32 + c;
       if (e < a.N) {
 #pragma unroll
@@ -280,6 +292,7 @@ __global__ void __launch_bounds__(256, QT > 1 ? 2 : EDT == KGE_F32 ? 3 : 4) few_
     wave_sync();
     if (!more) break;
   }
+  if constexpr (GRAD) epi.finish();
 }
 
 // ---- the best k from the tile maxima ----------------------------------------------------------------------
@@ -735,13 +748,13 @@ int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
   const int parts = dtype == KGE_F32 ? 3 : 1;
   a.nks = (a.d + 15) / 16;
   a.n_tiles = (a.N + 31) / 32;
-  const int qt = host::few_query_tiles(dtype, a.B, a.d, MODE == FEW_STORE ? 2 : 4);
+  const int qt = host::few_query_tiles(dtype, a.B, a.d, MODE >= FEW_STORE ? 2 : 4);
   a.n_qg = (a.B + 32 * qt - 1) / (32 * qt);
   // workgroups, as many per CU as registers and LDS allow, walk units of 4 * tpw tiles, each about the same number of them; runs of
   // eight tiles where there are more tiles than the selection reads one by one
   a.tpw = a.n_tiles > FEW_TILES_DIRECT ? FEW_RUN : 1;
   const size_t lds = (size_t)qt * a.nks * parts * 1024 + 4 * few_stage_bytes(dtype);
-  const size_t own = (lds + (MODE == FEW_MAX ? 4096 * qt : MODE == FEW_STORE ? 128 * qt : 0) + 1279) / 1280 * 1280;  // (granules of 1280)
+  const size_t own = (lds + (MODE == FEW_MAX ? 4096 * qt : MODE >= FEW_STORE ? 128 * qt : 0) + 1279) / 1280 * 1280;  // (granules of 1280)
   const size_t room = 163840 / own;
   const int64_t slots = 256 * std::max<int64_t>(1, std::min<int64_t>(room, qt > 1 ? 2 : dtype == KGE_F32 ? 3 : 4));
   const int64_t units = (a.n_tiles + 4 * a.tpw - 1) / (4 * a.tpw);
@@ -767,11 +780,13 @@ int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
     constexpr int EDT = decltype(edt)::value;
     if (qt == 1) hipLaunchKernelGGL((few_scan_kernel<EDT, 1, MODE>), grid, block, lds, st, a);
     else if (qt == 2) hipLaunchKernelGGL((few_scan_kernel<EDT, 2, MODE>), grid, block, lds, st, a);
-    else if constexpr (MODE != FEW_STORE) hipLaunchKernelGGL((few_scan_kernel<EDT, 4, MODE>), grid, block, lds, st, a);
+    else if constexpr (MODE < FEW_STORE) hipLaunchKernelGGL((few_scan_kernel<EDT, 4, MODE>), grid, block, lds, st, a);
   };
   if (dtype == KGE_F32) go(std::integral_constant<int, KGE_F32>{});
-  else if (dtype == KGE_BF16) go(std::integral_constant<int, KGE_BF16>{});
-  else go(std::integral_constant<int, KGE_I8>{});
+  else if constexpr (MODE != FEW_GRAD) {
+    if (dtype == KGE_BF16) go(std::integral_constant<int, KGE_BF16>{});
+    else go(std::integral_constant<int, KGE_I8>{});
+  }
   KGE_LAUNCH_CHECK("few_scan_kernel");
   return KGE_OK;
 }
@@ -779,8 +794,13 @@ int launch_few_scan(int dtype, FewArgs a, hipStream_t st) {
 
 int few_scores_launch(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
                       int64_t N, float* out, int64_t ldo, hipStream_t st) {
-  FewArgs a{Q, E, scale, bias, out, nullptr, nullptr, ldo, 0, N, 0, (int)B, (int)d, 0, 0, 0, 0};
+  FewArgs a{Q, E, scale, bias, out, nullptr, nullptr, ldo, 0, N, 0, (int)B, (int)d, 0, 0, 0, 0, {}};
   return launch_few_scan<FEW_STORE>(dtype, a, st);
+}
+
+int few_grad_launch(const float* Q, const float* E, int64_t B, int64_t d, int64_t N, const GradArgs& grad, hipStream_t st) {
+  FewArgs a{Q, E, nullptr, grad.bias, nullptr, nullptr, nullptr, 0, 0, N, 0, (int)B, (int)d, 0, 0, 0, 0, grad};
+  return launch_few_scan<FEW_GRAD>(KGE_F32, a, st);
 }
 
 int few_topk_launch(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
@@ -790,7 +810,7 @@ int few_topk_launch(const float* Q, const float* bias, const void* E, int dtype,
   float* maxima = (float*)workspace;
   float* runs = w.runs ? maxima + w.runs : nullptr;
   float* raw = w.raw ? maxima + w.raw : nullptr;
-  FewArgs a{Q, E, scale, nullptr, maxima, runs, raw, w.ldm, w.ldr, N, 0, (int)B, (int)d, 0, 0, 0, 0};
+  FewArgs a{Q, E, scale, nullptr, maxima, runs, raw, w.ldm, w.ldr, N, 0, (int)B, (int)d, 0, 0, 0, 0, {}};
   const int rc = raw ? launch_few_scan<FEW_MAX_RAW>(dtype, a, st) : launch_few_scan<FEW_MAX>(dtype, a, st);
   if (rc) return rc;
   FewFinishArgs f{Q, E, scale, bias, maxima, runs, raw, w.ldm, w.ldr, N, (N + 31) / 32, (int)d, (int)k, apply_sigmoid,

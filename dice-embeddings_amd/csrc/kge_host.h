@@ -378,6 +378,15 @@ inline bool few_scores_applies(int dtype, int64_t B, int64_t d, int64_t N) {
   if (dtype != KGE_F32 && d > 512 && B > 32 && N * d > 20000000) return false;
   return B >= 1 && B <= FEW_SCORES_MAX_B && few_rows_ok(dtype, d);
 }
+// The score gradients of a small batch (fp32), whole backward against the K-split kernel's in us, replayed from a graph: 135 entities d = 256
+// 32 queries 37.6 -> 27.6, d = 32 0.78 - 0.93 of the time, 14,541 x 128 0.88 - 0.97, 200,000 x 256 64 queries 0.75; faster at each of 96
+// shapes of 16 - 64 queries (a workgroup there walks the K chunks of 128 entities with a barrier between, here a wave those of 32).
+// With the gradient of the bias every wave adds its 32 sums per tile to the same B addresses: 1000 entities still 0.75 - 0.99, 5000 x 32 up
+// to 1.31, 40,943 x 32 1.70.
+constexpr int64_t FEW_GRAD_BIAS_MAX_N = 1024;
+inline bool few_grad_pays(int64_t B, int64_t d, int64_t N, bool with_dbias) {
+  return few_scores_applies(KGE_F32, B, d, N) && (!with_dbias || N <= FEW_GRAD_BIAS_MAX_N);
+}
 inline size_t few_topk_ws_bytes(int64_t B, int64_t N, int64_t k) {
   return (B <= FEW_MAX_B && k <= FEW_MAX_K && N <= FEW_MAX_N) ? (size_t)few_topk_ws(B, N).total * 4 : 0;
 }

@@ -47,6 +47,8 @@ int few_topk_launch(const float* Q, const float* bias, const void* E, int dtype,
                     hipStream_t st);
 int few_scores_launch(const float* Q, const float* bias, const void* E, int dtype, const float* scale, int64_t B, int64_t d,
                       int64_t N, float* out, int64_t ldo, hipStream_t st);
+struct GradArgs;
+int few_grad_launch(const float* Q, const float* E, int64_t B, int64_t d, int64_t N, const GradArgs& grad, hipStream_t st);
 
 // ---- MFMA 32x32 accumulator layout --------------------------------------------------------
 // acc[i] of lane l holds output (row_of(i, l / 32), l % 32).

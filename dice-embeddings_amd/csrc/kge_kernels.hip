@@ -2495,7 +2495,14 @@ int bce_backward_impl(const float* Q, const float* bias, const void* E, int dtyp
     }
   } else {
     const GradArgs ga{bias, sums, G, GT, dbias, p.ldG, p.ldT, inv_bn, uniform, want_s};
-    rc = launch_ksplit<GradEpi>(a, ga, 1, st, "kge_bce_multihot_backward: scores");
+    if (!GT && host::few_grad_pays(B, d, N, dbias != nullptr)) {
+      LaunchTimer timer;
+      if ((rc = timer.begin(st))) return rc;
+      if ((rc = few_grad_launch(Q, (const float*)E, B, d, N, ga, st))) return rc;
+      rc = timer.end("few_scan_kernel");
+    } else {
+      rc = launch_ksplit<GradEpi>(a, ga, 1, st, "kge_bce_multihot_backward: scores");
+    }
   }
   if (rc) return rc;
   if (csr_row && n_rows > 0) {

@@ -383,6 +383,8 @@ static void test_few_rules() {
   CHECK(!few_topk_pays(KGE_F32, 128, 256, 2000000) && !few_topk_pays(KGE_I8, 65, 1024, 500000));
   CHECK(few_scores_applies(KGE_BF16, 64, 1024, 14541) && !few_scores_applies(KGE_BF16, 33, 1024, 41000));
   CHECK(few_scores_applies(KGE_BF16, 32, 1024, 41000) && few_scores_applies(KGE_F32, 64, 336, 41000));
+  CHECK(few_grad_pays(64, 336, 41000, false) && !few_grad_pays(65, 64, 135, false) && !few_grad_pays(32, 30, 135, false));
+  CHECK(few_grad_pays(1, 4, FEW_GRAD_BIAS_MAX_N, true) && !few_grad_pays(1, 4, FEW_GRAD_BIAS_MAX_N + 1, true));
 }
 static void test_ks_plan() {
   const KsCost store{2.2, 1.2, 1.7, 0.2, {0, 0.74, 1.2, 1.56}}, rank{0.4, 1.0, 0.0, 0.65, {0, 0.82, 1.12, 1.6}};

@@ -194,3 +194,17 @@ def test_nan_rows_and_queries_where_scores_are_formed_again(storage, N, d, B):
             assert (idx[b] == -1).all() and vals[b].isnan().all()
         else:
             assert torch.equal(idx[b], want_i[b, :k]) and torch.equal(vals[b], want_v[b, :k])
+
+
+# one query, one short of / past a tile of 32, two tiles, their limit and the first batch past it; entities around a tile and past a
+# workgroup's four, the last table of the form with a bias gradient and the next; widths of one partial step, a partial line, whole lines, the widest that LDS holds and the first past it
+@pytest.mark.parametrize("B,N,d", [(1, 1, 4), (1, 33, 64), (31, 135, 256), (32, 135, 256), (33, 129, 36), (63, 1000, 100), (64, 14541, 200),
+                                   (64, 31, 336), (40, 257, 340), (65, 135, 256), (32, 40943, 64), (32, 1024, 64), (32, 1025, 64)])
+@pytest.mark.parametrize("eps,want_dbias", [(0.0, True), (0.1, False)])
+def test_gradients_of_few_queries(B, N, d, eps, want_dbias):
+    from test_gpu_split_rows import _step
+    got, want, bound, call = _step(B, N, d, eps, want_dbias, sums=6)
+    for g, w, b in zip(got, want, bound):
+        if g is not None:
+            assert ((g.double().reshape(w.shape) - w).abs() <= b).all()
+    assert all(torch.equal(a, b) for a, b in zip(call()[1::2], got[1::2]))      # dQ and dE: the same sums in the same order

@@ -8,13 +8,14 @@ pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
 
 
-def _step(B, N, d, eps, want_dbias, scale=0.3, spoil=None):
+def _step(B, N, d, eps, want_dbias, scale=0.3, spoil=None, sums=1):
     """(what the step returns, its float64 counterparts, their bounds).
 
     Bounds, per element: a product of two values of 22 - 23 bits is off by less than 8 u of itself, a sum of n of them by a
     rounding of the partial sum per 16 products more: (n / 16 + 8) u of the sum of their magnitudes.  So a score s is off by
     ds = (d / 16 + 8) u |q||e|, its sigmoid by ds / 4 and ten roundings of exponential, quotient, scale and subtraction (of
-    magnitude 1 where the label is 1), kept to 2 u."""
+    magnitude 1 where the label is 1), kept to 2 u.  ``sums``: the roundings of a partial sum per 16 products (six bf16 products
+    are added one by one: 6)."""
     from dicee_amd import ops
     rng = np.random.default_rng(B + N + d)
     Q, E = (torch.from_numpy((rng.standard_normal(s) * scale).astype(np.float32)).cuda() for s in ((B, d), (N, d)))
@@ -38,8 +39,8 @@ def _step(B, N, d, eps, want_dbias, scale=0.3, spoil=None):
     loss = torch.nn.functional.binary_cross_entropy_with_logits(S, y)
     c = 1.5 / (B * N)
     G = (torch.sigmoid(S) - y) * c
-    dG = c * (0.25 * (d / 16 + 8) * U * (q.abs() @ e.abs().T + bias.double().abs()[:, None]) + 12 * U * (torch.sigmoid(S) + y))
-    m = lambda n: (n / 16 + 8) * U  # noqa: E731
+    dG = c * (0.25 * (sums * d / 16 + 8) * U * (q.abs() @ e.abs().T + bias.double().abs()[:, None]) + 12 * U * (torch.sigmoid(S) + y))
+    m = lambda n: (sums * n / 16 + 8) * U  # noqa: E731
     want = (loss, G @ e, G.sum(1), G.T @ q)
     bound = (2e-6 * loss, dG @ e.abs() + m(N) * (G.abs() @ e.abs()), dG.sum(1) + N * U * G.abs().sum(1),
              dG.T @ q.abs() + m(B) * (G.abs().T @ q.abs()))
