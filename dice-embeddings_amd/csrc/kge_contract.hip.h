@@ -7,8 +7,6 @@
 //   qreg_i8_kernel      per-row int8 table, the same widths and walk, rows widened to bf16 on the way into LDS
 //   kchunk_kernel       bf16 / int8 with d > 256: K in chunks of 64 through LDS
 //   ksplit_kernel       fp32 tables, any d: every operand as three bf16 parts, six part products per product
-// (half_kernel in kge_half.hip.h, on the fp16 MFMA, is the one main loop beside them: the contractions of a training step, whose
-// sums need not be the scores' bits)
 // Reduction order of one score is fixed (k ascending in steps of the MFMA depth, nothing else), so
 // every kernel that forms dot(Q[b], E[e]) with these helpers produces the same fp32 bit pattern.
 //

@@ -5,7 +5,6 @@
 // -fsanitize=address,undefined) into the CPU test driver tests/host_model_test.cpp, so that every layout and
 // every packed field is exercised with bounds checks where there is no GPU.
 #pragma once
-#include <math.h>
 #include <stddef.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -36,7 +35,6 @@ constexpr int TOPK_CAP = 4096;           // candidates a query can collect in on
 constexpr int TOPK_MAX_K = 1024;
 constexpr int TOPK_FIRST_ROWS = 1024;    // first round takes everything: must not exceed TOPK_CAP
 constexpr int BCE_SLOTS = 128;
-constexpr int HALF_SLOTS = 256;          // partial maxima of an operand of the fp16 contraction
 constexpr int KS_WG_QUERIES = 128;       // workgroup shape of the fp32 contraction (also sizes the backward's K split)
 constexpr int KS_NARROW_ROWS = 128;      // entity rows of its narrow form, two or three workgroups per CU,
 constexpr int KS_WIDE_ROWS = 256;        // and of its wide form, one per CU
@@ -427,80 +425,11 @@ inline int64_t topk_growth(int64_t k) { return k <= 256 ? 4 : 2; }
 constexpr int BCE_POS_SLOTS = 128;  // partial sums over the positives (one atomic per workgroup, spread)
 inline size_t bce_ws_bytes() { return (2 * BCE_SLOTS + BCE_POS_SLOTS) * sizeof(double) + 128; }
 
-// A step's contractions on fp16 parts (half_kernel): the split rows of E, Q and G, with zeros up to whole chunks of 32 rows and
-// columns; allocated up to whole tiles of rows, and HALF_SLACK more for the columns of a last tile past the last row's end.
-constexpr int HALF_ROWS = 128;            // entity rows of a workgroup
-constexpr int HALF_SLACK = 4 * HALF_ROWS;
-struct HalfPlan {
-  bool on;
-  int64_t rows_e, rows_q, cols;  // rows that are written, and columns
-  // dE: the chunks of 128 entities from tail_chunk on have their sum over the batch split tail_splits ways (0: none), tail_len each
-  int64_t tail_chunk;
-  int tail_splits, tail_len;
-  int dq_splits;  // ranges of N that dQ is summed in, as equal as whole chunks allow
-  size_t off_max, off_E, off_Q, off_tail;
-};
-// Against the six bf16 products (the other form), a step's three contractions: 2048 x 40,943, d = 256 804 -> 512 us, 1024 x 3000,
-// d = 64 101 -> 60, 160 x 600, d = 32 37.5 -> 36.7, 128 x 600, d = 32 33.3 -> 33.9, 64 x 300, d = 32 31 -> 33 (d = 128 at that size 39.7 -> 37.1).  And a product of fp16 parts carries 8e-8 of its norm in
-// dropped parts, where that of bf16 parts carries roundings that grow with the length of the sum: measured against float64,
-// sums of 64 are about as far off either way (1e-7), shorter ones further, longer ones less (256: 1.1e-7 against 1.8e-7).  So
-// batches (dE) and tables (dQ) shorter than this keep the other form, and the scores of rows of fewer columns the bf16 chain.
-constexpr int HALF_MIN_SUM = 64;
-inline bool half_scores(int64_t d) { return d >= HALF_MIN_SUM; }
-inline bool half_pays(int64_t B, int64_t d, int64_t N) {
-  return B >= (half_scores(d) ? 128 : 160) && N >= HALF_MIN_SUM && N <= (1 << 22) && N * ((d + 31) / 32) < (1LL << 30) &&
-         B * ((d + 31) / 32) < (1LL << 30);
-}
-// dE's workgroups are one tile each, 512 at a time; those of a last round that would leave much of the chip idle split
-// their sums so that it fills (2048 x 40,943, d = 256: 640 tiles are one round and a quarter).
-inline void half_tail(int64_t N, int64_t d, HalfPlan& h) {
-  const int64_t groups = (d + KS_WG_QUERIES - 1) / KS_WG_QUERIES, chunks = (N + HALF_ROWS - 1) / HALF_ROWS, resident = 512;
-  h.tail_chunk = chunks * groups / resident * resident / groups;
-  const int64_t rest = (chunks - h.tail_chunk) * groups, k_chunks = h.rows_q / 32;
-  int best = 1;
-  double best_cost = 0.9;  // rounds of a whole sum's length; a split that gains less than a tenth is not worth its partial sums
-  for (int s = 2; s <= 8 && k_chunks >= 8 * s; ++s) {
-    const double cost = (double)((rest * s + resident - 1) / resident) / s + 0.02 * s;
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = s;
-    }
-  }
-  h.tail_splits = rest > 0 && best > 1 ? best : 0;
-  h.tail_len = h.tail_splits ? (int)((k_chunks + best - 1) / best * 32) : 0;
-  if (!h.tail_splits) h.tail_chunk = chunks;
-  else h.tail_splits = (int)((h.rows_q + h.tail_len - 1) / h.tail_len);  // (none of them empty)
-}
-// dQ: two workgroups per CU, at most 64 ranges, none shorter than four chunks; in eights where there are that many, so that an XCD
-// keeps to its ranges (the workgroups of a range read the same rows of E: a step of 1000 x 14,541, d = 200, in 31 ranges 30 - 40 us, in 32
-// 32)
-inline int half_dq_splits(int64_t B, int64_t d, int64_t N) {
-  const int64_t tiles = (B + KS_WG_QUERIES - 1) / KS_WG_QUERIES * ((d + HALF_ROWS - 1) / HALF_ROWS), chunks = (N + 31) / 32;
-  int64_t s = (512 + tiles - 1) / tiles;
-  if (s > 64) s = 64;
-  if (s > chunks / 4) s = chunks / 4;
-  if (s >= 6) s = (s + 3) / 8 * 8 > 0 ? (s + 3) / 8 * 8 : 8;
-  if (s * 2 > chunks) s = chunks / 2;
-  return (int)(s < 1 ? 1 : s);
-}
-inline unsigned half_split_blocks(int64_t rows, int64_t cols) {  // 32 lines at a time, four times over
-  const int64_t n = (rows * (cols / 32) + 127) / 128;
-  return (unsigned)(n < 2048 ? n : 2048);
-}
-// The power of two (its exponent) that brings every score gradient of a step below 2^15: a gradient is c (sigmoid - label)
-// with labels in [min(0, 1 - eps), max(1, 1 - eps)] + eps / N.
-inline int half_gradient_exponent(float c, float eps, int64_t N) {
-  const double bound = fabs((double)c) * (2.0 + fabs(1.0 - (double)eps) + 1.0 / (double)N);
-  if (!(bound > 0.0) || !(bound < 1e300)) return 0;
-  const int e = 14 - ilogb(bound);
-  return e > 116 ? 116 : e < -113 ? -113 : e;
-}
 struct BwdPlan {
   int64_t ldG, ldT;  // row strides of G [B, ldG] (a multiple of 32) and GT [N, ldT] (a multiple of 4)
   int k_splits, k_split_len;
   int dq_rows;  // dQ's form of the contraction
   bool kmajor;  // d a multiple of 4: the gradient contractions read G, E and Q where they lie (no GT, ET, QT)
-  HalfPlan half;
   size_t off_G, off_GT, off_ET, off_QT, off_part, total;
 };
 inline BwdPlan bwd_plan(int64_t B, int64_t d, int64_t N) {
@@ -513,9 +442,7 @@ inline BwdPlan bwd_plan(int64_t B, int64_t d, int64_t N) {
   // wide (d = 256, N = 41k, B = 1000 111 us for 118, B = 2048 211 for 228).
   const int64_t groups = (B + KS_WG_QUERIES - 1) / KS_WG_QUERIES;
   const int64_t wide = groups * ((d + KS_WIDE_ROWS - 1) / KS_WIDE_ROWS), narrow = groups * ((d + KS_NARROW_ROWS - 1) / KS_NARROW_ROWS);
-  p.kmajor = d % 4 == 0;
-  p.half.on = p.kmajor && half_pays(B, d, N);
-  p.dq_rows = (p.half.on || narrow < 2 * wide || wide * 64 < 256 || N * wide < 65536) ? KS_NARROW_ROWS : KS_WIDE_ROWS;
+  p.dq_rows = (narrow < 2 * wide || wide * 64 < 256 || N * wide < 65536) ? KS_NARROW_ROWS : KS_WIDE_ROWS;
   int64_t splits = p.dq_rows == KS_WIDE_ROWS ? (256 + wide - 1) / wide : (512 + narrow - 1) / narrow;
   if (splits > 64) splits = 64;
   if (splits < 1) splits = 1;
@@ -524,28 +451,12 @@ inline BwdPlan bwd_plan(int64_t B, int64_t d, int64_t N) {
   p.k_splits = (int)((N + len - 1) / len);
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
   size_t off = up(bce_ws_bytes());
-  HalfPlan& h = p.half;
-  if (h.on) {
-    auto rows = [](int64_t n, int64_t to) { return (n + to - 1) / to * to; };
-    h.rows_e = p.ldG;  // (N rounded to 32)
-    h.rows_q = rows(B, 32);
-    h.cols = rows(d, 32);
-    h.off_max = off;   off += up((2 * HALF_SLOTS + 2) * sizeof(uint32_t));
-    h.off_E = off;     off += up((size_t)rows(N, HALF_ROWS) * h.cols * 4 + HALF_SLACK);
-    h.off_Q = off;     off += up((size_t)rows(B, KS_WG_QUERIES) * h.cols * 4 + HALF_SLACK);
-    p.off_G = off;     off += up((size_t)rows(B, KS_WG_QUERIES) * p.ldG * 4 + HALF_SLACK);
-  } else {
-    p.off_G = off;     off += up((size_t)B * p.ldG * sizeof(float));
-  }
+  p.off_G = off;     off += up((size_t)B * p.ldG * sizeof(float));
+  p.kmajor = d % 4 == 0;
   p.off_GT = off;    off += p.kmajor ? 0 : up((size_t)N * p.ldT * sizeof(float));
   p.off_ET = off;    off += p.kmajor ? 0 : up((size_t)d * p.ldG * sizeof(float));
   p.off_QT = off;    off += p.kmajor ? 0 : up((size_t)d * p.ldT * sizeof(float));
-  if (h.on) h.dq_splits = half_dq_splits(B, d, N);
-  p.off_part = off;  off += up((size_t)(h.on && h.dq_splits > p.k_splits ? h.dq_splits : p.k_splits) * B * d * sizeof(float));
-  if (h.on) {
-    half_tail(N, d, h);
-    h.off_tail = off;  off += up((size_t)h.tail_splits * (N - h.tail_chunk * HALF_ROWS) * d * sizeof(float));
-  }
+  p.off_part = off;  off += up((size_t)p.k_splits * B * d * sizeof(float));
   p.total = off;
   return p;
 }

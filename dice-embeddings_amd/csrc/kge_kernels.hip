@@ -3,7 +3,6 @@
 #include "kge_contract.hip.h"
 #include "kge_rank128.hip.h"
 #include "kge_wide.hip.h"
-#include "kge_half.hip.h"
 #include "kge_topk_i8.hip.h"
 
 #include <string.h>
@@ -1070,8 +1069,6 @@ struct PosGrad {
   int64_t ldT;
   float* dbias;  // row sums of the gradient, or null
   float pos;
-  int split;     // G holds split rows of ldG columns ...
-  float up, down;  // ... with these powers of two: 2^s and 2^-s
 };
 constexpr int BCE_POS_SPLIT = 4;
 constexpr int BCE_POS_UNROLL = 4;
@@ -1110,16 +1107,7 @@ __global__ void __launch_bounds__(256) bce_pos_kernel(ContractArgs a, const floa
         on = sub == u ? ok[u] : on;
       }
       if (on) {
-        if (pg.split) {
-          _Float16* p = (_Float16*)pg.G + (q * pg.ldG + (mine & ~31ll)) * 2 + (mine & 31);
-          const float g = __builtin_fmaf((float)p[32], 1.f / 2048.f, (float)p[0]) * pg.down;
-          _Float16 h, l;
-          half_parts(g - pg.pos, pg.up, pg.up * 2048.f, h, l);
-          p[0] = h;
-          p[32] = l;
-        } else {
-          pg.G[q * pg.ldG + mine] -= pg.pos;
-        }
+        pg.G[q * pg.ldG + mine] -= pg.pos;
         if (pg.GT) pg.GT[mine * pg.ldT + q] -= pg.pos;
       }
     }
@@ -1251,29 +1239,15 @@ __global__ void __launch_bounds__(256) transpose_kernel(const float* in, int64_t
   }
 }
 
-// out[i] = sum over y of partial[y][i], y ascending, for one or two sets of partial sums: the first `blocks0` workgroups take the
-// first set
-// (and, in the first workgroup, the loss from its partial sums: a launch less on the way through the backward)
-struct SplitSums {
-  const float* partial;
-  float* out;
-  int64_t n;
-  int n_splits;
-};
-__global__ void reduce_splits_kernel(SplitSums s0, SplitSums s1, unsigned blocks0, BceFinal f) {
+// out[i] = sum over y of partial[y][i], y ascending
+// (and, in its first workgroup, the loss from its partial sums: a launch less on the way through the backward)
+__global__ void reduce_splits_kernel(const float* partial, int n_splits, int64_t n, float* out, BceFinal f) {
   if (f.loss && blockIdx.x == 0 && threadIdx.x < 64) bce_final(f, threadIdx.x);
-  const bool second = blockIdx.x >= blocks0;
-  const SplitSums s = second ? s1 : s0;
-  const unsigned block = second ? blockIdx.x - blocks0 : blockIdx.x, blocks = second ? gridDim.x - blocks0 : blocks0;
-  for (int64_t i = (int64_t)block * blockDim.x + threadIdx.x; i < s.n; i += (int64_t)blocks * blockDim.x) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     float v = 0.f;
-    for (int y = 0; y < s.n_splits; ++y) v += s.partial[(int64_t)y * s.n + i];
-    s.out[i] = v;
+    for (int y = 0; y < n_splits; ++y) v += partial[(int64_t)y * n + i];
+    out[i] = v;
   }
-}
-inline unsigned split_sums_blocks(const SplitSums& s) {
-  const int64_t b = (s.n + 255) / 256;
-  return s.n_splits < 2 ? 0u : (unsigned)(b < 2048 ? b : 2048);
 }
 
 // ============================================================================================
@@ -1376,9 +1350,7 @@ void plan_ksplit(ContractArgs& a, bool rows_aligned, int forced = 0) {
                                           : host::KsCost{0.4, 1.0, 0.0, 0.65, {0, 0.82, 1.12, 1.6}};
   const int64_t rows = a.e_end - a.e_begin;
   // the score gradients (sigmoids and a store per score) are always faster narrow: N = 41k, d = 256, B = 2048 375 -> 345 us
-  constexpr bool grad = std::is_same<E, GradEpi<2>>::value || std::is_same<E, GradSplitEpi<2>>::value ||
-                        std::is_same<E, GradSplitBiasEpi<2>>::value;
-  if (grad && !forced) forced = KS_NARROW_ROWS;
+  if (std::is_same<E, GradEpi<2>>::value && !forced) forced = KS_NARROW_ROWS;
   if (forced) {
     a.ks_rows = forced;
     a.chunk_rows = host::fullest_chunk(rows, a.n_qgroups, forced, forced == KS_NARROW_ROWS ? 512 : 256);
@@ -1429,19 +1401,12 @@ constexpr const char* epilogue_name() {
        : std::is_same<E, RankEpi<2>>::value ? "RankEpi"
        : std::is_same<E, TopkEpi<2>>::value ? "TopkEpi" : std::is_same<E, TopkKeyEpi<2>>::value ? "TopkKeyEpi"
        : std::is_same<E, TopkFirstEpi<2>>::value ? "TopkFirstEpi" : std::is_same<E, BceEpi<2>>::value ? "BceEpi"
-       : std::is_same<E, GradEpi<2>>::value ? "GradEpi" : std::is_same<E, GradSplitEpi<2>>::value ? "GradSplitEpi"
-       : std::is_same<E, GradSplitBiasEpi<2>>::value ? "GradSplitBiasEpi" : std::is_same<E, MinMaxEpi<2>>::value ? "MinMaxEpi" : "?";
+       : std::is_same<E, GradEpi<2>>::value ? "GradEpi" : std::is_same<E, MinMaxEpi<2>>::value ? "MinMaxEpi" : "?";
 }
 
 template <template <int> class EpiT, class EArgs>
 void ksplit_go(bool rows_aligned, dim3 grid, dim3 block, hipStream_t st, const ContractArgs& a, const EArgs& ea) {
-  using E = EpiT<2>;
-  constexpr bool grad_split = std::is_same<E, GradSplitEpi<2>>::value || std::is_same<E, GradSplitBiasEpi<2>>::value;
-  if constexpr (grad_split) {  // (rows are whole quads: host::HalfPlan)
-    hipLaunchKernelGGL((ksplit_kernel<EpiT, true, KS_NARROW_ROWS>), grid, block, 0, st, a, ea);
-    return;
-  } else {
-  constexpr bool narrow_only = std::is_same<E, GradEpi<2>>::value;
+  constexpr bool narrow_only = std::is_same<EpiT<2>, GradEpi<2>>::value;
   if constexpr (!narrow_only) {
     if (a.ks_rows == KS_WIDE_ROWS) {
       if (rows_aligned) hipLaunchKernelGGL((ksplit_kernel<EpiT, true, KS_WIDE_ROWS>), grid, block, 0, st, a, ea);
@@ -1451,7 +1416,6 @@ void ksplit_go(bool rows_aligned, dim3 grid, dim3 block, hipStream_t st, const C
   }
   if (rows_aligned) hipLaunchKernelGGL((ksplit_kernel<EpiT, true, KS_NARROW_ROWS>), grid, block, 0, st, a, ea);
   else hipLaunchKernelGGL((ksplit_kernel<EpiT, false, KS_NARROW_ROWS>), grid, block, 0, st, a, ea);
-  }
 }
 
 template <template <int> class EpiT, class EArgs>
@@ -1629,44 +1593,6 @@ int launch_ksplit(ContractArgs a, const EArgs& ea, unsigned k_splits, hipStream_
   else ksplit_go<EpiT>(rows_aligned, grid, block, st, a, ea);
   KGE_LAUNCH_CHECK(name);
   snprintf(kname, sizeof(kname), "ksplit_kernel<%s, %s, %d>", epilogue_name<EpiT>(), rows_aligned ? "true" : "false", a.ks_rows);
-  return timer.end(kname);
-}
-
-// half_kernel: split rows (StoreEpi with a K-major entity operand, StoreTEpi with both, the score gradients with neither).
-template <template <int> class EpiT, class EArgs>
-int launch_half(ContractArgs a, HalfArgs hs, const EArgs& ea, unsigned k_splits, hipStream_t st, const char* name) {
-  if (a.B == 0 || a.e_end <= a.e_begin) return KGE_OK;
-  constexpr bool store = std::is_same<EpiT<KS_NQT>, StoreEpi<KS_NQT>>::value;
-  constexpr bool store_t = std::is_same<EpiT<KS_NQT>, StoreTEpi<KS_NQT>>::value;
-  constexpr int KMAJ = store ? 1 : store_t ? 3 : 0;
-  KGE_REQUIRE(a.ldq % 32 == 0 && a.lde % 32 == 0 && a.ldq > 0 && a.lde > 0 && (((uintptr_t)a.E | (uintptr_t)a.Q) % 128 == 0) &&
-                  a.d % 32 == 0 && (k_splits == 1 || (store && (int64_t)k_splits <= a.d / 32)),
-              KGE_ERR_INVALID, "%s: split rows are whole lines", name);
-  hs.k_splits = (int)k_splits;
-  // (dE: a tile per workgroup, the tail's shared out; else as full a last round as whole tiles give)
-  a.chunk_rows = store_t ? host::HALF_ROWS : host::fullest_chunk(a.e_end - a.e_begin, a.n_qgroups, host::HALF_ROWS, 512);
-  a.n_chunks = (a.e_end - a.e_begin + a.chunk_rows - 1) / a.chunk_rows;
-  int64_t tail_wgs = 0;
-  if (store_t && hs.tail_splits) {
-    tail_wgs = (a.n_chunks - hs.tail_chunk) * a.n_qgroups * hs.tail_splits;
-    a.n_chunks = hs.tail_chunk;
-  }
-  hs.tail_first = contract_grid_wgs(a);
-  const int64_t nwg = hs.tail_first + tail_wgs;
-  if (!tail_wgs) hs.tail_first = nwg;
-  KGE_REQUIRE(nwg <= 0x7fffffffLL && k_splits >= 1 && k_splits <= 65535, KGE_ERR_INVALID,
-              "%s: grid of %lld x %u workgroups too large", name, (long long)nwg, k_splits);
-  dim3 grid((unsigned)nwg, k_splits), block(HALF_THREADS);
-  LaunchTimer timer;
-  if (int trc = timer.begin(st)) return trc;
-  if (store && k_splits % 8 == 0 && a.n_chunks < 8 && nwg * k_splits <= 0x7fffffffLL) {  // (as launch_ksplit)
-    a.k_split_xcd = (int)k_splits;
-    grid = dim3((unsigned)(nwg * k_splits), 1);
-  }
-  hipLaunchKernelGGL((half_kernel<EpiT, KMAJ>), grid, block, 0, st, a, hs, ea);
-  KGE_LAUNCH_CHECK(name);
-  char kname[160];
-  snprintf(kname, sizeof(kname), "half_kernel<%s, %d>", epilogue_name<EpiT>(), KMAJ);
   return timer.end(kname);
 }
 
@@ -2453,67 +2379,31 @@ int bce_backward_impl(const float* Q, const float* bias, const void* E, int dtyp
   float* part = (float*)(ws + p.off_part);
   const float inv_bn = grad_out / ((float)B * (float)N);
 
-  const unsigned prep_wgs = step_prepare_wgs(prep);
-  const host::HalfPlan& hp = p.half;
-  HalfArgs hs{};
-  const uint32_t* maxima = (const uint32_t*)(ws + hp.off_max);
-  const int32_t* exps = (const int32_t*)(maxima + 2 * HALF_SLOTS);
-  int exp_g = 0;
-  if (hp.on) {
-    exp_g = host::half_gradient_exponent(inv_bn, label_smoothing, N);
-    hipLaunchKernelGGL(half_max_kernel, dim3(2 * HALF_SLOTS + prep_wgs), dim3(HALF_MAX_THREADS), 0, st, (const float*)E, N * d, Q,
-                       B * d, (uint32_t*)maxima, sums, BCE_INIT_THREADS, dbias, B, prep);
-    KGE_LAUNCH_CHECK("half_max_kernel");
-    const HalfSplit se{(const float*)E, (unsigned char*)(ws + hp.off_E), N, hp.rows_e, (int)d, (int)(hp.cols / 32)};
-    const HalfSplit sq{Q, (unsigned char*)(ws + hp.off_Q), B, hp.rows_q, (int)d, (int)(hp.cols / 32)};
-    const unsigned be = host::half_split_blocks(hp.rows_e, hp.cols), bq = host::half_split_blocks(hp.rows_q, hp.cols);
-    hipLaunchKernelGGL(half_split_kernel, dim3(be + bq), dim3(256), 0, st, se, sq, be, maxima, (int32_t*)exps);
-    KGE_LAUNCH_CHECK("half_split_kernel");
-  } else {
-    const unsigned init_wgs = bce_init_blocks(B, dbias);
-    hipLaunchKernelGGL(bce_init_kernel, dim3(init_wgs + prep_wgs), dim3(BCE_INIT_THREADS), 0, st, sums, dbias, B, init_wgs, prep);
-    KGE_LAUNCH_CHECK("bce_init_kernel");
-  }
+  const unsigned init_wgs = bce_init_blocks(B, dbias);
+  hipLaunchKernelGGL(bce_init_kernel, dim3(init_wgs + step_prepare_wgs(prep)), dim3(BCE_INIT_THREADS), 0, st, sums, dbias, B, init_wgs,
+                     prep);
+  KGE_LAUNCH_CHECK("bce_init_kernel");
   // (1) scores -> g = (sigmoid(s) - dense part of y') * inv_bn, both layouts, and the loss sums
-  const float uniform = label_smoothing != 0.f ? inv_bn / (float)N : 0.f;
-  const int32_t want_s = label_smoothing != 0.f ? 1 : 0;
-  const float up = ldexpf(1.f, exp_g), down = ldexpf(1.f, -exp_g);
   ContractArgs a = make_args(Q, E, KGE_F32, nullptr, B, d, N, 0, N);
-  if (hp.on) {
-    const GradSplitArgs ga{bias, sums, (unsigned char*)G, dbias, p.ldG, inv_bn * up, uniform * up, down, want_s};
-    if (host::half_scores(d)) {
-      ContractArgs b = a;
-      b.Q = (const float*)(ws + hp.off_Q);
-      b.E = ws + hp.off_E;
-      b.d = b.ldq = b.lde = (int)hp.cols;
-      hs = HalfArgs{exps, exps + 1, 0, 0};
-      rc = dbias ? launch_half<GradSplitBiasEpi>(b, hs, ga, 1, st, "kge_bce_multihot_backward: scores")
-                 : launch_half<GradSplitEpi>(b, hs, ga, 1, st, "kge_bce_multihot_backward: scores");
-    } else {
-      rc = dbias ? launch_ksplit<GradSplitBiasEpi>(a, ga, 1, st, "kge_bce_multihot_backward: scores")
-                 : launch_ksplit<GradSplitEpi>(a, ga, 1, st, "kge_bce_multihot_backward: scores");
-    }
+  const GradArgs ga{bias, sums, G, GT, dbias, p.ldG, p.ldT, inv_bn, label_smoothing != 0.f ? inv_bn / (float)N : 0.f,
+                    label_smoothing != 0.f ? 1 : 0};
+  if (!GT && host::few_grad_pays(B, d, N, dbias != nullptr)) {
+    LaunchTimer timer;
+    if ((rc = timer.begin(st))) return rc;
+    if ((rc = few_grad_launch(Q, (const float*)E, B, d, N, ga, st))) return rc;
+    rc = timer.end("few_scan_kernel");
   } else {
-    const GradArgs ga{bias, sums, G, GT, dbias, p.ldG, p.ldT, inv_bn, uniform, want_s};
-    if (!GT && host::few_grad_pays(B, d, N, dbias != nullptr)) {
-      LaunchTimer timer;
-      if ((rc = timer.begin(st))) return rc;
-      if ((rc = few_grad_launch(Q, (const float*)E, B, d, N, ga, st))) return rc;
-      rc = timer.end("few_scan_kernel");
-    } else {
-      rc = launch_ksplit<GradEpi>(a, ga, 1, st, "kge_bce_multihot_backward: scores");
-    }
+    rc = launch_ksplit<GradEpi>(a, ga, 1, st, "kge_bce_multihot_backward: scores");
   }
   if (rc) return rc;
   if (csr_row && n_rows > 0) {
     const float pos = (label_smoothing != 0.f ? 1.0f - label_smoothing : 1.0f) * inv_bn;
     hipLaunchKernelGGL((bce_pos_kernel<KGE_F32>), dim3((unsigned)B, BCE_POS_SPLIT), dim3(256), 0, st, a, bias, csr_row,
-                       row_ptr, col, n_rows, loss ? sums : nullptr, PosGrad{G, p.ldG, GT, p.ldT, dbias, pos, hp.on, up, down});
+                       row_ptr, col, n_rows, loss ? sums : nullptr, PosGrad{G, p.ldG, GT, p.ldT, dbias, pos});
     KGE_LAUNCH_CHECK("bce_pos_kernel");
   }
   const BceFinal fin{sums, (double)B, (double)N, label_smoothing, loss};
-  const int dq_splits = hp.on ? hp.dq_splits : p.k_splits;
-  if (loss && dq_splits == 1 && hp.tail_splits < 2) {  // (else the reduction of partial sums does it)
+  if (loss && p.k_splits == 1) {  // (else dQ's reduction does it)
     hipLaunchKernelGGL(bce_final_kernel, dim3(1), dim3(64), 0, st, fin);
     KGE_LAUNCH_CHECK("bce_final_kernel");
   }
@@ -2526,7 +2416,6 @@ int bce_backward_impl(const float* Q, const float* bias, const void* E, int dtyp
                        B, d, d, QT, p.ldT);
     KGE_LAUNCH_CHECK("transpose_kernel");
   }
-  SplitSums tail_sums{};
   // (3) dQ [B, d] = G . E: rows of G against rows of ET (or E itself, K-major), K = N split over grid.y, partial sums
   // reduced in order
   {
@@ -2534,39 +2423,20 @@ int bce_backward_impl(const float* Q, const float* bias, const void* E, int dtyp
     b.ldq = (int)p.ldG;
     b.lde = kmajor ? (int)d : (int)p.ldG;
     b.k_split_len = p.k_split_len;
-    StoreArgs sa{dq_splits > 1 ? part : dQ, nullptr, d, (int64_t)B * d};
-    if (hp.on) {
-      b.E = ws + hp.off_E;
-      b.d = (int)p.ldG;
-      b.lde = (int)hp.cols;
-      b.k_split_len = 0;
-      hs = HalfArgs{exps, nullptr, 0, exp_g};
-      rc = launch_half<StoreEpi>(b, hs, sa, (unsigned)dq_splits, st, "kge_bce_multihot_backward: dQ");
-    } else {
-      rc = launch_ksplit<StoreEpi>(b, sa, (unsigned)p.k_splits, st, "kge_bce_multihot_backward: dQ", kmajor ? 1 : 0, p.dq_rows);
-    }
+    StoreArgs sa{p.k_splits > 1 ? part : dQ, nullptr, d, (int64_t)B * d};
+    rc = launch_ksplit<StoreEpi>(b, sa, (unsigned)p.k_splits, st, "kge_bce_multihot_backward: dQ", kmajor ? 1 : 0,
+                                 p.dq_rows);
     if (rc) return rc;
+    if (p.k_splits > 1) {
+      const int64_t n = B * d;
+      hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)((n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048)),
+                         dim3(256), 0, st, part, p.k_splits, n, dQ, fin);
+      KGE_LAUNCH_CHECK("reduce_splits_kernel");
+    }
   }
   // (4) dE [N, d] = G^T . Q: rows of GT against rows of QT, K = B (or G and Q themselves, both K-major)
   {
-    if (hp.on) {
-      ContractArgs b = make_args(Q, G, KGE_F32, nullptr, d, hp.rows_q, p.ldG, 0, p.ldG);
-      b.Q = (const float*)(ws + hp.off_Q);
-      b.ldq = (int)hp.cols;
-      b.lde = (int)p.ldG;
-      StoreArgs sa{dE, nullptr, d, 0, N};
-      hs = HalfArgs{nullptr, exps + 1, exp_g, 0};
-      const int64_t tail_row = hp.tail_chunk * host::HALF_ROWS;
-      if (hp.tail_splits) {
-        hs.tail_splits = hp.tail_splits;
-        hs.tail_chunk = hp.tail_chunk;
-        hs.tail_len = hp.tail_len;
-        hs.tail_stride = (N - tail_row) * d;
-        hs.tail = (float*)(ws + hp.off_tail) - tail_row * d;
-        tail_sums = SplitSums{(const float*)(ws + hp.off_tail), dE + tail_row * d, hs.tail_stride, hp.tail_splits};
-      }
-      rc = launch_half<StoreTEpi>(b, hs, sa, 1, st, "kge_bce_multihot_backward: dE");
-    } else if (kmajor) {
+    if (kmajor) {
       // the rows of Q as the "queries", the rows of G (N of them, read up to the padded pitch) as the "entities": a
       // workgroup's share of G is 256 or 128 neighbouring columns of every row, and the result is stored transposed
       ContractArgs b = make_args(Q, G, KGE_F32, nullptr, d, B, p.ldG, 0, p.ldG);
@@ -2582,13 +2452,6 @@ int bce_backward_impl(const float* Q, const float* bias, const void* E, int dtyp
       rc = launch_ksplit<StoreEpi>(b, sa, 1, st, "kge_bce_multihot_backward: dE");
     }
     if (rc) return rc;
-  }
-  // (5) partial sums
-  const SplitSums dq_sums{part, dQ, B * d, dq_splits};
-  const unsigned b0 = split_sums_blocks(dq_sums), b1 = split_sums_blocks(tail_sums);
-  if (b0 + b1) {
-    hipLaunchKernelGGL(reduce_splits_kernel, dim3(b0 + b1), dim3(256), 0, st, dq_sums, tail_sums, b0, fin);
-    KGE_LAUNCH_CHECK("reduce_splits_kernel");
   }
   return KGE_OK;
 }

@@ -154,48 +154,6 @@ static void test_layouts() {
                     {p.off_QT, copies * bdn[1] * p.ldT * 4}, {p.off_part, (size_t)p.k_splits * bdn[0] * bdn[1] * 4}},
                    p.total);
   }
-  // split rows: what the contractions read past an operand's own rows and columns (whole tiles, nothing is clamped) stays inside
-  // its region, the regions are disjoint, and dE's workgroups sum every (tile, K chunk) exactly once
-  for (int64_t B : {1, 127, 128, 129, 160, 300, 2048, 5000})
-    for (int64_t N : {1, 63, 64, 135, 1000, 14541, 40943, 1 << 22})
-      for (int64_t d : {4, 63, 64, 100, 128, 132, 256, 400}) {
-        const BwdPlan p = bwd_plan(B, d, N);
-        const HalfPlan& h = p.half;
-        CHECK(h.on == (p.kmajor && half_pays(B, d, N)));
-        if (!h.on) continue;
-        CHECK(h.rows_e == p.ldG && p.ldG % 32 == 0 && h.rows_q % 32 == 0 && h.rows_q >= B && h.cols % 32 == 0 && h.cols >= d);
-        CHECK(p.dq_rows == KS_NARROW_ROWS && h.off_E % 128 == 0 && h.off_Q % 128 == 0 && p.off_G % 128 == 0);
-        auto up = [](int64_t n, int64_t to) { return (n + to - 1) / to * to; };
-        const int64_t pe = 4 * h.cols, pg = 4 * p.ldG;  // row pitches, bytes
-        auto rows_end = [&](int64_t rows, int64_t pitch) { return up(rows, 128) * pitch; };                          // row-major
-        auto kmaj_end = [&](int64_t k, int64_t pitch, int64_t rows) { return (k - 1) * pitch + 4 * up(rows, 128); };  // K-major
-        const int64_t end_E = std::max(rows_end(N, pe), kmaj_end(p.ldG, pe, d)), end_Q = std::max(rows_end(B, pe), kmaj_end(h.rows_q, pe, d));
-        const int64_t end_G = std::max(rows_end(B, pg), kmaj_end(h.rows_q, pg, p.ldG));
-        const int64_t tail_row = h.tail_chunk * HALF_ROWS;
-        check_disjoint({{0, bce_ws_bytes()}, {h.off_max, (2 * HALF_SLOTS + 2) * 4}, {h.off_E, (size_t)end_E}, {h.off_Q, (size_t)end_Q},
-                        {p.off_G, (size_t)end_G}, {p.off_part, (size_t)h.dq_splits * B * d * 4},
-                        {h.off_tail, h.tail_splits ? (size_t)h.tail_splits * (N - tail_row) * d * 4 : 0}},
-                       p.total);
-        CHECK(h.dq_splits >= 1 && h.dq_splits <= 64 && (h.dq_splits < 8 || h.dq_splits % 8 == 0 || h.dq_splits == p.ldG / 32 / 2));
-        CHECK(h.dq_splits <= p.ldG / 32);                                                  // no range of dQ is empty
-        const int64_t groups = (d + 127) / 128, chunks = up(p.ldG, HALF_ROWS) / HALF_ROWS;
-        CHECK(h.tail_chunk >= 0 && h.tail_chunk <= chunks && (h.tail_splits == 0 || (h.tail_splits >= 2 && h.tail_splits <= 8)));
-        if (!h.tail_splits) CHECK(h.tail_chunk == chunks);
-        if (h.tail_splits) {
-          CHECK(tail_row < N && h.tail_len % 32 == 0 && (int64_t)(h.tail_splits - 1) * h.tail_len < h.rows_q &&
-                (int64_t)h.tail_splits * h.tail_len >= h.rows_q);
-          std::vector<char> seen((chunks - h.tail_chunk) * groups * h.tail_splits, 0);
-          for (size_t rest = 0; rest < seen.size(); ++rest) {  // as half_kernel deals them
-            const int64_t tile = rest / h.tail_splits, range = rest % h.tail_splits;
-            const int64_t at = ((tile / groups) * groups + tile % groups) * h.tail_splits + range;
-            CHECK(tile / groups < chunks - h.tail_chunk && !seen[at]);
-            seen[at] = 1;
-          }
-        }
-        const int exps[] = {half_gradient_exponent(1e-9f, 0.1f, N), half_gradient_exponent(0.f, 0.f, N), half_gradient_exponent(1e30f, 5.f, N)};
-        for (int e : exps) CHECK(e >= -113 && e <= 116);
-        CHECK(1e-9 * 3.1 * ldexp(1.0, exps[0]) < 32768.0);
-      }
 }
 
 static void test_csr_keys() {

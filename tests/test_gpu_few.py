@@ -203,7 +203,7 @@ def test_nan_rows_and_queries_where_scores_are_formed_again(storage, N, d, B):
 @pytest.mark.parametrize("eps,want_dbias", [(0.0, True), (0.1, False)])
 def test_gradients_of_few_queries(B, N, d, eps, want_dbias):
     from test_gpu_split_rows import _step
-    got, want, bound, call = _step(B, N, d, eps, want_dbias, sums=6)
+    got, want, bound, call = _step(B, N, d, eps, want_dbias)
     for g, w, b in zip(got, want, bound):
         if g is not None:
             assert ((g.double().reshape(w.shape) - w).abs() <= b).all()
