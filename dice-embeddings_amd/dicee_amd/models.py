@@ -385,9 +385,9 @@ class BaseKGE(torch.nn.Module):
         loss (detached) and ACCUMULATES the gradients into ``.grad`` of the parameters the step reads, as
         autograd would, so that any ``torch.optim`` optimizer can take the step."""
         loss, grads = self.kvsall_bce_gradients(x, csr, label_smoothing)
+        params = dict(self.named_parameters())
         for name, g in grads.items():
-            layer, attr = name.split(".")
-            prm = getattr(getattr(self, layer), attr)
+            prm = params[name]
             if not prm.requires_grad:
                 continue
             prm.grad = g if prm.grad is None else prm.grad + g

@@ -7,6 +7,7 @@ import re
 import numpy as np
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 from oracle import kge_oracle as ko
 
@@ -294,6 +295,21 @@ def test_one_call_forms_stand_for_unchanged_methods_only():
     assert calls == ["eval"]
     evaluator.eval_mode(plain.train())
     assert not plain.training
+
+
+def test_training_step_refuses_a_weight_that_is_no_parameter(monkeypatch):
+    """A computed weight (a parametrization, weight norm) has no ``.grad`` that an optimizer would read: a KeyError, and no
+    gradient left on a tensor that is thrown away."""
+    from dicee_amd import models
+    m = models.DistMult({"model": "DistMult", "embedding_dim": 32, "num_entities": 50, "num_relations": 5})
+    grads = {f"{t}_embeddings.weight": torch.ones(n, 32) for t, n in (("entity", 50), ("relation", 5))}
+    monkeypatch.setattr(m, "kvsall_bce_gradients", lambda *a: (torch.zeros(()), grads))
+    for times in (1, 2):
+        m.kvsall_training_step(None, None)
+        assert all(torch.equal(p.grad, times * grads[k]) for k, p in m.named_parameters())
+    torch.nn.utils.parametrize.register_parametrization(m.entity_embeddings, "weight", torch.nn.Identity())
+    with pytest.raises(KeyError):
+        m.kvsall_training_step(None, None)
 
 
 def test_synthetic_configs_small_scale():
