@@ -82,11 +82,11 @@ class KGE:
 
     def _best(self, pairs, topk, batch_size, heads=False):
         """(scores, ids) of the ``topk`` best entities per pair, flat, on the host (fused: no [B,N] matrix)."""
-        parts = [self._best_of_batch(pairs[i:i + batch_size], topk, heads) for i in range(0, pairs.size(0), batch_size)]
-        if len(parts) == 1:
-            return parts[0][0].flatten(), parts[0][1].flatten()
-        return (torch.cat([torch.zeros(0)] + [s.flatten() for s, _ in parts]),
-                torch.cat([torch.zeros(0, dtype=torch.long)] + [idx.flatten() for _, idx in parts]))
+        P = pairs.size(0)
+        scores, ids = torch.zeros(P, topk), torch.zeros(P, topk, dtype=torch.long)   # (the caller's own, not views of a copy)
+        for i in range(0, P, batch_size):
+            scores[i:i + batch_size, :], ids[i:i + batch_size, :] = self._best_of_batch(pairs[i:i + batch_size], topk, heads)
+        return scores.flatten(), ids.flatten()
 
     def predict_missing_tail_entity(self, head_entity: Union[List[str], str], relation: Union[List[str], str],
                                     within: List[str] = None, batch_size=2, topk=1, return_indices=False):

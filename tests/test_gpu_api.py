@@ -353,6 +353,24 @@ def test_predict_topk_and_predict_invariants():
         kge.predict_topk(h=3, r=["r0"])
 
 
+def test_answers_by_name_are_tensors_of_their_own(tmp_path):
+    """Scores and ids that can be saved together and share no memory, of one question and of several."""
+    from dicee_amd import KGE
+    m, _ = _toy("Keci", 32, p=0, q=1, seed=5)
+    kge = KGE(model=m.to("cuda"), entity_to_idx={f"e{i}": i for i in range(135)}, relation_to_idx={f"r{i}": i for i in range(46)})
+    for heads in (["e3"], ["e3", "e9", "e30"]):
+        x = torch.tensor([[int(e[1:]), 7] for e in heads], device="cuda")
+        for ask, by_head in ((kge.predict_missing_tail_entity, False), (lambda e, r, **kw: kge.predict_missing_head_entity(r, e, **kw), True)):
+            s, idx = ask(heads, "r7", topk=5, return_indices=True)
+            pairs = x.flip(1) if by_head else x
+            ws, widx = m.topk(pairs.contiguous(), 5, heads=by_head)
+            assert torch.equal(s, ws.cpu().flatten()) and torch.equal(idx, widx.cpu().flatten())
+            assert s.untyped_storage().data_ptr() != idx.untyped_storage().data_ptr()
+            torch.save((s, idx), tmp_path / "answers.pt")
+            again = torch.load(tmp_path / "answers.pt", weights_only=True)
+            assert torch.equal(again[0], s) and torch.equal(again[1], idx)
+
+
 @pytest.mark.parametrize("d", [32, 64, 96, 128, 192, 256, 320])   # LDS rows of 64, 128, 256 (exact and zero-padded); wider
 @pytest.mark.parametrize("storage", ["bf16", "int8"])
 def test_quantised_storage_follows_dequantised_fp32_math(storage, d):

@@ -312,6 +312,29 @@ def test_training_step_refuses_a_weight_that_is_no_parameter(monkeypatch):
         m.kvsall_training_step(None, None)
 
 
+def test_answers_by_name_have_types_and_shapes_of_their_own():
+    """Whatever a model's ``topk`` returns: fp32 scores and int64 ids, one row per pair, also of a single call."""
+    from types import SimpleNamespace
+
+    from dicee_amd import KGE
+    kge = KGE.__new__(KGE)
+    kge.entity_to_idx, kge.relation_to_idx = {"a": 0, "b": 1}, {"r": 0}
+    kge.all_have_inverse, kge.num_entities = False, 2
+
+    def topk(x, k, heads=False):
+        return torch.ones(len(x), width, dtype=torch.bfloat16), torch.ones(len(x), width, dtype=torch.int32)
+    kge.model = SimpleNamespace(entity_embeddings=SimpleNamespace(weight=torch.zeros(2, 4)), topk=topk)
+    for names in (["a"], ["a", "b"] * 3000):                # one call, and two (4096 pairs each)
+        for ask in (kge.predict_missing_tail_entity, lambda e, r, **kw: kge.predict_missing_head_entity(r, e, **kw)):
+            width = 2
+            scores, ids = ask(names, "r", topk=2, return_indices=True)
+            assert scores.dtype == torch.float32 and ids.dtype == torch.int64
+            assert scores.shape == ids.shape == (2 * len(names),)
+            width = 3
+            with pytest.raises(RuntimeError):
+                ask(names, "r", topk=2, return_indices=True)
+
+
 def test_synthetic_configs_small_scale():
     from dicee_amd import synthetic
     c1 = synthetic.make_config("c1")
