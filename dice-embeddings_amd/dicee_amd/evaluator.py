@@ -132,9 +132,11 @@ class _BatchStreams:
 
 
 def eval_mode(model):
-    """``model.eval()``, which walks and writes to every module, where some module is not in that mode yet."""
+    """``model.eval()``, which walks and writes to every module, where some module is not in that mode yet or has a ``train``
+    of its own."""
     from .models import BaseKGE, as_defined
-    if not as_defined(model, BaseKGE, "eval", "train", "modules") or any(m.training for m in model.modules()):
+    if (not as_defined(model, BaseKGE, "eval", "train", "modules")
+            or any(m.training or not as_defined(m, torch.nn.Module, "train") for m in model.modules())):
         model.eval()
 
 

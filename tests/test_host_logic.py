@@ -335,6 +335,27 @@ def test_answers_by_name_have_types_and_shapes_of_their_own():
                 ask(names, "r", topk=2, return_indices=True)
 
 
+def test_eval_reaches_modules_with_a_train_of_their_own():
+    """``model.eval()`` is left out only where it would change nothing: not where some module does more than keep a flag."""
+    from dicee_amd import evaluator, models
+    told = []
+
+    class Layer(torch.nn.Identity):
+        def train(self, mode=True):
+            told.append(mode)
+            return super().train(mode)
+    m = models.DistMult({"model": "DistMult", "embedding_dim": 32, "num_entities": 50, "num_relations": 5})
+    m.eval()
+    m.extra = Layer().eval()
+    told.clear()
+    evaluator.eval_mode(m)
+    assert told == [False]
+    m.extra = torch.nn.Identity().eval()
+    m.extra.train = lambda mode=True: told.append(mode)
+    evaluator.eval_mode(m)
+    assert told == [False, False]
+
+
 def test_synthetic_configs_small_scale():
     from dicee_amd import synthetic
     c1 = synthetic.make_config("c1")
