@@ -455,6 +455,8 @@ def rank_pass(model, ent, rel, pairs, targets, csr=None, *, ent_scale=None, p=0,
         raise ValueError("targets must be an int64 tensor of shape [n]")
     if rel.shape[1] != d:
         raise ValueError("entity and relation tables must have the same embedding dim")
+    if ent_scale is not None and (ent_scale.dtype != torch.float32 or ent_scale.numel() != N):
+        raise ValueError("ent_scale must be float32 [N]")
     if ent.dtype == torch.int8 and ent_scale is None:
         raise ValueError("int8 tables need per-row scales")
     if tie not in _lib.TIES:

@@ -79,3 +79,18 @@ def test_pass_argument_checks():
     with pytest.raises(RuntimeError):
         ops.rank_pass("DistMult", E, R, tri[:, :2].cpu(), tri[:, 2], csr["er"])
     assert ops.rank_pass("DistMult", E, R, tri[:0, :2], tri[:0, 2], csr["er"]).shape == (0,)
+
+
+def test_pass_of_an_int8_table_checks_its_scales():
+    """As the rank call per batch does: scales of another type or number are refused, nothing is launched."""
+    from dicee_amd import ops
+    from dicee_amd.evaluator import rank_in_batches
+    m, tri, csr = _setup("DistMult", 200, 5, 32, "int8", 30, 4)
+    good = m._scale
+    for bad in (good.double(), good[:-1].contiguous(), torch.cat([good, good])):
+        with pytest.raises(ValueError):
+            ops.rank_pass("DistMult", m._table, m._rel(), tri[:, :2], tri[:, 2], csr["er"], ent_scale=bad)
+        m._scale = bad
+        for call_queries in (0, 8192):
+            with pytest.raises(ValueError):
+                rank_in_batches(m, tri[:, :2], tri[:, 2], csr["er"], 10, call_queries=call_queries)
