@@ -64,3 +64,14 @@ def random_csr(rng, hr, targets, N, R, max_len=6, include_target=0.5, hub_rows=(
         key = (int(hr[j, 0]), int(hr[j, 1]))
         er[key].extend(int(v) for v in rng.choice(N, size=length, replace=False))
     return er
+
+
+def count_calls(monkeypatch, module, name):
+    """A list that grows by one with every call of ``module.name``, which goes on as before."""
+    calls, plain = [], getattr(module, name)
+
+    def counted(*args, **kw):
+        calls.append(name)
+        return plain(*args, **kw)
+    monkeypatch.setattr(module, name, counted)
+    return calls

@@ -208,3 +208,23 @@ def test_gradients_of_few_queries(B, N, d, eps, want_dbias):
         if g is not None:
             assert ((g.double().reshape(w.shape) - w).abs() <= b).all()
     assert all(torch.equal(a, b) for a, b in zip(call()[1::2], got[1::2]))      # dQ and dE: the same sums in the same order
+
+
+@pytest.mark.parametrize("B,N,d,want_dbias,scan", [
+    (1, 33, 64, True, True), (64, 14541, 336, False, True), (65, 135, 256, False, False), (32, 200, 340, False, False),
+    (32, 135, 30, False, False), (32, 1024, 64, True, True), (32, 1025, 64, True, False), (32, 40943, 64, False, True)])
+def test_gradients_of_few_queries_are_the_scans_where_its_rule_says_so(B, N, d, want_dbias, scan):
+    """By the names of the kernels launched: batch, row and table at the limits of the rule and past them."""
+    from torch.profiler import ProfilerActivity, profile
+
+    from dicee_amd import ops
+    Q, E = torch.randn(B, d, device="cuda"), torch.randn(N, d, device="cuda")
+    rows, ptr = torch.full((B,), -1, device="cuda"), torch.zeros(2, dtype=torch.int64, device="cuda")
+    col = torch.zeros(1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        ops.bce_multihot_backward(Q, None, E, rows, ptr, col, want_dbias=want_dbias)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages()]
+    assert any("few_scan_kernel" in n for n in names) == scan
+    assert any("GradEpi" in n for n in names) == (not scan)

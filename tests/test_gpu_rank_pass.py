@@ -3,6 +3,8 @@ import numpy as np
 import pytest
 import torch
 
+from helpers import count_calls
+
 pytestmark = pytest.mark.gpu
 
 
@@ -27,15 +29,20 @@ def _setup(name, N, R, d, storage, n, seed, norm=None, **args):
     ("QMult", 1000, 128, "bf16", 8192, None), ("QMult", 1000, 128, "bf16", 17001, None), ("ComplEx", 1000, 240, "int8", 8191, None),
     ("DistMult", 300, 320, "bf16", 9000, "BatchNorm1d"), ("DeCaL", 130, 24, "fp32", 1, None), ("OMult", 257, 64, "int8", 8200, None)])
 @pytest.mark.parametrize("heads", [False, True])
-def test_pass_equals_one_call_per_batch(name, N, d, storage, n, norm, heads):
+def test_pass_equals_one_call_per_batch(name, N, d, storage, n, norm, heads, monkeypatch):
+    from dicee_amd import ops
     from dicee_amd.evaluator import rank_in_batches
+    calls = count_calls(monkeypatch, ops, "rank_pass")
     m, tri, csr = _setup(name, N, 7, d, storage, n, n + d, norm, p=1, q=1, r=1)
     if heads and norm:
         m.normalize_head_entity_embeddings = m.normalize_relation_embeddings = type(m.hidden_normalizer)()
     x, t, c = (tri[:, 1:], tri[:, 0], csr["re"]) if heads else (tri[:, :2], tri[:, 2], csr["er"])
     for tie in ("stable", "optimistic", "pessimistic", "mean"):
         want = rank_in_batches(m, x, t, c, 1000, tie, heads=heads, call_queries=0)
+        assert not calls
         got = rank_in_batches(m, x, t, c, 1000, tie, heads=heads)
+        assert calls == ["rank_pass"]
+        calls.clear()
         assert got.dtype == want.dtype and torch.equal(got, want)
     assert torch.equal(rank_in_batches(m, x, t, None, 1000, heads=heads), rank_in_batches(m, x, t, None, 1000, heads=heads, call_queries=0))
     out = torch.empty(2, n, dtype=torch.int64, device="cuda")
@@ -53,7 +60,8 @@ def test_pass_of_ids_outside_the_tables():
     assert torch.equal(rank_in_batches(*args), rank_in_batches(*args, call_queries=0))
 
 
-def test_pass_of_a_model_with_a_query_of_its_own():
+def test_pass_of_a_model_with_a_query_of_its_own(monkeypatch):
+    from dicee_amd import ops
     from dicee_amd.evaluator import rank_in_batches
     m, tri, csr = _setup("DistMult", 200, 5, 32, "fp32", 300, 2)
     plain = rank_in_batches(m, tri[:, :2], tri[:, 2], csr["er"], 100)
@@ -63,8 +71,10 @@ def test_pass_of_a_model_with_a_query_of_its_own():
             Q, b = super().query(x, heads=heads, **kw)
             return -Q, b
     m.__class__ = Negated
+    calls = count_calls(monkeypatch, ops, "rank_pass")
     got = rank_in_batches(m, tri[:, :2], tri[:, 2], csr["er"], 100)
     assert torch.equal(got, rank_in_batches(m, tri[:, :2], tri[:, 2], csr["er"], 100, call_queries=0)) and not torch.equal(got, plain)
+    assert not calls
 
 
 def test_pass_argument_checks():

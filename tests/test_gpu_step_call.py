@@ -3,6 +3,8 @@ import numpy as np
 import pytest
 import torch
 
+from helpers import count_calls
+
 pytestmark = pytest.mark.gpu
 
 
@@ -12,9 +14,10 @@ pytestmark = pytest.mark.gpu
     ("CKeci", 135, 4, 60, 17, None, dict(p=1, q=1)), ("DeCaL", 130, 3, 28, 40, "LayerNorm", dict(p=2, q=2, r=2)),
     ("OMult", 257, 4, 64, 300, None, {})])
 @pytest.mark.parametrize("eps", [0.0, 0.1])
-def test_step_equals_the_calls_it_is_made_of(name, N, R, d, B, norm, kw, eps):
+def test_step_equals_the_calls_it_is_made_of(name, N, R, d, B, norm, kw, eps, monkeypatch):
     """The same kernels on the same operands: all but the sums that meet in atomics are equal, those to a few roundings."""
-    from dicee_amd import FilterCSR, MODEL_REGISTRY
+    from dicee_amd import FilterCSR, MODEL_REGISTRY, ops
+    calls = count_calls(monkeypatch, ops, "kvsall_step")
     torch.manual_seed(N + d)
     m = MODEL_REGISTRY[name](dict(model=name, embedding_dim=d, num_entities=N, num_relations=R, normalization=norm, **kw)).cuda()
     m.train(norm != "BatchNorm1d")                          # (batch statistics take another route)
@@ -27,12 +30,14 @@ def test_step_equals_the_calls_it_is_made_of(name, N, R, d, B, norm, kw, eps):
     x = tri[:B, :2].contiguous()
     x[0, 0] = (x[0, 0] + 1) % N                             # (a pair that may have no row)
     loss, grads = m.kvsall_bce_gradients(x, csr, eps)
+    assert calls == ["kvsall_step"]
 
     class Apart(type(m)):
         def query(self, x, heads=False, **k):
             return super().query(x, heads=heads, **k)
     m.__class__ = Apart
     wloss, want = m.kvsall_bce_gradients(x, csr, eps)
+    assert calls == ["kvsall_step"]                         # (not asked again)
     assert loss.shape == wloss.shape and abs(float(loss) - float(wloss)) <= 1e-6 * abs(float(wloss))
     assert grads.keys() == want.keys()
     for k in want:
