@@ -135,8 +135,9 @@ def eval_mode(model):
     """``model.eval()``, which walks and writes to every module, where some module is not in that mode yet or has a ``train``
     of its own."""
     from .models import BaseKGE, as_defined
+    plain = torch.nn.Module.train       # (asked without as_defined: 12 us of an evaluation's host, not 29)
     if (not as_defined(model, BaseKGE, "eval", "train", "modules")
-            or any(m.training or not as_defined(m, torch.nn.Module, "train") for m in model.modules())):
+            or any(m.training or type(m).train is not plain or "train" in vars(m) for m in model.modules())):
         model.eval()
 
 
