@@ -122,8 +122,8 @@ def main():
     ap.add_argument("--scale", type=float, default=1.0, help="shrink the workload (testing only)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--streams", type=int, default=1,
-                    help="consecutive steps on this many alternating streams, as dicee_amd.Evaluator runs the batches "
-                         "of an evaluation (2 there); a step short enough to be a chain of dependent launches gains "
+                    help="consecutive steps on this many alternating streams, as dicee_amd.Evaluator runs batches that it ranks "
+                         "one by one (2 there); a step short enough to be a chain of dependent launches gains "
                          "(c2: 0.117 -> 0.075 ms), and the main-loop kernel's own duration then includes what it "
                          "shares the GPU with")
     ap.add_argument("--graph", action="store_true",
@@ -135,8 +135,9 @@ def main():
     ap.add_argument("--no-ceiling", action="store_true",
                     help="skip the `ceiling` side figures (vendor bf16 GEMM on random and on zero operands)")
     ap.add_argument("--no-evaluation-pass", action="store_true",
-                    help="skip the `evaluation_pass` side figure (a profile of the step's own launches: the pass runs "
-                         "its batches on two streams, where a traced kernel's duration includes its wait for the other's CUs)")
+                    help="skip the `evaluation_pass` side figure (a profile of the step's own launches: the passes "
+                         "run the same kernels, the one by batches on two streams, where a traced kernel's duration includes "
+                         "its wait for the other's CUs)")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="also run one plain 1 GiB-in / 1 GiB-out elementwise kernel (reference point for "
                          "FETCH_SIZE / WRITE_SIZE counters under rocprofv3 --pmc)")
@@ -317,17 +318,16 @@ def main():
                             "roofline_achieved": a_sus, "roofline_frac": a_sus / PEAK_TFLOPS[compute] if a_sus else None,
                             "kernel_ms_avg": k_ms / max(k_n, 1), "launches": k_n}
     # side figure, outside the timed region: one whole evaluation pass over every query of the configuration as
-    # dicee_amd.Evaluator runs it (vectors, filter rows and thresholds of a group of batches from one launch each,
-    # batches alternating over two streams, the ranks formed at the end), wall clock of the best of four passes; and
-    # the same pass with every batch on the caller's stream
+    # dicee_amd.Evaluator runs it (one native call on the caller's stream, ids in, ranks out), wall clock of the best of
+    # four passes; and the same pass with one call per batch, alternating over two streams and on the caller's alone
     if mode in ("rank", "headrank") and not args.graph and not args.no_evaluation_pass:
         from dicee_amd.evaluator import rank_in_batches
         xq = (q_all[:, 1:] if mode == "headrank" else q_all[:, :2]).contiguous()
         tq = (q_all[:, 0] if mode == "headrank" else q_all[:, 2]).contiguous()
         f_csr = re_csr if mode == "headrank" else cfg.csr
         best = {}
-        # (streams, call_queries): the evaluator's default merges whole batches into calls of at least 8192 queries
-        # (a query's counters do not depend on what else is in its call); 0 keeps one call per batch
+        # (streams, call_queries): the evaluator's default, which is one call and has no use for either; call_queries 0
+        # keeps one call per batch (a query's counters do not depend on what else is in its call)
         for key in ((2, 8192), (2, 0), (1, 0)):
             for _ in range(4):
                 torch.cuda.synchronize()
@@ -339,11 +339,11 @@ def main():
                 best[key] = tp if key not in best else min(best[key], tp)
         n_batches = (int(xq.shape[0]) + cfg.B - 1) // cfg.B
         t_def, t_pb, t_pb1 = best[(2, 8192)], best[(2, 0)], best[(1, 0)]
-        out["evaluation_pass"] = {"queries": int(xq.shape[0]), "batch": cfg.B, "streams": 2, "call_queries": 8192,
+        out["evaluation_pass"] = {"queries": int(xq.shape[0]), "batch": cfg.B, "form": "kge_rank_pass",
                                   "ms": t_def * 1e3, "queries_per_sec": xq.shape[0] / t_def,
                                   "value": float(xq.shape[0]) * N / t_def, "unit": "scores/s",
                                   "mrr": float((1.0 / ranks_all.double()).mean().item()),
-                                  "one_call_per_batch": {"batches": n_batches, "ms": t_pb * 1e3,
+                                  "one_call_per_batch": {"batches": n_batches, "streams": 2, "ms": t_pb * 1e3,
                                                          "ms_per_batch": t_pb * 1e3 / n_batches,
                                                          "one_stream_ms": t_pb1 * 1e3,
                                                          "one_stream_ms_per_batch": t_pb1 * 1e3 / n_batches}}

@@ -5,8 +5,8 @@ Mirrors dicee's ``Evaluator`` for index-encoded (non byte-pair) models
 ``eval_with_vs_all``, :394-438 ``evaluate_lp_k_vs_all``, :440-471 the relation-prediction loop, :473-510 the
 entity-prediction loop, :622-643 ``evaluate_lp``) and its metric reduction
 (dicee/evaluation/utils.py:73-132).  Where the reference scores a batch, masks it row by row in
-Python and sorts every row, this evaluator makes one fused kernel call per batch and receives three
-counters per query.
+Python and sorts every row, this evaluator makes one native call per pass and receives a rank per query
+(models that build their queries otherwise: one fused rank call per run of batches, three counters per query).
 
 Tie rule.  The reference's rank of a tied target is whatever position an unstable ``torch.sort``
 gives it; every such position lies in ``[1 + n_greater, 1 + n_greater + n_equal]``.  ``tie`` picks
@@ -161,9 +161,9 @@ def rank_in_batches(model, x_all, target_all, csr, batch_size, tie="stable", str
     """Ranks (int64 tensor [n] on the model's device; ``out``: where to write them) of ``target_all`` [n] for the queries
     ``x_all`` [n,2].  The reference's batch size bounds the B x N score matrix it materialises (evaluator.py:484-508); the
     fused call forms no such matrix and a query's counters do not depend on what else is in its call, so that the pass is
-    one call (``ops.rank_pass``; one per 256 MB of query vectors): seven launches, one behind the other.  (Alternating whole
-    batches over two streams around calls per batch: 20,000 queries of a 14.5k graph 994 us on two streams and 1060 on one
-    against about 1000; 2 x 5000 queries of an int8 table 1005 and 925.)
+    one call (``ops.rank_pass``; one per 256 MB of query vectors): six launches and the main loop, which is one launch of an fp32
+    table and one per 8192 queries of a bf16 or int8 one, all on the caller's stream (``streams`` has no effect).  20,000
+    queries of a 14.5k graph: 1.13 ms, by one call per batch of 1024 1.62 - 1.97 on two streams and 1.86 on one.
 
     ``call_queries=0``, and models that build their queries otherwise: one fused rank call per batch of ``batch_size``
     queries (or, with ``call_queries``, per run of whole batches that together hold at least that many).  What does not
@@ -432,8 +432,8 @@ class Evaluator:
         return out.cpu().numpy()
 
     def _evaluate_entity_prediction(self, model, triple_idx, num_triples):
-        """Ranks (numpy int64 [n]) of the true tails; one fused kernel call per batch of
-        ``args.batch_size`` triples (the batching of evaluator.py:484-486)."""
+        """Ranks (numpy int64 [n]) of the true tails, by ``rank_in_batches`` (``args.batch_size``: the batching of
+        evaluator.py:484-486, which bounds nothing here but the calls of models that are asked batch by batch)."""
         triple_idx = np.asarray(triple_idx)
         if triple_idx.ndim != 2 or triple_idx.shape[1] != 3:
             raise ValueError("triple_idx must have shape [n, 3]")
